@@ -50,6 +50,8 @@ SIGNATURES = {
     "ave_fp4_quantize_nvfp4_bf16": [_vp, _vp, _vp, _vp, _int, _int, _vp],
     "ave_fp4_moe_route_top2": [_vp, _int, _int, _vp, _vp, _vp, _vp],
     "ave_fp4_moe_route_top2_ex": [_vp, _int, _int, _vp, _vp, _vp, _vp, _vp],
+    "ave_fp4_moe_route_top2_workspace_bytes": [_int, _int],
+    "ave_fp4_moe_route_top2_ws": [_vp, _int, _int, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp],
     "ave_fp4_moe_combine_top2": [_vp, _vp, _vp, _int, _int, _int, _vp, _vp],
     "ave_fp4_gather_rows_mxfp4": [_vp, _vp, _vp, _int, _int, _int, _vp, _vp, _vp],
     "ave_fp4_scales_to_blocked": [_vp, _int, _int, _vp, _vp],
@@ -73,7 +75,8 @@ SIGNATURES = {
 ABI_VERSION = 1   # what ave_fp4_abi_version() of a matching library returns
 
 _RESTYPES = {"ave_fp4_last_error": ctypes.c_char_p, "ave_fp4_gemm_mxfp4_workspace_bytes": ctypes.c_size_t,
-             "ave_fp4_gemm_nvfp4_workspace_bytes": ctypes.c_size_t}
+             "ave_fp4_gemm_nvfp4_workspace_bytes": ctypes.c_size_t,
+             "ave_fp4_moe_route_top2_workspace_bytes": ctypes.c_size_t}
 
 
 def library_path() -> str:

@@ -569,7 +569,7 @@ int ave_fp4_scales_from_blocked(const uint8_t* blocked, int rows, int cols, uint
 
 namespace {
 int route_common(const float* logits, int tokens, int E, int32_t* token_of_row, int32_t* row_offsets, float* row_weight,
-                 int32_t* rows_of_token, void* hip_stream) {
+                 int32_t* rows_of_token, void* workspace, size_t workspace_bytes, void* hip_stream) {
   g_err[0] = 0;
   if (tokens < 0) return fail_inval("tokens must be non-negative, got %d.", tokens);
   if (E < 2 || E > ave::route_top2_max_experts())
@@ -580,7 +580,10 @@ int route_common(const float* logits, int tokens, int E, int32_t* token_of_row, 
   if (!aligned(logits, 4) || !aligned(token_of_row, 4) || !aligned(row_offsets, 4) || !aligned(row_weight, 4) ||
       !aligned(rows_of_token, 4))
     return fail_inval("logits, token_of_row, row_offsets, row_weight and rows_of_token must be 4-byte aligned.");
-  return finish(ave::launch_route_top2(logits, tokens, E, token_of_row, row_offsets, row_weight, rows_of_token,
+  if (workspace_bytes > 0 && !workspace) return fail_inval("null workspace with workspace_bytes = %zu.", workspace_bytes);
+  if (workspace && !aligned(workspace, 16)) return fail_inval("workspace must be 16-byte aligned.");
+  if (workspace_bytes < ave::route_top2_workspace_bytes(tokens, E)) workspace = nullptr;
+  return finish(ave::launch_route_top2(logits, tokens, E, token_of_row, row_offsets, row_weight, rows_of_token, workspace,
                                        static_cast<hipStream_t>(hip_stream)),
                 "top-2 routing kernel");
 }
@@ -588,12 +591,24 @@ int route_common(const float* logits, int tokens, int E, int32_t* token_of_row, 
 
 int ave_fp4_moe_route_top2(const float* logits, int tokens, int E, int32_t* token_of_row, int32_t* row_offsets,
                            float* row_weight, void* hip_stream) {
-  return route_common(logits, tokens, E, token_of_row, row_offsets, row_weight, nullptr, hip_stream);
+  return route_common(logits, tokens, E, token_of_row, row_offsets, row_weight, nullptr, nullptr, 0, hip_stream);
 }
 
 int ave_fp4_moe_route_top2_ex(const float* logits, int tokens, int E, int32_t* token_of_row, int32_t* row_offsets,
                               float* row_weight, int32_t* rows_of_token, void* hip_stream) {
-  return route_common(logits, tokens, E, token_of_row, row_offsets, row_weight, rows_of_token, hip_stream);
+  return route_common(logits, tokens, E, token_of_row, row_offsets, row_weight, rows_of_token, nullptr, 0, hip_stream);
+}
+
+size_t ave_fp4_moe_route_top2_workspace_bytes(int tokens, int E) {
+  if (tokens < 0 || tokens > (1 << 29) || E < 2 || E > ave::route_top2_max_experts()) return 0;
+  return ave::route_top2_workspace_bytes(tokens, E);
+}
+
+int ave_fp4_moe_route_top2_ws(const float* logits, int tokens, int E, int32_t* token_of_row, int32_t* row_offsets,
+                              float* row_weight, int32_t* rows_of_token, void* workspace, size_t workspace_bytes,
+                              void* hip_stream) {
+  return route_common(logits, tokens, E, token_of_row, row_offsets, row_weight, rows_of_token, workspace, workspace_bytes,
+                      hip_stream);
 }
 
 int ave_fp4_moe_combine_top2(const uint16_t* rows, const int32_t* rows_of_token, const float* row_weight, int tokens,

@@ -127,10 +127,11 @@ hipError_t launch_quantize_mx(const void* x, int is_bf16, uint8_t* packed, uint8
 hipError_t launch_quantize_nv(const void* x, int is_bf16, const float* global_scale, uint8_t* packed, uint8_t* scales,
                               size_t n_blocks, hipStream_t s);
 
-// MoE routing (one workgroup) and row gather; see moe_route.hip
+// MoE routing and row gather; see moe_route.hip.  workspace: route_top2_workspace_bytes of them, 16-byte aligned, or null
 int route_top2_max_experts();
+size_t route_top2_workspace_bytes(int T, int E);
 hipError_t launch_route_top2(const float* logits, int T, int E, int32_t* token_of_row, int32_t* row_offsets,
-                             float* row_weight, int32_t* rows_of_token, hipStream_t s);
+                             float* row_weight, int32_t* rows_of_token, void* workspace, hipStream_t s);
 hipError_t launch_combine_top2(const uint16_t* rows, const int32_t* rows_of_token, const float* row_weight, int T, int H,
                                int n_rows, int renormalize, uint16_t* out, hipStream_t s);
 hipError_t launch_gather_rows(const uint8_t* src, const uint8_t* src_s, const int32_t* index, int rows, int src_rows,

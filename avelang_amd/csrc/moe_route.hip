@@ -9,12 +9,12 @@
 //   combine_top2_kernel the step behind the expert GEMMs: every token's two expert outputs, weighted with their
 //                       routing probabilities, summed back into token order.
 //
-// Both are integer/byte work.  Routing is a counting sort without any exchange between workgroups:
-// workgroup (e, part) scans ALL tokens once (token = iteration*1024 + thread, so loads are coalesced)
-// to count the routed rows of experts below e and the rows of e in front of its own token range --
-// that is the position of its first row -- and then places the rows of expert e for its range,
-// iteration by iteration, with a ballot per wave and a 16-entry prefix over the waves.  Tokens rise
-// with (iteration, wave, lane), so the order inside an expert is by token: the stable order.
+// Routing is a counting sort over chunks of tokens.  The tokens' choices are found once, by subgroups of lanes that read
+// a row of logits coalesced; a chunk's rows start where the experts below and the chunks before it end, and inside a chunk
+// 256 tokens at a time are ranked with ballots over the bits of the expert numbers.  Tokens rise with (chunk, block of
+// 256, wave, lane), so the order inside an expert is by token: the stable order.  A few tokens are one launch of one
+// workgroup; more tokens are two launches that pass the choices and the chunks' counts through a workspace, or, without
+// one, a single launch in which every workgroup counts all tokens.
 #include "fp4_common.hpp"
 #include "kernels.hpp"
 
@@ -22,141 +22,259 @@ namespace ave {
 namespace {
 
 constexpr int kRouteThreads = 1024;
+constexpr int kRouteBlock = 256;       // tokens that are ranked together
+constexpr int kRouteMaxE = 256;
+constexpr int kRouteMaxChunks = 256;
+constexpr int kRouteValues = 8;        // logits of one token that a lane holds
 
-struct Top2 {
-  int e0, e1;
-  float p0, p1;
+// Bound by latency: a few dependent trips to memory per kernel.  Every token's logits are read once (a version whose
+// workgroups -- one per expert -- each went through all tokens took 368 us for 2443 tokens and 141 experts and 27 us for
+// 16384 tokens and 8 experts; the two launches below 12 us and 9.7 us).  A chunk is what one workgroup takes: the tokens whose choices it
+// finds in one go (1024 lanes, E / 8 of them per token, at most 256 tokens), and never more than 256 chunks, so that a
+// workgroup's sum over the chunks before it stays a few loads per thread.  Up to two goes stay with one workgroup: the
+// second costs about what the second launch would.
+struct RouteShape {
+  int lanes_log2;                // lanes per token: the power of two from E / 8 up
+  int chunk_tokens, chunks;
 };
-
-// Highest and second-highest logit; among equal values the lower expert index ranks first.
-// Probabilities are those of the full softmax over the E logits.  The row is read eight values at a
-// time with all eight loads in flight together (two 16-byte loads when `vec`: E % 4 == 0 and an
-// aligned base), because a one-value-per-trip loop pays the memory latency E times per token.
-__device__ inline Top2 top2_of(const float* l, int E, bool vec, bool want_prob) {
-  float v0 = -__builtin_inff(), v1 = -__builtin_inff();
-  // the softmax denominator is added up in double: a float sum of E terms drifts by about sqrt(E) roundings, which for
-  // 200 and more experts is more than the 2e-6 relative error the probabilities are stated to keep
-  double sum = 0.0;
-  int e0 = -1, e1 = -1;
-  for (int c = 0; c < E; c += 8) {
-    float x[8];
-    if (vec) {
-      const v4f lo = *reinterpret_cast<const v4f*>(l + c);
-      const v4f hi = c + 4 < E ? *reinterpret_cast<const v4f*>(l + c + 4) : v4f{0, 0, 0, 0};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x[j] = lo[j];
-        x[4 + j] = hi[j];
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = c + j < E ? l[c + j] : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (c + j < E) {
-        const float v = x[j];
-        if (e0 < 0 || v > v0) {
-          if (want_prob) sum = e0 < 0 ? 1.0 : sum * (double)expf(v0 - v) + 1.0;   // running sum of exp(l - max)
-          v1 = v0;
-          e1 = e0;
-          v0 = v;
-          e0 = c + j;
-        } else {
-          if (want_prob) sum += (double)expf(v - v0);
-          if (e1 < 0 || v > v1) {
-            v1 = v;
-            e1 = c + j;
-          }
-        }
-      }
-    }
-  }
-  Top2 r{e0, e1, 0.f, 0.f};
-  if (want_prob) {
-    r.p0 = (float)(1.0 / sum);
-    r.p1 = (float)((double)expf(v1 - v0) / sum);
-  }
+inline RouteShape route_shape(int T, int E) {
+  RouteShape r{0, 0, 1};
+  while ((kRouteValues << r.lanes_log2) < E) ++r.lanes_log2;
+  const int go = (kRouteThreads >> r.lanes_log2) < kRouteBlock ? kRouteThreads >> r.lanes_log2 : kRouteBlock;
+  const int least = (T + kRouteMaxChunks - 1) / kRouteMaxChunks;
+  r.chunk_tokens = go > least ? go : least;
+  if (T <= 2 * go && T <= kRouteBlock) r.chunk_tokens = kRouteBlock;
+  r.chunks = T > 0 ? (T + r.chunk_tokens - 1) / r.chunk_tokens : 1;
   return r;
 }
 
-// sum over the workgroup; `buf` holds one int per wave; every thread returns the total
-__device__ inline int block_sum(int v, int* buf, int lane, int w) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-  __syncthreads();   // earlier readers of buf are done
-  if (lane == 0) buf[w] = v;
-  __syncthreads();
-  int total = 0;
-  for (int ww = 0; ww < kRouteThreads / 64; ++ww) total += buf[ww];
-  return total;
+struct RouteArgs {
+  const float* logits;
+  int T, E;
+  int lanes_log2;
+  int chunk_tokens, chunks;
+  int32_t* token_of_row;
+  int32_t* row_offsets;
+  float* row_weight;             // may be null
+  int32_t* rows_of_token;        // may be null: [T, 2], the routed row of every token's first and second choice
+  int* counts;                   // workspace: [chunks][E] routed rows, ...
+  unsigned* pairs;               // ... [T] first choice | second choice << 16,
+  v2f* probs;                    // ... [T] their probabilities
+};
+
+struct Choice {
+  float v;
+  int e;   // -1: none
+};
+__device__ inline bool ranks_before(const Choice& a, const Choice& b) {   // among equal scores the lower expert index
+  return a.e >= 0 && (b.e < 0 || a.v > b.v || (a.v == b.v && a.e < b.e));
 }
 
-// rows_of_token (optional, [T, 2]): the routed row of every token's first and second choice -- the inverse of
-// token_of_row, which the combine step reads.
-__global__ __launch_bounds__(kRouteThreads) void route_top2_kernel(const float* logits, int T, int E, int P,
-                                                                    int32_t* token_of_row, int32_t* row_offsets,
-                                                                    float* row_weight, int32_t* rows_of_token) {
-  __shared__ int wave_buf[2][kRouteThreads / 64];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int e = blockIdx.x / P, part = blockIdx.x % P;
-  const bool vec = (E & 3) == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0;
-  const int iters = (T + kRouteThreads - 1) / kRouteThreads;
-  const int per_part = (iters + P - 1) / P;
-  const int it0 = part * per_part < iters ? part * per_part : iters;
-  const int it1 = it0 + per_part < iters ? it0 + per_part : iters;
+// The choices of `n` tokens (at most 256) from token `t0` on, into pair[] and, when wanted, prob[] (both LDS):
+// highest and second-highest logit and their probabilities in the full softmax.  The softmax denominator is added up in
+// double: a float sum of E terms drifts by about sqrt(E) roundings, which for 200 and more experts is more than the
+// 2e-6 relative error the probabilities are stated to keep.  Its terms come from v_exp_f32: x exp(-x) 2^-24, what the
+// rounded product costs, is below 3e-8 for every x; the second choice's own probability takes expf.
+__device__ inline void choose_block(const RouteArgs& p, int t0, int n, bool want_prob, unsigned* pair, v2f* prob) {
+  const int L = 1 << p.lanes_log2, sub = threadIdx.x & (L - 1);
+  for (int i = threadIdx.x >> p.lanes_log2; i < n; i += kRouteThreads >> p.lanes_log2) {
+    const float* l = p.logits + (size_t)(t0 + i) * p.E;
+    float x[kRouteValues];
+#pragma unroll
+    for (int j = 0; j < kRouteValues; ++j) {
+      const int e = j * L + sub;
+      x[j] = e < p.E ? l[e] : 0.f;
+    }
+    Choice first{0.f, -1}, second{0.f, -1};
+#pragma unroll
+    for (int j = 0; j < kRouteValues; ++j) {   // selects, no branches
+      const int e = j * L + sub;
+      const Choice c{x[j], e < p.E ? e : -1};
+      const bool better = ranks_before(c, first), next = ranks_before(c, second);
+      second.v = better ? first.v : (next ? c.v : second.v);
+      second.e = better ? first.e : (next ? c.e : second.e);
+      first.v = better ? c.v : first.v;
+      first.e = better ? c.e : first.e;
+    }
+    for (int d = 1; d < L; d <<= 1) {
+      const Choice f{__shfl_xor(first.v, d, 64), __shfl_xor(first.e, d, 64)};
+      const Choice s{__shfl_xor(second.v, d, 64), __shfl_xor(second.e, d, 64)};
+      const bool better = ranks_before(f, first);
+      // the second of both is the loser of the two firsts or the winner's own second
+      const Choice lost = better ? first : f, own = better ? s : second;
+      first = better ? f : first;
+      second = ranks_before(lost, own) ? lost : own;
+    }
+    if (want_prob) {
+      const float top = __shfl(first.v, threadIdx.x & 63 & ~(L - 1), 64);
+      double sum = 0.0;
+#pragma unroll
+      for (int j = 0; j < kRouteValues; ++j)
+        sum += j * L + sub < p.E ? (double)__builtin_amdgcn_exp2f(1.4426950408889634f * (x[j] - top)) : 0.0;
+      for (int d = 1; d < L; d <<= 1) sum += __shfl_xor(sum, d, 64);
+      if (sub == 0) prob[i] = v2f{(float)(1.0 / sum), (float)((double)expf(second.v - first.v) / sum)};
+    }
+    if (sub == 0) pair[i] = (unsigned)first.e | (unsigned)second.e << 16;
+  }
+}
 
-  // ---- pass 1: where do this workgroup's rows start? ----------------------------------------
-  int below = 0, mine_before = 0, mine_all = 0;
-  for (int it = 0; it < iters; ++it) {
-    const int t = it * kRouteThreads + tid;
-    if (t < T) {
-      const Top2 r = top2_of(logits + (size_t)t * E, E, vec, false);
-      below += (r.e0 < e) + (r.e1 < e);
-      const int hit = (r.e0 == e) | (r.e1 == e);
-      mine_all += hit;
-      if (it < it0) mine_before += hit;
+// First of the two launches: a chunk's choices and its routed rows per expert, into the workspace.
+__global__ __launch_bounds__(kRouteThreads) void route_choose_kernel(RouteArgs p) {
+  __shared__ unsigned pair[kRouteBlock];
+  __shared__ v2f prob[kRouteBlock];
+  __shared__ int count[kRouteMaxE];
+  const int tid = threadIdx.x;
+  const int t_begin = blockIdx.x * p.chunk_tokens;
+  const int t_end = t_begin + p.chunk_tokens < p.T ? t_begin + p.chunk_tokens : p.T;
+  if (tid < kRouteMaxE) count[tid] = 0;
+  for (int t0 = t_begin; t0 < t_end; t0 += kRouteBlock) {
+    const int n = t_end - t0 < kRouteBlock ? t_end - t0 : kRouteBlock;
+    choose_block(p, t0, n, p.row_weight != nullptr, pair, prob);
+    __syncthreads();
+    if (tid < n) {
+      const unsigned c = pair[tid];
+      p.pairs[t0 + tid] = c;
+      if (p.row_weight) p.probs[t0 + tid] = prob[tid];
+      atomicAdd(&count[c & 0xFFFF], 1);
+      atomicAdd(&count[c >> 16], 1);
+    }
+    __syncthreads();
+  }
+  if (tid < p.E) p.counts[(size_t)blockIdx.x * p.E + tid] = count[tid];
+}
+
+// Places the rows of one chunk per workgroup.  CHOSEN: choices and counts come from the workspace; otherwise the
+// workgroup makes them itself, for all tokens (there is one chunk, or the caller gave no workspace).
+template <bool CHOSEN>
+__global__ __launch_bounds__(kRouteThreads) void route_place_kernel(RouteArgs p) {
+  __shared__ unsigned pair[kRouteBlock];
+  __shared__ v2f prob[kRouteBlock];
+  __shared__ int before[kRouteMaxE], total[kRouteMaxE];   // rows of an expert in the chunks before this one; in all
+  __shared__ int next[kRouteMaxE];                        // where an expert's next row goes
+  __shared__ int of_wave[kRouteBlock / 64][kRouteMaxE];
+  __shared__ int wave_total[kRouteMaxE / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int t_begin = blockIdx.x * p.chunk_tokens;
+  const int t_end = t_begin + p.chunk_tokens < p.T ? t_begin + p.chunk_tokens : p.T;
+
+  if (tid < kRouteMaxE) before[tid] = total[tid] = 0;
+  __syncthreads();
+  if constexpr (CHOSEN) {
+    // thread = (group of chunks, expert): a table row of counts is read coalesced
+    int width = 1;
+    while (width < p.E) width <<= 1;
+    const int e = tid & (width - 1);
+    if (e < p.E) {
+      int sum_before = 0, sum = 0;
+#pragma unroll 8
+      for (int c = tid / width; c < p.chunks; c += kRouteThreads / width) {
+        const int v = p.counts[(size_t)c * p.E + e];
+        sum += v;
+        sum_before += c < (int)blockIdx.x ? v : 0;
+      }
+      if (sum) atomicAdd(&total[e], sum);
+      if (sum_before) atomicAdd(&before[e], sum_before);
+    }
+    __syncthreads();
+  } else {
+    for (int t0 = 0; t0 < p.T; t0 += kRouteBlock) {
+      const int n = p.T - t0 < kRouteBlock ? p.T - t0 : kRouteBlock;
+      choose_block(p, t0, n, p.row_weight != nullptr && p.chunks == 1, pair, prob);
+      __syncthreads();
+      if (tid < n) {
+        const unsigned c = pair[tid];
+        atomicAdd(&total[c & 0xFFFF], 1);
+        atomicAdd(&total[c >> 16], 1);
+        if (t0 + tid < t_begin) {
+          atomicAdd(&before[c & 0xFFFF], 1);
+          atomicAdd(&before[c >> 16], 1);
+        }
+      }
+      __syncthreads();
     }
   }
-  below = block_sum(below, wave_buf[0], lane, w);
-  mine_before = block_sum(mine_before, wave_buf[0], lane, w);
-  mine_all = block_sum(mine_all, wave_buf[0], lane, w);
-  if (part == 0 && tid == 0) {
-    row_offsets[e + 1] = below + mine_all;
-    if (e == 0) row_offsets[0] = 0;
+
+  // exclusive sum of the totals over the experts
+  if (tid < kRouteMaxE) {
+    const int mine = total[tid];
+    int run = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(run, d, 64);
+      run += lane >= d ? o : 0;
+    }
+    if (lane == 63) wave_total[w] = run;
+    next[tid] = run - mine;
   }
   __syncthreads();
+  if (tid < kRouteMaxE) {
+    int start = next[tid];
+    for (int ww = 0; ww < w; ++ww) start += wave_total[ww];
+    if (blockIdx.x == 0 && tid < p.E) {
+      p.row_offsets[tid + 1] = start + total[tid];
+      if (tid == 0) p.row_offsets[0] = 0;
+    }
+    next[tid] = start + before[tid];
+  }
 
-  // ---- pass 2: place the rows of expert e for tokens of iterations [it0, it1) -----------------
-  int run = below + mine_before;
-  for (int it = it0; it < it1; ++it) {
-    const int t = it * kRouteThreads + tid;
-    bool hit = false;
-    float prob = 0.f;
-    int rank = 0;
-    if (t < T) {
-      const Top2 r = top2_of(logits + (size_t)t * E, E, vec, row_weight != nullptr);
-      hit = r.e0 == e || r.e1 == e;
-      prob = r.e0 == e ? r.p0 : r.p1;
-      rank = r.e0 == e ? 0 : 1;
+  for (int t0 = t_begin; t0 < t_end; t0 += kRouteBlock) {
+    const int n = t_end - t0 < kRouteBlock ? t_end - t0 : kRouteBlock;
+    if constexpr (!CHOSEN) {
+      if (p.chunks > 1 || p.T > kRouteBlock) {   // (else pair[] and prob[] still hold this block)
+        __syncthreads();
+        choose_block(p, t0, n, p.row_weight != nullptr, pair, prob);
+      }
     }
-    const unsigned long long mask = __ballot(hit);
-    int* buf = wave_buf[it & 1];   // alternating buffers: one barrier per iteration is enough
-    if (lane == 0) buf[w] = __popcll(mask);
+    for (int i = tid; i < kRouteBlock / 64 * kRouteMaxE; i += kRouteThreads) of_wave[i / kRouteMaxE][i % kRouteMaxE] = 0;
     __syncthreads();
-    int before = 0, total = 0;
-    for (int ww = 0; ww < kRouteThreads / 64; ++ww) {
-      const int c = buf[ww];
-      before += ww < w ? c : 0;
-      total += c;
+    int expert[2] = {0, 0}, rank[2] = {0, 0};
+    v2f weight = {0.f, 0.f};
+    const bool on = tid < n;
+    if (tid < kRouteBlock) {   // whole waves
+      unsigned c = 0;
+      if (on) {
+        c = CHOSEN ? p.pairs[t0 + tid] : pair[tid];
+        if (p.row_weight) weight = CHOSEN ? p.probs[t0 + tid] : prob[tid];
+      }
+      expert[0] = (int)(c & 0xFFFF);
+      expert[1] = (int)(c >> 16);
+      // lanes whose token goes to expert x, as first or as second choice: bits of their expert numbers against x's
+      unsigned long long same[2][2];
+      const unsigned long long live = __ballot(on);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) same[k][0] = same[k][1] = live;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const unsigned long long has[2] = {__ballot((expert[0] >> b) & 1), __ballot((expert[1] >> b) & 1)};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const bool bit = (expert[k] >> b) & 1;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) same[k][j] &= bit ? has[j] : ~has[j];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const unsigned long long all = same[k][0] | same[k][1];
+        rank[k] = __popcll(all & ((1ull << lane) - 1ull));
+        if (on && rank[k] == 0) of_wave[w][expert[k]] = __popcll(all);
+      }
     }
-    if (hit) {
-      const int pos = run + before + __popcll(mask & ((1ull << lane) - 1ull));
-      token_of_row[pos] = t;
-      if (row_weight) row_weight[pos] = prob;
-      if (rows_of_token) rows_of_token[2 * (size_t)t + rank] = pos;
+    __syncthreads();
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        int pos = next[expert[k]] + rank[k];
+        for (int ww = 0; ww < w; ++ww) pos += of_wave[ww][expert[k]];
+        p.token_of_row[pos] = t0 + tid;
+        if (p.row_weight) p.row_weight[pos] = weight[k];
+        if (p.rows_of_token) p.rows_of_token[2 * (size_t)(t0 + tid) + k] = pos;
+      }
     }
-    run += total;
+    __syncthreads();
+    if (tid < kRouteMaxE)
+      for (int ww = 0; ww < kRouteBlock / 64; ++ww) next[tid] += of_wave[ww][tid];
+    __syncthreads();
   }
 }
 
@@ -253,18 +371,35 @@ __global__ __launch_bounds__(256) void combine_top2_kernel(const uint16_t* rows,
 
 }  // namespace
 
-int route_top2_max_experts() { return 256; }
+int route_top2_max_experts() { return kRouteMaxE; }
+
+// [chunks][E] counts, then [T] probabilities (8 bytes), then [T] choices
+size_t route_top2_workspace_bytes(int T, int E) {
+  const RouteShape r = route_shape(T, E);
+  if (r.chunks <= 1) return 0;
+  return ((size_t)r.chunks * E * sizeof(int) + 15) / 16 * 16 + (size_t)T * (sizeof(v2f) + sizeof(unsigned));
+}
 
 hipError_t launch_route_top2(const float* logits, int T, int E, int32_t* token_of_row, int32_t* row_offsets,
-                             float* row_weight, int32_t* rows_of_token, hipStream_t s) {
-  // token ranges per expert: enough workgroups to occupy the chip, at least one iteration each
-  const int iters = (T + kRouteThreads - 1) / kRouteThreads;
-  int parts = 256 / E;
-  parts = parts > 8 ? 8 : parts;
-  parts = parts > iters ? iters : parts;
-  parts = parts < 1 ? 1 : parts;
-  hipLaunchKernelGGL(route_top2_kernel, dim3((unsigned)(E * parts)), dim3(kRouteThreads), 0, s, logits, T, E, parts,
-                     token_of_row, row_offsets, row_weight, rows_of_token);
+                             float* row_weight, int32_t* rows_of_token, void* workspace, hipStream_t s) {
+  const RouteShape r = route_shape(T, E);
+  RouteArgs p{logits, T, E, r.lanes_log2, r.chunk_tokens, r.chunks, token_of_row, row_offsets, row_weight, rows_of_token, nullptr, nullptr, nullptr};
+  if (r.chunks > 1 && workspace) {
+    uint8_t* at = static_cast<uint8_t*>(workspace);
+    p.counts = reinterpret_cast<int*>(at);
+    at += ((size_t)r.chunks * E * sizeof(int) + 15) / 16 * 16;
+    p.probs = reinterpret_cast<v2f*>(at);
+    p.pairs = reinterpret_cast<unsigned*>(at + (size_t)T * sizeof(v2f));
+    hipLaunchKernelGGL(route_choose_kernel, dim3((unsigned)r.chunks), dim3(kRouteThreads), 0, s, p);
+    hipLaunchKernelGGL(route_place_kernel<true>, dim3((unsigned)r.chunks), dim3(kRouteThreads), 0, s, p);
+    return hipGetLastError();
+  }
+  if (r.chunks > 1) {   // every workgroup goes through all tokens: more than a few of them only repeat that work
+    const int parts = r.chunks < 8 ? r.chunks : 8;
+    p.chunk_tokens = (T + parts - 1) / parts;
+    p.chunks = (T + p.chunk_tokens - 1) / p.chunk_tokens;
+  }
+  hipLaunchKernelGGL(route_place_kernel<false>, dim3((unsigned)p.chunks), dim3(kRouteThreads), 0, s, p);
   return hipGetLastError();
 }
 

@@ -52,10 +52,13 @@ def moe_route_top2(logits, token_of_row=None, row_offsets=None, row_weight=None,
         rows_of_token = _out_tensor(rows_of_token, "rows_of_token", (t, 2), torch.int32, dev)
     lib = _lib.load()
     with torch.cuda.device(dev):
-        rc = lib.ave_fp4_moe_route_top2_ex(logits.data_ptr(), t, e, token_of_row.data_ptr(), row_offsets.data_ptr(),
+        # the choices and the counts between the two launches (torch's allocator, stream-ordered, part of a graph's pool)
+        ws_bytes = lib.ave_fp4_moe_route_top2_workspace_bytes(t, e)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        rc = lib.ave_fp4_moe_route_top2_ws(logits.data_ptr(), t, e, token_of_row.data_ptr(), row_offsets.data_ptr(),
                                            row_weight.data_ptr(),
                                            rows_of_token.data_ptr() if rows_of_token is not None else None,
-                                           _stream_ptr(dev))
+                                           workspace.data_ptr() if ws_bytes else None, ws_bytes, _stream_ptr(dev))
     _lib.check(rc)
     return token_of_row, row_offsets, row_weight
 

@@ -280,6 +280,19 @@ int ave_fp4_moe_route_top2_ex(const float* logits, int tokens, int E, int32_t* t
                               float* row_weight, int32_t* rows_of_token, void* hip_stream);
 
 /*
+ * The same routing with a caller-provided device workspace (16-byte aligned, no initialisation needed, garbage
+ * afterwards): the tokens' choices and the counts of every 128 or 256 tokens are passed through it from one launch to a
+ * second, so that the logits are read once.  ave_fp4_moe_route_top2_workspace_bytes gives its size, 0 where a single
+ * workgroup does all the work; with a smaller (or null) workspace the call is ave_fp4_moe_route_top2_ex, which goes
+ * through the logits once per eighth of the tokens.  Same integer outputs; calls that may overlap need workspaces of
+ * their own.
+ */
+size_t ave_fp4_moe_route_top2_workspace_bytes(int tokens, int E);
+int ave_fp4_moe_route_top2_ws(const float* logits, int tokens, int E, int32_t* token_of_row, int32_t* row_offsets,
+                              float* row_weight, int32_t* rows_of_token, void* workspace, size_t workspace_bytes,
+                              void* hip_stream);
+
+/*
  * The step behind the expert GEMMs: out[t, :] = w0 * rows[r0, :] + w1 * rows[r1, :] with (r0, r1) =
  * rows_of_token[t], w = row_weight of those rows, divided by w0 + w1 when `renormalize` is non-zero.  rows
  * [2*tokens, H] bf16 (the down projection's output in routed order), out [tokens, H] bf16, both 16-byte aligned;

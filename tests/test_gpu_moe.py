@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from avelang_amd import _lib
 from avelang_amd import (gather_rows_mxfp4, grouped_gemm_mxfp4_swiglu_quant_transposed_b, grouped_gemm_mxfp4_transposed_b,
                          moe_combine_top2, moe_route_top2, quantize_mxfp4)
 from oracle import fp4_oracle as orc
@@ -44,6 +45,28 @@ def test_route_top2_probabilities_with_hundreds_of_experts(gpu, t, e, seed):
     tok, off, w = _route(gpu, logits)
     assert np.array_equal(off, want_off) and np.array_equal(tok, want_tok)
     assert np.allclose(w, want_w, rtol=2e-6, atol=1e-30), float(np.max(np.abs(w - want_w) / want_w))
+
+
+@pytest.mark.parametrize("t,e", [(1, 256), (32, 129), (64, 200), (65, 200), (129, 128), (256, 64), (255, 32), (256, 8),
+                                 (257, 9), (513, 65), (33000, 256), (66000, 5)])
+def test_route_top2_chunks_with_and_without_a_workspace(gpu, t, e):
+    """Around one and two goes of a workgroup (256, 128, 64 or 32 tokens by the number of experts), more tokens than 256
+    such chunks, and chunks of more than one block of 256; the entry point without a workspace gives the same integers."""
+    logits = orc.randn((t, e), t + e)
+    logits[t // 2] = 0.5
+    want_tok, want_off, want_w = orc.route_top2(logits)
+    dev = torch.from_numpy(logits).to(gpu)
+    inv = torch.full((t, 2), -7, dtype=torch.int32, device=gpu)
+    tok, off, w = moe_route_top2(dev, rows_of_token=inv)
+    torch.cuda.synchronize()
+    assert np.array_equal(off.cpu().numpy(), want_off) and np.array_equal(tok.cpu().numpy(), want_tok)
+    assert np.allclose(w.cpu().numpy(), want_w, rtol=2e-6, atol=1e-30)
+    assert np.array_equal(inv.cpu().numpy(), orc.rows_of_token(want_tok, logits))
+    tok2, off2, w2, inv2 = torch.zeros_like(tok), torch.zeros_like(off), torch.zeros_like(w), torch.zeros_like(inv)
+    _lib.check(_lib.load().ave_fp4_moe_route_top2_ex(dev.data_ptr(), t, e, tok2.data_ptr(), off2.data_ptr(), w2.data_ptr(),
+                                                     inv2.data_ptr(), torch.cuda.current_stream(gpu).cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(tok, tok2) and torch.equal(off, off2) and torch.equal(w, w2) and torch.equal(inv, inv2)
 
 
 def test_route_top2_skewed_and_empty_experts(gpu):
