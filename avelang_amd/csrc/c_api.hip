@@ -348,6 +348,28 @@ int ave_fp4_debug_gemm_mxfp4_splitk(const uint8_t* A, const uint8_t* A_scale, co
   return gemm_mxfp4_split(A, A_scale, B, B_scale, C, M, N, K, workspace, workspace_bytes, plan, hip_stream);
 }
 
+// The planned kernel, or, where the operands' alignment (or a small K) rules it out, the first of the others that runs.
+static int nv_dispatch(const ave::NvArgs& p, const ave::NvPlan& plan, hipStream_t s) {
+  using Plan = ave::NvPlan;
+  if (plan.kernel == Plan::kNarrow && ave::nv_narrow_supports(p))
+    return finish(ave::launch_nv_narrow(p, plan.tile_rows, plan.slices > 1, s), "nvfp4 narrow-tile kernel");
+  if (plan.kernel == Plan::kTile && ave::nv_tile_supports(p))
+    return finish(ave::launch_nv_tile(p, plan.slices > 1, s), "nvfp4 tile kernel");
+  if (plan.kernel == Plan::kTileF16 && ave::nv_f16_tile_supports(p))
+    return finish(ave::launch_nv_f16_tile(p, s), "nvfp4 f16-staged tile kernel");
+  if (ave::nv_decode_supports(p)) return finish(ave::launch_nv_decode(p, s), "nvfp4 decode kernel");
+  if (ave::nv_tile_supports(p)) return finish(ave::launch_nv_tile(p, false, s), "nvfp4 tile kernel");
+  if (p.K >= 1024 && ave::nv_narrow_supports(p)) return finish(ave::launch_nv_narrow(p, 64, false, s), "nvfp4 narrow-tile kernel");   // A and B 8-byte aligned
+  // What is left is a K below 1024 that is no multiple of 256, or a K of 256 and 512 on operands that are not 16-byte aligned.  The f16-staged
+  // kernel converts and multiplies whole 256 x 256 tiles at about 1.7 us per 64 elements of K whatever the tile holds; the
+  // shape-agnostic kernel runs one wave per 32 x 32 block.  Measured crossover (N = 4096 and 28672, K = 320 / 2112 / 4160,
+  // 20..300 rows): up to about 1500 such blocks the one-wave kernel is faster (300 x 4096 x 2112: 38 against 46 us; 20 x
+  // 28672 x 4160: 79 against 86), above it the tile kernel (65 x 28672 x 4160: 90 against 131 us).
+  if (ave::nv_f16_tile_supports(p) && ((long)(p.M + 31) / 32) * ((long)(p.N + 31) / 32) > 1536)
+    return finish(ave::launch_nv_f16_tile(p, s), "nvfp4 f16-staged tile kernel");
+  return finish(ave::launch_nv_generic(p, s), "nvfp4 generic kernel");
+}
+
 int ave_fp4_gemm_nvfp4_ex(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,
                           const uint8_t* B_scale, const float* B_global, uint16_t* C, int M, int N, int K,
                           void* hip_stream, int variant) {
@@ -359,16 +381,10 @@ int ave_fp4_gemm_nvfp4_ex(const uint8_t* A, const uint8_t* A_scale, const float*
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
   switch (variant) {
     case AVE_FP4_AUTO:
-      if (ave::nv_decode_supports(p)) return finish(ave::launch_nv_decode(p, s), "nvfp4 decode kernel");
-      if (ave::nv_tile_supports(p)) return finish(ave::launch_nv_tile(p, s), "nvfp4 tile kernel");
-      // What is left is every other K (a multiple of 16).  The f16-staged kernel converts and multiplies
-      // whole 256 x 256 tiles at about 1 us per 64 elements of K whatever the tile holds; the shape-agnostic kernel
-      // runs one wave per 32 x 32 block.  Measured crossover (N = 4096 and 28672, K = 320 / 2112 / 4160, 20..300
-      // rows): up to about 1500 such blocks the one-wave kernel is faster (300 x 4096 x 2112: 38 against 46 us; 20 x
-      // 28672 x 4160: 79 against 86), above it the tile kernel (65 x 28672 x 4160: 90 against 131 us).
-      if (ave::nv_f16_tile_supports(p) && ((long)(M + 31) / 32) * ((long)(N + 31) / 32) > 1536)
-        return finish(ave::launch_nv_f16_tile(p, s), "nvfp4 f16-staged tile kernel");
-      return finish(ave::launch_nv_generic(p, s), "nvfp4 generic kernel");
+      return nv_dispatch(p, ave::nv_plan(M, N, K, ave::compute_units(), false), s);
+    case AVE_FP4_NARROW:
+      if (!ave::nv_narrow_supports(p)) return fail_inval("narrow-tile kernel does not support M=%d N=%d K=%d.", M, N, K);
+      return finish(ave::launch_nv_narrow(p, M <= 64 ? 64 : 128, false, s), "nvfp4 narrow-tile kernel");
     case AVE_FP4_TILE_F16:
       if (!ave::nv_f16_tile_supports(p))
         return fail_inval("f16-staged tile kernel does not support M=%d N=%d K=%d (16-byte aligned A and B and 4-byte aligned scales for K %% 64 == 0, 8-byte aligned A and B otherwise).", M, N, K);
@@ -380,13 +396,38 @@ int ave_fp4_gemm_nvfp4_ex(const uint8_t* A, const uint8_t* A_scale, const float*
       return finish(ave::launch_nv_generic(p, s), "nvfp4 generic kernel");
     case AVE_FP4_TILE:
       if (!ave::nv_tile_supports(p)) return fail_inval("tile kernel does not support M=%d N=%d K=%d.", M, N, K);
-      return finish(ave::launch_nv_tile(p, s), "nvfp4 tile kernel");
+      return finish(ave::launch_nv_tile(p, false, s), "nvfp4 tile kernel");
     default:
       return fail_inval("unknown kernel variant %d.", variant);
   }
 }
 
-size_t ave_fp4_gemm_nvfp4_workspace_bytes(int M, int N, int K) { return ave::nv_tile_split_plan(M, N, K).workspace_bytes; }
+int ave_fp4_debug_gemm_nvfp4_narrow(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,
+                                    const uint8_t* B_scale, const float* B_global, uint16_t* C, int M, int N, int K,
+                                    void* workspace, size_t workspace_bytes, int tile_rows, int slice_stages, void* hip_stream) {
+  g_err[0] = 0;
+  if (int rc = check_common(A, A_scale, B, B_scale, C, M, N, K, 16, 8)) return rc;
+  if (M == 0 || N == 0) return 0;
+  if (!A_global || !B_global) return fail_inval("null per-tensor scale pointer.");
+  ave::NvArgs p{A, A_scale, A_global, B, B_scale, B_global, C, M, N, K};
+  if (!ave::nv_narrow_supports(p)) return fail_inval("narrow-tile kernel does not support M=%d N=%d K=%d.", M, N, K);
+  if (tile_rows != 64 && tile_rows != 128) return fail_inval("tile_rows must be 64 or 128, got %d.", tile_rows);
+  const int stages = K / 256;
+  if (slice_stages < 0 || slice_stages > stages) return fail_inval("slice_stages must be in 0..%d, got %d.", stages, slice_stages);
+  if (slice_stages > 0) {
+    p.slices = (stages + slice_stages - 1) / slice_stages;
+    p.slice_stages = slice_stages;
+    p.P = static_cast<float*>(workspace);
+    const size_t need = (size_t)p.slices * (size_t)M * (size_t)N * sizeof(float);
+    if (!workspace || !aligned(workspace, 16) || workspace_bytes < need)
+      return fail_inval("workspace must be 16-byte aligned and hold %zu bytes, got %zu.", need, workspace_bytes);
+  }
+  return finish(ave::launch_nv_narrow(p, tile_rows, slice_stages > 0, static_cast<hipStream_t>(hip_stream)), "nvfp4 narrow-tile kernel");
+}
+
+size_t ave_fp4_gemm_nvfp4_workspace_bytes(int M, int N, int K) {
+  return ave::nv_plan(M, N, K, ave::compute_units(), true).workspace_bytes;
+}
 
 int ave_fp4_gemm_nvfp4_ws(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,
                           const uint8_t* B_scale, const float* B_global, uint16_t* C, int M, int N, int K, void* workspace,
@@ -398,14 +439,14 @@ int ave_fp4_gemm_nvfp4_ws(const uint8_t* A, const uint8_t* A_scale, const float*
   if (workspace_bytes > 0 && !workspace) return fail_inval("null workspace with workspace_bytes = %zu.", workspace_bytes);
   if (workspace && !aligned(workspace, 16)) return fail_inval("workspace must be 16-byte aligned.");
   ave::NvArgs p{A, A_scale, A_global, B, B_scale, B_global, C, M, N, K};
-  const ave::SplitPlan plan = ave::nv_tile_split_plan(M, N, K);
-  if (plan.slices > 1 && workspace_bytes >= plan.workspace_bytes && ave::nv_tile_supports(p)) {
-    p.P = static_cast<float*>(workspace);
-    p.slices = plan.slices;
-    p.slice_stages = plan.slice_pairs;
-    return finish(ave::launch_nv_tile_splitk(p, static_cast<hipStream_t>(hip_stream)), "nvfp4 tile kernel, split K");
-  }
-  return ave_fp4_gemm_nvfp4_ex(A, A_scale, A_global, B, B_scale, B_global, C, M, N, K, hip_stream, AVE_FP4_AUTO);
+  const ave::NvPlan plan = ave::nv_plan(M, N, K, ave::compute_units(), true);
+  const bool runs = plan.kernel == ave::NvPlan::kTile ? ave::nv_tile_supports(p) : ave::nv_narrow_supports(p);
+  if (plan.slices > 1 && (workspace_bytes < plan.workspace_bytes || !runs))
+    return ave_fp4_gemm_nvfp4_ex(A, A_scale, A_global, B, B_scale, B_global, C, M, N, K, hip_stream, AVE_FP4_AUTO);
+  p.P = static_cast<float*>(workspace);
+  p.slices = plan.slices;
+  p.slice_stages = plan.slice_stages;
+  return nv_dispatch(p, plan, static_cast<hipStream_t>(hip_stream));
 }
 
 int ave_fp4_gemm_nvfp4(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,

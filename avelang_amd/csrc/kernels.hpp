@@ -46,9 +46,16 @@ struct SplitPlan {
 SplitPlan mx_tile_split_plan(int M, int N, int K, size_t max_workspace_bytes = ~(size_t)0);
 SplitPlan mx_tile_split_plan_for(int M, int N, int K, int compute_units,
                                  size_t max_workspace_bytes = ~(size_t)0);   // host arithmetic only
-// the NVFP4 tile kernel's split: slice_pairs holds the 256-element stages per slice
-SplitPlan nv_tile_split_plan(int M, int N, int K);
-SplitPlan nv_tile_split_plan_for(int M, int N, int K, int compute_units);
+
+// Which NVFP4 kernel shape-based dispatch takes (gemm_nv_narrow.hip); alignment is checked against the pointers afterwards.
+struct NvPlan {
+  enum Kernel { kOther, kDecode, kNarrow, kTile, kTileF16 } kernel = kOther;   // kOther: small K, the caller's rules
+  int tile_rows = 0;            // kNarrow: 64 or 128
+  int slices = 1;               // kNarrow, kTile: K in slices of slice_stages x 256 elements (a K tail with the last one)
+  int slice_stages = 0;
+  size_t workspace_bytes = 0;   // what the slices' partial sums take, 0 for one slice
+};
+NvPlan nv_plan(int M, int N, int K, int compute_units, bool may_split);   // host arithmetic only
 
 struct NvArgs {
   const uint8_t* A;        // [M, K/2]
@@ -112,11 +119,11 @@ hipError_t launch_mx_narrow_splitk(const MxArgs& p, hipStream_t s);
 hipError_t launch_splitk_reduce(const float* P, uint16_t* C, size_t mn, int slices, hipStream_t s);
 hipError_t launch_mx_narrow(const MxArgs& p, hipStream_t s);
 hipError_t launch_mx_decode(const MxArgs& p, hipStream_t s);
-hipError_t launch_nv_tile(const NvArgs& p, hipStream_t s);
+hipError_t launch_nv_tile(const NvArgs& p, bool split, hipStream_t s);
 hipError_t launch_nv_f16_tile(const NvArgs& p, hipStream_t s);   // any K % 16 == 0: every element dequantised once per workgroup
 hipError_t launch_nv_decode(const NvArgs& p, hipStream_t s);
 hipError_t launch_nv_ring(const NvArgs& p, hipStream_t s);          // the LDS-ring weight-streaming kernel, M <= 64
-hipError_t launch_nv_tile_splitk(const NvArgs& p, hipStream_t s);   // p.P, p.slices, p.slice_stages from nv_tile_split_plan
+hipError_t launch_nv_narrow(const NvArgs& p, int tile_rows, bool split, hipStream_t s);   // tiles of 64 or 128 rows by 128 columns
 
 // x: [rows, k] fp32 or bf16 -> packed [rows, k_padded/2] bytes, scales [rows, k_padded/32] bytes; the blocks behind
 // column k of a row are written as blocks of zeros (k_padded >= k, both multiples of 32)
@@ -165,6 +172,7 @@ bool mx_decode_swiglu_supports(const MxArgs& p);
 bool mx_decode_swiglu_quant_supports(const MxArgs& p);   // ... with the fused quantiser (p.Q, p.Qs): up to 32 rows
 bool nv_tile_supports(const NvArgs& p);
 bool nv_f16_tile_supports(const NvArgs& p);
+bool nv_narrow_supports(const NvArgs& p);
 bool nv_decode_supports(const NvArgs& p);
 bool nv_ring_supports(const NvArgs& p);
 

@@ -46,15 +46,16 @@ enum ave_fp4_variant {
                           K % 128 == 0 (K % 32 == 0 for up to 16 MB of weights);
                           NVFP4: M <= 64 and K % 128 == 0, or M <= 32 and K a multiple of 32 from 512 up, or
                           M <= 64 and K a multiple of 32 from 1024 up with an even number of whole 512-element units */
-  AVE_FP4_NARROW = 4,  /* MXFP4 only: 256x128 tiles, three stage buffers; needs K a multiple of 32 from 512 up and 16-byte aligned scale
+  AVE_FP4_NARROW = 4,  /* NVFP4: 64x128 (up to 64 rows) or 128x128 tiles, any K from 256 up (a multiple of 16; A and B 8-byte
+                          aligned).  MXFP4: 256x128 tiles, three stage buffers; needs K a multiple of 32 from 512 up and 16-byte aligned scale
                           tensors; shape-based dispatch takes it for more than 64 rows when its tiles fit the compute units,
                           and for 33..64 rows against a nearly full round of 128-row tiles (N around 28672..32768 on 256
                           compute units) */
   AVE_FP4_TILE_F16 = 5, /* NVFP4 only: 256x256 tiles whose operands are dequantised to f16 once per workgroup on their way
                           into LDS, in steps of 64 elements of K; any K (a multiple of 16: a last step of 16, 32 or 48
-                          elements is staged with zeros behind it).  Shape-based dispatch takes it for K % 256 != 0,
-                          where AVE_FP4_TILE cannot run (for K % 256 == 0 AVE_FP4_TILE is faster), when C holds more
-                          than 1536 blocks of 32 x 32 (below that AVE_FP4_GENERIC is the faster one) */
+                          elements is staged with zeros behind it).  Shape-based dispatch takes it for prefill shapes with
+                          K % 64 == 0 and K % 256 != 0, where AVE_FP4_TILE cannot run, and below K = 1024 for K % 256 != 0
+                          when C holds more than 1536 blocks of 32 x 32 */
   AVE_FP4_TILE_STREAMED = 6 /* MXFP4 plain GEMM only: AVE_FP4_TILE with look-ahead touches -- eight K stages before a
                           tile's end the workgroups request the weight panels of their next tiles, so that weights
                           which come from HBM (a model's layers, each with weights of its own) are in the last-level
@@ -157,12 +158,11 @@ int ave_fp4_gemm_nvfp4_ex(const uint8_t* A, const uint8_t* A_scale, const float*
                           const uint8_t* B_scale, const float* B_global, uint16_t* C, int M, int N, int K,
                           void* hip_stream, int variant);
 /*
- * The NVFP4 GEMM with a caller-provided device workspace, the counterpart of ave_fp4_gemm_mxfp4_ws: for more than 64
- * rows and at most half as many 256 x 256 tiles as compute units, K is cut into slices that run on different
- * compute units (the NVFP4 tile kernel is bound by its fp4 -> f16 conversions, several microseconds per 256
- * elements of K, so few tiles over a long K are slow: 270 us for 128 x 4096 x 14336 unsplit).  Same contract as the
- * MXFP4 form: ave_fp4_gemm_nvfp4_workspace_bytes gives the size (0: no split), a smaller or null workspace makes
- * the call ave_fp4_gemm_nvfp4, the result is deterministic and within the GEMM's tolerance.
+ * The NVFP4 GEMM with a caller-provided device workspace, the counterpart of ave_fp4_gemm_mxfp4_ws: where the output
+ * tiles number at most half the compute units and a model of the times says that it pays, K is cut into slices that run
+ * on different compute units (128 x 4096 x 14336: 25 us instead of 59).  Same contract as the MXFP4 form:
+ * ave_fp4_gemm_nvfp4_workspace_bytes gives the size (0: no split), a smaller or null workspace makes the call
+ * ave_fp4_gemm_nvfp4, the result is deterministic and within the GEMM's tolerance.
  */
 size_t ave_fp4_gemm_nvfp4_workspace_bytes(int M, int N, int K);
 int ave_fp4_gemm_nvfp4_ws(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,

@@ -28,6 +28,12 @@ int ave_fp4_debug_split_plan(int M, int N, int K, int compute_units, int* slices
 int ave_fp4_debug_gemm_mxfp4_splitk(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                                     uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes,
                                     int slice_pairs, int narrow_tiles, void* hip_stream);
+/* The same for the NVFP4 GEMM on the 128-column tiles of AVE_FP4_NARROW: tile_rows is 64 or 128, K is cut into slices of
+ * slice_stages x 256 elements (0: not at all, the workspace may be null; the elements behind the last whole 256 go with
+ * the last slice); the workspace must hold ceil(K / 256 / slice_stages) * M * N * 4 bytes. */
+int ave_fp4_debug_gemm_nvfp4_narrow(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,
+                                    const uint8_t* B_scale, const float* B_global, uint16_t* C, int M, int N, int K,
+                                    void* workspace, size_t workspace_bytes, int tile_rows, int slice_stages, void* hip_stream);
 /* The same plan when the partial sums may take at most max_workspace_bytes: the best split that fits, or none.  This is
  * what ave_fp4_gemm_mxfp4_noalloc runs with max_workspace_bytes = AVE_FP4_NOALLOC_SCRATCH_BYTES. */
 int ave_fp4_debug_split_plan_capped(int M, int N, int K, int compute_units, size_t max_workspace_bytes, int* slices,
