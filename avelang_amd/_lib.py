@@ -9,8 +9,28 @@ from __future__ import annotations
 import ctypes
 import os
 
+import torch  # noqa: F401  (its libraries are what the extension below links against)
+
 _LIB_NAME = "libave_fp4.so"
 _lib = None
+
+
+class _NotBuilt:
+    """Stands in for the extension where it has not been built: nothing is done in C++, the wrappers go through their own
+    checks, and :func:`load` then says what is missing."""
+
+    def __init__(self, error):
+        self.error = error
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+# The entry points on torch tensors in C++ (csrc/torch_calls.cc): each function does the whole call or returns None.
+try:
+    from . import _torch_calls as native
+except ImportError as _error:
+    native = _NotBuilt(_error)
 
 AUTO, GENERIC, TILE, DECODE, NARROW, TILE_F16, TILE_STREAMED = 0, 1, 2, 3, 4, 5, 6
 
@@ -95,6 +115,9 @@ def load() -> ctypes.CDLL:
             f"{_LIB_NAME} not found at {path}: build it with `make -C avelang_amd/csrc` "
             "(or __graft_entry__.build()); there is no fallback path."
         )
+    if isinstance(native, _NotBuilt):
+        raise RuntimeError("avelang_amd._torch_calls is not built (or not for this torch): build it with `make -C avelang_amd/csrc` "
+                           "(or __graft_entry__.build())") from native.error
     lib = ctypes.CDLL(path)
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)  # AttributeError if the library lacks a declared symbol

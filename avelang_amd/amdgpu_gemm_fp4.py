@@ -13,12 +13,17 @@
 What differs from the bf16 reference: ``A``/``B`` hold packed E2M1 codes (two per byte,
 low nibble = even k) and each comes with a block-scale tensor; the reference's
 ``M % 128 == N % 128 == 0`` restriction is dropped.
+
+Every wrapper first hands its arguments to the C++ function of the same name (``csrc/torch_calls.cc``), which makes the whole
+call when they are exactly what the kernels take; what follows it in the wrapper is for everything else -- the checks that
+say what is wrong with an argument, tensor subclasses, another binding (``lib``).
 """
 from __future__ import annotations
 
 import torch
 
 from . import _lib
+from ._lib import native as _native
 
 GROUP_K_MXFP4 = 32  # K elements per E8M0 scale
 GROUP_K_NVFP4 = 16  # K elements per E4M3 scale
@@ -141,6 +146,10 @@ def gemm_mxfp4_transposed_b(A, A_scale, B, B_scale, out=None, *, variant: int = 
     ``split_k=False`` keeps every shape on the one-launch kernels (bit-identical to ``ave_fp4_gemm_mxfp4``).
     ``lib``: the binding to call through -- the ctypes binding of ``libave_fp4.so`` unless given (the pybind11
     extension built from ``python/src`` offers the same functions)."""
+    if lib is None:
+        done = _native.gemm_mxfp4(A, A_scale, B, B_scale, out, variant, split_k)
+        if done is not None:
+            return done
     A, A_scale, B, B_scale, m, n, k, _, dev = _gemm_operands(A, A_scale, B, B_scale, GROUP_K_MXFP4)
     out = _prepare_out(out, (m, n), dev)
     lib = lib or _lib.load()
@@ -169,6 +178,10 @@ def gemm_mxfp4_blocked_scales_transposed_b(A, A_scale_blocked, B, B_scale_blocke
     flat uint8 tensors of ``ceil(rows / 128) * 128 * K / 32`` bytes; ``K`` must be a multiple of 512 (``ValueError``
     otherwise: convert with :func:`avelang_amd.scales_from_blocked`).  Bit-identical to
     :func:`gemm_mxfp4_transposed_b` on the row-major scales with ``variant`` DECODE (up to 64 rows) or TILE."""
+    if lib is None:
+        done = _native.gemm_mxfp4_blocked_scales(A, A_scale_blocked, B, B_scale_blocked, out)
+        if done is not None:
+            return done
     A = _as_bytes(A, "A")
     B = _as_bytes(B, "B")
     A_scale_blocked = _as_bytes(A_scale_blocked, "A_scale_blocked")
@@ -197,6 +210,9 @@ def gemm_mxfp4_swiglu_transposed_b(A, A_scale, B, B_scale, out=None, *, variant:
     """MXFP4 gate+up GEMM with SwiGLU fused: ``B`` ``[2N, K/2]`` holds the ``N`` gate rows followed by the
     ``N`` up rows (``B_scale`` ``[2N, K/32]`` likewise); returns bf16 ``[M, N]`` with
     ``out[m, n] = silu(A[m] . B[n]) * (A[m] . B[N + n])``, evaluated in fp32."""
+    done = _native.gemm_mxfp4_swiglu(A, A_scale, B, B_scale, out, variant)
+    if done is not None:
+        return done
     A, A_scale, B, B_scale, m, n, k, _, dev = _gemm_operands(A, A_scale, B, B_scale, GROUP_K_MXFP4, gate_up=True)
     out = _prepare_out(out, (m, n), dev)
     lib = _lib.load()
@@ -217,6 +233,9 @@ def gemm_mxfp4_swiglu_quant_transposed_b(A, A_scale, B, B_scale, out=None, out_s
     ``ValueError`` otherwise.  ``n_pad`` (a multiple of 32, at least N): the rows of both results are laid out for
     ``n_pad`` columns, for a consumer that runs over a padded K (see :func:`quantize_mxfp4`); the columns from N on are
     not written -- tensors allocated here are zero-filled, tensors passed in must hold zero bytes there."""
+    done = _native.gemm_mxfp4_swiglu_quant(A, A_scale, B, B_scale, out, out_scale, n_pad)
+    if done is not None:
+        return done
     A, A_scale, B, B_scale, m, n, k, _, dev = _gemm_operands(A, A_scale, B, B_scale, GROUP_K_MXFP4, gate_up=True,
                                                              quantised_out=True)
     out, out_scale, n_pad = _quantised_outputs(out, out_scale, m, n, dev, n_pad)
@@ -236,6 +255,10 @@ def gemm_nvfp4_transposed_b(A, A_scale, A_global, B, B_scale, B_global, out=None
                             split_k: bool = True, lib=None):
     """NVFP4 GEMM. Scales are E4M3 bytes per 16 k (``[M, K/16]``, ``[N, K/16]``);
     ``A_global`` / ``B_global`` are one-element fp32 tensors on the same device."""
+    if lib is None:
+        done = _native.gemm_nvfp4(A, A_scale, A_global, B, B_scale, B_global, out, variant, split_k)
+        if done is not None:
+            return done
     A, A_scale, B, B_scale, m, n, k, _, dev = _gemm_operands(A, A_scale, B, B_scale, GROUP_K_NVFP4)
     for name, g in (("A_global", A_global), ("B_global", B_global)):
         if not isinstance(g, torch.Tensor) or g.dtype != torch.float32 or g.numel() != 1:
@@ -266,6 +289,10 @@ def grouped_gemm_mxfp4_transposed_b(A, A_scale, B, B_scale, row_offsets, out=Non
     """Grouped (MoE) MXFP4 GEMM in one launch. ``A`` ``[total_M, K/2]`` holds the rows of
     all experts back to back; ``B`` ``[E, N, K/2]``; ``row_offsets`` int32 ``[E+1]`` on the
     device (rows ``row_offsets[e]:row_offsets[e+1]`` use ``B[e]``). Returns bf16 ``[total_M, N]``."""
+    if lib is None:
+        done = _native.grouped_gemm_mxfp4(A, A_scale, B, B_scale, row_offsets, out, variant)
+        if done is not None:
+            return done
     A, A_scale, B, B_scale, m, n, k, e, dev = _gemm_operands(A, A_scale, B, B_scale, GROUP_K_MXFP4, grouped=True,
                                                              row_offsets=row_offsets)
     out = _prepare_out(out, (m, n), dev)
@@ -283,6 +310,9 @@ def grouped_gemm_mxfp4_swiglu_transposed_b(A, A_scale, B, B_scale, row_offsets, 
     """Grouped (MoE) gate+up GEMM with SwiGLU in one launch: ``B`` ``[E, 2N, K/2]`` holds, per expert, the ``N`` gate
     rows followed by the ``N`` up rows; rows ``row_offsets[e]:row_offsets[e+1]`` of ``A`` use ``B[e]``.  Returns bf16
     ``[total_M, N]``, every expert's rows equal to :func:`gemm_mxfp4_swiglu_transposed_b` on that expert alone."""
+    done = _native.grouped_gemm_mxfp4_swiglu(A, A_scale, B, B_scale, row_offsets, out)
+    if done is not None:
+        return done
     A, A_scale, B, B_scale, m, n, k, e, dev = _gemm_operands(A, A_scale, B, B_scale, GROUP_K_MXFP4, grouped=True,
                                                              gate_up=True, row_offsets=row_offsets)
     out = _prepare_out(out, (m, n), dev)
@@ -302,6 +332,9 @@ def grouped_gemm_mxfp4_swiglu_quant_transposed_b(A, A_scale, B, B_scale, row_off
     behind it: returns ``(codes [total_M, N/2], scales [total_M, N/32])``, bit-identical to ``quantize_mxfp4`` of the
     bf16 result.  ``N % 32 == 0``; needs ``K`` to be a multiple of 32 from 512 up and raises ``ValueError`` otherwise.
     ``n_pad``: as in :func:`gemm_mxfp4_swiglu_quant_transposed_b`."""
+    done = _native.grouped_gemm_mxfp4_swiglu_quant(A, A_scale, B, B_scale, row_offsets, out, out_scale, n_pad)
+    if done is not None:
+        return done
     A, A_scale, B, B_scale, m, n, k, e, dev = _gemm_operands(A, A_scale, B, B_scale, GROUP_K_MXFP4, grouped=True,
                                                              gate_up=True, row_offsets=row_offsets, quantised_out=True)
     out, out_scale, n_pad = _quantised_outputs(out, out_scale, m, n, dev, n_pad)
@@ -356,6 +389,9 @@ def quantize_mxfp4(x, packed=None, scales=None, *, k_pad=None):
     on written as zero blocks.  A GEMM over ``k_pad`` with weights padded the same way (:func:`pad_k_mxfp4`) gives the
     same sums, and the tuned kernels run faster on a K that is a multiple of 512 than on one whose packed rows are no
     multiple of 128 bytes (2880 -> 3072: 14 % less time at 8192 x 2880 x 2880)."""
+    done = _native.quantize_mxfp4(x, packed, scales, k_pad)
+    if done is not None:
+        return done
     if k_pad is not None and isinstance(x, torch.Tensor) and x.dim() == 2:
         k_pad = _padded_columns(x.shape[1], k_pad, "k_pad")
     r, k, dev, packed, scales = _quantiser_operands(x, GROUP_K_MXFP4, packed, scales, k_pad)
@@ -388,6 +424,9 @@ def quantize_nvfp4(x, global_scale, packed=None, scales=None):
     the caller, e.g. ``amax / (448 * 6)``): returns ``(packed uint8 [R, K/2], scales uint8 [R, K/16])`` in the
     layout :func:`gemm_nvfp4_transposed_b` takes together with the same ``global_scale``.  A block that holds an
     infinity or a NaN gets scale byte 0x7F (the E4M3 NaN) and zero codes."""
+    done = _native.quantize_nvfp4(x, global_scale, packed, scales)
+    if done is not None:
+        return done
     r, k, dev, packed, scales = _quantiser_operands(x, GROUP_K_NVFP4, packed, scales)
     if not isinstance(global_scale, torch.Tensor) or global_scale.dtype != torch.float32 or global_scale.numel() != 1:
         raise ValueError("global_scale must be a torch.float32 tensor with one element.")

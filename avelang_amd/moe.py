@@ -9,6 +9,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from ._lib import native as _native
 from .amdgpu_gemm_fp4 import GROUP_K_MXFP4, _as_bytes, _check_matrix, _stream_ptr
 
 MAX_EXPERTS = 256
@@ -31,6 +32,9 @@ def moe_route_top2(logits, token_of_row=None, row_offsets=None, row_weight=None,
     offsets :func:`grouped_gemm_mxfp4_transposed_b` takes, and the softmax probability of each row.
     ``rows_of_token`` (int32 ``[T, 2]``, optional) is filled with the inverse map that
     :func:`moe_combine_top2` reads: the routed row of every token's first and second choice."""
+    done = _native.moe_route_top2(logits, token_of_row, row_offsets, row_weight, rows_of_token)
+    if done is not None:
+        return done
     if not isinstance(logits, torch.Tensor):
         raise TypeError(f"logits must be a torch.Tensor, got {type(logits).__name__}.")
     if logits.dtype != torch.float32:
@@ -68,6 +72,9 @@ def moe_combine_top2(rows, rows_of_token, row_weight, out=None, *, renormalize=F
     probabilities of those rows (divided by their sum when ``renormalize``): the expert outputs back in token
     order.  ``rows`` bf16 ``[2T, H]`` (``H % 8 == 0``), ``rows_of_token`` int32 ``[T, 2]``, ``row_weight`` fp32
     ``[2T]``; returns bf16 ``[T, H]``."""
+    done = _native.moe_combine_top2(rows, rows_of_token, row_weight, out, renormalize)
+    if done is not None:
+        return done
     if not isinstance(rows, torch.Tensor) or rows.dtype != torch.bfloat16:
         raise ValueError("rows must be a torch.bfloat16 tensor.")
     if rows.dim() != 2 or rows.shape[0] % 2 != 0:
@@ -97,6 +104,9 @@ def gather_rows_mxfp4(A, A_scale, index, out=None, out_scale=None):
     """``out[i] = A[index[i]]``, ``out_scale[i] = A_scale[index[i]]``: ``A`` ``[R, K/2]`` packed E2M1,
     ``A_scale`` ``[R, K/32]`` E8M0 bytes, ``index`` int32 ``[rows]``.  An index outside ``[0, R)`` gives
     a row of zero bytes.  Returns ``(out uint8 [rows, K/2], out_scale uint8 [rows, K/32])``."""
+    done = _native.gather_rows_mxfp4(A, A_scale, index, out, out_scale)
+    if done is not None:
+        return done
     A = _as_bytes(A, "A")
     A_scale = _as_bytes(A_scale, "A_scale")
     if A.dim() != 2:
