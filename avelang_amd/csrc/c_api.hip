@@ -683,6 +683,29 @@ int ave_fp4_gather_rows_mxfp4(const uint8_t* A, const uint8_t* A_scale, const in
                 "row gather kernel");
 }
 
+// The streaming kernel where shape-based dispatch takes it; false: somebody else's shape.
+static bool grouped_stream(ave::MxArgs& p, void* hip_stream, int* rc) {
+  const int rows = ave::mx_stream_rows(p);
+  if (rows == 0) return false;
+  p.tail_four_apart = (long)p.M > 128L * p.E;   // where the 256 x 256 kernel is the other choice: its bits
+  *rc = finish(ave::launch_mx_stream(p, rows, static_cast<hipStream_t>(hip_stream)), "grouped mxfp4 streaming kernel");
+  return true;
+}
+
+int ave_fp4_debug_grouped_gemm_mxfp4_stream(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                            const int32_t* row_offsets, uint16_t* C, uint8_t* Q, uint8_t* Q_scale, int total_M,
+                                            int E, int N, int K, int swiglu, int tile_rows, void* hip_stream) {
+  g_err[0] = 0;
+  if (E <= 0) return fail_inval("E must be positive, got %d.", E);
+  if (int rc = check_common(A, A_scale, B, B_scale, Q ? static_cast<const void*>(Q) : C, total_M, N, K, 32, 16)) return rc;
+  if (total_M == 0 || N == 0) return 0;
+  if (!row_offsets) return fail_inval("null row_offsets pointer.");
+  if (tile_rows != 32 && tile_rows != 64 && tile_rows != 128) return fail_inval("tile_rows must be 32, 64 or 128, got %d.", tile_rows);
+  ave::MxArgs p{A, A_scale, B, B_scale, Q ? nullptr : C, total_M, N, K, row_offsets, E, swiglu ? 1 : 0, Q, Q_scale};
+  if (!ave::mx_stream_supports(p)) return fail_inval("streaming kernel does not support total_M=%d N=%d K=%d.", total_M, N, K);
+  return finish(ave::launch_mx_stream(p, tile_rows, static_cast<hipStream_t>(hip_stream)), "grouped mxfp4 streaming kernel");
+}
+
 int ave_fp4_grouped_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B,
                                   const uint8_t* B_scale, const int32_t* row_offsets, uint16_t* C, int total_M,
                                   int E, int N, int K, void* hip_stream, int variant) {
@@ -695,13 +718,13 @@ int ave_fp4_grouped_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, cons
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
   switch (variant) {
     case AVE_FP4_AUTO:
-      if (ave::mx_narrow_preferred(p)) return finish(ave::launch_mx_narrow(p, s), "grouped mxfp4 narrow-tile kernel");
+      if (int rc; grouped_stream(p, s, &rc)) return rc;
       if (ave::mx_tile_supports(p)) return finish(ave::launch_mx_tile(p, s), "grouped mxfp4 tile kernel");
       return finish(ave::launch_mx_generic(p, s), "grouped mxfp4 generic kernel");
     case AVE_FP4_NARROW:
-      if (!ave::mx_narrow_supports(p))
+      if (!ave::mx_stream_supports(p))
         return fail_inval("narrow-tile kernel does not support total_M=%d N=%d K=%d.", total_M, N, K);
-      return finish(ave::launch_mx_narrow(p, s), "grouped mxfp4 narrow-tile kernel");
+      return finish(ave::launch_mx_stream(p, 128, s), "grouped mxfp4 streaming kernel");
     case AVE_FP4_GENERIC:
       return finish(ave::launch_mx_generic(p, s), "grouped mxfp4 generic kernel");
     case AVE_FP4_TILE:
@@ -724,7 +747,7 @@ int ave_fp4_grouped_gemm_mxfp4_swiglu(const uint8_t* A, const uint8_t* A_scale, 
   if (!row_offsets) return fail_inval("null row_offsets pointer.");
   ave::MxArgs p{A, A_scale, B, B_scale, C, total_M, N, K, row_offsets, E, 1};
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
-  if (ave::mx_narrow_preferred(p)) return finish(ave::launch_mx_narrow(p, s), "grouped mxfp4 swiglu narrow-tile kernel");
+  if (int rc; grouped_stream(p, s, &rc)) return rc;
   if (ave::mx_tile_supports(p)) return finish(ave::launch_mx_tile(p, s), "grouped mxfp4 swiglu tile kernel");
   return finish(ave::launch_mx_generic(p, s), "grouped mxfp4 swiglu generic kernel");
 }
@@ -753,8 +776,7 @@ int ave_fp4_grouped_gemm_mxfp4_swiglu_quant_padded(const uint8_t* A, const uint8
     return fail_inval("N_padded must be a multiple of 32 and at least N = %d, got %d.", N, N_padded);
   ave::MxArgs p{A, A_scale, B, B_scale, nullptr, total_M, N, K, row_offsets, E, 1, Q, Q_scale};
   p.q_n = N_padded;
-  if (ave::mx_narrow_preferred(p))
-    return finish(ave::launch_mx_narrow(p, static_cast<hipStream_t>(hip_stream)), "grouped mxfp4 swiglu + quantise narrow-tile kernel");
+  if (int rc; grouped_stream(p, hip_stream, &rc)) return rc;
   if (!ave::mx_tile_supports(p))
     return fail_inval("the fused SwiGLU + quantiser runs on the LDS-staged kernels only: K %% 512 == 0 with 16-byte aligned "
                       "scale tensors, or another multiple of 32 from 512 up with 16-byte aligned A and B (got total_M=%d N=%d K=%d).", total_M, N, K);

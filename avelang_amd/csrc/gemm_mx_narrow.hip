@@ -17,11 +17,6 @@
 // B-image rows of wave (wm, wn) are the gate rows (first 32) and the up rows (last 32) of outputs 32 wn .. 32 wn + 31,
 // so the wave's two accumulator blocks of a row block hold the gate and the up value of the same outputs and
 // silu(gate) * up is evaluated in registers, in fp32, exactly as in the 256 x 256 kernel's fused form.
-// GROUPED: the rows of A belong to p.E experts (p.row_offsets, on the device) with weights of their own; the m-tile
-// list is the concatenation of the experts' tile lists, as in the 256 x 256 kernel.  For expert layers at decode
-// batch sizes, where an expert has a few dozen rows: 128-row tiles, and PERSISTENT -- such a launch is several rounds
-// of tiles (8 experts x 224 tiles of gate+up rows), so one workgroup per compute unit walks them and the loads of
-// the next tile go out before the current tile has ended (inside the kernel: PERSIST, cross).
 // QUANT (with SWIGLU): the bf16 result is not stored but quantised to MXFP4 (p.Q, p.Qs) with the stand-alone
 // quantiser's steps: the 32 outputs of a block are the 2 x 8 values of lane l and the 2 x 8 of lane l ^ 32.
 #include "fp4_common.hpp"
@@ -36,7 +31,7 @@ constexpr int NM = 256, NN = 128, BK = 256;
 constexpr int kRowBytes = BK / 2;                       // 128
 // Geometry of the two forms.  Full: 256 rows of A per tile, stages of 48 KB, a ring of three.  HALF: 128 rows of A
 // per tile -- waves 0-3 multiply, waves 4-7 load, always -- stages of 32 KB, a ring of four: a third more weight
-// bytes in flight per compute unit, for shapes and expert layers with at most 128 rows (per expert), where the
+// bytes in flight per compute unit, for shapes with at most 128 rows, where the
 // upper half of a 256-row tile would be loaded for nothing.
 template <bool HALF>
 struct Geo {
@@ -126,14 +121,13 @@ __device__ inline void mma_quarter(v16f (&acc)[2][2], const v4i (&bf)[2], const 
   }                                                           \
   __builtin_amdgcn_sched_barrier(0);
 
-template <bool SWIGLU, bool QUANT = false, bool SPLITK = false, bool GROUPED = false, bool HALF = false>
+template <bool SWIGLU, bool QUANT = false, bool SPLITK = false, bool HALF = false>
 __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, int n_tiles) {
   using G = Geo<HALF>;
   constexpr int kRowsTile = G::kRows, kOffB = G::kOffB, kStage = G::kStage, kRing = G::kRing, kScaleBase = G::kScaleBase;
   constexpr int kDataLoads = G::kDataLoads;
   static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
   static_assert(!SPLITK || !SWIGLU, "K is split for the plain GEMM");
-  static_assert(!SPLITK || !GROUPED, "K is split for the plain GEMM");
   constexpr int kTileN = SWIGLU ? NN / 2 : NN;   // output columns per tile
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x;
@@ -142,79 +136,17 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   const int wm = w >> 1, wn = w & 1;   // wave (wm, wn) owns rows 64 wm .., columns 64 wn .. of the tile
   // SPLITK: workgroup pid is tile pid % tiles of K slice pid / tiles; a slice is p.slice_pairs pairs of stages (the
   // last one what is left), its fp32 sums go to p.P[slice][M][N] and launch_splitk_reduce adds the slices up.
-  // GROUPED: persistent -- an expert layer at a decode batch is several rounds of tiles with few rows each, so one
-  // workgroup per compute unit walks the tiles pid, pid + gridDim.x, ... and requests the next tile's first stages
-  // before the finished tile's results leave (a workgroup per tile pays the start of the pipeline once per tile).
-  constexpr bool PERSIST = GROUPED;
-  // GROUPED, up to 256 experts (what the routing kernel takes): lane l keeps {first m-tile, m-tiles, first row, end
-  // row} (clamped to [0, M]) of experts l, l + 64, l + 128 and l + 192 in registers, read once; the list's true length
-  // replaces the host's bound (rows / tile + experts).  More experts than that: the caller's table is walked entry by
-  // entry for every tile (locate_group_tile).
-  constexpr int kExpertSets = 4;
-  int g_first[kExpertSets], g_nt[kExpertSets], g_r0[kExpertSets], g_r1[kExpertSets];
-  if (GROUPED && p.E <= 64 * kExpertSets) {
-    int carry = 0;   // m-tiles of the experts in the sets before
-#pragma unroll
-    for (int q = 0; q < kExpertSets; ++q) {
-      const int e = 64 * q + lane;
-      int r0 = 0, r1 = 0;
-      if (e < p.E) {
-        r0 = p.row_offsets[e];
-        r1 = p.row_offsets[e + 1];
-        r0 = r0 < 0 ? 0 : (r0 > p.M ? p.M : r0);
-        r1 = r1 < 0 ? 0 : (r1 > p.M ? p.M : r1);
-      }
-      const int nt = r1 > r0 ? (r1 - r0 + kRowsTile - 1) / kRowsTile : 0;
-      int incl = nt;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(incl, d);
-        if (lane >= d) incl += up;
-      }
-      g_first[q] = carry + incl - nt;
-      g_nt[q] = nt;
-      g_r0[q] = r0;
-      g_r1[q] = r1;
-      carry += __builtin_amdgcn_readlane(incl, 63);
-    }
-    m_tiles = carry;
-  }
-  const int total = m_tiles * n_tiles * (SPLITK ? p.slices : 1);
-  int pid = blockIdx.x;
-  // rows [m_begin, m_end) of A and C: m_end is the end of the matrix, or of the expert
-  int tm, tn, slice = 0, m_begin, m_end, expert, n_begin;
-  auto locate = [&](int id) {   // false: a slot behind the last tile of the grouped list; uniform for the workgroup
+  const int m_end = p.M;
+  int tm, tn, slice = 0;
+  {
+    int id = blockIdx.x;
     if (SPLITK) {
       slice = id / (m_tiles * n_tiles);
       id -= slice * (m_tiles * n_tiles);
     }
     map_tile(id, m_tiles, n_tiles, tm, tn);
-    m_begin = tm * kRowsTile;
-    m_end = p.M;
-    expert = 0;
-    n_begin = tn * kTileN;
-    if (!GROUPED) return true;
-    if (p.E <= 64 * kExpertSets) {
-#pragma unroll
-      for (int q = 0; q < kExpertSets; ++q) {
-        const unsigned long long hits = __ballot(tm >= g_first[q] && tm < g_first[q] + g_nt[q]);
-        if (hits) {
-          const int e = __builtin_ctzll(hits);
-          expert = 64 * q + e;
-          m_begin = __builtin_amdgcn_readlane(g_r0[q], e) + (tm - __builtin_amdgcn_readlane(g_first[q], e)) * kRowsTile;
-          m_end = __builtin_amdgcn_readlane(g_r1[q], e);
-          return true;
-        }
-      }
-      return false;
-    }
-    return locate_group_tile(p.row_offsets, p.E, p.M, kRowsTile, tm, expert, m_begin, m_end);
-  };
-  {
-    bool have = pid < total && locate(pid);
-    while (PERSIST && !have && (pid += (int)gridDim.x) < total) have = locate(pid);
-    if (!have) return;
   }
+  const int m_begin = tm * kRowsTile, n_begin = tn * kTileN;
   const int k_pair0 = SPLITK ? slice * p.slice_pairs : 0;
   const unsigned row_bytes = (unsigned)p.K / 2, row_scales = (unsigned)p.K / 32;
   const int pairs_left = p.K / (2 * BK) - k_pair0;
@@ -227,9 +159,6 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   // Rows past the end of a matrix are clamped to its last row: their products land in C elements never stored.
   const int wi = w & 3;
   unsigned a_off[8], b_off[4], as_off, bs_off;
-  bool upper_idle;
-  int issuers;
-  size_t expert_rows;
   const uint8_t *ga, *gb, *gas, *gbs;   // data advance by a stage, scales by a pair per issue
   // row of B behind row `row` (0..127) of the tile's B image, clamped to a valid row
   auto b_image_row = [&](int row) {
@@ -242,7 +171,7 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     const int n = n_begin + row;
     return n < p.N ? n : p.N - 1;
   };
-  auto setup_tile = [&]() {   // of the tile that locate() has just described
+  {
     const int lr = lane >> 3, cprime = lane & 7;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -264,19 +193,17 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     const int bn = b_image_row(brow);
     as_off = (unsigned)am * row_scales;
     bs_off = (unsigned)bn * row_scales;
-    // Waves 4-7 own rows 128 .. 255 of the tile.  When those rows lie past the end of A (at most 128 rows in all)
-    // they multiply nothing, and they take over the loads from waves 0-3: every SIMD then has one wave that
-    // multiplies and one that loads, and a stalled load instruction stalls no MFMA.
-    upper_idle = HALF || m_begin + 128 >= m_end;
-    issuers = __builtin_amdgcn_readfirstlane(upper_idle ? 1 : 0);
     // a pair of stages is 256 bytes of a data row and 16 scale bytes
-    expert_rows = (size_t)expert * (SWIGLU ? 2 : 1) * p.N;   // an expert holds N, or N gate + N up rows
     ga = p.A + (size_t)k_pair0 * (2 * kRowBytes);
-    gb = p.B + expert_rows * row_bytes + (size_t)k_pair0 * (2 * kRowBytes);
+    gb = p.B + (size_t)k_pair0 * (2 * kRowBytes);
     gas = p.As + (size_t)k_pair0 * 16;
-    gbs = p.Bs + expert_rows * row_scales + (size_t)k_pair0 * 16;
-  };
-  setup_tile();
+    gbs = p.Bs + (size_t)k_pair0 * 16;
+  }
+  // Waves 4-7 own rows 128 .. 255 of the tile.  When those rows lie past the end of A (at most 128 rows in all)
+  // they multiply nothing, and they take over the loads from waves 0-3: every SIMD then has one wave that
+  // multiplies and one that loads, and a stalled load instruction stalls no MFMA.
+  const bool upper_idle = HALF || m_begin + 128 >= m_end;
+  const int issuers = __builtin_amdgcn_readfirstlane(upper_idle ? 1 : 0);
   const unsigned lds_base = (unsigned)(uintptr_t)lds;
   auto issue_data = [&](unsigned sb) {
     if constexpr (HALF) dma16_stage_half(w >> 2, issuers, sb + (unsigned)wi * 4096, sb + kOffB + (unsigned)wi * 4096, ga, gb, a_off, b_off);
@@ -326,45 +253,19 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   constexpr int kWaitOdd = (kRing - 2) * kDataLoads + (kRing == 4 ? kScaleLoads : 0);
   constexpr int kWaitTailOdd = kDataLoads;       // in front of the last two stages: D(stages-1) alone
   constexpr bool kTailIssues = kRing == 3;       // four stages from the end, stage s + R still exists for R = 3 only
-  auto issue_first_stages = [&]() {
-    issue_scale_pair(0);
-    issue_data(stage_buffer(0));
-    issue_data(stage_buffer(1));
-    if (stages > 2) {
-      issue_scale_pair(1);
-      issue_data(stage_buffer(2));
-      if (kRing == 4) issue_data(stage_buffer(3));
-    }
-  };
-  issue_first_stages();
-  bool first_tile = true;
-  for (;;) {   // one tile per trip; a single trip unless PERSIST
-  // Stage 0 has landed when only the loads issued behind it are outstanding.  From the second tile on that count holds
-  // for the waves that only load (the 128-row tiles: waves 4-7); a wave that has also stored the previous tile's
-  // results waits for everything it has in flight.
-  if (first_tile || HALF) {
-    if (stages > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 1) * kDataLoads + kScaleLoads) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDataLoads) : "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  issue_scale_pair(0);
+  issue_data(stage_buffer(0));
+  issue_data(stage_buffer(1));
+  if (stages > 2) {
+    issue_scale_pair(1);
+    issue_data(stage_buffer(2));
+    if (kRing == 4) issue_data(stage_buffer(3));
   }
+  // stage 0 has landed when only the loads issued behind it are outstanding
+  if (stages > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 1) * kDataLoads + kScaleLoads) : "memory");
+  else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDataLoads) : "memory");
   __syncthreads();
-  const bool loader = w >= 4 && upper_idle;   // of the tile being computed (setup_tile below is for the next one)
-  const int c_m_begin = m_begin, c_m_end = m_end, c_n_begin = n_begin;   // the tile being computed
-  // PERSIST, whole groups of four stages and no K tail: the ring does not run dry between two tiles.  Four stages
-  // before the tile's end -- where the loads of a single tile stop -- the next tile is looked up and the loading waves
-  // send its first four stages out one by one into the buffers as they are consumed, in the order and with the wait
-  // counts of the steady state (a tile's stage j then sits in buffer j % 4 and its pair of scales in buffer
-  // (j / 2) % 2, as ever).  With 128-row tiles the roles are fixed: waves 0-3 multiply and never load.
-  const bool can_cross = PERSIST && HALF && stages >= 4 && (stages & 3) == 0 && p.K % (2 * BK) == 0;
-  bool have_next = false, crossed = false;
-  auto cross = [&](bool loads) {
-    if (can_cross) {
-      while (!have_next && (pid += (int)gridDim.x) < total) have_next = locate(pid);
-      crossed = true;
-      if (loads && have_next) setup_tile();
-    }
-  };
+  const bool loader = w >= 4 && upper_idle;
   if (loader) {
     // the loading waves of a tile without upper rows: the waits, barriers and issues of the stages below, nothing else
 #define AVE_LOAD_STAGE(WAIT, ISSUE, PARITY)                                  \
@@ -382,16 +283,6 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
       ++s;
       AVE_LOAD_STAGE(kWaitOdd, true, 1)
     }
-    cross(true);
-    if (have_next) {   // only after cross(): the tile's last four stages issue the next tile's first four
-      AVE_LOAD_STAGE(kWaitEven, true, 0)
-      ++s;
-      AVE_LOAD_STAGE(kWaitOdd, true, 1)
-      ++s;
-      AVE_LOAD_STAGE(kWaitEven, true, 0)
-      ++s;
-      AVE_LOAD_STAGE(kWaitOdd, true, 1)
-    } else {
     if (stages > 2) {
       AVE_LOAD_STAGE(kWaitEven, kTailIssues, 0)
       ++s;
@@ -401,10 +292,9 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     AVE_LOAD_STAGE(0, false, 0)
     ++s;
     AVE_LOAD_STAGE(0, false, 1)
-    }
 #undef AVE_LOAD_STAGE
-    if (!PERSIST) return;
-  } else {
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -454,7 +344,6 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     ++s;
     AVE_STAGE(kWaitOdd, true, true, 1)
   }
-  cross(false);   // the loading waves do the same four stages before their tile's end and issue the next tile's loads
   if (stages > 2) {               // four stages left: with a ring of three the last load goes out in the first of them
     AVE_STAGE(kWaitEven, kTailIssues, true, 0)
     ++s;
@@ -478,8 +367,8 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     const int tail_blocks = (p.K % (2 * BK)) / 32;
     if (tail_blocks != 0) {
       const unsigned first_block = (unsigned)(p.K / (2 * BK)) * 16u;
-      const uint8_t* tB = p.B + expert_rows * row_bytes;
-      const uint8_t* tBs = p.Bs + expert_rows * row_scales;
+      const uint8_t* tB = p.B;
+      const uint8_t* tBs = p.Bs;
       unsigned ar[2], br[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -514,17 +403,6 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) asm volatile("" : "+v"(acc[i][j]));
-  }   // multiplying waves
-  // ---- end of the tile: the next one's first stages go out before this one's results do (unless they already have) --
-  if (PERSIST && !crossed) {
-    while (!have_next && (pid += (int)gridDim.x) < total) have_next = locate(pid);
-    __syncthreads();   // every wave is done reading the ring
-    if (have_next) {
-      setup_tile();
-      issue_first_stages();
-    }
-  }
-  if (!loader) {
   if constexpr (SWIGLU) {
     // acc[0][mi] holds the gate and acc[1][mi] the up values of row m_begin + 64 wm + 32 mi + c, outputs
     // n_begin + 32 wn + 16 piece + 8 q + 0..7 (registers 8 piece .. 8 piece + 7)
@@ -532,15 +410,15 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     const bool vec_ok = (p.N % 8 == 0) && ((reinterpret_cast<uintptr_t>(p.C) & 15) == 0);
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi) {
-      const int m = c_m_begin + wm * 64 + 32 * mi + c;
-      if (m >= c_m_end) continue;
+      const int m = m_begin + wm * 64 + 32 * mi + c;
+      if (m >= m_end) continue;
       uint16_t* crow = QUANT ? nullptr : p.C + (size_t)m * p.N;
       const v16f& g = acc[0][mi];
       const v16f& u = acc[1][mi];
       v4i obits[2];   // QUANT: the 2 x 8 bf16 results of this lane
 #pragma unroll
       for (int piece = 0; piece < 2; ++piece) {
-        const int n = c_n_begin + 32 * wn + 16 * piece + 8 * q;
+        const int n = n_begin + 32 * wn + 16 * piece + 8 * q;
         float hv[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) hv[e] = silu(g[8 * piece + e]) * u[8 * piece + e];
@@ -580,7 +458,7 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
         amax = lane_xor_max_bits(amax, 32);
         const int byte = mx_scale_byte(amax);
         const float scale = mx_scale_value(byte);
-        const int n0 = c_n_begin + 32 * wn;   // first output of the block
+        const int n0 = n_begin + 32 * wn;   // first output of the block
         if (n0 < p.N) {
 #pragma unroll
           for (int piece = 0; piece < 2; ++piece) {
@@ -596,23 +474,19 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
       }
     }
   } else if constexpr (SPLITK) {
-    store_wave_block_f32<2, 2>(acc, p.P + (size_t)slice * (size_t)p.M * (size_t)p.N, p.N, c_m_begin + wm * 64, p.M,
-                               c_n_begin + wn * 64, lane);
+    store_wave_block_f32<2, 2>(acc, p.P + (size_t)slice * (size_t)p.M * (size_t)p.N, p.N, m_begin + wm * 64, p.M,
+                               n_begin + wn * 64, lane);
   } else {
-    store_wave_block<2, 2>(acc, p.C, p.N, c_m_begin + wm * 64, c_m_end, c_n_begin + wn * 64, lane, 1.0f);
+    store_wave_block<2, 2>(acc, p.C, p.N, m_begin + wm * 64, m_end, n_begin + wn * 64, lane, 1.0f);
   }
-  }   // multiplying waves
-  if (!PERSIST || !have_next) return;
-  first_tile = false;
-  }   // next tile
 }
 
 }  // namespace
 
-// What the kernel needs: the plain or the SwiGLU-fused GEMM (also grouped) on whole pairs of stages, aligned scale
-// rows, 32-bit offsets over the rows of A and over one expert's weight rows (2N of them with SwiGLU).
+// What the kernel needs: the plain or the SwiGLU-fused GEMM (expert layers: gemm_mx_stream.hip) on whole pairs of stages, aligned scale
+// rows, 32-bit offsets over the rows of A and over the weight rows (2N of them with SwiGLU).
 bool mx_narrow_supports(const MxArgs& p) {
-  if (p.row_offsets && p.E <= 0) return false;
+  if (p.row_offsets) return false;
   if (p.Q && (!p.swiglu || !p.Qs || p.N % 32 != 0 || (reinterpret_cast<uintptr_t>(p.Q) & 3))) return false;
   if (p.M <= 0 || p.N <= 0 || p.K < 2 * BK || p.K % 32 != 0) return false;
   // a K tail is fetched in 16-byte pieces straight from A and B
@@ -625,12 +499,9 @@ bool mx_narrow_supports(const MxArgs& p) {
 
 // Where it pays: more rows than the weight-streaming kernel takes (that kernel has no fused quantiser: with one,
 // any number of rows), and no more tiles than compute units -- the shapes whose 256 x 256 tiling would leave half of
-// the chip idle.  Grouped: an expert layer at a decode batch, at most 128 rows per expert on average (the host
-// does not know the distribution) -- every expert then streams its weights through tiles with few rows, where the
-// ring of three stage buffers and the idle upper waves count.
+// the chip idle.
 bool mx_narrow_preferred(const MxArgs& p) {
   if (!mx_narrow_supports(p)) return false;
-  if (p.row_offsets) return (long)p.M <= 128L * p.E;
   const int cus = compute_units(), tile_n = p.swiglu ? NN / 2 : NN;
   if (p.M <= 64 && !p.Q) {
     // Up to 64 rows belong to the weight-streaming kernel -- except 33..64 rows against so many weight rows that the
@@ -646,48 +517,40 @@ bool mx_narrow_preferred(const MxArgs& p) {
 }
 
 namespace {
-template <bool SWIGLU, bool QUANT, bool GROUPED, bool HALF>
+template <bool SWIGLU, bool QUANT, bool HALF>
 hipError_t launch_narrow(const MxArgs& p, hipStream_t s, int n_tiles) {
-  // grouped: upper bound of the concatenated tile list, one partly filled tile per expert at most
-  const int m_tiles = (p.M + Geo<HALF>::kRows - 1) / Geo<HALF>::kRows + (GROUPED ? p.E : 0);
-  if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<SWIGLU, QUANT, false, GROUPED, HALF>>(kLds<HALF>); e != hipSuccess) return e;
-  long grid = (long)m_tiles * n_tiles;
-  if (GROUPED) {   // persistent: one workgroup per compute unit (a multiple of 8, so that a workgroup's tiles stay on its XCD)
-    const int cus = compute_units();
-    if (cus <= 0) return hipErrorInvalidDevice;
-    grid = grid < cus ? grid : cus;
-  }
-  hipLaunchKernelGGL((mx_narrow_kernel<SWIGLU, QUANT, false, GROUPED, HALF>), dim3((unsigned)grid), dim3(512),
-                     kLds<HALF>, s, p, m_tiles, n_tiles);
+  const int m_tiles = (p.M + Geo<HALF>::kRows - 1) / Geo<HALF>::kRows;
+  if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<SWIGLU, QUANT, false, HALF>>(kLds<HALF>); e != hipSuccess) return e;
+  hipLaunchKernelGGL((mx_narrow_kernel<SWIGLU, QUANT, false, HALF>), dim3((unsigned)((long)m_tiles * n_tiles)), dim3(512), kLds<HALF>, s, p,
+                     m_tiles, n_tiles);
   return hipGetLastError();
 }
-template <bool GROUPED, bool HALF>
+template <bool HALF>
 hipError_t launch_narrow_form(const MxArgs& p, hipStream_t s, int n_tiles) {
-  if (p.swiglu && p.Q) return launch_narrow<true, true, GROUPED, HALF>(p, s, n_tiles);
-  if (p.swiglu) return launch_narrow<true, false, GROUPED, HALF>(p, s, n_tiles);
-  return launch_narrow<false, false, GROUPED, HALF>(p, s, n_tiles);
+  if (p.swiglu && p.Q) return launch_narrow<true, true, HALF>(p, s, n_tiles);
+  if (p.swiglu) return launch_narrow<true, false, HALF>(p, s, n_tiles);
+  return launch_narrow<false, false, HALF>(p, s, n_tiles);
 }
 }  // namespace
 
 // 128-row tiles (waves 0-3 multiply, waves 4-7 load, a ring of four stages) where no tile would have upper rows
-// -- at most 128 rows in all, and every grouped launch (experts with more rows get more tiles) -- and wherever they
+// -- at most 128 rows in all -- and wherever they
 // do not outnumber the compute units.
 hipError_t launch_mx_narrow(const MxArgs& p, hipStream_t s) {
   const int tile_n = p.swiglu ? NN / 2 : NN;
   const int n_tiles = (p.N + tile_n - 1) / tile_n;
-  if (p.row_offsets) return launch_narrow_form<true, true>(p, s, n_tiles);
   // 128-row tiles also for more rows while they do not outnumber the compute units: twice the workgroups
   const int cus = compute_units();
-  if (p.M <= 128 || (cus > 0 && (long)((p.M + 127) / 128) * n_tiles <= cus)) return launch_narrow_form<false, true>(p, s, n_tiles);
-  return launch_narrow_form<false, false>(p, s, n_tiles);
+  if (p.M <= 128 || (cus > 0 && (long)((p.M + 127) / 128) * n_tiles <= cus)) return launch_narrow_form<true>(p, s, n_tiles);
+  return launch_narrow_form<false>(p, s, n_tiles);
 }
 
 hipError_t launch_mx_narrow_splitk(const MxArgs& p, hipStream_t s) {
   const int n_tiles = (p.N + NN - 1) / NN;
   if (p.M <= 128 || p.half_rows) {
     const int m_tiles = (p.M + 127) / 128;
-    if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<false, false, true, false, true>>(kLds<true>); e != hipSuccess) return e;
-    hipLaunchKernelGGL((mx_narrow_kernel<false, false, true, false, true>), dim3((unsigned)(m_tiles * n_tiles * p.slices)),
+    if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<false, false, true, true>>(kLds<true>); e != hipSuccess) return e;
+    hipLaunchKernelGGL((mx_narrow_kernel<false, false, true, true>), dim3((unsigned)(m_tiles * n_tiles * p.slices)),
                        dim3(512), kLds<true>, s, p, m_tiles, n_tiles);
   } else {
     const int m_tiles = (p.M + NM - 1) / NM;

@@ -1,0 +1,509 @@
+// Grouped MXFP4 GEMM for gfx950 for expert layers with a few rows per expert (a decode batch, or many experts): 32 or 64 rows
+// of A by 128 weight rows per tile, and a ring of LDS buffers that never runs dry between tiles.
+//
+// Bound by HBM: every expert's weights are read once, 1.06 bytes per two elements, and what a compute unit gets through its
+// load path is about 22 - 25 KB per us.  The 128-row tiles of gemm_mx_narrow.hip spend half of that on rows of A -- for 16
+// rows an expert, on 112 repeats of its last row -- and start their ring anew for every tile where K is no multiple of 1024, with a
+// K tail read from global memory at the end of each.  Here a stage (256 elements of K) is 20 or 24 KB of which 16 are weights, six or
+// five stages are in flight, and tile boundaries and K tails are ordinary stages of one continuous stream.
+//
+// Six wavefronts: waves 0 and 1 multiply -- 64 weight rows each, two 32-row blocks, so that with SWIGLU the gate and the up value of
+// an output meet in one lane as in gemm_mx_narrow.hip -- and waves 2 - 5 load, a quarter of a stage each, with one
+// barrier per stage: behind the barrier of stage j, which says that stage j has landed and stage j - 1 is consumed, stage j + ring - 1
+// is requested into the buffer of stage j - 1.  One workgroup per compute unit walks the tiles pid, pid + gridDim.x, ...
+//
+// Layout, swizzle, K order inside a stage and the epilogues are those of gemm_mx_narrow.hip; the scale rows of a pair of stages
+// (16 bytes) travel with its first stage into slots of their own.  K tail: stages = ceil(K / 256); in the last one 16-byte chunks behind
+// the row's end repeat its last chunk, the 16 scale bytes are the row's last 16 (the row may be the tensor's last), and the
+// multiplying waves find them there and zero what is not in the row.
+#include <cmath>
+
+#include "fp4_common.hpp"
+#include "kernels.hpp"
+#include "tile_common.hpp"
+#include "tile_map.hpp"
+
+namespace ave {
+namespace {
+
+constexpr int BN = 128, BK = 256;
+constexpr int kRowBytes = BK / 2;   // 128
+constexpr int kLoadWaves = 4;
+
+template <int R>   // rows of A per tile
+struct Geo {
+  static constexpr int kWM = R == 128 ? 2 : 1;               // multiplying waves along M, R / kWM rows each
+  static constexpr int kMI = R / 32 / kWM;                   // 32-row blocks of such a wave
+  static constexpr int kMulWaves = 2 * kWM;
+  static constexpr int kThreads = (kMulWaves + kLoadWaves) * 64;
+  static constexpr int kOffB = R * kRowBytes;
+  static constexpr int kStage = kOffB + BN * kRowBytes;      // 20480 / 24576 / 32768
+  static constexpr int kRing = R == 32 ? 7 : (R == 64 ? 6 : 4);
+  static constexpr int kScaleRows = R + BN;                  // of a pair of stages: A's, then B's, 16 bytes each
+  static constexpr int kSlot = kScaleRows * 16;              // 2560 / 3072 / 4096
+  // Pairs that stages j .. j + kRing - 1 touch at most (tiles of three stages: pairs of two and of one in turn).
+  static constexpr int kSlots = R == 128 ? 3 : 5;
+  static constexpr int kScaleBase = kRing * kStage;
+  static constexpr int kLds = kScaleBase + kSlots * kSlot;   // 156160 / 162816 / 143360
+  static constexpr int kALoads = R / 32;                     // 1 KB pieces (8 rows) of A per loading wave and stage
+  static constexpr int kData = kALoads + 4;                  // loads of a loading wave for a stage; one more with a pair's scales
+  static constexpr int kScaleLanes = kScaleRows / kLoadWaves;   // 40 / 48 / 64
+};
+static_assert(Geo<32>::kLds <= 160 * 1024 && Geo<64>::kLds <= 160 * 1024 && Geo<128>::kLds <= 160 * 1024, "LDS of one compute unit");
+
+__device__ inline int lds_read1(unsigned addr) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) unsigned char*>((uintptr_t)addr);
+}
+template <int N>
+__device__ inline void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// 16 bytes per lane from an address of its own, lanes below `lanes` only (the instruction counts on vmcnt all the same)
+template <int LANES>
+__device__ inline void load_scale_rows(const uint8_t* from, unsigned to) {
+  unsigned long long saved;
+  asm volatile(
+      "s_mov_b32 m0, %[to]\n\t"
+      "s_mov_b64 %[sv], exec\n\t"
+      "s_mov_b64 exec, %[mask]\n\t"
+      "global_load_lds_dwordx4 %[from], off\n\t"
+      "s_mov_b64 exec, %[sv]\n\t"
+      : [sv] "=&s"(saved)
+      : [to] "s"(to), [mask] "s"(LANES == 64 ? ~0ull : (1ull << (LANES & 63)) - 1), [from] "v"(from)
+      : "m0", "memory");
+}
+
+// a pointer that is the same in every lane, in scalar registers
+__device__ inline const uint8_t* uniform(const uint8_t* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+  return reinterpret_cast<const uint8_t*>((uint64_t)hi << 32 | lo);
+}
+
+template <int R, bool SWIGLU, bool QUANT>
+__global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, int n_tiles) {
+  using G = Geo<R>;
+  static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
+  constexpr int kTileN = SWIGLU ? BN / 2 : BN;   // output columns per tile
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const unsigned lds_base = (unsigned)(uintptr_t)lds;
+  const unsigned row_bytes = (unsigned)p.K / 2, row_scales = (unsigned)p.K / 32;
+  const int stages = (p.K + BK - 1) / BK;
+  const int tail_blocks = (p.K % BK) / 32;             // blocks of 32 in the last stage, 0: it is a whole one
+  const int pair_tail = (p.K % (2 * BK)) / 32;         // scale bytes in the last pair, 0: all 16
+
+  // Lane l keeps {first m-tile, m-tiles, first row, end row} (clamped to [0, M]) of experts l, l + 64, l + 128 and l + 192;
+  // with more than 256 experts the caller's table is walked for every tile.
+  constexpr int kSets = 4;
+  int g_first[kSets], g_nt[kSets], g_r0[kSets], g_r1[kSets];
+  int m_tiles = 0;
+  const bool in_registers = p.E <= 64 * kSets;
+  if (in_registers) {
+#pragma unroll
+    for (int q = 0; q < kSets; ++q) {
+      const int e = 64 * q + lane;
+      int r0 = 0, r1 = 0;
+      if (e < p.E) {
+        r0 = p.row_offsets[e];
+        r1 = p.row_offsets[e + 1];
+        r0 = r0 < 0 ? 0 : (r0 > p.M ? p.M : r0);
+        r1 = r1 < 0 ? 0 : (r1 > p.M ? p.M : r1);
+      }
+      const int nt = r1 > r0 ? (r1 - r0 + R - 1) / R : 0;
+      int incl = nt;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(incl, d);
+        if (lane >= d) incl += up;
+      }
+      g_first[q] = m_tiles + incl - nt;
+      g_nt[q] = nt;
+      g_r0[q] = r0;
+      g_r1[q] = r1;
+      m_tiles += __builtin_amdgcn_readlane(incl, 63);
+    }
+  } else {
+    m_tiles = (p.M + R - 1) / R + p.E;   // upper bound
+  }
+  const int total = m_tiles * n_tiles;
+
+  int pid = (int)blockIdx.x - (int)gridDim.x;
+  int m_begin = 0, m_end = 0, expert = 0, n_begin = 0;
+  auto next_tile = [&]() {   // false: no tile left; uniform for the workgroup
+    while ((pid += (int)gridDim.x) < total) {
+      int tm, tn;
+      map_tile(pid, m_tiles, n_tiles, tm, tn);
+      n_begin = tn * kTileN;
+      if (!in_registers) {
+        int e, r0, r1;
+        if (!__builtin_amdgcn_readfirstlane(locate_group_tile(p.row_offsets, p.E, p.M, R, tm, e, r0, r1) ? 1 : 0)) continue;
+        expert = __builtin_amdgcn_readfirstlane(e);
+        m_begin = __builtin_amdgcn_readfirstlane(r0);
+        m_end = __builtin_amdgcn_readfirstlane(r1);
+        return true;
+      }
+#pragma unroll
+      for (int q = 0; q < kSets; ++q) {
+        const unsigned long long hits = __ballot(tm >= g_first[q] && tm < g_first[q] + g_nt[q]);
+        if (hits) {
+          const int e = __builtin_ctzll(hits);
+          expert = 64 * q + e;
+          m_begin = __builtin_amdgcn_readlane(g_r0[q], e) + (tm - __builtin_amdgcn_readlane(g_first[q], e)) * R;
+          m_end = __builtin_amdgcn_readlane(g_r1[q], e);
+          return true;
+        }
+      }
+    }
+    return false;
+  };
+  // row of B behind row `row` (0 .. 127) of the tile's B image, clamped to a valid row
+  auto b_image_row = [&](int row) {
+    if (SWIGLU) {   // rows 64 w + j: j < 32 the gate row, j >= 32 the up row of output column 32 w + (j & 31)
+      int n = n_begin + 32 * (row >> 6) + (row & 31);
+      n = n < p.N ? n : p.N - 1;
+      return (row & 32) ? p.N + n : n;
+    }
+    const int n = n_begin + row;
+    return n < p.N ? n : p.N - 1;
+  };
+
+  if (w >= G::kMulWaves) {
+    // ---- loading waves ---------------------------------------------------------------------------------------------------
+    const int wi = w - G::kMulWaves;
+    unsigned a_off[G::kALoads], b_off[4];
+    int a_chunk[G::kALoads], b_chunk[4];
+    const uint8_t *ga = nullptr, *gb = nullptr, *gs = nullptr;
+    int s = stages;            // stage of the tile that goes out next
+    unsigned to = lds_base, slot_to = lds_base + G::kScaleBase;
+    unsigned with_scales = 0;  // bit i: the stage issued i stages ago brought a pair of scale rows
+    int issued = 0;
+    auto issue = [&]() {       // false: nothing left
+      if (s == stages) {
+        if (!next_tile()) return false;
+        s = 0;
+        const int lr = lane >> 3, cprime = lane & 7;
+#pragma unroll
+        for (int i = 0; i < G::kALoads; ++i) {
+          const int row = (wi * G::kALoads + i) * 8 + lr;
+          int am = m_begin + row;
+          am = am < m_end ? am : m_end - 1;
+          a_chunk[i] = cprime ^ ((row >> 1) & 7);
+          a_off[i] = (unsigned)am * row_bytes + (unsigned)a_chunk[i] * 16;
+        }
+        const size_t expert_rows = (size_t)expert * (SWIGLU ? 2 : 1) * p.N;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = (wi * 4 + i) * 8 + lr;
+          b_chunk[i] = cprime ^ ((row >> 1) & 7);
+          b_off[i] = (unsigned)b_image_row(row) * row_bytes + (unsigned)b_chunk[i] * 16;
+        }
+        ga = p.A;
+        gb = p.B + expert_rows * row_bytes;
+        const int sr = wi * G::kScaleLanes + (lane < G::kScaleLanes ? lane : 0);
+        int am = m_begin + sr;
+        am = am < m_end ? am : m_end - 1;
+        gs = sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
+      }
+      if (tail_blocks != 0 && s == stages - 1) {   // chunks behind the row's end: its last chunk again
+#pragma unroll
+        for (int i = 0; i < G::kALoads; ++i)
+          if (a_chunk[i] >= tail_blocks) a_off[i] -= (unsigned)(a_chunk[i] - (tail_blocks - 1)) * 16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (b_chunk[i] >= tail_blocks) b_off[i] -= (unsigned)(b_chunk[i] - (tail_blocks - 1)) * 16;
+      }
+      const bool scales = (s & 1) == 0;
+      if (scales) {
+        if (pair_tail != 0 && s + 2 >= stages) gs -= 16 - pair_tail;   // (K >= 512: there are 16 bytes in front of the row's end)
+        load_scale_rows<G::kScaleLanes>(gs, __builtin_amdgcn_readfirstlane(slot_to) + (unsigned)wi * (G::kScaleLanes * 16));
+        gs += 16;
+        slot_to = slot_to + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot_to + G::kSlot;
+      }
+      with_scales = (with_scales << 1) | (scales ? 1u : 0u);
+#pragma unroll
+      for (int i = 0; i < G::kALoads; ++i) dma16(uniform(ga), a_off[i], to + (unsigned)(wi * G::kALoads + i) * 1024);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dma16(uniform(gb), b_off[i], to + G::kOffB + (unsigned)(wi * 4 + i) * 1024);
+      ga += kRowBytes;
+      gb += kRowBytes;
+      to = to + G::kStage == lds_base + G::kScaleBase ? lds_base : to + G::kStage;
+      ++s;
+      ++issued;
+      return true;
+    };
+    bool more = true;
+    for (int i = 0; i < G::kRing - 1 && more; ++i) more = issue();
+    for (int j = 0; j < issued; ++j) {
+      // Stage j has landed when only the loads of the stages behind it are outstanding: `ahead` of them, each kData loads
+      // and one more for those that brought scale rows (fewer than there are is safe, and waits a little longer).
+      const int ahead = __builtin_amdgcn_readfirstlane(issued - 1 - j);
+      if (ahead >= G::kRing - 2) {
+        const int c = __popc(__builtin_amdgcn_readfirstlane((int)(with_scales & ((1u << (G::kRing - 2)) - 1))));
+        if (c >= 3) wait_vm<(G::kRing - 2) * G::kData + 3>();
+        else if (c == 2) wait_vm<(G::kRing - 2) * G::kData + 2>();
+        else wait_vm<(G::kRing - 2) * G::kData + 1>();   // every two stages in a row hold the first stage of a pair
+      } else if (ahead == 4) {
+        wait_vm<4 * G::kData>();
+      } else if (ahead == 3) {
+        wait_vm<3 * G::kData>();
+      } else if (ahead == 2) {
+        wait_vm<2 * G::kData>();
+      } else if (ahead == 1) {
+        wait_vm<G::kData>();
+      } else {
+        wait_vm<0>();
+      }
+      __syncthreads();
+      if (more) more = issue();
+    }
+    return;
+  }
+
+  // ---- multiplying waves ----------------------------------------------------------------------------------------------------
+  constexpr int MI = G::kMI;
+  const int rho = lane & 31, h = lane >> 5;
+  const int wn = w & 1, m_wave = (w >> 1) * (32 * MI);   // this wave's weight rows start at 64 wn, its rows of A at m_wave
+  const int a_row = m_wave + rho;             // + 32 mi
+  const int b_row = wn * 64 + pi_row(rho);    // + 32 nj
+  const unsigned a_frag = (unsigned)(a_row * kRowBytes + (((4 * h) ^ ((a_row >> 1) & 7)) * 16));
+  const unsigned b_frag = (unsigned)(G::kOffB + b_row * kRowBytes + (((4 * h) ^ ((b_row >> 1) & 7)) * 16));
+  const unsigned a_sc = (unsigned)a_row * 16, b_sc = (unsigned)(R + b_row) * 16;   // in a slot, + 512 per 32 rows
+  unsigned sb = lds_base, slot = lds_base + G::kLds - G::kSlot;
+  while (next_tile()) {
+    v16f acc[2][MI];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < MI; ++j) acc[i][j] = v16f{};
+    int as_cur[MI], bs_cur[2];
+    // the dword of a row's 16 scale bytes for stage parity P and this lane's half: 2 P + h
+    auto read_scales = [&](int P) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) as_cur[i] = lds_read4(slot + a_sc + i * 512 + (unsigned)(2 * P + h) * 4);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) bs_cur[i] = lds_read4(slot + b_sc + i * 512 + (unsigned)(2 * P + h) * 4);
+    };
+    v4i af[4][MI], bf[4][2];   // the fragments of a whole stage: all requested before the first is waited for
+    auto read_frags = [&]() {
+#pragma unroll
+      for (int kj = 0; kj < 4; ++kj) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) af[kj][i] = lds_read16(sb + (a_frag ^ ((unsigned)kj * 16)) + i * 4096);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) bf[kj][i] = lds_read16(sb + (b_frag ^ ((unsigned)kj * 16)) + i * 4096);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    const int whole = pair_tail == 0 ? stages : (stages - 1) & ~1;   // stages of whole pairs
+    auto next_slot = [&]() { slot = slot + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot + G::kSlot; };
+    auto next_buffer = [&]() { sb = sb + G::kStage == lds_base + G::kScaleBase ? lds_base : sb + G::kStage; };
+    int s = 0;
+    if (G::kWM > 1 && m_begin + m_wave >= m_end) {   // no rows for this wave: the barriers and the positions, nothing else
+      for (; s < stages; ++s) {
+        __syncthreads();
+        if ((s & 1) == 0) next_slot();
+        next_buffer();
+      }
+      continue;
+    }
+    for (; s < whole; ++s) {
+      __syncthreads();   // the stage has landed
+      if ((s & 1) == 0) next_slot();
+      read_scales(s & 1);
+      read_frags();
+#pragma unroll
+      for (int nj = 0; nj < 2; ++nj)
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<0, 0>(bf[0][nj], af[0][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
+#pragma unroll
+      for (int nj = 0; nj < 2; ++nj)
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<1, 1>(bf[1][nj], af[1][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
+#pragma unroll
+      for (int nj = 0; nj < 2; ++nj)
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<2, 2>(bf[2][nj], af[2][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
+#pragma unroll
+      for (int nj = 0; nj < 2; ++nj)
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<3, 3>(bf[3][nj], af[3][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
+      next_buffer();
+    }
+    // The one or two stages behind the last whole pair.  Their blocks are added up in the order of the kernel that runs the
+    // ungrouped GEMM of these rows: two by two (gemm_mx_narrow.hip), or four apart as in every other stage (gemm_mx_tile.hip).
+    // A block that is not there is zeros under the scale 2^0.
+    for (; s < stages; ++s) {
+      __syncthreads();
+      if ((s & 1) == 0) next_slot();
+      const int blocks = s == stages - 1 && tail_blocks != 0 ? tail_blocks : 8;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int block = p.tail_four_apart ? 4 * h + j : 2 * j + h;
+        const bool have = block < blocks;
+        const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (have ? block : 0));
+        const v4i none = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          const v4i f = lds_read16(sb + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
+          const int sc = lds_read1(at + a_sc + i * 512);
+          af[j][i] = have ? f : none;
+          as_cur[i] = have ? sc : 0x7f;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const v4i f = lds_read16(sb + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
+          const int sc = lds_read1(at + b_sc + i * 512);
+          bf[j][i] = have ? f : none;
+          bs_cur[i] = have ? sc : 0x7f;
+        }
+#pragma unroll
+        for (int nj = 0; nj < 2; ++nj)
+#pragma unroll
+          for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<0, 0>(bf[j][nj], af[j][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
+      }
+      next_buffer();
+    }
+
+    if constexpr (SWIGLU) {
+      // acc[0][mi] holds the gate and acc[1][mi] the up values of row m_begin + m_wave + 32 mi + c, outputs n_begin + 32 wn + 16 piece + 8 q
+      // + 0..7 (registers 8 piece .. 8 piece + 7)
+      const int c = lane & 31, q = lane >> 5;
+      const bool vec_ok = (p.N % 8 == 0) && ((reinterpret_cast<uintptr_t>(p.C) & 15) == 0);
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi) {
+        const int m = m_begin + m_wave + 32 * mi + c;
+        if (m >= m_end) continue;
+        uint16_t* crow = QUANT ? nullptr : p.C + (size_t)m * p.N;
+        v4i o[2];
+#pragma unroll
+        for (int piece = 0; piece < 2; ++piece) {
+          float hv[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) hv[e] = silu(acc[0][mi][8 * piece + e]) * acc[1][mi][8 * piece + e];
+          o[piece] = v4i{(int)pack_bf16x2(hv[0], hv[1]), (int)pack_bf16x2(hv[2], hv[3]), (int)pack_bf16x2(hv[4], hv[5]), (int)pack_bf16x2(hv[6], hv[7])};
+          if constexpr (!QUANT) {
+            const int n = n_begin + 32 * wn + 16 * piece + 8 * q;
+            if (vec_ok && n + 8 <= p.N) {
+              *reinterpret_cast<v4i*>(crow + n) = o[piece];
+            } else {
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                if (n + e < p.N) crow[n + e] = (uint16_t)(((unsigned)o[piece][e >> 1] >> (16 * (e & 1))) & 0xFFFF);
+            }
+          }
+        }
+        if constexpr (QUANT) {
+          // the stand-alone quantiser's steps on the bf16 values (N % 32 == 0: a block lies inside the matrix or outside it as
+          // a whole, so both lanes of the exchange are in the same state)
+          float v[2][8];
+#pragma unroll
+          for (int piece = 0; piece < 2; ++piece)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              v[piece][2 * j] = __builtin_bit_cast(float, (unsigned)o[piece][j] << 16);
+              v[piece][2 * j + 1] = __builtin_bit_cast(float, (unsigned)o[piece][j] & 0xFFFF0000u);
+            }
+          unsigned amax = abs_max_bits(v[0]);
+          const unsigned second = abs_max_bits(v[1]);
+          amax = lane_xor_max_bits(amax > second ? amax : second, 32);
+          const int byte = mx_scale_byte(amax);
+          const float scale = mx_scale_value(byte);
+          const int n0 = n_begin + 32 * wn;   // first output of the block
+          if (n0 < p.N) {
+#pragma unroll
+            for (int piece = 0; piece < 2; ++piece) {
+              unsigned codes = 0;
+              codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[piece][0], v[piece][1], scale, 0);
+              codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[piece][2], v[piece][3], scale, 1);
+              codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[piece][4], v[piece][5], scale, 2);
+              codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[piece][6], v[piece][7], scale, 3);
+              *reinterpret_cast<unsigned*>(p.Q + (size_t)m * (q_row_cols(p) / 2) + (n0 + 16 * piece + 8 * q) / 2) = byte == 0xFF ? 0u : codes;
+            }
+            if (q == 0) p.Qs[(size_t)m * (q_row_cols(p) / 32) + n0 / 32] = (uint8_t)byte;
+          }
+        }
+      }
+    } else {
+      store_wave_block<MI, 2>(acc, p.C, p.N, m_begin + m_wave, m_end, n_begin + wn * 64, lane, 1.0f);
+    }
+  }
+}
+
+template <int R, bool SWIGLU, bool QUANT>
+hipError_t launch(const MxArgs& p, hipStream_t s) {
+  constexpr int kTileN = SWIGLU ? BN / 2 : BN;
+  const int n_tiles = (p.N + kTileN - 1) / kTileN;
+  const int cus = compute_units();
+  if (cus <= 0) return hipErrorInvalidDevice;
+  if (hipError_t e = allow_dynamic_lds<mx_stream_kernel<R, SWIGLU, QUANT>>(Geo<R>::kLds); e != hipSuccess) return e;
+  const long tiles = ((long)(p.M + R - 1) / R + p.E) * n_tiles;   // upper bound of the experts' tile lists
+  hipLaunchKernelGGL((mx_stream_kernel<R, SWIGLU, QUANT>), dim3((unsigned)(tiles < cus ? tiles : cus)), dim3(Geo<R>::kThreads), Geo<R>::kLds, s, p,
+                     n_tiles);
+  return hipGetLastError();
+}
+template <int R>
+hipError_t launch_form(const MxArgs& p, hipStream_t s) {
+  if (p.swiglu && p.Q) return launch<R, true, true>(p, s);
+  if (p.swiglu) return launch<R, true, false>(p, s);
+  return launch<R, false, false>(p, s);
+}
+
+}  // namespace
+
+// K a multiple of 32 from 512 up, 16-byte aligned A and B, 32-bit offsets over the rows of A and over one expert's weight rows,
+// a tile count that fits an int.  Scale rows may start anywhere.
+bool mx_stream_supports(const MxArgs& p) {
+  if (!p.row_offsets || p.E <= 0 || p.M <= 0 || p.N <= 0 || p.K < 2 * BK || p.K % 32 != 0) return false;
+  if (p.Q && (!p.swiglu || !p.Qs || p.N % 32 != 0 || (reinterpret_cast<uintptr_t>(p.Q) & 3))) return false;
+  if (((reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.B)) & 15) != 0) return false;
+  const uint64_t b_rows = (uint64_t)p.N * (p.swiglu ? 2 : 1);
+  if ((uint64_t)p.M * (uint64_t)(p.K / 2) >= (1ull << 32) || b_rows * (uint64_t)(p.K / 2) >= (1ull << 32)) return false;
+  const uint64_t tiles = ((uint64_t)(p.M + 31) / 32 + (uint64_t)p.E) * (uint64_t)((p.N + BN / 2 - 1) / (BN / 2));
+  return tiles < (1ull << 30);
+}
+
+namespace {
+// m-tiles of R rows that E experts with `rows` rows on average (and the spread of random routing) are expected to fill
+double expected_m_tiles(int E, double rows, int R) {
+  double per_expert = 1.0;
+  const double sigma = sqrt(rows < 1.0 ? 1.0 : rows);
+  for (int k = 1; k * R < rows + 6 * sigma; ++k) per_expert += 0.5 * erfc((k * R + 0.5 - rows) / (sigma * 1.41421356));
+  return E * per_expert;
+}
+}  // namespace
+
+// Shape-based dispatch; the host knows the average number of rows per expert only.  Up to 128 this kernel: it reads
+// the weights once at 4 - 5.5 TB/s (gate+up of 8 experts x 16 rows, 28672 x 4096, 92 us; 128 experts x 16 rows, 5760 x 2880, 247 us where
+// the 128-row tiles with a ring per tile took 318; 78 experts x 4 rows, 21504 x 1184, 205 against 306).  32 rows a tile up to 18 rows per
+// expert (an expert with more rows takes a second tile and its weights a second time through the load path: 36 rows on
+// average 105 us, on 64-row tiles 87 us), 64 up to 44 (64 rows on average 137 us, on 128-row tiles 111), 128 above.
+// More than 128 rows per expert: against the 256 x 256 kernel, by a model of both in microseconds on 256 compute units -- 0.84 per stage and round
+// here; there 2.1 - 2.8 per stage and round and 4 - 14 around a tile, more where few tiles share a weight panel or K has a tail
+// (22 experts x 134 rows, 3072 x 12800: 171 us here, 220 there; 25600 x 3072: 310 here, 272 there).
+int mx_stream_rows(const MxArgs& p) {
+  if (!mx_stream_supports(p)) return 0;
+  const double rows = (double)p.M / p.E;
+  if (rows <= 18) return 32;
+  if (rows <= 44) return 64;
+  if (rows <= 128) return 128;
+  if (rows > 1024) return 0;
+  int cus = compute_units();
+  if (cus <= 0) cus = 256;
+  const int stages = (p.K + BK - 1) / BK;
+  const long n_here = p.swiglu ? (p.N + 63) / 64 : (p.N + 127) / 128, n_there = p.swiglu ? (p.N + 127) / 128 : (p.N + 255) / 256;
+  const double here = ceil(expected_m_tiles(p.E, rows, 128) * n_here / cus) * stages * 0.84 + 4.0;
+  const double m_there = expected_m_tiles(p.E, rows, 256);
+  const bool whole = p.K % (2 * BK) == 0, wide = n_there >= 64;
+  const double per_stage = !whole ? 2.8 : (wide ? 2.1 : 2.3), around = whole && wide ? 6.0 : (m_there < 1.3 * p.E ? 14.0 : 4.0);
+  const double there = ceil(m_there * n_there / cus) * (stages * per_stage + around);
+  return here < there ? 128 : 0;
+}
+
+hipError_t launch_mx_stream(const MxArgs& p, int tile_rows, hipStream_t s) {
+  return tile_rows == 32 ? launch_form<32>(p, s) : (tile_rows == 64 ? launch_form<64>(p, s) : launch_form<128>(p, s));
+}
+
+}  // namespace ave

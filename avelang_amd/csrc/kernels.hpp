@@ -27,6 +27,8 @@ struct MxArgs {
   int half_rows = 0;           //   narrow-tile kernel only: 1 = the slices run on its 128-row tiles
   int touch = 0;               // 256 x 256 kernel, plain GEMM: 1 = look-ahead touches of the next round's panels (weights
                                //   expected to come from HBM rather than from the last-level cache)
+  int tail_four_apart = 0;     // grouped streaming kernel: order of addition behind the last whole 512 elements of K, as in the
+                               //   256 x 256 kernel (1) or as in the narrow-tile kernel (0)
   int blocked_scales = 0;      // 1: As and Bs are in the 128 x 4 blocked layout (plain GEMM, K % 512 == 0): padded to
                                //   128 rows and 4 columns, 512-byte tiles in row-major tile order, scale (r, c) of a
                                //   tile at byte (r % 32) * 16 + (r / 32) * 4 + c
@@ -118,6 +120,7 @@ hipError_t launch_mx_narrow_splitk(const MxArgs& p, hipStream_t s);
 // C = bf16(P[0] + ... + P[slices-1]) in slice order; P[s] is [mn] floats
 hipError_t launch_splitk_reduce(const float* P, uint16_t* C, size_t mn, int slices, hipStream_t s);
 hipError_t launch_mx_narrow(const MxArgs& p, hipStream_t s);
+hipError_t launch_mx_stream(const MxArgs& p, int tile_rows, hipStream_t s);   // grouped, tiles of 32, 64 or 128 rows by 128 weight rows
 hipError_t launch_mx_decode(const MxArgs& p, hipStream_t s);
 hipError_t launch_nv_tile(const NvArgs& p, bool split, hipStream_t s);
 hipError_t launch_nv_f16_tile(const NvArgs& p, hipStream_t s);   // any K % 16 == 0: every element dequantised once per workgroup
@@ -167,6 +170,8 @@ bool mx_tile_blocked_supports(const MxArgs& p);     // p.blocked_scales: the 256
 bool mx_decode_blocked_supports(const MxArgs& p);   // ... the weight-streaming kernel does
 bool mx_narrow_supports(const MxArgs& p);    // the 256 x 128 tile kernel can run the shape
 bool mx_narrow_preferred(const MxArgs& p);   // ... and shape-based dispatch picks it
+bool mx_stream_supports(const MxArgs& p);
+int mx_stream_rows(const MxArgs& p);         // rows per tile (32, 64, 128) with which shape-based dispatch takes that kernel, or 0
 bool mx_decode_supports(const MxArgs& p);
 bool mx_decode_swiglu_supports(const MxArgs& p);
 bool mx_decode_swiglu_quant_supports(const MxArgs& p);   // ... with the fused quantiser (p.Q, p.Qs): up to 32 rows

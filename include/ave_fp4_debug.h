@@ -34,6 +34,12 @@ int ave_fp4_debug_gemm_mxfp4_splitk(const uint8_t* A, const uint8_t* A_scale, co
 int ave_fp4_debug_gemm_nvfp4_narrow(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,
                                     const uint8_t* B_scale, const float* B_global, uint16_t* C, int M, int N, int K,
                                     void* workspace, size_t workspace_bytes, int tile_rows, int slice_stages, void* hip_stream);
+/* Diagnostic and test hook: the grouped MXFP4 GEMM on tiles of tile_rows (32, 64 or 128) rows of A by 128 weight rows, whatever the
+ * shape (K a multiple of 32 from 512 up, 16-byte aligned A and B).  swiglu: B holds 2N rows per expert; with Q and Q_scale
+ * (C null) the result is quantised, rows laid out for N columns. */
+int ave_fp4_debug_grouped_gemm_mxfp4_stream(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                            const int32_t* row_offsets, uint16_t* C, uint8_t* Q, uint8_t* Q_scale, int total_M,
+                                            int E, int N, int K, int swiglu, int tile_rows, void* hip_stream);
 /* The same plan when the partial sums may take at most max_workspace_bytes: the best split that fits, or none.  This is
  * what ave_fp4_gemm_mxfp4_noalloc runs with max_workspace_bytes = AVE_FP4_NOALLOC_SCRATCH_BYTES. */
 int ave_fp4_debug_split_plan_capped(int M, int N, int K, int compute_units, size_t max_workspace_bytes, int* slices,

@@ -1,0 +1,64 @@
+"""GPU parity of the grouped MXFP4 kernel for a few rows per expert: every tile height, tiles of two and more stages with
+every kind of K tail, experts around a tile's rows, plain, with SwiGLU and with SwiGLU and the quantiser."""
+import numpy as np
+import pytest
+import torch
+
+from avelang_amd import _lib, quantize_mxfp4
+from oracle import fp4_oracle as orc
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def _stream(gpu, ops, ro, n, tile_rows, swiglu, quant):
+    m, k, e = ops[0].shape[0], ops[0].shape[1] * 2, ops[2].shape[0]
+    c = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu)
+    q = torch.full((m, n // 2), 0xEE, dtype=torch.uint8, device=gpu)
+    qs = torch.full((m, n // 32), 0xEE, dtype=torch.uint8, device=gpu)
+    _lib.check(_lib.load().ave_fp4_debug_grouped_gemm_mxfp4_stream(
+        *(t.data_ptr() for t in ops), ro.data_ptr(), None if quant else c.data_ptr(), q.data_ptr() if quant else None,
+        qs.data_ptr() if quant else None, m, e, n, k, swiglu, tile_rows, torch.cuda.current_stream(gpu).cuda_stream))
+    torch.cuda.synchronize(gpu)
+    return (q, qs) if quant else c
+
+
+# rows per expert around 32, 64 and 128 and several tiles; two, three, four and more stages; K % 512 of 1, 7, 8, 9 and 15 blocks
+@pytest.mark.parametrize("rows,n,k", [([3, 0, 31, 33], 64, 512), ([1], 32, 544), ([64, 65, 0, 127], 96, 736), ([129, 5], 160, 768),
+                                      ([32, 200, 1, 70], 128, 800), ([40, 130, 0, 300], 192, 992), ([17] * 20, 352, 1024),
+                                      ([2] * 70, 64, 1312), ([66, 0, 140], 224, 2880), ([5] * 40 + [90], 512, 1792)])
+@pytest.mark.parametrize("tile_rows", [32, 64, 128])
+def test_stream_matches_oracle_and_its_own_fused_forms(gpu, rows, n, k, tile_rows):
+    e, m = len(rows), sum(rows)
+    ro = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    a, a_s = H.mx_operand(m, k, seed=m + k)
+    b, b_s = H.mx_operand(e * 2 * n, k, seed=n + k, std=0.05)
+    b, b_s = b.reshape(e, 2 * n, k // 2), b_s.reshape(e, 2 * n, k // 32)
+    ops = [H.to_dev(t, gpu) for t in (a, a_s, b, b_s)]
+    dro = torch.from_numpy(ro).to(gpu)
+    plain = H.bits(_stream(gpu, ops, dro, 2 * n, tile_rows, 0, False))
+    fused = _stream(gpu, ops, dro, n, tile_rows, 1, False)
+    q, qs = _stream(gpu, ops, dro, n, tile_rows, 1, True)
+    for x in range(e):
+        r0, r1 = int(ro[x]), int(ro[x + 1])
+        if r1 > r0:
+            H.assert_mx_close(plain[r0:r1], a[r0:r1], a_s[r0:r1], b[x], b_s[x])
+            ok, rep = orc.check_swiglu_bf16(H.bits(fused[r0:r1]), a[r0:r1], a_s[r0:r1], b[x], b_s[x])
+            assert ok, (x, rep)
+    want_q, want_s = quantize_mxfp4(fused)
+    assert torch.equal(q, want_q) and torch.equal(qs, want_s)
+
+
+def test_stream_walks_a_table_of_more_than_256_experts(gpu):
+    n, k, e = 64, 736, 300
+    rows = np.zeros(e, dtype=np.int64)
+    rows[[0, 7, 255, 256, 299]] = [5, 40, 129, 1, 33]
+    ro = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    a, a_s = H.mx_operand(int(ro[-1]), k, seed=1)
+    b, b_s = H.mx_operand(e * n, k, seed=2, std=0.05)
+    b, b_s = b.reshape(e, n, k // 2), b_s.reshape(e, n, k // 32)
+    ops = [H.to_dev(t, gpu) for t in (a, a_s, b, b_s)]
+    for tile_rows in (32, 128):
+        c = H.bits(_stream(gpu, ops, torch.from_numpy(ro).to(gpu), n, tile_rows, 0, False))
+        for x in np.nonzero(rows)[0]:
+            H.assert_mx_close(c[ro[x]:ro[x + 1]], a[ro[x]:ro[x + 1]], a_s[ro[x]:ro[x + 1]], b[x], b_s[x])
