@@ -49,10 +49,16 @@ SIGNATURES = {
     "ave_fp4_debug_split_plan_capped": [_int, _int, _int, _int, ctypes.c_size_t, ctypes.POINTER(_int), ctypes.POINTER(_int),
                                         ctypes.POINTER(_int), ctypes.POINTER(ctypes.c_size_t)],
     "ave_fp4_debug_gemm_mxfp4_splitk": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _int, _int, _vp],
+    "ave_fp4_debug_gemm_mxfp4_stream_splitk": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _int, _int, _vp],
     "ave_fp4_debug_grouped_gemm_mxfp4_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _int, _vp],
     "ave_fp4_debug_gemm_nvfp4_narrow": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _int, _int, _vp],
     "ave_fp4_gemm_mxfp4_swiglu": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp],
     "ave_fp4_gemm_mxfp4_swiglu_ex": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, _int],
+    "ave_fp4_gemm_mxfp4_planned_workspace_bytes": [_int, _int, _int],
+    "ave_fp4_gemm_mxfp4_planned": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _vp],
+    "ave_fp4_gemm_mxfp4_swiglu_workspace_bytes": [_int, _int, _int, _int],
+    "ave_fp4_gemm_mxfp4_swiglu_ws": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _vp],
+    "ave_fp4_gemm_mxfp4_swiglu_quant_ws": [_vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _vp, ctypes.c_size_t, _vp],
     "ave_fp4_gemm_nvfp4": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp],
     "ave_fp4_gemm_nvfp4_ex": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, _int],
     "ave_fp4_gemm_nvfp4_workspace_bytes": [_int, _int, _int],
@@ -97,6 +103,8 @@ SIGNATURES = {
 ABI_VERSION = 1   # what ave_fp4_abi_version() of a matching library returns
 
 _RESTYPES = {"ave_fp4_last_error": ctypes.c_char_p, "ave_fp4_gemm_mxfp4_workspace_bytes": ctypes.c_size_t,
+             "ave_fp4_gemm_mxfp4_planned_workspace_bytes": ctypes.c_size_t,
+             "ave_fp4_gemm_mxfp4_swiglu_workspace_bytes": ctypes.c_size_t,
              "ave_fp4_gemm_nvfp4_workspace_bytes": ctypes.c_size_t,
              "ave_fp4_moe_route_top2_workspace_bytes": ctypes.c_size_t}
 

@@ -156,10 +156,10 @@ def gemm_mxfp4_transposed_b(A, A_scale, B, B_scale, out=None, *, variant: int = 
     with torch.cuda.device(dev):
         # shapes with few output tiles and a long K are split along K through a workspace from torch's allocator
         # (stream-ordered like `out`, and part of the graph's pool under capture); the library never allocates
-        ws_bytes = lib.ave_fp4_gemm_mxfp4_workspace_bytes(m, n, k) if int(variant) == _lib.AUTO and split_k else 0
+        ws_bytes = lib.ave_fp4_gemm_mxfp4_planned_workspace_bytes(m, n, k) if int(variant) == _lib.AUTO and split_k else 0
         if ws_bytes:
             workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            rc = lib.ave_fp4_gemm_mxfp4_ws(
+            rc = lib.ave_fp4_gemm_mxfp4_planned(
                 A.data_ptr(), A_scale.data_ptr(), B.data_ptr(), B_scale.data_ptr(), out.data_ptr(),
                 m, n, k, workspace.data_ptr(), ws_bytes, _stream_ptr(dev),
             )
@@ -217,10 +217,18 @@ def gemm_mxfp4_swiglu_transposed_b(A, A_scale, B, B_scale, out=None, *, variant:
     out = _prepare_out(out, (m, n), dev)
     lib = _lib.load()
     with torch.cuda.device(dev):
-        rc = lib.ave_fp4_gemm_mxfp4_swiglu_ex(
-            A.data_ptr(), A_scale.data_ptr(), B.data_ptr(), B_scale.data_ptr(), out.data_ptr(),
-            m, n, k, _stream_ptr(dev), int(variant),
-        )
+        ws_bytes = lib.ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(m, n, k, 0) if int(variant) == _lib.AUTO else 0
+        if ws_bytes:
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            rc = lib.ave_fp4_gemm_mxfp4_swiglu_ws(
+                A.data_ptr(), A_scale.data_ptr(), B.data_ptr(), B_scale.data_ptr(), out.data_ptr(),
+                m, n, k, workspace.data_ptr(), ws_bytes, _stream_ptr(dev),
+            )
+        else:
+            rc = lib.ave_fp4_gemm_mxfp4_swiglu_ex(
+                A.data_ptr(), A_scale.data_ptr(), B.data_ptr(), B_scale.data_ptr(), out.data_ptr(),
+                m, n, k, _stream_ptr(dev), int(variant),
+            )
     _lib.check(rc)
     return out
 
@@ -243,9 +251,11 @@ def gemm_mxfp4_swiglu_quant_transposed_b(A, A_scale, B, B_scale, out=None, out_s
         return out, out_scale
     lib = _lib.load()
     with torch.cuda.device(dev):
-        rc = lib.ave_fp4_gemm_mxfp4_swiglu_quant_padded(
+        ws_bytes = lib.ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(m, n, k, 1)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        rc = lib.ave_fp4_gemm_mxfp4_swiglu_quant_ws(
             A.data_ptr(), A_scale.data_ptr(), B.data_ptr(), B_scale.data_ptr(), out.data_ptr(), out_scale.data_ptr(),
-            m, n, n_pad, k, _stream_ptr(dev),
+            m, n, n_pad, k, workspace.data_ptr() if ws_bytes else None, ws_bytes, _stream_ptr(dev),
         )
     _lib.check(rc)
     return out, out_scale

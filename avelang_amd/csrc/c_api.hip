@@ -201,6 +201,38 @@ int ave_fp4_debug_stream_read_write(const void* src, size_t bytes, void* dst, si
                 "streaming-read-and-write probe");
 }
 
+static ave::MxStreamPlan stream_plan(int M, int N, int K, bool swiglu, bool quant, bool may_split) {
+  const int cus = ave::compute_units();
+  return ave::kept_plan(M, N, K, cus * 8 + swiglu * 4 + quant * 2 + may_split,
+                        [&] { return ave::mx_stream_plan(M, N, K, swiglu, quant, cus, may_split); });
+}
+static ave::NvPlan nv_plan(int M, int N, int K, bool may_split) {
+  const int cus = ave::compute_units();
+  return ave::kept_plan(M, N, K, cus * 2 + may_split, [&] { return ave::nv_plan(M, N, K, cus, may_split); });
+}
+static ave::SplitPlan split_plan(int M, int N, int K) {
+  return ave::kept_plan(M, N, K, ave::compute_units(), [&] { return ave::mx_tile_split_plan(M, N, K); });
+}
+
+// The ungrouped GEMM (or a fused SwiGLU form of it) on the streaming kernel with K in one piece, where that is planned.
+static bool stream_whole(const ave::MxArgs& p, void* hip_stream, int* rc) {
+  const ave::MxStreamPlan plan = stream_plan(p.M, p.N, p.K, p.swiglu != 0, p.Q != nullptr, false);
+  if (plan.rows == 0 || !ave::mx_stream_supports(p)) return false;
+  *rc = finish(ave::launch_mx_stream(p, plan.rows, static_cast<hipStream_t>(hip_stream)), "mxfp4 streaming kernel");
+  return true;
+}
+// The same with K in slices, where that is planned and the workspace holds their sums.
+static bool stream_split(ave::MxArgs p, void* workspace, size_t workspace_bytes, void* hip_stream, int* rc) {
+  const ave::MxStreamPlan plan = stream_plan(p.M, p.N, p.K, p.swiglu != 0, p.Q != nullptr, true);
+  if (plan.rows == 0 || plan.slices < 2 || workspace_bytes < plan.workspace_bytes || !ave::mx_stream_supports(p)) return false;
+  if (p.C && p.swiglu && !aligned(p.C, 16)) return false;   // stored 16 bytes at a time
+  p.P = static_cast<float*>(workspace);
+  p.slices = plan.slices;
+  p.slice_pairs = plan.slice_pairs;
+  *rc = finish(ave::launch_mx_stream(p, plan.rows, static_cast<hipStream_t>(hip_stream)), "mxfp4 streaming kernel, split K");
+  return true;
+}
+
 int ave_fp4_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                           uint16_t* C, int M, int N, int K, void* hip_stream, int variant) {
   g_err[0] = 0;
@@ -210,6 +242,7 @@ int ave_fp4_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
   switch (variant) {
     case AVE_FP4_AUTO:
+      if (int rc; stream_whole(p, s, &rc)) return rc;
       // (33..64 rows against a nearly full round of 128-row tiles: the narrow-tile kernel ahead of the rings)
       if (M > 32 && M <= 64 && ave::mx_narrow_preferred(p)) return finish(ave::launch_mx_narrow(p, s), "mxfp4 narrow-tile kernel");
       if (ave::mx_decode_supports(p)) return finish(ave::launch_mx_decode(p, s), "mxfp4 decode kernel");
@@ -262,7 +295,7 @@ int ave_fp4_gemm_mxfp4_blocked_scales(const uint8_t* A, const uint8_t* A_scale_b
                     "ave_fp4_scales_from_blocked and call ave_fp4_gemm_mxfp4.", M, N, K);
 }
 
-size_t ave_fp4_gemm_mxfp4_workspace_bytes(int M, int N, int K) { return ave::mx_tile_split_plan(M, N, K).workspace_bytes; }
+size_t ave_fp4_gemm_mxfp4_workspace_bytes(int M, int N, int K) { return split_plan(M, N, K).workspace_bytes; }
 
 int ave_fp4_debug_split_plan_capped(int M, int N, int K, int compute_units, size_t max_workspace_bytes, int* slices,
                                     int* slice_pairs, int* narrow_tiles, size_t* workspace_bytes) {
@@ -302,10 +335,32 @@ int ave_fp4_gemm_mxfp4_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_
   if (M == 0 || N == 0) return 0;
   if (workspace_bytes > 0 && !workspace) return fail_inval("null workspace with workspace_bytes = %zu.", workspace_bytes);
   if (workspace && !aligned(workspace, 16)) return fail_inval("workspace must be 16-byte aligned.");
-  const ave::SplitPlan plan = ave::mx_tile_split_plan(M, N, K);
+  const ave::SplitPlan plan = split_plan(M, N, K);
   if (plan.slices > 1 && workspace_bytes >= plan.workspace_bytes && aligned(A_scale, 16) && aligned(B_scale, 16))
     return gemm_mxfp4_split(A, A_scale, B, B_scale, C, M, N, K, workspace, workspace_bytes, plan, hip_stream);
   return ave_fp4_gemm_mxfp4_ex(A, A_scale, B, B_scale, C, M, N, K, hip_stream, AVE_FP4_AUTO);
+}
+
+static int check_workspace(const void* workspace, size_t workspace_bytes) {
+  if (workspace_bytes > 0 && !workspace) return fail_inval("null workspace with workspace_bytes = %zu.", workspace_bytes);
+  if (workspace && !aligned(workspace, 16)) return fail_inval("workspace must be 16-byte aligned.");
+  return 0;
+}
+
+size_t ave_fp4_gemm_mxfp4_planned_workspace_bytes(int M, int N, int K) {
+  const ave::MxStreamPlan plan = stream_plan(M, N, K, false, false, true);
+  return plan.rows ? plan.workspace_bytes : ave_fp4_gemm_mxfp4_workspace_bytes(M, N, K);
+}
+
+int ave_fp4_gemm_mxfp4_planned(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                               uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes, void* hip_stream) {
+  g_err[0] = 0;
+  if (int rc = check_common(A, A_scale, B, B_scale, C, M, N, K, 32, 16)) return rc;
+  if (M == 0 || N == 0) return 0;
+  if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
+  int rc;
+  if (stream_split(ave::MxArgs{A, A_scale, B, B_scale, C, M, N, K, nullptr, 0}, workspace, workspace_bytes, hip_stream, &rc)) return rc;
+  return ave_fp4_gemm_mxfp4_ws(A, A_scale, B, B_scale, C, M, N, K, workspace, workspace_bytes, hip_stream);
 }
 
 int ave_fp4_gemm_mxfp4_noalloc(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
@@ -381,7 +436,7 @@ int ave_fp4_gemm_nvfp4_ex(const uint8_t* A, const uint8_t* A_scale, const float*
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
   switch (variant) {
     case AVE_FP4_AUTO:
-      return nv_dispatch(p, ave::nv_plan(M, N, K, ave::compute_units(), false), s);
+      return nv_dispatch(p, nv_plan(M, N, K, false), s);
     case AVE_FP4_NARROW:
       if (!ave::nv_narrow_supports(p)) return fail_inval("narrow-tile kernel does not support M=%d N=%d K=%d.", M, N, K);
       return finish(ave::launch_nv_narrow(p, M <= 64 ? 64 : 128, false, s), "nvfp4 narrow-tile kernel");
@@ -426,7 +481,7 @@ int ave_fp4_debug_gemm_nvfp4_narrow(const uint8_t* A, const uint8_t* A_scale, co
 }
 
 size_t ave_fp4_gemm_nvfp4_workspace_bytes(int M, int N, int K) {
-  return ave::nv_plan(M, N, K, ave::compute_units(), true).workspace_bytes;
+  return nv_plan(M, N, K, true).workspace_bytes;
 }
 
 int ave_fp4_gemm_nvfp4_ws(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,
@@ -439,7 +494,7 @@ int ave_fp4_gemm_nvfp4_ws(const uint8_t* A, const uint8_t* A_scale, const float*
   if (workspace_bytes > 0 && !workspace) return fail_inval("null workspace with workspace_bytes = %zu.", workspace_bytes);
   if (workspace && !aligned(workspace, 16)) return fail_inval("workspace must be 16-byte aligned.");
   ave::NvArgs p{A, A_scale, A_global, B, B_scale, B_global, C, M, N, K};
-  const ave::NvPlan plan = ave::nv_plan(M, N, K, ave::compute_units(), true);
+  const ave::NvPlan plan = nv_plan(M, N, K, true);
   const bool runs = plan.kernel == ave::NvPlan::kTile ? ave::nv_tile_supports(p) : ave::nv_narrow_supports(p);
   if (plan.slices > 1 && (workspace_bytes < plan.workspace_bytes || !runs))
     return ave_fp4_gemm_nvfp4_ex(A, A_scale, A_global, B, B_scale, B_global, C, M, N, K, hip_stream, AVE_FP4_AUTO);
@@ -523,6 +578,7 @@ int ave_fp4_gemm_mxfp4_swiglu_ex(const uint8_t* A, const uint8_t* A_scale, const
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
   switch (variant) {
     case AVE_FP4_AUTO:
+      if (int rc; stream_whole(p, s, &rc)) return rc;
       // (33..64 rows against a nearly full round of 128-row tiles: the narrow-tile kernel ahead of the rings)
       if (M > 32 && M <= 64 && ave::mx_narrow_preferred(p)) return finish(ave::launch_mx_narrow(p, s), "mxfp4 swiglu narrow-tile kernel");
       if (ave::mx_decode_swiglu_supports(p)) return finish(ave::launch_mx_decode(p, s), "mxfp4 swiglu decode kernel");
@@ -555,12 +611,22 @@ int ave_fp4_gemm_mxfp4_swiglu_ex(const uint8_t* A, const uint8_t* A_scale, const
 
 int ave_fp4_gemm_mxfp4_swiglu_quant(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                                     uint8_t* Q, uint8_t* Q_scale, int M, int N, int K, void* hip_stream) {
-  return ave_fp4_gemm_mxfp4_swiglu_quant_padded(A, A_scale, B, B_scale, Q, Q_scale, M, N, N, K, hip_stream);
+  return ave_fp4_gemm_mxfp4_swiglu_quant_ws(A, A_scale, B, B_scale, Q, Q_scale, M, N, N, K, nullptr, 0, hip_stream);
 }
 
 int ave_fp4_gemm_mxfp4_swiglu_quant_padded(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B,
                                            const uint8_t* B_scale, uint8_t* Q, uint8_t* Q_scale, int M, int N,
                                            int N_padded, int K, void* hip_stream) {
+  return ave_fp4_gemm_mxfp4_swiglu_quant_ws(A, A_scale, B, B_scale, Q, Q_scale, M, N, N_padded, K, nullptr, 0, hip_stream);
+}
+
+size_t ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(int M, int N, int K, int quant) {
+  return stream_plan(M, N, K, true, quant != 0, true).workspace_bytes;
+}
+
+int ave_fp4_gemm_mxfp4_swiglu_quant_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                       uint8_t* Q, uint8_t* Q_scale, int M, int N, int N_padded, int K, void* workspace,
+                                       size_t workspace_bytes, void* hip_stream) {
   g_err[0] = 0;
   // Q stands in for C in the common checks (non-null, 2-byte aligned is implied by the 16 bytes asked below)
   if (int rc = check_common(A, A_scale, B, B_scale, Q, M, N, K, 32, 16)) return rc;
@@ -571,8 +637,11 @@ int ave_fp4_gemm_mxfp4_swiglu_quant_padded(const uint8_t* A, const uint8_t* A_sc
   if (!aligned(Q, 16)) return fail_inval("Q must be 16-byte aligned.");
   if (N_padded < N || N_padded % 32 != 0)
     return fail_inval("N_padded must be a multiple of 32 and at least N = %d, got %d.", N, N_padded);
+  if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
   ave::MxArgs p{A, A_scale, B, B_scale, nullptr, M, N, K, nullptr, 0, 1, Q, Q_scale};
   p.q_n = N_padded;
+  if (int rc; stream_split(p, workspace, workspace_bytes, hip_stream, &rc)) return rc;
+  if (int rc; stream_whole(p, hip_stream, &rc)) return rc;
   if (ave::mx_decode_swiglu_quant_supports(p))
     return finish(ave::launch_mx_decode(p, static_cast<hipStream_t>(hip_stream)), "mxfp4 swiglu + quantise decode kernel");
   if (ave::mx_narrow_preferred(p))
@@ -582,6 +651,17 @@ int ave_fp4_gemm_mxfp4_swiglu_quant_padded(const uint8_t* A, const uint8_t* A_sc
                       "scale tensors, or another multiple of 32 from 512 up with 16-byte aligned A and B (got M=%d N=%d K=%d).", M, N, K);
   p.touch = weights_likely_from_hbm(B, 2 * (size_t)N * (size_t)(K / 2 + K / 32)) ? 1 : 0;
   return finish(ave::launch_mx_tile(p, static_cast<hipStream_t>(hip_stream)), "mxfp4 swiglu + quantise tile kernel");
+}
+
+int ave_fp4_gemm_mxfp4_swiglu_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                 uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes, void* hip_stream) {
+  g_err[0] = 0;
+  if (int rc = check_common(A, A_scale, B, B_scale, C, M, N, K, 32, 16)) return rc;
+  if (M == 0 || N == 0) return 0;
+  if (N > (1 << 30)) return fail_inval("N must not exceed 2^30, got %d.", N);
+  if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
+  if (int rc; stream_split(ave::MxArgs{A, A_scale, B, B_scale, C, M, N, K, nullptr, 0, 1}, workspace, workspace_bytes, hip_stream, &rc)) return rc;
+  return ave_fp4_gemm_mxfp4_swiglu_ex(A, A_scale, B, B_scale, C, M, N, K, hip_stream, AVE_FP4_AUTO);
 }
 
 int ave_fp4_gemm_mxfp4_swiglu(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
@@ -681,6 +761,28 @@ int ave_fp4_gather_rows_mxfp4(const uint8_t* A, const uint8_t* A_scale, const in
   return finish(ave::launch_gather_rows(A, A_scale, index, rows, src_rows, K, out, out_scale,
                                         static_cast<hipStream_t>(hip_stream)),
                 "row gather kernel");
+}
+
+int ave_fp4_debug_gemm_mxfp4_stream_splitk(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                           uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes, int tile_rows,
+                                           int slice_pairs, void* hip_stream) {
+  g_err[0] = 0;
+  if (int rc = check_common(A, A_scale, B, B_scale, C, M, N, K, 32, 16)) return rc;
+  if (M == 0 || N == 0) return 0;
+  if (tile_rows != 32 && tile_rows != 64 && tile_rows != 128) return fail_inval("tile_rows must be 32, 64 or 128, got %d.", tile_rows);
+  const int pairs = K / 512;
+  if (slice_pairs <= 0 || slice_pairs > pairs) return fail_inval("slice_pairs must be in 1..%d, got %d.", pairs, slice_pairs);
+  ave::MxArgs p{A, A_scale, B, B_scale, C, M, N, K, nullptr, 0};
+  p.slices = (pairs + slice_pairs - 1) / slice_pairs;
+  p.slice_pairs = slice_pairs;
+  p.P = static_cast<float*>(workspace);
+  const size_t need = (size_t)p.slices * (size_t)M * (size_t)N * sizeof(float);
+  if (!workspace || !aligned(workspace, 16) || workspace_bytes < need)
+    return fail_inval("workspace must be 16-byte aligned and hold %zu bytes, got %zu.", need, workspace_bytes);
+  if (!ave::mx_stream_supports(p)) return fail_inval("streaming kernel does not support M=%d N=%d K=%d.", M, N, K);
+  hipStream_t s = static_cast<hipStream_t>(hip_stream);
+  if (hipError_t e = ave::launch_mx_stream(p, tile_rows, s); e != hipSuccess) return finish(e, "mxfp4 streaming kernel, split K");
+  return finish(ave::launch_splitk_reduce(p.P, C, (size_t)M * (size_t)N, p.slices, s), "reduction of the K slices");
 }
 
 // The streaming kernel where shape-based dispatch takes it; false: somebody else's shape.

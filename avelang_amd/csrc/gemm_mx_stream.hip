@@ -80,10 +80,14 @@ __device__ inline const uint8_t* uniform(const uint8_t* p) {
   return reinterpret_cast<const uint8_t*>((uint64_t)hi << 32 | lo);
 }
 
-template <int R, bool SWIGLU, bool QUANT>
+// GROUPED: the rows of A belong to p.E experts (p.row_offsets) with weights of their own; otherwise one matrix of p.M rows.
+// SPLITK (plain form, not grouped): a work item is a tile and a slice of p.slice_pairs pairs of stages (the last one what is left, the
+// K tail with it); its fp32 sums go to p.P[slice][M][N].
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK>
 __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, int n_tiles) {
   using G = Geo<R>;
   static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
+  static_assert(!SPLITK || (!SWIGLU && !GROUPED), "K is split for the plain GEMM");
   constexpr int kTileN = SWIGLU ? BN / 2 : BN;   // output columns per tile
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x;
@@ -101,7 +105,9 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
   int g_first[kSets], g_nt[kSets], g_r0[kSets], g_r1[kSets];
   int m_tiles = 0;
   const bool in_registers = p.E <= 64 * kSets;
-  if (in_registers) {
+  if (!GROUPED) {
+    m_tiles = (p.M + R - 1) / R;
+  } else if (in_registers) {
 #pragma unroll
     for (int q = 0; q < kSets; ++q) {
       const int e = 64 * q + lane;
@@ -128,15 +134,27 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
   } else {
     m_tiles = (p.M + R - 1) / R + p.E;   // upper bound
   }
-  const int total = m_tiles * n_tiles;
+  const int total = m_tiles * n_tiles * (SPLITK ? p.slices : 1);
 
   int pid = (int)blockIdx.x - (int)gridDim.x;
   int m_begin = 0, m_end = 0, expert = 0, n_begin = 0;
+  int slice = 0, s_first = 0, s_last = stages;   // stages of the tile: all of them, or those of a slice
   auto next_tile = [&]() {   // false: no tile left; uniform for the workgroup
     while ((pid += (int)gridDim.x) < total) {
-      int tm, tn;
-      map_tile(pid, m_tiles, n_tiles, tm, tn);
+      int tm, tn, id = pid;
+      if (SPLITK) {
+        slice = id / (m_tiles * n_tiles);
+        id -= slice * (m_tiles * n_tiles);
+        s_first = slice * 2 * p.slice_pairs;
+        s_last = s_first + 2 * p.slice_pairs < stages && slice + 1 < p.slices ? s_first + 2 * p.slice_pairs : stages;
+      }
+      map_tile(id, m_tiles, n_tiles, tm, tn);
       n_begin = tn * kTileN;
+      if (!GROUPED) {
+        m_begin = tm * R;
+        m_end = p.M;
+        return true;
+      }
       if (!in_registers) {
         int e, r0, r1;
         if (!__builtin_amdgcn_readfirstlane(locate_group_tile(p.row_offsets, p.E, p.M, R, tm, e, r0, r1) ? 1 : 0)) continue;
@@ -176,14 +194,14 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
     unsigned a_off[G::kALoads], b_off[4];
     int a_chunk[G::kALoads], b_chunk[4];
     const uint8_t *ga = nullptr, *gb = nullptr, *gs = nullptr;
-    int s = stages;            // stage of the tile that goes out next
+    int s = s_last;            // stage of the tile that goes out next
     unsigned to = lds_base, slot_to = lds_base + G::kScaleBase;
     unsigned with_scales = 0;  // bit i: the stage issued i stages ago brought a pair of scale rows
     int issued = 0;
     auto issue = [&]() {       // false: nothing left
-      if (s == stages) {
+      if (s == s_last) {
         if (!next_tile()) return false;
-        s = 0;
+        s = s_first;
         const int lr = lane >> 3, cprime = lane & 7;
 #pragma unroll
         for (int i = 0; i < G::kALoads; ++i) {
@@ -200,12 +218,13 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
           b_chunk[i] = cprime ^ ((row >> 1) & 7);
           b_off[i] = (unsigned)b_image_row(row) * row_bytes + (unsigned)b_chunk[i] * 16;
         }
-        ga = p.A;
-        gb = p.B + expert_rows * row_bytes;
+        ga = p.A + (size_t)s * kRowBytes;
+        gb = p.B + expert_rows * row_bytes + (size_t)s * kRowBytes;
         const int sr = wi * G::kScaleLanes + (lane < G::kScaleLanes ? lane : 0);
         int am = m_begin + sr;
         am = am < m_end ? am : m_end - 1;
         gs = sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
+        gs += (size_t)(s >> 1) * 16;
       }
       if (tail_blocks != 0 && s == stages - 1) {   // chunks behind the row's end: its last chunk again
 #pragma unroll
@@ -297,12 +316,13 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    const int whole = pair_tail == 0 ? stages : (stages - 1) & ~1;   // stages of whole pairs
+    // stages of whole pairs end here
+    const int whole = pair_tail == 0 || s_last < stages ? s_last : (stages - 1) & ~1;
     auto next_slot = [&]() { slot = slot + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot + G::kSlot; };
     auto next_buffer = [&]() { sb = sb + G::kStage == lds_base + G::kScaleBase ? lds_base : sb + G::kStage; };
-    int s = 0;
+    int s = s_first;
     if (G::kWM > 1 && m_begin + m_wave >= m_end) {   // no rows for this wave: the barriers and the positions, nothing else
-      for (; s < stages; ++s) {
+      for (; s < s_last; ++s) {
         __syncthreads();
         if ((s & 1) == 0) next_slot();
         next_buffer();
@@ -335,7 +355,7 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
     // The one or two stages behind the last whole pair.  Their blocks are added up in the order of the kernel that runs the
     // ungrouped GEMM of these rows: two by two (gemm_mx_narrow.hip), or four apart as in every other stage (gemm_mx_tile.hip).
     // A block that is not there is zeros under the scale 2^0.
-    for (; s < stages; ++s) {
+    for (; s < s_last; ++s) {
       __syncthreads();
       if ((s & 1) == 0) next_slot();
       const int blocks = s == stages - 1 && tail_blocks != 0 ? tail_blocks : 8;
@@ -426,29 +446,100 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
           }
         }
       }
+    } else if constexpr (SPLITK) {
+      store_wave_block_f32<MI, 2>(acc, p.P + (size_t)slice * (size_t)p.M * (size_t)p.N, p.N, m_begin + m_wave, m_end, n_begin + wn * 64, lane);
     } else {
       store_wave_block<MI, 2>(acc, p.C, p.N, m_begin + m_wave, m_end, n_begin + wn * 64, lane, 1.0f);
     }
   }
 }
 
-template <int R, bool SWIGLU, bool QUANT>
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK>
 hipError_t launch(const MxArgs& p, hipStream_t s) {
   constexpr int kTileN = SWIGLU ? BN / 2 : BN;
   const int n_tiles = (p.N + kTileN - 1) / kTileN;
   const int cus = compute_units();
   if (cus <= 0) return hipErrorInvalidDevice;
-  if (hipError_t e = allow_dynamic_lds<mx_stream_kernel<R, SWIGLU, QUANT>>(Geo<R>::kLds); e != hipSuccess) return e;
-  const long tiles = ((long)(p.M + R - 1) / R + p.E) * n_tiles;   // upper bound of the experts' tile lists
-  hipLaunchKernelGGL((mx_stream_kernel<R, SWIGLU, QUANT>), dim3((unsigned)(tiles < cus ? tiles : cus)), dim3(Geo<R>::kThreads), Geo<R>::kLds, s, p,
-                     n_tiles);
+  constexpr auto kernel = mx_stream_kernel<R, SWIGLU, QUANT, GROUPED, SPLITK>;
+  if (hipError_t e = allow_dynamic_lds<kernel>(Geo<R>::kLds); e != hipSuccess) return e;
+  // grouped: upper bound of the experts' tile lists
+  const long tiles = ((long)(p.M + R - 1) / R + (GROUPED ? p.E : 0)) * n_tiles * (SPLITK ? p.slices : 1);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < cus ? tiles : cus)), dim3(Geo<R>::kThreads), Geo<R>::kLds, s, p, n_tiles);
+  return hipGetLastError();
+}
+// silu(gate) * up of K slices' sums P[slices][M][2N] (N gate columns, then N up columns), added up in slice order: bf16 into C, or
+// (QUANT) quantised to MXFP4 with the stand-alone quantiser's steps on the bf16 values.  A lane owns 8 outputs of one row, so a block
+// of 32 is four neighbouring lanes (N % 32 == 0: blocks never leave a row).  Bound by the sums' way through the memory system.
+template <bool QUANT>
+__global__ __launch_bounds__(256) void reduce_swiglu_kernel(MxArgs p) {
+  const unsigned per_row = (unsigned)p.N / 8;
+  const size_t lanes = (size_t)p.M * per_row, step = (size_t)p.M * 2 * p.N;
+  for (size_t g = (size_t)blockIdx.x * 256 + threadIdx.x; g < lanes; g += (size_t)gridDim.x * 256) {
+    const size_t m = g / per_row;
+    const unsigned n = (unsigned)(g % per_row) * 8;
+    const float* at = p.P + m * 2 * p.N + n;
+    v4f gate[2] = {}, up[2] = {};
+#pragma unroll 4
+    for (int sl = 0; sl < p.slices; ++sl) {
+      const v4f* x = reinterpret_cast<const v4f*>(at + sl * step);
+      const v4f* y = reinterpret_cast<const v4f*>(at + sl * step + p.N);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        gate[i] += x[i];
+        up[i] += y[i];
+      }
+    }
+    float hv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) hv[e] = silu(gate[e >> 2][e & 3]) * up[e >> 2][e & 3];
+    const v4i o = {(int)pack_bf16x2(hv[0], hv[1]), (int)pack_bf16x2(hv[2], hv[3]), (int)pack_bf16x2(hv[4], hv[5]), (int)pack_bf16x2(hv[6], hv[7])};
+    if constexpr (!QUANT) {
+      *reinterpret_cast<v4i*>(p.C + m * p.N + n) = o;
+    } else {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[2 * j] = __builtin_bit_cast(float, (unsigned)o[j] << 16);
+        v[2 * j + 1] = __builtin_bit_cast(float, (unsigned)o[j] & 0xFFFF0000u);
+      }
+      const int byte = mx_scale_byte(lane_xor_max_bits(lane_xor_max_bits(abs_max_bits(v), 1), 2));
+      const float scale = mx_scale_value(byte);
+      unsigned codes = 0;
+      codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[0], v[1], scale, 0);
+      codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[2], v[3], scale, 1);
+      codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[4], v[5], scale, 2);
+      codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, v[6], v[7], scale, 3);
+      *reinterpret_cast<unsigned*>(p.Q + m * (q_row_cols(p) / 2) + n / 2) = byte == 0xFF ? 0u : codes;
+      if ((n & 31) == 0) p.Qs[m * (q_row_cols(p) / 32) + n / 32] = (uint8_t)byte;
+    }
+  }
+}
+
+// The K slices' sums of all weight rows (gate and up rows alike), then the sum over the slices.
+template <int R>
+hipError_t launch_split(const MxArgs& p, hipStream_t s) {
+  MxArgs q = p;
+  q.swiglu = 0;
+  q.N = p.swiglu ? 2 * p.N : p.N;
+  if (hipError_t e = launch<R, false, false, false, true>(q, s); e != hipSuccess) return e;
+  if (!p.swiglu) return launch_splitk_reduce(p.P, p.C, (size_t)p.M * (size_t)p.N, p.slices, s);
+  const size_t blocks = ((size_t)p.M * (p.N / 8) + 255) / 256;
+  const dim3 grid((unsigned)(blocks < 4096 ? blocks : 4096));
+  if (p.Q) hipLaunchKernelGGL(reduce_swiglu_kernel<true>, grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL(reduce_swiglu_kernel<false>, grid, dim3(256), 0, s, p);
   return hipGetLastError();
 }
 template <int R>
 hipError_t launch_form(const MxArgs& p, hipStream_t s) {
-  if (p.swiglu && p.Q) return launch<R, true, true>(p, s);
-  if (p.swiglu) return launch<R, true, false>(p, s);
-  return launch<R, false, false>(p, s);
+  if (p.P) return launch_split<R>(p, s);
+  if (!p.row_offsets) {
+    if (p.swiglu && p.Q) return launch<R, true, true, false, false>(p, s);
+    if (p.swiglu) return launch<R, true, false, false, false>(p, s);
+    return launch<R, false, false, false, false>(p, s);
+  }
+  if (p.swiglu && p.Q) return launch<R, true, true, true, false>(p, s);
+  if (p.swiglu) return launch<R, true, false, true, false>(p, s);
+  return launch<R, false, false, true, false>(p, s);
 }
 
 }  // namespace
@@ -456,13 +547,13 @@ hipError_t launch_form(const MxArgs& p, hipStream_t s) {
 // K a multiple of 32 from 512 up, 16-byte aligned A and B, 32-bit offsets over the rows of A and over one expert's weight rows,
 // a tile count that fits an int.  Scale rows may start anywhere.
 bool mx_stream_supports(const MxArgs& p) {
-  if (!p.row_offsets || p.E <= 0 || p.M <= 0 || p.N <= 0 || p.K < 2 * BK || p.K % 32 != 0) return false;
+  if ((p.row_offsets ? p.E <= 0 : p.E != 0) || p.M <= 0 || p.N <= 0 || p.K < 2 * BK || p.K % 32 != 0) return false;
   if (p.Q && (!p.swiglu || !p.Qs || p.N % 32 != 0 || (reinterpret_cast<uintptr_t>(p.Q) & 3))) return false;
   if (((reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.B)) & 15) != 0) return false;
   const uint64_t b_rows = (uint64_t)p.N * (p.swiglu ? 2 : 1);
   if ((uint64_t)p.M * (uint64_t)(p.K / 2) >= (1ull << 32) || b_rows * (uint64_t)(p.K / 2) >= (1ull << 32)) return false;
   const uint64_t tiles = ((uint64_t)(p.M + 31) / 32 + (uint64_t)p.E) * (uint64_t)((p.N + BN / 2 - 1) / (BN / 2));
-  return tiles < (1ull << 30);
+  return tiles * (uint64_t)(p.row_offsets ? 1 : p.slices) < (1ull << 30);
 }
 
 namespace {
@@ -484,7 +575,7 @@ double expected_m_tiles(int E, double rows, int R) {
 // here; there 2.1 - 2.8 per stage and round and 4 - 14 around a tile, more where few tiles share a weight panel or K has a tail
 // (22 experts x 134 rows, 3072 x 12800: 171 us here, 220 there; 25600 x 3072: 310 here, 272 there).
 int mx_stream_rows(const MxArgs& p) {
-  if (!mx_stream_supports(p)) return 0;
+  if (!p.row_offsets || !mx_stream_supports(p)) return 0;
   const double rows = (double)p.M / p.E;
   if (rows <= 18) return 32;
   if (rows <= 44) return 64;
@@ -500,6 +591,93 @@ int mx_stream_rows(const MxArgs& p) {
   const double per_stage = !whole ? 2.8 : (wide ? 2.1 : 2.3), around = whole && wide ? 6.0 : (m_there < 1.3 * p.E ? 14.0 : 4.0);
   const double there = ceil(m_there * n_there / cus) * (stages * per_stage + around);
   return here < there ? 128 : 0;
+}
+
+// The plain GEMM and the fused SwiGLU forms of one matrix of M rows.  The other kernels tile N alone (the weight-streaming kernel: 16
+// weight rows a tile, the fused quantiser whole blocks of 32 outputs; the narrow-tile kernel 128 weight rows), so few weight rows leave
+// compute units idle for the whole of K, and a K that is no multiple of 512 costs the narrow-tile kernel 5 us.  The best of them and
+// of this kernel, K whole or in slices, by a model in microseconds fitted to graph replays of 72 plain shapes (1 .. 256 rows; most
+// within 15 %):
+//  * weight-streaming kernel: 2.3 + rounds x (tiles per workgroup x a + row blocks' b) x K in whole panels of 2048, 1.2 for a K tail;
+//  * narrow-tile kernel: 3 + the larger of 0.40 - 0.47 a stage and the memory time, 5 for a K tail; 256 x 256 tiles 1.65 a stage;
+//  * here: 3.3 + the larger of 0.42 - 0.5 a stage and the memory time, slices' sums 3.5 for the second launch and 7 TB/s there and back;
+//  * memory time: the weights at 7 TB/s and what is read again from L2 at 16 TB/s; a third more where rows do not start at whole
+//    128-byte lines.
+// Measured, before -> after: 128 x 1792 x 16096 52 -> 16 us, 128 x 9216 x 8832 26.8 -> 20.7, 62 x 1792 x 16096 18.5 -> 13.0,
+// 128 x 4096 x 14336 17.8 -> 15.8.
+MxStreamPlan mx_stream_plan(int M, int N, int K, bool swiglu, bool quant, int cus, bool may_split) {
+  MxStreamPlan plan;
+  if (cus <= 0) cus = 256;
+  if (M <= 0 || N <= 0 || K < 2 * BK || K % 32 != 0 || M > 2048 || (swiglu && N % 8 != 0)) return plan;
+  // The plain GEMM of up to 64 rows (above 32: below K = 12288) gives the weight-streaming kernel's bits whether or not the
+  // caller provides a workspace; its slices would save 1 - 3 us of 10 - 16 in places (32 x 5120 x 13824: 15.7 -> 12.8).
+  if (!swiglu && (M <= 32 || (M <= 64 && K < 12288))) return plan;
+  auto ceil_div = [](long a, long b) { return (a + b - 1) / b; };
+  const long rows_b = (long)N * (swiglu ? 2 : 1);
+  const double pitch = K % 256 != 0 ? 1.35 : 1.0, weights = (double)rows_b * K * 0.53;
+  const int stages = (K + BK - 1) / BK, pairs = K / (2 * BK);
+  auto memory = [&](double items, double item_stages, int rows_a) {
+    const double all = items * item_stages * (rows_a + BN) * 136.0;
+    return (weights / 7e6 + (all > weights ? all - weights : 0.0) / 16e6) * pitch;
+  };
+  auto larger = [](double a, double b) { return a > b ? a : b; };
+  // ---- what the other kernels take --------------------------------------------------------------------------------------
+  double other = 1e30;
+  if (M <= (quant ? 32 : 64)) {
+    const int mb = M <= 16 ? 0 : (M <= 32 ? 1 : 2), units = K / 512;
+    const double a[3] = {3.1e-4, 3.5e-4, 4.4e-4}, b[3] = {1.35e-4, 2.8e-4, 5.4e-4};
+    const int tiles = (int)ceil_div(rows_b, 16), t = quant ? tiles_per_workgroup(tiles, cus, 8, 4) : tiles_per_workgroup(tiles, cus, 7);
+    const double panels = units >= 4 ? ceil_div(units, 4) * 2048.0 : units * 512.0;
+    other = 2.3 + ceil_div(ceil_div(tiles, t), cus) * (t * a[mb] + b[mb]) * panels + (K % 512 ? 1.2 : 0.0);
+  }
+  if (M > 32) {
+    const long half = ceil_div(M, 128) * ceil_div(rows_b, 128), full = ceil_div(M, 256) * ceil_div(rows_b, 128);
+    if (full <= cus) {
+      const bool h = M <= 128 || half <= cus;
+      const double per_stage = !h ? 0.85 : (M <= 64 ? 0.40 : 0.47);
+      const double t = 3.0 + larger(stages * per_stage, memory(h ? half : full, stages, h ? (M < 128 ? M : 128) : 256)) + (K % 512 ? 5.0 : 0.0);
+      other = other < t ? other : t;
+    } else {
+      const double t = 3.0 + ceil_div(ceil_div(M, 256) * ceil_div(rows_b, 256), cus) * stages * 1.65 + (K % 512 ? 5.0 : 0.0);
+      other = other < t ? other : t;
+    }
+  }
+  if (may_split && !swiglu) {   // the split that mx_tile_split_plan would take
+    const SplitPlan split = mx_tile_split_plan_for(M, N, K, cus);
+    if (split.slices > 1) {
+      const double per_stage = !split.narrow ? 1.65 : (!split.half ? 0.85 : (M <= 64 ? 0.40 : 0.47));
+      const long tiles = ceil_div(M, split.half ? 128 : 256) * ceil_div(N, split.narrow ? 128 : 256);
+      const double t = 6.0 + larger(2 * split.slice_pairs * per_stage, memory(tiles * split.slices, 2 * split.slice_pairs, split.half ? (M < 128 ? M : 128) : 256)) +
+                       8.0 * split.slices * M * N / 7e6;
+      other = other < t ? other : t;
+    }
+  }
+  // ---- this kernel ----------------------------------------------------------------------------------------------------------
+  double best = other * 0.92;   // (the model is no better than that)
+  for (int rows = 32; rows <= 128; rows *= 2) {
+    if ((rows == 32 && M > 64) || (rows == 128 && M <= 32)) continue;
+    const long tiles = ceil_div(M, rows) * ceil_div(rows_b, BN);
+    const int rows_a = M < rows ? M : rows;
+    const double per_stage = rows == 128 ? 0.50 : 0.42;
+    const double whole = 3.3 + larger(ceil_div(tiles, cus) * stages * per_stage, memory(tiles, stages, rows_a));
+    if (tiles <= cus && M > 32 && whole < best) {
+      best = whole;
+      plan = {rows, 1, 0, 0};
+    }
+    if (!may_split) continue;
+    for (int want = 2; want <= pairs && tiles * want <= cus; ++want) {
+      const int per = (int)ceil_div(pairs, want);
+      if (ceil_div(pairs, per) != want) continue;
+      const double sums = 4.0 * want * M * rows_b;
+      const double item_stages = 2.0 * per + (K % 512) / 256.0;
+      const double t = 6.8 + larger(item_stages * per_stage, memory(tiles * want, item_stages, rows_a)) + 2.0 * sums / 7e6;
+      if (t < best) {
+        best = t;
+        plan = {rows, want, per, (size_t)want * (size_t)M * (size_t)rows_b * sizeof(float)};
+      }
+    }
+  }
+  return plan;
 }
 
 hipError_t launch_mx_stream(const MxArgs& p, int tile_rows, hipStream_t s) {

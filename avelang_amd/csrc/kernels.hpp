@@ -49,6 +49,17 @@ SplitPlan mx_tile_split_plan(int M, int N, int K, size_t max_workspace_bytes = ~
 SplitPlan mx_tile_split_plan_for(int M, int N, int K, int compute_units,
                                  size_t max_workspace_bytes = ~(size_t)0);   // host arithmetic only
 
+// The streaming kernel for the ungrouped MXFP4 GEMM and its fused SwiGLU forms (gemm_mx_stream.hip): rows per tile, 0 where
+// another kernel is the faster one; K in slices of slice_pairs x 512 elements (a K tail with the last one) whose sums take
+// workspace_bytes, when it may be split.
+struct MxStreamPlan {
+  int rows = 0;
+  int slices = 1;
+  int slice_pairs = 0;
+  size_t workspace_bytes = 0;
+};
+MxStreamPlan mx_stream_plan(int M, int N, int K, bool swiglu, bool quant, int compute_units, bool may_split);   // host arithmetic only
+
 // Which NVFP4 kernel shape-based dispatch takes (gemm_nv_narrow.hip); alignment is checked against the pointers afterwards.
 struct NvPlan {
   enum Kernel { kOther, kDecode, kNarrow, kTile, kTileF16 } kernel = kOther;   // kOther: small K, the caller's rules
@@ -106,6 +117,24 @@ inline int tiles_per_workgroup(int n_tiles, int cus, int t_max, int step = 1) {
     }
   }
   return best;
+}
+
+// A plan is a pure function of a shape and costs 1 - 2 us of host arithmetic, a third of a short call: every thread keeps the last
+// plan of each of 64 hash slots (one table per `make`, whose type is a lambda's own).
+template <typename F>
+auto kept_plan(int a, int b, int c, int d, F make) {
+  struct Slot {
+    int key[4] = {-1, -1, -1, -1};
+    decltype(make()) plan;
+  };
+  thread_local Slot slots[64];
+  const unsigned h = ((unsigned)a * 0x9E3779B1u) ^ ((unsigned)b * 0x85EBCA77u) ^ ((unsigned)c * 0xC2B2AE3Du) ^ ((unsigned)d * 0x27D4EB2Fu);
+  Slot& s = slots[(h >> 16) & 63];
+  if (s.key[0] != a || s.key[1] != b || s.key[2] != c || s.key[3] != d) {
+    s.plan = make();
+    s.key[0] = a, s.key[1] = b, s.key[2] = c, s.key[3] = d;
+  }
+  return s.plan;
 }
 
 // Each launcher validates nothing: callers (the C ABI) check shapes and alignment first.

@@ -157,11 +157,11 @@ PyObject* gemm_mxfp4(PyObject* const* arg) {
   if (!g.take(arg, 32, false) || !as_int(arg[5], &variant) || !out.take(arg[4], {g.m, g.n}, at::kBFloat16, g.dev)) NOT_MINE;
   const int split = PyObject_IsTrue(arg[6]);
   if (split < 0) return nullptr;
-  const size_t bytes = variant == AVE_FP4_AUTO && split ? on_device(g.dev, [&] { return ave_fp4_gemm_mxfp4_workspace_bytes(g.m, g.n, g.k); }) : 0;
+  const size_t bytes = variant == AVE_FP4_AUTO && split ? on_device(g.dev, [&] { return ave_fp4_gemm_mxfp4_planned_workspace_bytes(g.m, g.n, g.k); }) : 0;
   Tensor ws;
   if (bytes) ws = empty({(int64_t)bytes}, at::kByte, g.dev);
   const bool ok = launch(g.dev, [&](void* s) {
-    if (bytes) return ave_fp4_gemm_mxfp4_ws(u8(g.a), u8(g.as), u8(g.b), u8(g.bs), ptr_as<uint16_t>(out.t), g.m, g.n, g.k, ptr(ws), bytes, s);
+    if (bytes) return ave_fp4_gemm_mxfp4_planned(u8(g.a), u8(g.as), u8(g.b), u8(g.bs), ptr_as<uint16_t>(out.t), g.m, g.n, g.k, ptr(ws), bytes, s);
     return ave_fp4_gemm_mxfp4_ex(u8(g.a), u8(g.as), u8(g.b), u8(g.bs), ptr_as<uint16_t>(out.t), g.m, g.n, g.k, s, variant);
   });
   return ok ? out.object() : nullptr;
@@ -215,7 +215,11 @@ PyObject* gemm_mxfp4_swiglu(PyObject* const* arg) {
   Out out;
   int variant;
   if (!g.take(arg, 32, false) || g.n % 2 != 0 || !as_int(arg[5], &variant) || !out.take(arg[4], {g.m, g.n / 2}, at::kBFloat16, g.dev)) NOT_MINE;
+  const size_t bytes = variant == AVE_FP4_AUTO ? on_device(g.dev, [&] { return ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(g.m, g.n / 2, g.k, 0); }) : 0;
+  Tensor ws;
+  if (bytes) ws = empty({(int64_t)bytes}, at::kByte, g.dev);
   const bool ok = launch(g.dev, [&](void* s) {
+    if (bytes) return ave_fp4_gemm_mxfp4_swiglu_ws(u8(g.a), u8(g.as), u8(g.b), u8(g.bs), ptr_as<uint16_t>(out.t), g.m, g.n / 2, g.k, ptr(ws), bytes, s);
     return ave_fp4_gemm_mxfp4_swiglu_ex(u8(g.a), u8(g.as), u8(g.b), u8(g.bs), ptr_as<uint16_t>(out.t), g.m, g.n / 2, g.k, s, variant);
   });
   return ok ? out.object() : nullptr;
@@ -240,9 +244,12 @@ PyObject* gemm_mxfp4_swiglu_quant(PyObject* const* arg) {
   Out out, scale;
   int padded;
   if (!g.take(arg, 32, false) || !quantised(arg[4], arg[5], arg[6], g, g.n / 2, &out, &scale, &padded)) NOT_MINE;
+  const size_t bytes = on_device(g.dev, [&] { return ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(g.m, g.n / 2, g.k, 1); });
+  Tensor ws;
+  if (bytes) ws = empty({(int64_t)bytes}, at::kByte, g.dev);
   const bool ok = launch(g.dev, [&](void* s) {
-    return ave_fp4_gemm_mxfp4_swiglu_quant_padded(u8(g.a), u8(g.as), u8(g.b), u8(g.bs), ptr_as<uint8_t>(out.t), ptr_as<uint8_t>(scale.t), g.m,
-                                                  g.n / 2, padded, g.k, s);
+    return ave_fp4_gemm_mxfp4_swiglu_quant_ws(u8(g.a), u8(g.as), u8(g.b), u8(g.bs), ptr_as<uint8_t>(out.t), ptr_as<uint8_t>(scale.t), g.m, g.n / 2,
+                                              padded, g.k, bytes ? ptr(ws) : nullptr, bytes, s);
   });
   return ok ? pair_of(out, scale) : nullptr;
 }

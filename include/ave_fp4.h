@@ -116,6 +116,17 @@ int ave_fp4_gemm_mxfp4_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_
 #define AVE_FP4_NOALLOC_SCRATCH_BYTES (32u << 20)
 int ave_fp4_gemm_mxfp4_noalloc(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                                uint16_t* C, int M, int N, int K, void* hip_stream);
+
+/*
+ * The GEMM as the library would run it when it may use a workspace: ave_fp4_gemm_mxfp4_ws's splits and those of the streaming kernel,
+ * which also cuts K for up to 64 rows and for any K % 32 == 0, whichever a model of the times puts first.
+ * ave_fp4_gemm_mxfp4_planned_workspace_bytes gives the size, 0 where K is not split; the contract is that of
+ * ave_fp4_gemm_mxfp4_ws.
+ */
+size_t ave_fp4_gemm_mxfp4_planned_workspace_bytes(int M, int N, int K);
+int ave_fp4_gemm_mxfp4_planned(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                               uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes, void* hip_stream);
+
 /*
  * MXFP4 gate+up GEMM with the SwiGLU activation fused into the epilogue:
  *   C[m, n] = silu(g) * u,  g = sum_k A[m,k] B[n,k],  u = sum_k A[m,k] B[N+n,k],  silu(x) = x / (1 + exp(-x)),
@@ -144,6 +155,20 @@ int ave_fp4_gemm_mxfp4_swiglu_ex(const uint8_t* A, const uint8_t* A_scale, const
  */
 int ave_fp4_gemm_mxfp4_swiglu_quant(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                                     uint8_t* Q, uint8_t* Q_scale, int M, int N, int K, void* hip_stream);
+
+/*
+ * Both fused forms with a caller-provided workspace (the contract of ave_fp4_gemm_mxfp4_ws): where few weight rows leave compute
+ * units idle, K is cut into slices whose fp32 sums of gate and up values meet in a second launch, which applies the
+ * activation and, in the quantising form, the quantiser.  ave_fp4_gemm_mxfp4_swiglu_workspace_bytes gives the size for either form
+ * (quant = 0 or 1), 0 where K is not split; quantising the result of the one is what the other gives wherever both are
+ * split alike.
+ */
+size_t ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(int M, int N, int K, int quant);
+int ave_fp4_gemm_mxfp4_swiglu_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                 uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes, void* hip_stream);
+int ave_fp4_gemm_mxfp4_swiglu_quant_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                       uint8_t* Q, uint8_t* Q_scale, int M, int N, int N_padded, int K, void* workspace,
+                                       size_t workspace_bytes, void* hip_stream);
 
 /*
  * NVFP4: A_scale [M, K/16] and B_scale [N, K/16] are E4M3 bytes (one per 16

@@ -34,6 +34,12 @@ int ave_fp4_debug_gemm_mxfp4_splitk(const uint8_t* A, const uint8_t* A_scale, co
 int ave_fp4_debug_gemm_nvfp4_narrow(const uint8_t* A, const uint8_t* A_scale, const float* A_global, const uint8_t* B,
                                     const uint8_t* B_scale, const float* B_global, uint16_t* C, int M, int N, int K,
                                     void* workspace, size_t workspace_bytes, int tile_rows, int slice_stages, void* hip_stream);
+/* Diagnostic and test hook: the MXFP4 GEMM on the streaming kernel's tiles of tile_rows (32, 64 or 128) rows, K in slices of
+ * slice_pairs x 512 elements (a K tail goes with the last one) whose partial sums are added up by a second launch; the workspace
+ * must hold ceil(K / 512 / slice_pairs) * M * N * 4 bytes (the quotient K / 512 rounded down). */
+int ave_fp4_debug_gemm_mxfp4_stream_splitk(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                           uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes, int tile_rows,
+                                           int slice_pairs, void* hip_stream);
 /* Diagnostic and test hook: the grouped MXFP4 GEMM on tiles of tile_rows (32, 64 or 128) rows of A by 128 weight rows, whatever the
  * shape (K a multiple of 32 from 512 up, 16-byte aligned A and B).  swiglu: B holds 2N rows per expert; with Q and Q_scale
  * (C null) the result is quantised, rows laid out for N columns. */

@@ -97,6 +97,9 @@ PYBIND11_MODULE(_ave_fp4_bindings, m) {
   AVE_BIND(ave_fp4_gemm_mxfp4_ex);
   AVE_BIND(ave_fp4_gemm_mxfp4_ws);
   AVE_BIND(ave_fp4_gemm_mxfp4_noalloc);
+  AVE_BIND(ave_fp4_gemm_mxfp4_planned);
+  AVE_BIND(ave_fp4_gemm_mxfp4_swiglu_ws);
+  AVE_BIND(ave_fp4_gemm_mxfp4_swiglu_quant_ws);
   AVE_BIND(ave_fp4_gemm_mxfp4_blocked_scales);
   AVE_BIND(ave_fp4_gemm_mxfp4_swiglu);
   AVE_BIND(ave_fp4_gemm_mxfp4_swiglu_ex);
@@ -117,6 +120,8 @@ PYBIND11_MODULE(_ave_fp4_bindings, m) {
   AVE_BIND(ave_fp4_quantize_nvfp4_f32);
   AVE_BIND(ave_fp4_quantize_nvfp4_bf16);
   m.def("ave_fp4_gemm_mxfp4_workspace_bytes", &ave_fp4_gemm_mxfp4_workspace_bytes);
+  m.def("ave_fp4_gemm_mxfp4_planned_workspace_bytes", &ave_fp4_gemm_mxfp4_planned_workspace_bytes);
+  m.def("ave_fp4_gemm_mxfp4_swiglu_workspace_bytes", &ave_fp4_gemm_mxfp4_swiglu_workspace_bytes);
   m.def("ave_fp4_gemm_nvfp4_workspace_bytes", &ave_fp4_gemm_nvfp4_workspace_bytes);
   m.def("ave_fp4_abi_version", &ave_fp4_abi_version);
   m.def("ave_fp4_last_error", []() { return std::string(ave_fp4_last_error()); });

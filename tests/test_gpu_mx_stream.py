@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from avelang_amd import _lib, quantize_mxfp4
+from avelang_amd import _lib, gemm_mxfp4_swiglu_quant_transposed_b, gemm_mxfp4_swiglu_transposed_b, quantize_mxfp4
 from oracle import fp4_oracle as orc
 from tests import helpers as H
 
@@ -62,3 +62,51 @@ def test_stream_walks_a_table_of_more_than_256_experts(gpu):
         c = H.bits(_stream(gpu, ops, torch.from_numpy(ro).to(gpu), n, tile_rows, 0, False))
         for x in np.nonzero(rows)[0]:
             H.assert_mx_close(c[ro[x]:ro[x + 1]], a[ro[x]:ro[x + 1]], a_s[ro[x]:ro[x + 1]], b[x], b_s[x])
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 5, 512), (33, 130, 544), (65, 200, 1248), (128, 300, 2880), (200, 128, 1536)])
+@pytest.mark.parametrize("tile_rows", [32, 64, 128])
+def test_stream_split_k(gpu, m, n, k, tile_rows):
+    """K in slices of one to three pairs of stages, the tail with the last one; unit scales make the sums exact."""
+    rng = np.random.default_rng(m + k)
+    a = rng.integers(0, 256, size=(m, k // 2), dtype=np.uint8)
+    b = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    a_s, b_s = (rng.integers(118, 132, size=(r, k // 32), dtype=np.uint8) for r in (m, n))
+    one_a, one_b = np.full_like(a_s, 127), np.full_like(b_s, 127)
+    exact = orc.f64_to_bf16_bits(orc.gemm_mxfp4_fp64(a, one_a, b, one_b))
+    for slice_pairs in range(1, min(3, k // 512) + 1):
+        slices = -(-(k // 512) // slice_pairs)
+        for sa, sb in ((a_s, b_s), (one_a, one_b)):
+            ws = torch.full((slices * m * n,), float("nan"), dtype=torch.float32, device=gpu)
+            out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu)
+            da, dsa, db, dsb = (H.to_dev(t, gpu) for t in (a, sa, b, sb))
+            _lib.check(_lib.load().ave_fp4_debug_gemm_mxfp4_stream_splitk(
+                da.data_ptr(), dsa.data_ptr(), db.data_ptr(), dsb.data_ptr(), out.data_ptr(), m, n, k, ws.data_ptr(), ws.numel() * 4,
+                tile_rows, slice_pairs, torch.cuda.current_stream(gpu).cuda_stream))
+            torch.cuda.synchronize(gpu)
+            if sa is one_a:
+                assert np.array_equal(H.bits(out), exact)
+            else:
+                H.assert_mx_close(H.bits(out), a, sa, b, sb)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 512, 8192), (20, 1536, 4992), (48, 512, 7168), (100, 256, 3776), (200, 128, 2880)])
+def test_swiglu_forms_on_few_weight_rows(gpu, m, n, k):
+    """Shapes whose K is cut over idle compute units: the fused quantiser gives the quantised bf16 result, within tolerance."""
+    a, a_s = H.mx_operand(m, k, seed=m)
+    b, b_s = H.mx_operand(2 * n, k, seed=n, std=0.05)
+    ops = [H.to_dev(t, gpu) for t in (a, a_s, b, b_s)]
+    with torch.cuda.device(gpu):
+        split = [_lib.load().ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(m, n, k, quant) for quant in (0, 1)]
+    c = gemm_mxfp4_swiglu_transposed_b(*ops)
+    ok, rep = orc.check_swiglu_bf16(H.bits(c), a, a_s, b, b_s)
+    assert ok, rep
+    q, qs = gemm_mxfp4_swiglu_quant_transposed_b(*ops)
+    want_q, want_s = quantize_mxfp4(c)
+    if split[0] == split[1]:
+        assert torch.equal(q, want_q) and torch.equal(qs, want_s)
+    codes, scales = q.cpu().numpy(), qs.cpu().numpy()
+    assert np.mean(codes != want_q.cpu().numpy()) < 1e-3 and np.mean(scales != want_s.cpu().numpy()) < 1e-3
+    padded = gemm_mxfp4_swiglu_quant_transposed_b(*ops, n_pad=n + 64)
+    assert torch.equal(padded[0][:, :n // 2], q) and torch.equal(padded[1][:, :n // 32], qs)
+    assert not padded[0][:, n // 2:].any() and not padded[1][:, n // 32:].any()
