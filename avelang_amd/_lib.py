@@ -32,7 +32,7 @@ try:
 except ImportError as _error:
     native = _NotBuilt(_error)
 
-AUTO, GENERIC, TILE, DECODE, NARROW, TILE_F16, TILE_STREAMED = 0, 1, 2, 3, 4, 5, 6
+AUTO, GENERIC, TILE, DECODE, NARROW, TILE_F16, TILE_STREAMED, SHORT = 0, 1, 2, 3, 4, 5, 6, 7
 
 _vp = ctypes.c_void_p
 _int = ctypes.c_int

@@ -233,6 +233,8 @@ static bool stream_split(ave::MxArgs p, void* workspace, size_t workspace_bytes,
   return true;
 }
 
+static bool short_preferred(int M, int N, int K) { return ave::mx_short_preferred(M, N, K, ave::compute_units()); }
+
 int ave_fp4_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                           uint16_t* C, int M, int N, int K, void* hip_stream, int variant) {
   g_err[0] = 0;
@@ -242,6 +244,7 @@ int ave_fp4_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
   switch (variant) {
     case AVE_FP4_AUTO:
+      if (short_preferred(M, N, K)) return finish(ave::launch_mx_short(p, s), "mxfp4 short-K kernel");
       if (int rc; stream_whole(p, s, &rc)) return rc;
       // (33..64 rows against a nearly full round of 128-row tiles: the narrow-tile kernel ahead of the rings)
       if (M > 32 && M <= 64 && ave::mx_narrow_preferred(p)) return finish(ave::launch_mx_narrow(p, s), "mxfp4 narrow-tile kernel");
@@ -267,6 +270,9 @@ int ave_fp4_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_
     case AVE_FP4_NARROW:
       if (!ave::mx_narrow_supports(p)) return fail_inval("narrow-tile kernel does not support M=%d N=%d K=%d.", M, N, K);
       return finish(ave::launch_mx_narrow(p, s), "mxfp4 narrow-tile kernel");
+    case AVE_FP4_SHORT:
+      if (!ave::mx_short_supports(p)) return fail_inval("short-K kernel does not support M=%d N=%d K=%d.", M, N, K);
+      return finish(ave::launch_mx_short(p, s), "mxfp4 short-K kernel");
     default:
       return fail_inval("unknown kernel variant %d.", variant);
   }
@@ -336,7 +342,7 @@ int ave_fp4_gemm_mxfp4_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_
   if (workspace_bytes > 0 && !workspace) return fail_inval("null workspace with workspace_bytes = %zu.", workspace_bytes);
   if (workspace && !aligned(workspace, 16)) return fail_inval("workspace must be 16-byte aligned.");
   const ave::SplitPlan plan = split_plan(M, N, K);
-  if (plan.slices > 1 && workspace_bytes >= plan.workspace_bytes && aligned(A_scale, 16) && aligned(B_scale, 16))
+  if (!short_preferred(M, N, K) && plan.slices > 1 && workspace_bytes >= plan.workspace_bytes && aligned(A_scale, 16) && aligned(B_scale, 16))
     return gemm_mxfp4_split(A, A_scale, B, B_scale, C, M, N, K, workspace, workspace_bytes, plan, hip_stream);
   return ave_fp4_gemm_mxfp4_ex(A, A_scale, B, B_scale, C, M, N, K, hip_stream, AVE_FP4_AUTO);
 }
@@ -348,6 +354,7 @@ static int check_workspace(const void* workspace, size_t workspace_bytes) {
 }
 
 size_t ave_fp4_gemm_mxfp4_planned_workspace_bytes(int M, int N, int K) {
+  if (short_preferred(M, N, K)) return 0;
   const ave::MxStreamPlan plan = stream_plan(M, N, K, false, false, true);
   return plan.rows ? plan.workspace_bytes : ave_fp4_gemm_mxfp4_workspace_bytes(M, N, K);
 }
@@ -359,7 +366,7 @@ int ave_fp4_gemm_mxfp4_planned(const uint8_t* A, const uint8_t* A_scale, const u
   if (M == 0 || N == 0) return 0;
   if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
   int rc;
-  if (stream_split(ave::MxArgs{A, A_scale, B, B_scale, C, M, N, K, nullptr, 0}, workspace, workspace_bytes, hip_stream, &rc)) return rc;
+  if (!short_preferred(M, N, K) && stream_split(ave::MxArgs{A, A_scale, B, B_scale, C, M, N, K, nullptr, 0}, workspace, workspace_bytes, hip_stream, &rc)) return rc;
   return ave_fp4_gemm_mxfp4_ws(A, A_scale, B, B_scale, C, M, N, K, workspace, workspace_bytes, hip_stream);
 }
 
@@ -371,7 +378,7 @@ int ave_fp4_gemm_mxfp4_noalloc(const uint8_t* A, const uint8_t* A_scale, const u
   // the best split whose partial sums fit the scratch (for nearly every shape the plan of ave_fp4_gemm_mxfp4_ws; a few
   // hundred rows against a K of 30000 and more would want up to twice the scratch and get fewer, longer slices here)
   const ave::SplitPlan plan = ave::mx_tile_split_plan(M, N, K, (size_t)AVE_FP4_NOALLOC_SCRATCH_BYTES);
-  if (plan.slices > 1 && aligned(A_scale, 16) && aligned(B_scale, 16)) {
+  if (!short_preferred(M, N, K) && plan.slices > 1 && aligned(A_scale, 16) && aligned(B_scale, 16)) {
     hipError_t e;
     void* scratch = scratch_pointer(&e);
     if (!scratch) return finish(e, "address of the library's scratch buffer");

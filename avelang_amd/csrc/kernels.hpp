@@ -150,6 +150,7 @@ hipError_t launch_mx_narrow_splitk(const MxArgs& p, hipStream_t s);
 hipError_t launch_splitk_reduce(const float* P, uint16_t* C, size_t mn, int slices, hipStream_t s);
 hipError_t launch_mx_narrow(const MxArgs& p, hipStream_t s);
 hipError_t launch_mx_stream(const MxArgs& p, int tile_rows, hipStream_t s);   // grouped, tiles of 32, 64 or 128 rows by 128 weight rows
+hipError_t launch_mx_short(const MxArgs& p, hipStream_t s);    // small calls, K up to 2048
 hipError_t launch_mx_decode(const MxArgs& p, hipStream_t s);
 hipError_t launch_nv_tile(const NvArgs& p, bool split, hipStream_t s);
 hipError_t launch_nv_f16_tile(const NvArgs& p, hipStream_t s);   // any K % 16 == 0: every element dequantised once per workgroup
@@ -199,6 +200,8 @@ bool mx_tile_blocked_supports(const MxArgs& p);     // p.blocked_scales: the 256
 bool mx_decode_blocked_supports(const MxArgs& p);   // ... the weight-streaming kernel does
 bool mx_narrow_supports(const MxArgs& p);    // the 256 x 128 tile kernel can run the shape
 bool mx_narrow_preferred(const MxArgs& p);   // ... and shape-based dispatch picks it
+bool mx_short_supports(const MxArgs& p);
+bool mx_short_preferred(int M, int N, int K, int compute_units);   // host arithmetic only
 bool mx_stream_supports(const MxArgs& p);
 int mx_stream_rows(const MxArgs& p);         // rows per tile (32, 64, 128) with which shape-based dispatch takes that kernel, or 0
 bool mx_decode_supports(const MxArgs& p);

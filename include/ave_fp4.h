@@ -56,7 +56,7 @@ enum ave_fp4_variant {
                           elements is staged with zeros behind it).  Shape-based dispatch takes it for prefill shapes with
                           K % 64 == 0 and K % 256 != 0, where AVE_FP4_TILE cannot run, and below K = 1024 for K % 256 != 0
                           when C holds more than 1536 blocks of 32 x 32 */
-  AVE_FP4_TILE_STREAMED = 6 /* MXFP4 plain GEMM only: AVE_FP4_TILE with look-ahead touches -- eight K stages before a
+  AVE_FP4_TILE_STREAMED = 6, /* MXFP4 plain GEMM only: AVE_FP4_TILE with look-ahead touches -- eight K stages before a
                           tile's end the workgroups request the weight panels of their next tiles, so that weights
                           which come from HBM (a model's layers, each with weights of its own) are in the last-level
                           cache when their stage loads ask for them; takes effect with K % 512 == 0, 16-byte aligned
@@ -66,6 +66,8 @@ enum ave_fp4_variant {
                           per device, the weight tensors of its latest MXFP4 GEMMs: weights found among the most
                           recent ones that add up to 192 MB at most are taken to be in the 256 MB last-level cache
                           (one GEMM replayed on the same operands) and run as AVE_FP4_TILE, all others as this form */
+  AVE_FP4_SHORT = 7    /* MXFP4 plain GEMM only: 32x32 blocks of C, one wave each up to K = 512 and four waves that share K up
+                          to 2048, operands straight into registers; for small calls */
 };
 
 /*
