@@ -73,6 +73,21 @@ __device__ inline void load_scale_rows(const uint8_t* from, unsigned to) {
       : "m0", "memory");
 }
 
+// dma16 for the lanes of `lanes` only (with no lane left it counts on vmcnt all the same)
+__device__ inline void dma16_lanes(const void* gbase, unsigned voff, unsigned lds_addr, unsigned long long lanes) {
+  unsigned long long saved;
+  asm volatile(
+      "s_mov_b32 m0, %[to]\n\t"
+      "s_mov_b64 %[sv], exec\n\t"
+      "s_mov_b64 exec, %[mask]\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %[off], %[base]\n\t"
+      "s_mov_b64 exec, %[sv]\n\t"
+      : [sv] "=&s"(saved)
+      : [to] "s"(__builtin_amdgcn_readfirstlane(lds_addr)), [mask] "s"(lanes), [off] "v"(voff), [base] "s"(gbase)
+      : "m0", "memory");
+}
+
 // a pointer that is the same in every lane, in scalar registers
 __device__ inline const uint8_t* uniform(const uint8_t* p) {
   const uint64_t v = reinterpret_cast<uint64_t>(p);
@@ -83,11 +98,19 @@ __device__ inline const uint8_t* uniform(const uint8_t* p) {
 // GROUPED: the rows of A belong to p.E experts (p.row_offsets) with weights of their own; otherwise one matrix of p.M rows.
 // SPLITK (plain form, not grouped): a work item is a tile and a slice of p.slice_pairs pairs of stages (the last one what is left, the
 // K tail with it); its fp32 sums go to p.P[slice][M][N].
-template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK>
+// SHIFT: rows that do not all start at a cache line.  A stage cut at the row's start then touches two lines of 128 bytes per row and
+// half of what the load path moves is thrown away (5760 x 2880, 16 rows of each of 128 experts: 255 us, with K = 2816 instead 203).
+// So a ring buffer holds one LINE per row -- line j of a row that starts 16 sh bytes behind a line boundary is its chunks
+// 8 j - sh .. + 7 -- and a stage is read from two buffers: chunk c of stage s lies in line s where c + sh < 8 and in line s + 1
+// otherwise (a "late" chunk), in either case in the slot that it has without SHIFT, so that reads stay free of bank conflicts.  Stage s waits for line
+// s + 1, one stage earlier than without; a tile whose last stage has late chunks takes one line more.  Chunks of a line that are not the
+// row's are not loaded.  Measured: 255 -> 220 us, with 2880 weight rows 131 -> 112.
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
 __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, int n_tiles) {
   using G = Geo<R>;
   static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
   static_assert(!SPLITK || (!SWIGLU && !GROUPED), "K is split for the plain GEMM");
+  static_assert(!SHIFT || GROUPED, "by lines: the experts' weights only");
   constexpr int kTileN = SWIGLU ? BN / 2 : BN;   // output columns per tile
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x;
@@ -98,6 +121,11 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
   const int stages = (p.K + BK - 1) / BK;
   const int tail_blocks = (p.K % BK) / 32;             // blocks of 32 in the last stage, 0: it is a whole one
   const int pair_tail = (p.K % (2 * BK)) / 32;         // scale bytes in the last pair, 0: all 16
+  // SHIFT: rows start at multiples of `unit` chunks behind a line boundary; row r of a matrix at chunk (base + r * row16) % 8
+  const unsigned row16 = row_bytes / 16, a16 = (unsigned)(reinterpret_cast<uintptr_t>(p.A) >> 4), b16 = (unsigned)(reinterpret_cast<uintptr_t>(p.B) >> 4);
+  const unsigned bits16 = row16 | a16 | b16 | 8;
+  const int unit = (int)(bits16 & (0u - bits16));
+  const bool late_at_end = SHIFT && (tail_blocks != 0 ? tail_blocks : 8) > unit;   // the last stage of K has late chunks in some row
 
   // Lane l keeps {first m-tile, m-tiles, first row, end row} (clamped to [0, M]) of experts l, l + 64, l + 128 and l + 192;
   // with more than 256 experts the caller's table is walked for every tile.
@@ -193,15 +221,18 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
     const int wi = w - G::kMulWaves;
     unsigned a_off[G::kALoads], b_off[4];
     int a_chunk[G::kALoads], b_chunk[4];
+    unsigned a_late = 0, b_late = 0;   // SHIFT: bit i: this lane's chunk of load i is a late one
     const uint8_t *ga = nullptr, *gb = nullptr, *gs = nullptr;
-    int s = s_last;            // stage of the tile that goes out next
+    int s = 0, s_end = 0;      // stage (SHIFT: line) of the tile that goes out next, and the one behind its last
     unsigned to = lds_base, slot_to = lds_base + G::kScaleBase;
     unsigned with_scales = 0;  // bit i: the stage issued i stages ago brought a pair of scale rows
     int issued = 0;
     auto issue = [&]() {       // false: nothing left
-      if (s == s_last) {
+      if (s == s_end) {
         if (!next_tile()) return false;
         s = s_first;
+        s_end = s_last + (late_at_end ? 1 : 0);
+        a_late = b_late = 0;
         const int lr = lane >> 3, cprime = lane & 7;
 #pragma unroll
         for (int i = 0; i < G::kALoads; ++i) {
@@ -210,23 +241,33 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
           am = am < m_end ? am : m_end - 1;
           a_chunk[i] = cprime ^ ((row >> 1) & 7);
           a_off[i] = (unsigned)am * row_bytes + (unsigned)a_chunk[i] * 16;
+          if (SHIFT) {
+            if (a_chunk[i] + (int)((a16 + (unsigned)am * row16) & 7) >= 8) a_late |= 1u << i;
+            else a_off[i] += kRowBytes;
+          }
         }
         const size_t expert_rows = (size_t)expert * (SWIGLU ? 2 : 1) * p.N;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int row = (wi * 4 + i) * 8 + lr;
           b_chunk[i] = cprime ^ ((row >> 1) & 7);
-          b_off[i] = (unsigned)b_image_row(row) * row_bytes + (unsigned)b_chunk[i] * 16;
+          const unsigned bn = (unsigned)b_image_row(row);
+          b_off[i] = bn * row_bytes + (unsigned)b_chunk[i] * 16;
+          if (SHIFT) {
+            if (b_chunk[i] + (int)((b16 + ((unsigned)expert_rows + bn) * row16) & 7) >= 8) b_late |= 1u << i;
+            else b_off[i] += kRowBytes;
+          }
         }
-        ga = p.A + (size_t)s * kRowBytes;
-        gb = p.B + expert_rows * row_bytes + (size_t)s * kRowBytes;
+        // (SHIFT: a late chunk is that of the stage before; the offsets are from one stage in front of line s)
+        ga = p.A + (size_t)s * kRowBytes - (SHIFT ? kRowBytes : 0);
+        gb = p.B + expert_rows * row_bytes + (size_t)s * kRowBytes - (SHIFT ? kRowBytes : 0);
         const int sr = wi * G::kScaleLanes + (lane < G::kScaleLanes ? lane : 0);
         int am = m_begin + sr;
         am = am < m_end ? am : m_end - 1;
         gs = sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
         gs += (size_t)(s >> 1) * 16;
       }
-      if (tail_blocks != 0 && s == stages - 1) {   // chunks behind the row's end: its last chunk again
+      if (!SHIFT && tail_blocks != 0 && s == stages - 1) {   // chunks behind the row's end: its last chunk again
 #pragma unroll
         for (int i = 0; i < G::kALoads; ++i)
           if (a_chunk[i] >= tail_blocks) a_off[i] -= (unsigned)(a_chunk[i] - (tail_blocks - 1)) * 16;
@@ -234,7 +275,7 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
         for (int i = 0; i < 4; ++i)
           if (b_chunk[i] >= tail_blocks) b_off[i] -= (unsigned)(b_chunk[i] - (tail_blocks - 1)) * 16;
       }
-      const bool scales = (s & 1) == 0;
+      const bool scales = (s & 1) == 0 && (!SHIFT || s < s_last);
       if (scales) {
         if (pair_tail != 0 && s + 2 >= stages) gs -= 16 - pair_tail;   // (K >= 512: there are 16 bytes in front of the row's end)
         load_scale_rows<G::kScaleLanes>(gs, __builtin_amdgcn_readfirstlane(slot_to) + (unsigned)wi * (G::kScaleLanes * 16));
@@ -242,10 +283,21 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
         slot_to = slot_to + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot_to + G::kSlot;
       }
       with_scales = (with_scales << 1) | (scales ? 1u : 0u);
+      if (SHIFT && (s == 0 || s >= stages - 1)) {   // a line with chunks that are not the row's: these lanes stay out
+        auto mine = [&](unsigned late, int i, int chunk) {
+          const int at = 8 * s + chunk - (late >> i & 1 ? 8 : 0);
+          return __ballot(at >= 0 && at < (int)row_scales);
+        };
 #pragma unroll
-      for (int i = 0; i < G::kALoads; ++i) dma16(uniform(ga), a_off[i], to + (unsigned)(wi * G::kALoads + i) * 1024);
+        for (int i = 0; i < G::kALoads; ++i) dma16_lanes(uniform(ga), a_off[i], to + (unsigned)(wi * G::kALoads + i) * 1024, mine(a_late, i, a_chunk[i]));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) dma16(uniform(gb), b_off[i], to + G::kOffB + (unsigned)(wi * 4 + i) * 1024);
+        for (int i = 0; i < 4; ++i) dma16_lanes(uniform(gb), b_off[i], to + G::kOffB + (unsigned)(wi * 4 + i) * 1024, mine(b_late, i, b_chunk[i]));
+      } else {
+#pragma unroll
+        for (int i = 0; i < G::kALoads; ++i) dma16(uniform(ga), a_off[i], to + (unsigned)(wi * G::kALoads + i) * 1024);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dma16(uniform(gb), b_off[i], to + G::kOffB + (unsigned)(wi * 4 + i) * 1024);
+      }
       ga += kRowBytes;
       gb += kRowBytes;
       to = to + G::kStage == lds_base + G::kScaleBase ? lds_base : to + G::kStage;
@@ -256,14 +308,16 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
     bool more = true;
     for (int i = 0; i < G::kRing - 1 && more; ++i) more = issue();
     for (int j = 0; j < issued; ++j) {
-      // Stage j has landed when only the loads of the stages behind it are outstanding: `ahead` of them, each kData loads
-      // and one more for those that brought scale rows (fewer than there are is safe, and waits a little longer).
-      const int ahead = __builtin_amdgcn_readfirstlane(issued - 1 - j);
-      if (ahead >= G::kRing - 2) {
-        const int c = __popc(__builtin_amdgcn_readfirstlane((int)(with_scales & ((1u << (G::kRing - 2)) - 1))));
-        if (c >= 3) wait_vm<(G::kRing - 2) * G::kData + 3>();
-        else if (c == 2) wait_vm<(G::kRing - 2) * G::kData + 2>();
-        else wait_vm<(G::kRing - 2) * G::kData + 1>();   // every two stages in a row hold the first stage of a pair
+      // Stage j (SHIFT: line j + 1) has landed when only the loads of the stages behind it are outstanding: `ahead` of them, each kData
+      // loads and one more for those that brought scale rows (fewer than there are is safe, and waits a little longer).
+      constexpr int kAhead = G::kRing - 2 - (SHIFT ? 1 : 0);   // (while there is more to issue)
+      const int ahead = __builtin_amdgcn_readfirstlane(issued - 1 - (SHIFT ? 1 : 0) - j);
+      if (ahead >= kAhead) {
+        const int c = __popc(__builtin_amdgcn_readfirstlane((int)(with_scales & ((1u << kAhead) - 1))));
+        if (c >= 3) wait_vm<kAhead * G::kData + 3>();
+        else if (c == 2) wait_vm<kAhead * G::kData + 2>();
+        else if (!SHIFT || c == 1) wait_vm<kAhead * G::kData + 1>();   // (not SHIFT: every two stages in a row hold the first stage of a pair)
+        else wait_vm<kAhead * G::kData>();
       } else if (ahead == 4) {
         wait_vm<4 * G::kData>();
       } else if (ahead == 3) {
@@ -291,7 +345,27 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
   const unsigned b_frag = (unsigned)(G::kOffB + b_row * kRowBytes + (((4 * h) ^ ((b_row >> 1) & 7)) * 16));
   const unsigned a_sc = (unsigned)a_row * 16, b_sc = (unsigned)(R + b_row) * 16;   // in a slot, + 512 per 32 rows
   unsigned sb = lds_base, slot = lds_base + G::kLds - G::kSlot;
+  auto next_buffer = [&]() { sb = sb + G::kStage == lds_base + G::kScaleBase ? lds_base : sb + G::kStage; };
   while (next_tile()) {
+    // SHIFT: bit c: chunk c of the fragment row is a late one
+    unsigned a_late[MI] = {}, b_late[2] = {};
+    if (SHIFT) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        int am = m_begin + a_row + 32 * i;
+        am = am < m_end ? am : m_end - 1;
+        a_late[i] = 0xFF00u >> ((a16 + (unsigned)am * row16) & 7);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        b_late[i] = 0xFF00u >> ((b16 + ((unsigned)expert * (SWIGLU ? 2 : 1) * (unsigned)p.N + (unsigned)b_image_row(b_row + 32 * i)) * row16) & 7);
+    }
+    // where a fragment row's chunk `chunk` lies, from the buffer of its stage
+    auto late = [&](unsigned mask, int chunk) {
+      if (!SHIFT) return 0u;
+      const unsigned to_next = sb + G::kStage == lds_base + G::kScaleBase ? lds_base - sb : (unsigned)G::kStage;
+      return (0u - (mask >> chunk & 1)) & to_next;
+    };
     v16f acc[2][MI];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -310,23 +384,29 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
 #pragma unroll
       for (int kj = 0; kj < 4; ++kj) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) af[kj][i] = lds_read16(sb + (a_frag ^ ((unsigned)kj * 16)) + i * 4096);
+        for (int i = 0; i < MI; ++i) af[kj][i] = lds_read16(sb + late(a_late[i], 4 * h + kj) + (a_frag ^ ((unsigned)kj * 16)) + i * 4096);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) bf[kj][i] = lds_read16(sb + (b_frag ^ ((unsigned)kj * 16)) + i * 4096);
+        for (int i = 0; i < 2; ++i) bf[kj][i] = lds_read16(sb + late(b_late[i], 4 * h + kj) + (b_frag ^ ((unsigned)kj * 16)) + i * 4096);
       }
       __builtin_amdgcn_sched_barrier(0);
     };
     // stages of whole pairs end here
     const int whole = pair_tail == 0 || s_last < stages ? s_last : (stages - 1) & ~1;
     auto next_slot = [&]() { slot = slot + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot + G::kSlot; };
-    auto next_buffer = [&]() { sb = sb + G::kStage == lds_base + G::kScaleBase ? lds_base : sb + G::kStage; };
     int s = s_first;
+    auto behind_the_last_stage = [&]() {
+      if (late_at_end) {
+        __syncthreads();
+        next_buffer();
+      }
+    };
     if (G::kWM > 1 && m_begin + m_wave >= m_end) {   // no rows for this wave: the barriers and the positions, nothing else
       for (; s < s_last; ++s) {
         __syncthreads();
         if ((s & 1) == 0) next_slot();
         next_buffer();
       }
+      behind_the_last_stage();
       continue;
     }
     for (; s < whole; ++s) {
@@ -367,14 +447,14 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
         const v4i none = {0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-          const v4i f = lds_read16(sb + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
+          const v4i f = lds_read16(sb + late(a_late[i], block) + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
           const int sc = lds_read1(at + a_sc + i * 512);
           af[j][i] = have ? f : none;
           as_cur[i] = have ? sc : 0x7f;
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          const v4i f = lds_read16(sb + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
+          const v4i f = lds_read16(sb + late(b_late[i], block) + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
           const int sc = lds_read1(at + b_sc + i * 512);
           bf[j][i] = have ? f : none;
           bs_cur[i] = have ? sc : 0x7f;
@@ -386,6 +466,7 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
       }
       next_buffer();
     }
+    behind_the_last_stage();
 
     if constexpr (SWIGLU) {
       // acc[0][mi] holds the gate and acc[1][mi] the up values of row m_begin + m_wave + 32 mi + c, outputs n_begin + 32 wn + 16 piece + 8 q
@@ -454,19 +535,41 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
   }
 }
 
-template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK>
-hipError_t launch(const MxArgs& p, hipStream_t s) {
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
+hipError_t launch_rows(const MxArgs& p, hipStream_t s) {
   constexpr int kTileN = SWIGLU ? BN / 2 : BN;
   const int n_tiles = (p.N + kTileN - 1) / kTileN;
   const int cus = compute_units();
   if (cus <= 0) return hipErrorInvalidDevice;
-  constexpr auto kernel = mx_stream_kernel<R, SWIGLU, QUANT, GROUPED, SPLITK>;
+  constexpr auto kernel = mx_stream_kernel<R, SWIGLU, QUANT, GROUPED, SPLITK, SHIFT>;
   if (hipError_t e = allow_dynamic_lds<kernel>(Geo<R>::kLds); e != hipSuccess) return e;
   // grouped: upper bound of the experts' tile lists
   const long tiles = ((long)(p.M + R - 1) / R + (GROUPED ? p.E : 0)) * n_tiles * (SPLITK ? p.slices : 1);
   hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < cus ? tiles : cus)), dim3(Geo<R>::kThreads), Geo<R>::kLds, s, p, n_tiles);
   return hipGetLastError();
 }
+// SHIFT for experts' weights whose rows do not all start at a cache line, from HBM and over a few lines: the start of a tile costs it
+// more, and where a launch is short or its weights are in the last-level cache the lines that it saves do not bound it.  Measured on
+// weights beyond that cache (200 experts x 8 and x 40 rows, 4096 weight rows; 78 x 4, 21504; 120 x 100, 8192), without against with: K = 544 and 800 0.83 - 1.06,
+// 1056 1.03 - 1.13, 1120 and 1184 (five stages and a line more) 0.94 - 1.08, 1312 - 1696 1.02 - 1.18, 2080 - 4256 1.10 - 1.21.  One
+// matrix (1 - 300 rows): 0.87 - 1.04, so not there.
+template <bool SWIGLU>
+bool by_lines(const MxArgs& p) {
+  if (p.K <= 4 * BK && !p.by_lines) return false;
+  const uint64_t row = (uint64_t)p.K / 2, b_rows = (uint64_t)p.N * (SWIGLU ? 2 : 1);
+  const uint64_t at = (reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.B) | row) & (kRowBytes - 1);
+  if (at == 0 || ((uint64_t)p.E * b_rows * row < (64u << 20) && !p.by_lines)) return false;
+  const uint64_t unit = at & (0 - at), tail = row % kRowBytes != 0 ? row % kRowBytes : kRowBytes;
+  if (tail > unit && p.K <= 5 * BK && !p.by_lines) return false;
+  return (uint64_t)p.M * row + 256 < (1ull << 32) && b_rows * row + 256 < (1ull << 32);   // room for the 128 bytes on top of an offset
+}
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK>
+hipError_t launch(const MxArgs& p, hipStream_t s) {
+  if constexpr (GROUPED)
+    if (by_lines<SWIGLU>(p)) return launch_rows<R, SWIGLU, QUANT, GROUPED, SPLITK, true>(p, s);
+  return launch_rows<R, SWIGLU, QUANT, GROUPED, SPLITK, false>(p, s);
+}
+
 // silu(gate) * up of K slices' sums P[slices][M][2N] (N gate columns, then N up columns), added up in slice order: bf16 into C, or
 // (QUANT) quantised to MXFP4 with the stand-alone quantiser's steps on the bf16 values.  A lane owns 8 outputs of one row, so a block
 // of 32 is four neighbouring lanes (N % 32 == 0: blocks never leave a row).  Bound by the sums' way through the memory system.

@@ -49,6 +49,33 @@ def test_stream_matches_oracle_and_its_own_fused_forms(gpu, rows, n, k, tile_row
     assert torch.equal(q, want_q) and torch.equal(qs, want_s)
 
 
+# every offset of a row from its line (K / 32 mod 8), last stages that end in front of, at and behind a line's end, two to nine stages
+@pytest.mark.parametrize("rows,n,k", [([3, 0, 31, 33], 64, 544), ([1, 64], 32, 576), ([64, 65, 0, 127], 96, 736), ([129, 5], 160, 768),
+                                      ([32, 200, 1, 70], 128, 800), ([40, 130, 0, 300], 192, 992), ([17] * 20, 352, 1184),
+                                      ([2] * 70, 64, 1312), ([66, 0, 140], 224, 2208), ([5] * 40 + [90], 96, 1056)])
+@pytest.mark.parametrize("tile_rows", [32, 64, 128])
+@pytest.mark.parametrize("off", [0, 16, 80])
+def test_stream_by_lines_gives_the_same_bits(gpu, rows, n, k, tile_rows, off):
+    """Rows loaded by whole cache lines: the same sums in the same order; `off`: operands that start 16 bytes behind each other's lines."""
+    e, m = len(rows), sum(rows)
+    ro = torch.from_numpy(np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)).to(gpu)
+    rng = np.random.default_rng(k + off)
+
+    def behind(shape, at):
+        t = torch.empty(int(np.prod(shape)) + at, dtype=torch.uint8, device=gpu)
+        t[at:] = torch.from_numpy(rng.integers(0, 256, size=int(np.prod(shape)), dtype=np.uint8)).to(gpu)
+        return t[at:].reshape(shape)
+
+    a, b = behind((m, k // 2), off), behind((e, 2 * n, k // 2), 2 * off)
+    a_s, b_s = (torch.from_numpy(rng.integers(118, 132, size=s, dtype=np.uint8)).to(gpu) for s in ((m, k // 32), (e, 2 * n, k // 32)))
+    ops = (a, a_s, b, b_s)
+    for cols, swiglu, quant in ((2 * n, 0, False), (n, 1, False), (n, 1, True)):
+        want = _stream(gpu, ops, ro, cols, tile_rows, swiglu, quant)
+        got = _stream(gpu, ops, ro, cols, tile_rows | 0x1000, swiglu, quant)
+        for x, y in zip(want, got) if quant else ((want, got),):
+            assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
+
+
 def test_stream_walks_a_table_of_more_than_256_experts(gpu):
     n, k, e = 64, 736, 300
     rows = np.zeros(e, dtype=np.int64)
