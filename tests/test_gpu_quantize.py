@@ -197,3 +197,32 @@ def test_quantisers_mark_blocks_with_non_finite_values(gpu, dtype):
     assert (want_s == 0x7F).sum() == 9 + 16
     assert np.array_equal(s.cpu().numpy(), want_s)
     assert np.array_equal(_canon(p.cpu().numpy()), _canon(want_p))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows, k, k_pad", [
+    (1, 32, None), (7, 224, None), (3, 4064, None),          # one block; a last workgroup that is nearly empty
+    (5, 224, 512),                                           # padded rows
+    (2048, 4096, None), (2049, 4096, None),                  # fp32: the two sides of 32 MB
+    (4097, 4096, None),                                      # bf16: above 32 MB, a last workgroup of one row's end
+    (8193, 2080, 2560),                                      # above 32 MB with padded rows
+])
+def test_quantise_mx_sizes_bit_for_bit(gpu, dtype, rows, k, k_pad):
+    """Every form of the kernel (chosen by the size of the input) against the oracle on the first, middle and last row and, bit
+    for bit, against calls on a fifth of the rows."""
+    g = torch.Generator(device=gpu).manual_seed(rows + k)
+    x = (torch.randn((rows, k), generator=g, device=gpu) * torch.exp2(torch.randint(-8, 9, (rows, k // 32), generator=g, device=gpu)
+                                                                      .float()).repeat_interleave(32, 1)).to(dtype)
+    x[-1, -1] = float("inf")
+    x[0, :32] = 0
+    p, s = quantize_mxfp4(x, k_pad=k_pad)
+    picked = sorted({0, rows // 2, rows - 1})
+    want_p, want_s = orc.quantize_mxfp4(x[picked].float().cpu().numpy())
+    assert np.array_equal(s[picked, : k // 32].cpu().numpy(), want_s)
+    assert np.array_equal(_canon(p[picked, : k // 2].cpu().numpy()), _canon(want_p))
+    if k_pad:
+        assert int(p[:, k // 2:].max()) == 0 and bool((s[:, k // 32:] == 127).all())
+    step = max(1, rows // 5)
+    for r in range(0, rows, step):
+        hp, hs = quantize_mxfp4(x[r:r + step], k_pad=k_pad)
+        assert torch.equal(hp, p[r:r + step]) and torch.equal(hs, s[r:r + step])
