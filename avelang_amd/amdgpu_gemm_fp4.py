@@ -235,8 +235,9 @@ def gemm_mxfp4_swiglu_transposed_b(A, A_scale, B, B_scale, out=None, *, variant:
 
 def gemm_mxfp4_swiglu_quant_transposed_b(A, A_scale, B, B_scale, out=None, out_scale=None, *, n_pad=None):
     """Gate+up GEMM, SwiGLU and the MXFP4 quantiser of the next GEMM's activations in one launch: returns
-    ``(codes, scales)``, uint8 ``[M, N/2]`` and ``[M, N/32]``, bit-identical to
-    ``quantize_mxfp4`` applied to the bf16 result of :func:`gemm_mxfp4_swiglu_transposed_b`.  ``N % 32 == 0``;
+    ``(codes, scales)``, uint8 ``[M, N/2]`` and ``[M, N/32]``: ``quantize_mxfp4`` applied to the bf16 result of
+    :func:`gemm_mxfp4_swiglu_transposed_b`, bit for bit above 64 rows and wherever both add K up in the same order; up to 64 rows
+    each call picks its own kernel and its own slices of K, and a sum may round the other way.  ``N % 32 == 0``;
     needs ``K`` to be a multiple of 32 from 512 up (the LDS-staged kernels; multiples of 512 are fastest) and raises
     ``ValueError`` otherwise.  ``n_pad`` (a multiple of 32, at least N): the rows of both results are laid out for
     ``n_pad`` columns, for a consumer that runs over a padded K (see :func:`quantize_mxfp4`); the columns from N on are
@@ -319,7 +320,8 @@ def grouped_gemm_mxfp4_transposed_b(A, A_scale, B, B_scale, row_offsets, out=Non
 def grouped_gemm_mxfp4_swiglu_transposed_b(A, A_scale, B, B_scale, row_offsets, out=None):
     """Grouped (MoE) gate+up GEMM with SwiGLU in one launch: ``B`` ``[E, 2N, K/2]`` holds, per expert, the ``N`` gate
     rows followed by the ``N`` up rows; rows ``row_offsets[e]:row_offsets[e+1]`` of ``A`` use ``B[e]``.  Returns bf16
-    ``[total_M, N]``, every expert's rows equal to :func:`gemm_mxfp4_swiglu_transposed_b` on that expert alone."""
+    ``[total_M, N]``, every expert's rows those of :func:`gemm_mxfp4_swiglu_transposed_b` on that expert alone, bit for bit
+    where that call does not cut K into slices (or run on the weight-streaming kernel, up to 64 rows)."""
     done = _native.grouped_gemm_mxfp4_swiglu(A, A_scale, B, B_scale, row_offsets, out)
     if done is not None:
         return done

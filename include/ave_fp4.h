@@ -120,8 +120,8 @@ int ave_fp4_gemm_mxfp4_noalloc(const uint8_t* A, const uint8_t* A_scale, const u
                                uint16_t* C, int M, int N, int K, void* hip_stream);
 
 /*
- * The GEMM as the library would run it when it may use a workspace: ave_fp4_gemm_mxfp4_ws's splits and those of the streaming kernel,
- * which also cuts K for up to 64 rows and for any K % 32 == 0, whichever a model of the times puts first.
+ * The GEMM as the library would run it when it may use a workspace: ave_fp4_gemm_mxfp4_ws's splits and those of the streaming kernel
+ * (more than 64 rows, or 33 - 64 from K = 12288; any K % 32 == 0), whichever a model of the times puts first.
  * ave_fp4_gemm_mxfp4_planned_workspace_bytes gives the size, 0 where K is not split; the contract is that of
  * ave_fp4_gemm_mxfp4_ws.
  */
@@ -163,7 +163,7 @@ int ave_fp4_gemm_mxfp4_swiglu_quant(const uint8_t* A, const uint8_t* A_scale, co
  * units idle, K is cut into slices whose fp32 sums of gate and up values meet in a second launch, which applies the
  * activation and, in the quantising form, the quantiser.  ave_fp4_gemm_mxfp4_swiglu_workspace_bytes gives the size for either form
  * (quant = 0 or 1), 0 where K is not split; quantising the result of the one is what the other gives wherever both are
- * split alike.
+ * split alike: always above 64 rows, up to there often only the quantising form is split.
  */
 size_t ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(int M, int N, int K, int quant);
 int ave_fp4_gemm_mxfp4_swiglu_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
