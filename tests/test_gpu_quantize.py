@@ -226,3 +226,24 @@ def test_quantise_mx_sizes_bit_for_bit(gpu, dtype, rows, k, k_pad):
     for r in range(0, rows, step):
         hp, hs = quantize_mxfp4(x[r:r + step], k_pad=k_pad)
         assert torch.equal(hp, p[r:r + step]) and torch.equal(hs, s[r:r + step])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows, k", [(1, 16), (3, 4080), (4096, 4096), (4097, 4112)])   # bf16: 4096 x 4096 is 32 MB, the largest not streamed
+def test_quantise_nv_sizes_bit_for_bit(gpu, dtype, rows, k):
+    """Every form of the kernel against the oracle on the first, middle and last row and, bit for bit, against calls on a
+    fifth of the rows."""
+    g = torch.Generator(device=gpu).manual_seed(rows + k)
+    x = torch.randn((rows, k), generator=g, device=gpu).to(dtype)
+    x[-1, -1] = float("nan")
+    x[0, :16] = 0
+    scale = torch.tensor([0.002], device=gpu)
+    p, s = quantize_nvfp4(x, scale)
+    picked = sorted({0, rows // 2, rows - 1})
+    want_p, want_s = orc.quantize_nvfp4_fp32(x[picked].float().cpu().numpy(), np.float32(scale.item()))[:2]
+    assert np.array_equal(s[picked].cpu().numpy(), want_s)
+    assert np.array_equal(_canon(p[picked].cpu().numpy()), _canon(want_p))
+    step = max(1, rows // 5)
+    for r in range(0, rows, step):
+        hp, hs = quantize_nvfp4(x[r:r + step], scale)
+        assert torch.equal(hp, p[r:r + step]) and torch.equal(hs, s[r:r + step])
