@@ -115,6 +115,8 @@ hipError_t launch(const void* x, uint8_t* packed, uint8_t* scales, size_t rows, 
   if constexpr (sizeof(T) == 4)
     return streamed ? launch_form<T, 4, 2, true>(x, packed, scales, n_blocks, k, k_padded, s)
                     : launch_form<T, 8, 1, false>(x, packed, scales, n_blocks, k, k_padded, s);
+  else if (n_blocks <= (1u << 15))   // a decode batch (1 M elements): one piece a lane keeps twice the compute units busy, 2.7 us against 2.8
+    return launch_form<T, 8, 1, false>(x, packed, scales, n_blocks, k, k_padded, s);
   else
     return streamed ? launch_form<T, 8, 2, true>(x, packed, scales, n_blocks, k, k_padded, s)
                     : launch_form<T, 8, 2, false>(x, packed, scales, n_blocks, k, k_padded, s);

@@ -113,6 +113,7 @@ template <typename T>
 hipError_t launch(const void* x, const float* g, uint8_t* packed, uint8_t* scales, size_t n_blocks, hipStream_t s) {
   if (n_blocks == 0) return hipSuccess;
   if constexpr (sizeof(T) == 4) return launch_form<T, 1, false>(x, g, packed, scales, n_blocks, s);
+  else if (n_blocks <= (1u << 16)) return launch_form<T, 1, false>(x, g, packed, scales, n_blocks, s);   // 1 M elements: all units busy
   else   // streamed above the 32 MB that the L2s hold together
     return n_blocks * 32 > (32u << 20) ? launch_form<T, 2, true>(x, g, packed, scales, n_blocks, s)
                                        : launch_form<T, 2, false>(x, g, packed, scales, n_blocks, s);
