@@ -66,12 +66,15 @@ struct Choice {
   float v;
   int e;   // -1: none
 };
-__device__ inline bool ranks_before(const Choice& a, const Choice& b) {   // among equal scores the lower expert index
+// Among equal scores the lower expert index; no order over NaN, which must not become a choice's v.
+__device__ inline bool ranks_before(const Choice& a, const Choice& b) {
   return a.e >= 0 && (b.e < 0 || a.v > b.v || (a.v == b.v && a.e < b.e));
 }
 
 // The choices of `n` tokens (at most 256) from token `t0` on, into pair[] and, when wanted, prob[] (both LDS):
-// highest and second-highest logit and their probabilities in the full softmax.  The softmax denominator is added up in
+// highest and second-highest logit and their probabilities in the full softmax.  A NaN never hides the finite logits: the
+// choices are those of a scan over the experts that starts with experts 0 and 1 and replaces a choice only by a greater
+// score -- a NaN of expert 0 stays the first choice, one of expert 1 the second behind expert 0, any other is passed over.  The softmax denominator is added up in
 // double: a float sum of E terms drifts by about sqrt(E) roundings, which for 200 and more experts is more than the
 // 2e-6 relative error the probabilities are stated to keep.  Its terms come from v_exp_f32: x exp(-x) 2^-24, what the
 // rounded product costs, is below 3e-8 for every x; the second choice's own probability takes expf.
@@ -89,7 +92,8 @@ __device__ inline void choose_block(const RouteArgs& p, int t0, int n, bool want
 #pragma unroll
     for (int j = 0; j < kRouteValues; ++j) {   // selects, no branches
       const int e = j * L + sub;
-      const Choice c{x[j], e < p.E ? e : -1};
+      const bool nan = x[j] != x[j];
+      const Choice c{nan ? __builtin_inff() : x[j], e < p.E && (!nan || e == 0) ? e : -1};
       const bool better = ranks_before(c, first), next = ranks_before(c, second);
       second.v = better ? first.v : (next ? c.v : second.v);
       second.e = better ? first.e : (next ? c.e : second.e);
@@ -105,6 +109,8 @@ __device__ inline void choose_block(const RouteArgs& p, int t0, int n, bool want
       first = better ? f : first;
       second = ranks_before(lost, own) ? lost : own;
     }
+    const float x1 = L == 1 ? x[1] : __shfl(x[0], (threadIdx.x & 63 & ~(L - 1)) + 1, 64);   // of expert 1
+    if (first.e == 0 && x1 != x1) second = {x1, 1};
     if (want_prob) {
       const float top = __shfl(first.v, threadIdx.x & 63 & ~(L - 1), 64);
       double sum = 0.0;

@@ -93,6 +93,41 @@ def test_route_top2_no_tokens_and_validation(gpu):
         moe_route_top2(torch.zeros((4, 8), device=gpu), row_offsets=torch.zeros(8, dtype=torch.int32, device=gpu))
 
 
+def _scan_top2(row):
+    """Experts 0 and 1, replaced only by a greater score: what routing does with a NaN among the logits."""
+    first, second = 0, None
+    for e in range(1, len(row)):
+        if row[e] > row[first]:
+            first, second = e, first
+        elif second is None or row[e] > row[second]:
+            second = e
+    return first, second
+
+
+@pytest.mark.parametrize("t,e", [(40, 2), (300, 8), (64, 9), (500, 64), (70, 200), (33000, 16)])
+def test_route_top2_nan_does_not_hide_finite_logits(gpu, t, e):
+    """One or several NaNs at every place of a row (a lane's first logit among them): the choices of a plain scan, in the
+    one-workgroup form, through the workspace and without it."""
+    logits = orc.randn((t, e), t + e)
+    for i in range(0, t, 2):
+        logits[i, i // 2 % e] = np.nan
+    logits[3::10, : e // 2] = np.nan
+    logits[5 % t] = np.nan
+    top = np.array([_scan_top2(r) for r in logits])
+    order = np.argsort(top.reshape(-1), kind="stable")
+    want_tok, want_off = (order // 2).astype(np.int32), np.concatenate([[0], np.cumsum(np.bincount(top.reshape(-1), minlength=e))])
+    dev = torch.from_numpy(logits).to(gpu)
+    tok, off, w = moe_route_top2(dev)
+    tok2, off2 = torch.zeros_like(tok), torch.zeros_like(off)
+    _lib.check(_lib.load().ave_fp4_moe_route_top2(dev.data_ptr(), t, e, tok2.data_ptr(), off2.data_ptr(), None,
+                                                  torch.cuda.current_stream(gpu).cuda_stream))
+    torch.cuda.synchronize()
+    for x, y in ((tok, off), (tok2, off2)):
+        assert np.array_equal(y.cpu().numpy(), want_off) and np.array_equal(x.cpu().numpy(), want_tok)
+    has_nan = np.isnan(logits).any(axis=1)
+    assert np.array_equal(np.isnan(w.cpu().numpy()), has_nan[want_tok])
+
+
 @pytest.mark.parametrize("rows,src,k", [(64, 16, 4096), (37, 9, 512), (50, 20, 128), (33, 7, 32), (20, 5, 96),
                                         (4096, 1000, 1024)])
 def test_gather_rows_equals_oracle(gpu, rows, src, k):
