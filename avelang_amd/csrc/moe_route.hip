@@ -116,7 +116,8 @@ __device__ inline void choose_block(const RouteArgs& p, int t0, int n, bool want
       double sum = 0.0;
 #pragma unroll
       for (int j = 0; j < kRouteValues; ++j)
-        sum += j * L + sub < p.E ? (double)__builtin_amdgcn_exp2f(1.4426950408889634f * (x[j] - top)) : 0.0;
+        if (j * L + sub < p.E)   // (the first choice's own term is 1 also where it is an infinity)
+          sum += j * L + sub == first.e && x[j] == x[j] ? 1.0 : (double)__builtin_amdgcn_exp2f(1.4426950408889634f * (x[j] - top));
       for (int d = 1; d < L; d <<= 1) sum += __shfl_xor(sum, d, 64);
       if (sub == 0) prob[i] = v2f{(float)(1.0 / sum), (float)((double)expf(second.v - first.v) / sum)};
     }

@@ -128,6 +128,22 @@ def test_route_top2_nan_does_not_hide_finite_logits(gpu, t, e):
     assert np.array_equal(np.isnan(w.cpu().numpy()), has_nan[want_tok])
 
 
+@pytest.mark.parametrize("t,e", [(50, 2), (300, 8), (500, 64), (70, 200)])
+def test_route_top2_infinite_logits(gpu, t, e):
+    """An infinite score has probability 1 and its companion 0; experts at minus infinity are never taken before others
+    and add nothing to the denominator."""
+    logits = orc.randn((t, e), t + e)
+    masked = np.zeros_like(logits, dtype=bool)
+    masked[1::3, 1:-1] = e > 2
+    logits[masked] = -np.inf
+    best = np.arange(0, t, 3)
+    logits[best, best % e] = np.inf
+    want_tok, want_off, want_w = orc.route_top2(np.where(np.isposinf(logits), 1e4, logits))   # exp(-1e4) is 0 in float and in double
+    tok, off, w = _route(gpu, logits)
+    assert np.array_equal(off, want_off) and np.array_equal(tok, want_tok)
+    assert np.allclose(w, want_w, rtol=2e-6, atol=1e-30)
+
+
 @pytest.mark.parametrize("rows,src,k", [(64, 16, 4096), (37, 9, 512), (50, 20, 128), (33, 7, 32), (20, 5, 96),
                                         (4096, 1000, 1024)])
 def test_gather_rows_equals_oracle(gpu, rows, src, k):
