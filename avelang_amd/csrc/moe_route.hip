@@ -74,10 +74,11 @@ __device__ inline bool ranks_before(const Choice& a, const Choice& b) {
 // The choices of `n` tokens (at most 256) from token `t0` on, into pair[] and, when wanted, prob[] (both LDS):
 // highest and second-highest logit and their probabilities in the full softmax.  A NaN never hides the finite logits: the
 // choices are those of a scan over the experts that starts with experts 0 and 1 and replaces a choice only by a greater
-// score -- a NaN of expert 0 stays the first choice, one of expert 1 the second behind expert 0, any other is passed over.  The softmax denominator is added up in
-// double: a float sum of E terms drifts by about sqrt(E) roundings, which for 200 and more experts is more than the
-// 2e-6 relative error the probabilities are stated to keep.  Its terms come from v_exp_f32: x exp(-x) 2^-24, what the
-// rounded product costs, is below 3e-8 for every x; the second choice's own probability takes expf.
+// score -- a NaN of expert 0 stays the first choice, one of expert 1 the second behind expert 0, any other is passed over.
+// The softmax denominator is added up in double: a float sum of E terms drifts by about sqrt(E) roundings, which for 200 and more experts is more than the
+// 2e-6 relative error the probabilities are stated to keep.  Its terms take expf: v_exp_f32 on x log2(e) is off by
+// |x| 2^-24 where that product is rounded, which shows in the sum of 64 and more (rms error of the probabilities, 64 .. 256
+// experts: 3.4 - 3.6e-8, with expf 3.0e-8), and the kernel waits for memory either way.
 __device__ inline void choose_block(const RouteArgs& p, int t0, int n, bool want_prob, unsigned* pair, v2f* prob) {
   const int L = 1 << p.lanes_log2, sub = threadIdx.x & (L - 1);
   for (int i = threadIdx.x >> p.lanes_log2; i < n; i += kRouteThreads >> p.lanes_log2) {
@@ -115,9 +116,10 @@ __device__ inline void choose_block(const RouteArgs& p, int t0, int n, bool want
       const float top = __shfl(first.v, threadIdx.x & 63 & ~(L - 1), 64);
       double sum = 0.0;
 #pragma unroll
-      for (int j = 0; j < kRouteValues; ++j)
-        if (j * L + sub < p.E)   // (the first choice's own term is 1 also where it is an infinity)
-          sum += j * L + sub == first.e && x[j] == x[j] ? 1.0 : (double)__builtin_amdgcn_exp2f(1.4426950408889634f * (x[j] - top));
+      for (int j = 0; j < kRouteValues; ++j) {   // (the first choice's own term is 1 also where it is an infinity)
+        const float d = j * L + sub == first.e && x[j] == x[j] ? 0.f : x[j] - top;
+        sum += (double)expf(j * L + sub < p.E ? d : -__builtin_inff());
+      }
       for (int d = 1; d < L; d <<= 1) sum += __shfl_xor(sum, d, 64);
       if (sub == 0) prob[i] = v2f{(float)(1.0 / sum), (float)((double)expf(second.v - first.v) / sum)};
     }

@@ -144,6 +144,17 @@ def test_route_top2_infinite_logits(gpu, t, e):
     assert np.allclose(w, want_w, rtol=2e-6, atol=1e-30)
 
 
+@pytest.mark.parametrize("e", [64, 128, 256])
+def test_route_top2_probabilities_keep_float_accuracy(gpu, e):
+    """Rounding the result to float costs 2.5e-8 (rms, relative: 2^-24 sqrt(E[1/m^2] / 3) for mantissas m spread evenly in the
+    logarithm), an exponential that is right to one unit 1 - 2e-8 beside it: 3.25e-8 at most together."""
+    logits = orc.randn((40000, e), e, 3.0)
+    want_tok, _, want_w = orc.route_top2(logits)
+    tok, _, w = _route(gpu, logits)
+    assert np.array_equal(tok, want_tok)
+    assert np.sqrt(np.mean((w / want_w - 1.0) ** 2)) < 3.25e-8
+
+
 @pytest.mark.parametrize("rows,src,k", [(64, 16, 4096), (37, 9, 512), (50, 20, 128), (33, 7, 32), (20, 5, 96),
                                         (4096, 1000, 1024)])
 def test_gather_rows_equals_oracle(gpu, rows, src, k):
