@@ -308,11 +308,11 @@ int ave_fp4_moe_route_top2_ex(const float* logits, int tokens, int E, int32_t* t
 
 /*
  * The same routing with a caller-provided device workspace (16-byte aligned, no initialisation needed, garbage
- * afterwards): the tokens' choices and the counts of every 128 or 256 tokens are passed through it from one launch to a
- * second, so that the logits are read once.  ave_fp4_moe_route_top2_workspace_bytes gives its size, 0 where a single
- * workgroup does all the work; with a smaller (or null) workspace the call is ave_fp4_moe_route_top2_ex, which goes
- * through the logits once per eighth of the tokens.  Same integer outputs; calls that may overlap need workspaces of
- * their own.
+ * afterwards): the tokens' choices and the counts of every chunk of tokens (32 and more, by E and the number of tokens) are passed
+ * through it from one launch to a second, so that the logits are read once.  ave_fp4_moe_route_top2_workspace_bytes gives
+ * its size, 0 where a single workgroup does all the work; with a smaller (or null) workspace the call is
+ * ave_fp4_moe_route_top2_ex, every workgroup of which goes through all logits (16384 tokens: 21 us against 8.4 with 8 experts,
+ * 280 against 13 with 128).  Same results; calls that may overlap need workspaces of their own.
  */
 size_t ave_fp4_moe_route_top2_workspace_bytes(int tokens, int E);
 int ave_fp4_moe_route_top2_ws(const float* logits, int tokens, int E, int32_t* token_of_row, int32_t* row_offsets,

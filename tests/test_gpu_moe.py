@@ -155,6 +155,34 @@ def test_route_top2_probabilities_keep_float_accuracy(gpu, e):
     assert np.sqrt(np.mean((w / want_w - 1.0) ** 2)) < 3.25e-8
 
 
+@pytest.mark.parametrize("t,e,times", [(16384, 8, 6), (16384, 128, 40), (131072, 8, 25)])
+def test_route_top2_without_a_workspace_stays_within_reach_of_the_one_with(gpu, t, e, times):
+    """Every workgroup of the single launch goes through all tokens; what it does for a token has to be little (measured: 2.5, 22
+    and 11 times the two launches through a workspace; a loop with barriers and atomics per 256 tokens was 20, 69 and 100)."""
+    logits = torch.randn(t, e, device=gpu)
+    tok, w = torch.empty(2 * t, dtype=torch.int32, device=gpu), torch.empty(2 * t, device=gpu)
+    off, inv = torch.empty(e + 1, dtype=torch.int32, device=gpu), torch.empty(t, 2, dtype=torch.int32, device=gpu)
+    lib = _lib.load()
+
+    def best(call):
+        call()
+        us = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                call()
+            b.record()
+            b.synchronize()
+            us.append(a.elapsed_time(b) * 100)
+        return min(us)
+
+    with_ws = best(lambda: moe_route_top2(logits, tok, off, w, inv))
+    without = best(lambda: _lib.check(lib.ave_fp4_moe_route_top2_ex(logits.data_ptr(), t, e, tok.data_ptr(), off.data_ptr(), w.data_ptr(),
+                                                                    inv.data_ptr(), torch.cuda.current_stream(gpu).cuda_stream)))
+    assert without < times * with_ws, (without, with_ws)
+
+
 @pytest.mark.parametrize("rows,src,k", [(64, 16, 4096), (37, 9, 512), (50, 20, 128), (33, 7, 32), (20, 5, 96),
                                         (4096, 1000, 1024)])
 def test_gather_rows_equals_oracle(gpu, rows, src, k):
@@ -328,3 +356,28 @@ def test_whole_expert_layer_with_swiglu_and_combine_in_one_graph(gpu):
     torch.cuda.synchronize()
     assert torch.equal(out, replayed)
     assert not torch.equal(replayed, eager)
+
+
+@pytest.mark.parametrize("t,e", [(257, 8), (512, 8), (513, 8), (512, 16), (513, 16), (1025, 6), (5000, 32), (3001, 33), (2100, 250),
+                                 (270000, 2)])
+def test_route_top2_counts_of_all_tokens(gpu, t, e):
+    """The entry without a workspace around one workgroup's tokens, with one and several lanes per token, experts that fill no group of
+    four, and more trips than a byte counts (270000 tokens): the integers and probabilities of the one with a workspace."""
+    logits = orc.randn((t, e), t + e)
+    logits[::7, : max(1, e - 1)] = 0.25          # ties
+    logits[5::11, 1:] = -np.inf                  # one logit above minus infinity
+    logits[8::13] = -np.inf
+    logits[9::17, e // 2] = np.nan
+    dev = torch.from_numpy(logits).to(gpu)
+    inv = torch.full((t, 2), -7, dtype=torch.int32, device=gpu)
+    want = (*moe_route_top2(dev, rows_of_token=inv), inv)
+    got = [torch.zeros_like(x) for x in want]
+    _lib.check(_lib.load().ave_fp4_moe_route_top2_ex(dev.data_ptr(), t, e, *(x.data_ptr() for x in got),
+                                                     torch.cuda.current_stream(gpu).cuda_stream))
+    torch.cuda.synchronize()
+    for x, y in zip(got, want):
+        assert torch.equal(x.view(torch.int32), y.view(torch.int32))
+    if t < 2000:
+        top = np.array([_scan_top2(r) for r in logits])
+        order = np.argsort(top.reshape(-1), kind="stable")
+        assert np.array_equal(got[0].cpu().numpy(), order // 2)
