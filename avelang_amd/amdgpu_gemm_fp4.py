@@ -234,10 +234,10 @@ def gemm_mxfp4_swiglu_transposed_b(A, A_scale, B, B_scale, out=None, *, variant:
 
 
 def gemm_mxfp4_swiglu_quant_transposed_b(A, A_scale, B, B_scale, out=None, out_scale=None, *, n_pad=None):
-    """Gate+up GEMM, SwiGLU and the MXFP4 quantiser of the next GEMM's activations in one launch: returns
+    """Gate+up GEMM, SwiGLU and the MXFP4 quantiser of the next GEMM's activations in one call: returns
     ``(codes, scales)``, uint8 ``[M, N/2]`` and ``[M, N/32]``: ``quantize_mxfp4`` applied to the bf16 result of
-    :func:`gemm_mxfp4_swiglu_transposed_b`, bit for bit above 64 rows and wherever both add K up in the same order; up to 64 rows
-    each call picks its own kernel and its own slices of K, and a sum may round the other way.  ``N % 32 == 0``;
+    :func:`gemm_mxfp4_swiglu_transposed_b`, bit for bit up to 32 rows and above 64; from 33 to 64 rows each call picks its own
+    kernel and its own slices of K, and a sum may round the other way.  ``N % 32 == 0``;
     needs ``K`` to be a multiple of 32 from 512 up (the LDS-staged kernels; multiples of 512 are fastest) and raises
     ``ValueError`` otherwise.  ``n_pad`` (a multiple of 32, at least N): the rows of both results are laid out for
     ``n_pad`` columns, for a consumer that runs over a padded K (see :func:`quantize_mxfp4`); the columns from N on are

@@ -233,6 +233,21 @@ static bool stream_split(ave::MxArgs p, void* workspace, size_t workspace_bytes,
   return true;
 }
 
+// SwiGLU and quantiser of a few rows in two launches, the bf16 result in the workspace, where that is planned.
+static size_t in_two_bytes(int M, int N, int K) {
+  return ave::mx_swiglu_quant_in_two(M, N, K, ave::compute_units()) ? (size_t)M * (size_t)N * sizeof(uint16_t) : 0;
+}
+static bool swiglu_quant_in_two(const ave::MxArgs& p, void* workspace, size_t workspace_bytes, hipStream_t s, int* rc) {
+  if (p.M > 32 || workspace_bytes < (size_t)p.M * (size_t)p.N * sizeof(uint16_t) || in_two_bytes(p.M, p.N, p.K) == 0) return false;
+  if (ave::q_row_cols(p) != p.N) return false;   // (the quantiser would write a padded row's end)
+  const ave::MxArgs h{p.A, p.As, p.B, p.Bs, static_cast<uint16_t*>(workspace), p.M, p.N, p.K, nullptr, 0, 1};
+  if (!ave::mx_decode_swiglu_supports(h)) return false;
+  hipError_t e = ave::launch_mx_decode(h, s);
+  if (e == hipSuccess) e = ave::launch_quantize_mx(workspace, 1, p.Q, p.Qs, (size_t)p.M, p.N, p.N, s);
+  *rc = finish(e, "mxfp4 swiglu decode kernel and quantiser");
+  return true;
+}
+
 static bool short_preferred(int M, int N, int K) { return ave::mx_short_preferred(M, N, K, ave::compute_units()); }
 
 int ave_fp4_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
@@ -628,7 +643,8 @@ int ave_fp4_gemm_mxfp4_swiglu_quant_padded(const uint8_t* A, const uint8_t* A_sc
 }
 
 size_t ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(int M, int N, int K, int quant) {
-  return stream_plan(M, N, K, true, quant != 0, true).workspace_bytes;
+  const size_t slices = stream_plan(M, N, K, true, quant != 0, true).workspace_bytes;
+  return slices == 0 && quant != 0 ? in_two_bytes(M, N, K) : slices;
 }
 
 int ave_fp4_gemm_mxfp4_swiglu_quant_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
@@ -649,6 +665,7 @@ int ave_fp4_gemm_mxfp4_swiglu_quant_ws(const uint8_t* A, const uint8_t* A_scale,
   p.q_n = N_padded;
   if (int rc; stream_split(p, workspace, workspace_bytes, hip_stream, &rc)) return rc;
   if (int rc; stream_whole(p, hip_stream, &rc)) return rc;
+  if (int rc; swiglu_quant_in_two(p, workspace, workspace_bytes, static_cast<hipStream_t>(hip_stream), &rc)) return rc;
   if (ave::mx_decode_swiglu_quant_supports(p))
     return finish(ave::launch_mx_decode(p, static_cast<hipStream_t>(hip_stream)), "mxfp4 swiglu + quantise decode kernel");
   if (ave::mx_narrow_preferred(p))

@@ -696,6 +696,29 @@ int mx_stream_rows(const MxArgs& p) {
   return here < there ? 128 : 0;
 }
 
+namespace {
+// The weight-streaming kernel's time in microseconds for `rows_b` weight rows (see mx_stream_plan); its fused quantiser takes whole
+// blocks of 32 outputs, four tiles, to a workgroup.
+double ring_us(int M, long rows_b, int K, bool quant, int cus) {
+  auto ceil_div = [](long a, long b) { return (a + b - 1) / b; };
+  const int mb = M <= 16 ? 0 : (M <= 32 ? 1 : 2), units = K / 512;
+  const double a[3] = {3.1e-4, 3.5e-4, 4.4e-4}, b[3] = {1.35e-4, 2.8e-4, 5.4e-4};
+  const int tiles = (int)ceil_div(rows_b, 16), t = quant ? tiles_per_workgroup(tiles, cus, 8, 4) : tiles_per_workgroup(tiles, cus, 7);
+  const double panels = units >= 4 ? ceil_div(units, 4) * 2048.0 : units * 512.0;
+  return 2.3 + ceil_div(ceil_div(tiles, t), cus) * (t * a[mb] + b[mb]) * panels + (K % 512 ? 1.2 : 0.0);
+}
+}  // namespace
+
+// SwiGLU and quantiser of up to 32 rows as two launches, the bf16 form and the quantiser: where the fused quantiser's four tiles a
+// workgroup leave most compute units idle.  The second launch takes 1.6 - 2.2 us; the model is good to about one.  Fused -> two
+// launches: 1 x 512 x 8192 11.0 -> 6.8 us, 20 x 1536 x 5184 12.4 -> 9.0, 2 x 3072 x 7424 16.4 -> 13.1; kept fused: 4 x 4608 x 7680
+// (14.6, two launches 15.1), 32 x 4096 x 4096 (9.7, 10.4), 16 x 1024 x 1024 (4.6, 5.2).
+bool mx_swiglu_quant_in_two(int M, int N, int K, int cus) {
+  if (cus <= 0) cus = 256;
+  if (M <= 0 || M > 32 || N <= 0 || N % 32 != 0 || K < 2 * BK || K % 32 != 0) return false;
+  return ring_us(M, 2L * N, K, true, cus) > ring_us(M, 2L * N, K, false, cus) + 3.0;
+}
+
 // The plain GEMM and the fused SwiGLU forms of one matrix of M rows.  The other kernels tile N alone (the weight-streaming kernel: 16
 // weight rows a tile, the fused quantiser whole blocks of 32 outputs; the narrow-tile kernel 128 weight rows), so few weight rows leave
 // compute units idle for the whole of K, and a K that is no multiple of 512 costs the narrow-tile kernel 5 us.  The best of them and
@@ -726,13 +749,9 @@ MxStreamPlan mx_stream_plan(int M, int N, int K, bool swiglu, bool quant, int cu
   auto larger = [](double a, double b) { return a > b ? a : b; };
   // ---- what the other kernels take --------------------------------------------------------------------------------------
   double other = 1e30;
-  if (M <= (quant ? 32 : 64)) {
-    const int mb = M <= 16 ? 0 : (M <= 32 ? 1 : 2), units = K / 512;
-    const double a[3] = {3.1e-4, 3.5e-4, 4.4e-4}, b[3] = {1.35e-4, 2.8e-4, 5.4e-4};
-    const int tiles = (int)ceil_div(rows_b, 16), t = quant ? tiles_per_workgroup(tiles, cus, 8, 4) : tiles_per_workgroup(tiles, cus, 7);
-    const double panels = units >= 4 ? ceil_div(units, 4) * 2048.0 : units * 512.0;
-    other = 2.3 + ceil_div(ceil_div(tiles, t), cus) * (t * a[mb] + b[mb]) * panels + (K % 512 ? 1.2 : 0.0);
-  }
+  // Up to 32 rows both fused forms cut K alike (or not at all), so that quantising the one's result is the other, bit for bit: the
+  // plan is that of the bf16 form.  Above, the weight-streaming kernel has no quantiser.
+  if (M <= (quant ? 32 : 64)) other = ring_us(M, rows_b, K, false, cus);
   if (M > 32) {
     const long half = ceil_div(M, 128) * ceil_div(rows_b, 128), full = ceil_div(M, 256) * ceil_div(rows_b, 128);
     if (full <= cus) {

@@ -60,6 +60,8 @@ struct MxStreamPlan {
   size_t workspace_bytes = 0;
 };
 MxStreamPlan mx_stream_plan(int M, int N, int K, bool swiglu, bool quant, int compute_units, bool may_split);   // host arithmetic only
+// Up to 32 rows, one matrix, no split planned: the SwiGLU form's bf16 result and the quantiser as two launches are the faster ones.
+bool mx_swiglu_quant_in_two(int M, int N, int K, int compute_units);   // host arithmetic only
 
 // Which NVFP4 kernel shape-based dispatch takes (gemm_nv_narrow.hip); alignment is checked against the pointers afterwards.
 struct NvPlan {

@@ -148,8 +148,9 @@ int ave_fp4_gemm_mxfp4_swiglu_ex(const uint8_t* A, const uint8_t* A_scale, const
 /*
  * The same gate+up GEMM and SwiGLU, with the MXFP4 quantiser of the next GEMM's activations fused behind it:
  * the fp32 result is rounded to bf16 and quantised per 32 consecutive n exactly as ave_fp4_quantize_mxfp4_bf16
- * would quantise the bf16 output of ave_fp4_gemm_mxfp4_swiglu (bit-identical codes and scales), without that
- * output ever being written.  Q [M, N/2] packed E2M1 (16-byte aligned), Q_scale [M, N/32] E8M0; N % 32 == 0.
+ * would quantise the bf16 output of ave_fp4_gemm_mxfp4_swiglu, without that output ever being written: codes and scales
+ * are bit-identical up to 32 rows and above 64; from 33 to 64 rows each call picks its own kernel, and a sum may round the other
+ * way.  Q [M, N/2] packed E2M1 (16-byte aligned), Q_scale [M, N/32] E8M0; N % 32 == 0.
  * Up to 32 rows run on the weight-streaming kernel (K a multiple of 32 from 512 up, 16-byte aligned operands), everything
  * else on the LDS-staged kernels: K % 512 == 0 with 16-byte-aligned scale tensors, or any other multiple of
  * 32 from 512 up with 16-byte-aligned A and B; else AVE_FP4_EINVAL (use the two calls then).  No counterpart in the reference, whose kernel ends at the bf16 store
@@ -161,9 +162,10 @@ int ave_fp4_gemm_mxfp4_swiglu_quant(const uint8_t* A, const uint8_t* A_scale, co
 /*
  * Both fused forms with a caller-provided workspace (the contract of ave_fp4_gemm_mxfp4_ws): where few weight rows leave compute
  * units idle, K is cut into slices whose fp32 sums of gate and up values meet in a second launch, which applies the
- * activation and, in the quantising form, the quantiser.  ave_fp4_gemm_mxfp4_swiglu_workspace_bytes gives the size for either form
- * (quant = 0 or 1), 0 where K is not split; quantising the result of the one is what the other gives wherever both are
- * split alike: always above 64 rows, up to there often only the quantising form is split.
+ * activation and, in the quantising form, the quantiser.  Up to 32 rows the quantising form without row padding may also run as two
+ * launches, the bf16 form into the workspace and the quantiser.  ave_fp4_gemm_mxfp4_swiglu_workspace_bytes gives the size for
+ * either form (quant = 0 or 1), 0 where none is used.  Quantising the result of the one form is what the other gives, bit for bit, up to
+ * 32 rows and above 64, both called with their workspace (C 16-byte aligned) or both without.
  */
 size_t ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(int M, int N, int K, int quant);
 int ave_fp4_gemm_mxfp4_swiglu_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,

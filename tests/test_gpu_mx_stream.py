@@ -137,3 +137,19 @@ def test_swiglu_forms_on_few_weight_rows(gpu, m, n, k):
     padded = gemm_mxfp4_swiglu_quant_transposed_b(*ops, n_pad=n + 64)
     assert torch.equal(padded[0][:, :n // 2], q) and torch.equal(padded[1][:, :n // 32], qs)
     assert not padded[0][:, n // 2:].any() and not padded[1][:, n // 32:].any()
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 512, 8192), (3, 1024, 2816), (4, 1408, 5376), (8, 1024, 7680), (18, 1536, 3584), (25, 3936, 6912),
+                                   (32, 64, 2080), (16, 1024, 1024), (65, 512, 4096), (130, 256, 7200)])
+def test_swiglu_quant_is_the_quantised_swiglu_result(gpu, m, n, k):
+    """Up to 32 rows and above 64 the fused quantiser's codes and scales are those of the two calls, bit for bit, whatever the forms do
+    about compute units that few weight rows leave idle; with padded rows as well."""
+    a, a_s = H.mx_operand(m, k, seed=m + n)
+    b, b_s = H.mx_operand(2 * n, k, seed=n + k, std=0.05)
+    ops = [H.to_dev(t, gpu) for t in (a, a_s, b, b_s)]
+    want_q, want_s = quantize_mxfp4(gemm_mxfp4_swiglu_transposed_b(*ops))
+    q, qs = gemm_mxfp4_swiglu_quant_transposed_b(*ops)
+    assert torch.equal(q, want_q) and torch.equal(qs, want_s)
+    q, qs = gemm_mxfp4_swiglu_quant_transposed_b(*ops, n_pad=n + 96)
+    assert torch.equal(q[:, :n // 2], want_q) and torch.equal(qs[:, :n // 32], want_s)
+    assert not q[:, n // 2:].any() and not qs[:, n // 32:].any()
