@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 import torch  # noqa: F401  (its libraries are what the extension below links against)
 
@@ -16,8 +17,8 @@ _lib = None
 
 
 class _NotBuilt:
-    """Stands in for the extension where it has not been built: nothing is done in C++, the wrappers go through their own
-    checks, and :func:`load` then says what is missing."""
+    """Stands in for the extension where it cannot be imported (not built, or built against another torch): nothing is done in
+    C++ and every call goes through its wrapper and ctypes, with the same kernels; :func:`load` says once what is missing."""
 
     def __init__(self, error):
         self.error = error
@@ -125,8 +126,9 @@ def load() -> ctypes.CDLL:
             "(or __graft_entry__.build()); there is no fallback path."
         )
     if isinstance(native, _NotBuilt):
-        raise RuntimeError("avelang_amd._torch_calls is not built (or not for this torch): build it with `make -C avelang_amd/csrc` "
-                           "(or __graft_entry__.build())") from native.error
+        warnings.warn(f"avelang_amd._torch_calls cannot be imported ({native.error}): calls take about 10 us more on the host; "
+                      "build it for this torch with `make -C avelang_amd/csrc` (or __graft_entry__.build())", RuntimeWarning,
+                      stacklevel=2)
     lib = ctypes.CDLL(path)
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)  # AttributeError if the library lacks a declared symbol

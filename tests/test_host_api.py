@@ -43,6 +43,31 @@ def test_library_exports_every_declared_symbol():
     assert lib.ave_fp4_abi_version() == 1
 
 
+def test_library_loads_without_the_extension_on_torch_tensors():
+    """The entry points in C++ save host time only: where they cannot be imported the ctypes binding serves every call."""
+    import subprocess
+    import sys
+    code = """
+import sys, warnings
+sys.modules["avelang_amd._torch_calls"] = None      # what an extension built against another torch looks like: ImportError
+import torch
+from avelang_amd import _lib, gemm_mxfp4_transposed_b
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    assert _lib.load().ave_fp4_abi_version() == 1
+    assert _lib.load().ave_fp4_gemm_mxfp4(None, None, None, None, None, 4, 4, 33, None) == -1
+assert [w.category for w in seen] == [RuntimeWarning] and "_torch_calls cannot be imported" in str(seen[0].message)
+try:
+    gemm_mxfp4_transposed_b(*[torch.zeros(4, 8, dtype=torch.uint8)] * 4)
+except ValueError as e:
+    assert "K must be a multiple of 32" in str(e)
+else:
+    raise AssertionError("the wrapper's checks did not run")
+"""
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr
+
+
 def test_plain_c_caller_links_against_declared_symbols_only():
     """The C program the GPU tests run is built with the library and imports nothing the header lacks."""
     import subprocess
