@@ -577,6 +577,7 @@ template <bool QUANT>
 __global__ __launch_bounds__(256) void reduce_swiglu_kernel(MxArgs p) {
   const unsigned per_row = (unsigned)p.N / 8;
   const size_t lanes = (size_t)p.M * per_row, step = (size_t)p.M * 2 * p.N;
+  const bool vec_ok = (reinterpret_cast<uintptr_t>(p.C) & 15) == 0;   // (N % 8 == 0)
   for (size_t g = (size_t)blockIdx.x * 256 + threadIdx.x; g < lanes; g += (size_t)gridDim.x * 256) {
     const size_t m = g / per_row;
     const unsigned n = (unsigned)(g % per_row) * 8;
@@ -597,7 +598,13 @@ __global__ __launch_bounds__(256) void reduce_swiglu_kernel(MxArgs p) {
     for (int e = 0; e < 8; ++e) hv[e] = silu(gate[e >> 2][e & 3]) * up[e >> 2][e & 3];
     const v4i o = {(int)pack_bf16x2(hv[0], hv[1]), (int)pack_bf16x2(hv[2], hv[3]), (int)pack_bf16x2(hv[4], hv[5]), (int)pack_bf16x2(hv[6], hv[7])};
     if constexpr (!QUANT) {
-      *reinterpret_cast<v4i*>(p.C + m * p.N + n) = o;
+      uint16_t* c = p.C + m * p.N + n;
+      if (vec_ok) {
+        *reinterpret_cast<v4i*>(c) = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[e] = (uint16_t)(((unsigned)o[e >> 1] >> (16 * (e & 1))) & 0xFFFF);
+      }
     } else {
       float v[8];
 #pragma unroll

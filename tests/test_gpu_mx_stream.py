@@ -153,3 +153,18 @@ def test_swiglu_quant_is_the_quantised_swiglu_result(gpu, m, n, k):
     q, qs = gemm_mxfp4_swiglu_quant_transposed_b(*ops, n_pad=n + 96)
     assert torch.equal(q[:, :n // 2], want_q) and torch.equal(qs[:, :n // 32], want_s)
     assert not q[:, n // 2:].any() and not qs[:, n // 32:].any()
+
+
+@pytest.mark.parametrize("off", [1, 2, 4])
+def test_swiglu_of_k_slices_into_a_result_at_any_element(gpu, off):
+    """A result that starts 2, 4 or 8 bytes behind a 16-byte boundary (a view into a larger tensor): the same bits, and nothing beside it."""
+    m, n, k = 100, 256, 3776
+    ops = [H.to_dev(t, gpu) for t in (*H.mx_operand(m, k, seed=m), *H.mx_operand(2 * n, k, seed=n, std=0.05))]
+    with torch.cuda.device(gpu):
+        assert _lib.load().ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(m, n, k, 0) > 0
+    want = gemm_mxfp4_swiglu_transposed_b(*ops)
+    buffer = torch.full((m * n + 16,), 7.0, dtype=torch.bfloat16, device=gpu)
+    out = buffer[off:off + m * n].view(m, n)
+    assert gemm_mxfp4_swiglu_transposed_b(*ops, out) is out and out.data_ptr() % 16 == 2 * off
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert (buffer[:off] == 7).all() and (buffer[off + m * n:] == 7).all()
