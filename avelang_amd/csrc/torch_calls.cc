@@ -57,7 +57,19 @@ bool as_int(PyObject* o, int* v) {
   return x >= INT_MIN && x <= INT_MAX;
 }
 
-Tensor empty(at::IntArrayRef shape, at::ScalarType dtype, c10::Device dev) { return at::empty(shape, at::TensorOptions().dtype(dtype).device(dev)); }
+// Other Python threads run while this one is inside: an allocation may have to wait for the driver, as torch.empty's may.
+struct NoGil {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+Tensor empty(at::IntArrayRef shape, at::ScalarType dtype, c10::Device dev) {
+  NoGil no_gil;
+  return at::empty(shape, at::TensorOptions().dtype(dtype).device(dev));
+}
+Tensor zeros(at::IntArrayRef shape, at::ScalarType dtype, c10::Device dev) {
+  NoGil no_gil;
+  return at::zeros(shape, at::TensorOptions().dtype(dtype).device(dev));
+}
 
 // `given` (None: a new tensor) as the output of this shape and dtype; false when a given one does not fit.
 struct Out {
@@ -65,7 +77,7 @@ struct Out {
   PyObject* given = nullptr;
   bool take(PyObject* o, at::IntArrayRef shape, at::ScalarType dtype, c10::Device dev, bool zero = false) {
     if (o == Py_None) {
-      t = zero ? at::zeros(shape, at::TensorOptions().dtype(dtype).device(dev)) : empty(shape, dtype, dev);
+      t = zero ? zeros(shape, dtype, dev) : empty(shape, dtype, dev);
       return true;
     }
     const Tensor* p = tensor(o);
@@ -100,9 +112,10 @@ bool launch(c10::Device dev, F f) {
   const auto current = c10::hip::current_device();
   if (current != dev.index()) c10::hip::set_device(dev.index());
   void* stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
-  Py_BEGIN_ALLOW_THREADS
-  rc = f(stream);
-  Py_END_ALLOW_THREADS
+  {
+    NoGil no_gil;
+    rc = f(stream);
+  }
   if (current != dev.index()) c10::hip::set_device(current);
   if (rc == 0) return true;
   const char* msg = ave_fp4_last_error();

@@ -1,5 +1,9 @@
 """The C++ entry points on torch tensors (avelang_amd._torch_calls): a call they take gives what the Python wrapper gives
 through ctypes, ``out`` comes back as the object that was passed, and what they do not take reaches the wrapper's checks."""
+import ctypes.util
+import threading
+import time
+
 import pytest
 import torch
 
@@ -76,3 +80,32 @@ def test_out_is_returned_and_wrong_arguments_reach_the_checks(gpu):
         api.gemm_mxfp4_transposed_b(a, a_s, w, w_s, variant=99)
     with pytest.raises(TypeError, match="7 arguments expected, got 1"):
         api._native.gemm_mxfp4(a)
+
+
+@pytest.mark.parametrize("n_pad", [None, 128])   # (padded results are allocated and cleared)
+def test_other_threads_run_while_memory_is_allocated(gpu, n_pad):
+    """A pool whose driver allocation is usleep: it takes as many microseconds as bytes are asked for (2 MB, a few tries) and hands out
+    nothing.  Another Python thread counts on meanwhile; with the interpreter's lock held it would stand still."""
+    a, a_s, w, w_s = (H.to_dev(t, gpu) for t in (*H.mx_operand(16, 512, seed=1), *H.mx_operand(64, 512, seed=2)))
+    slow = torch.cuda.memory.CUDAPluggableAllocator(ctypes.util.find_library("c"), "usleep", "abs")
+    pool = torch.cuda.MemPool(slow.allocator())
+    stop, ticks = threading.Event(), [0]
+
+    def count():
+        while not stop.wait(0.01):
+            ticks[0] += 1
+
+    thread = threading.Thread(target=count)
+    thread.start()
+    try:
+        start = time.monotonic()
+        with torch.cuda.use_mem_pool(pool), pytest.raises(torch.OutOfMemoryError):
+            ticks[0] = 0
+            if api._native.gemm_mxfp4_swiglu_quant(a, a_s, w, w_s, None, None, n_pad) is not None:
+                raise AssertionError("the pool had memory")
+        counted, seconds = ticks[0], time.monotonic() - start
+    finally:
+        stop.set()
+        thread.join()
+    assert seconds > 1.0, seconds
+    assert counted > 20 * seconds, (counted, seconds)   # 100 a second when nothing holds it up
