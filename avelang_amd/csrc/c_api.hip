@@ -225,7 +225,6 @@ static bool stream_whole(const ave::MxArgs& p, void* hip_stream, int* rc) {
 static bool stream_split(ave::MxArgs p, void* workspace, size_t workspace_bytes, void* hip_stream, int* rc) {
   const ave::MxStreamPlan plan = stream_plan(p.M, p.N, p.K, p.swiglu != 0, p.Q != nullptr, true);
   if (plan.rows == 0 || plan.slices < 2 || workspace_bytes < plan.workspace_bytes || !ave::mx_stream_supports(p)) return false;
-  if (p.C && p.swiglu && !aligned(p.C, 16)) return false;   // stored 16 bytes at a time
   p.P = static_cast<float*>(workspace);
   p.slices = plan.slices;
   p.slice_pairs = plan.slice_pairs;

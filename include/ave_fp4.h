@@ -165,7 +165,7 @@ int ave_fp4_gemm_mxfp4_swiglu_quant(const uint8_t* A, const uint8_t* A_scale, co
  * activation and, in the quantising form, the quantiser.  Up to 32 rows the quantising form without row padding may also run as two
  * launches, the bf16 form into the workspace and the quantiser.  ave_fp4_gemm_mxfp4_swiglu_workspace_bytes gives the size for
  * either form (quant = 0 or 1), 0 where none is used.  Quantising the result of the one form is what the other gives, bit for bit, up to
- * 32 rows and above 64, both called with their workspace (C 16-byte aligned) or both without.
+ * 32 rows and above 64, both called with their workspace or both without.
  */
 size_t ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(int M, int N, int K, int quant);
 int ave_fp4_gemm_mxfp4_swiglu_ws(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,

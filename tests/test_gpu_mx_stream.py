@@ -168,3 +168,17 @@ def test_swiglu_of_k_slices_into_a_result_at_any_element(gpu, off):
     assert gemm_mxfp4_swiglu_transposed_b(*ops, out) is out and out.data_ptr() % 16 == 2 * off
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
     assert (buffer[:off] == 7).all() and (buffer[off + m * n:] == 7).all()
+
+
+def test_swiglu_of_k_slices_is_cut_alike_whatever_the_result_address(gpu):
+    """Scales over 2^24, so that the order of the sums shows in the bits: a result at an odd element is still made of the same K slices."""
+    m, n, k = 100, 256, 3776
+    rng = np.random.default_rng(5)
+    ops = [torch.from_numpy(rng.integers(lo, hi, size=s, dtype=np.uint8)).to(gpu)
+           for lo, hi, s in ((0, 256, (m, k // 2)), (108, 132, (m, k // 32)), (0, 256, (2 * n, k // 2)), (100, 124, (2 * n, k // 32)))]
+    with torch.cuda.device(gpu):
+        assert _lib.load().ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(m, n, k, 0) > 0
+    want = gemm_mxfp4_swiglu_transposed_b(*ops)
+    out = torch.empty(m * n + 1, dtype=torch.bfloat16, device=gpu)[1:].view(m, n)
+    gemm_mxfp4_swiglu_transposed_b(*ops, out)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
