@@ -803,9 +803,7 @@ int ave_fp4_debug_gemm_mxfp4_stream_splitk(const uint8_t* A, const uint8_t* A_sc
   if (!workspace || !aligned(workspace, 16) || workspace_bytes < need)
     return fail_inval("workspace must be 16-byte aligned and hold %zu bytes, got %zu.", need, workspace_bytes);
   if (!ave::mx_stream_supports(p)) return fail_inval("streaming kernel does not support M=%d N=%d K=%d.", M, N, K);
-  hipStream_t s = static_cast<hipStream_t>(hip_stream);
-  if (hipError_t e = ave::launch_mx_stream(p, tile_rows, s); e != hipSuccess) return finish(e, "mxfp4 streaming kernel, split K");
-  return finish(ave::launch_splitk_reduce(p.P, C, (size_t)M * (size_t)N, p.slices, s), "reduction of the K slices");
+  return finish(ave::launch_mx_stream(p, tile_rows, static_cast<hipStream_t>(hip_stream)), "mxfp4 streaming kernel, split K");
 }
 
 // The streaming kernel where shape-based dispatch takes it; false: somebody else's shape.
