@@ -811,6 +811,7 @@ static bool grouped_stream(ave::MxArgs& p, void* hip_stream, int* rc) {
   const int rows = ave::mx_stream_rows(p);
   if (rows == 0) return false;
   p.tail_four_apart = (long)p.M > 128L * p.E;   // where the 256 x 256 kernel is the other choice: its bits
+  p.rows_by_table = 1;
   *rc = finish(ave::launch_mx_stream(p, rows, static_cast<hipStream_t>(hip_stream)), "grouped mxfp4 streaming kernel");
   return true;
 }

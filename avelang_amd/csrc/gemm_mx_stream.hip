@@ -1,14 +1,15 @@
-// Grouped MXFP4 GEMM for gfx950 for expert layers with a few rows per expert (a decode batch, or many experts): 32 or 64 rows
-// of A by 128 weight rows per tile, and a ring of LDS buffers that never runs dry between tiles.
+// MXFP4 GEMM for gfx950 for expert layers with a few rows per expert (a decode batch, or many experts), and for one matrix with few
+// weight rows, K whole or in slices: 32, 64 or 128 rows of A by 128 weight rows per tile, and a ring of LDS buffers that never runs
+// dry between tiles.
 //
-// Bound by HBM: every expert's weights are read once, 1.06 bytes per two elements, and what a compute unit gets through its
-// load path is about 22 - 25 KB per us.  The 128-row tiles of gemm_mx_narrow.hip spend half of that on rows of A -- for 16
-// rows an expert, on 112 repeats of its last row -- and start their ring anew for every tile where K is no multiple of 1024, with a
-// K tail read from global memory at the end of each.  Here a stage (256 elements of K) is 20 or 24 KB of which 16 are weights, six or
-// five stages are in flight, and tile boundaries and K tails are ordinary stages of one continuous stream.
+// Bound by HBM: every expert's weights are read once, 1.06 bytes per two elements, at 5.2 - 5.7 TB/s over all compute units (21 - 22 KB
+// per us each).  The rows of A come from L2 (a stage of 32 KB has been seen to pass in 0.47 us), but a tile of 128 rows brings 112
+// repeats of its last row for an expert with 16, and the ring that 128-row tiles started anew for every tile, with a K tail read from global
+// memory at its end, ran dry where K is no multiple of 1024.  Here a stage (256 elements of K) is 20, 24 or 32 KB of which 16 are weights;
+// six, five or three of them are in flight, and tile boundaries and K tails are ordinary stages of one continuous stream.
 //
-// Six wavefronts: waves 0 and 1 multiply -- 64 weight rows each, two 32-row blocks, so that with SWIGLU the gate and the up value of
-// an output meet in one lane as in gemm_mx_narrow.hip -- and waves 2 - 5 load, a quarter of a stage each, with one
+// Six wavefronts (128 rows: eight): waves 0 and 1 (0 - 3) multiply -- 64 weight rows each, two 32-row blocks, so that with SWIGLU the gate and
+// the up value of an output meet in one lane as in gemm_mx_narrow.hip -- and the last four load, a quarter of a stage each, with one
 // barrier per stage: behind the barrier of stage j, which says that stage j has landed and stage j - 1 is consumed, stage j + ring - 1
 // is requested into the buffer of stage j - 1.  One workgroup per compute unit walks the tiles pid, pid + gridDim.x, ...
 //
@@ -95,6 +96,25 @@ __device__ inline const uint8_t* uniform(const uint8_t* p) {
   return reinterpret_cast<const uint8_t*>((uint64_t)hi << 32 | lo);
 }
 
+// Experts' first and end rows, clamped to [0, M]: lane l keeps those of experts l, l + 64, l + 128 and l + 192 (none: 0, 0).
+constexpr int kSets = 4;
+__device__ __forceinline__ void load_table(const MxArgs& p, int (&g_r0)[kSets], int (&g_r1)[kSets]) {
+#pragma unroll
+  for (int q = 0; q < kSets; ++q) {
+    const int e = 64 * q + (int)(threadIdx.x & 63);
+    int r0 = 0, r1 = 0;
+    if (e < p.E) {
+      r0 = p.row_offsets[e];
+      r1 = p.row_offsets[e + 1];
+      r0 = r0 < 0 ? 0 : (r0 > p.M ? p.M : r0);
+      r1 = r1 < 0 ? 0 : (r1 > p.M ? p.M : r1);
+    }
+    g_r0[q] = r0;
+    g_r1[q] = r1;
+  }
+}
+__device__ inline bool table_in_registers(const MxArgs& p) { return p.E <= 64 * kSets; }
+
 // GROUPED: the rows of A belong to p.E experts (p.row_offsets) with weights of their own; otherwise one matrix of p.M rows.
 // SPLITK (plain form, not grouped): a work item is a tile and a slice of p.slice_pairs pairs of stages (the last one what is left, the
 // K tail with it); its fp32 sums go to p.P[slice][M][N].
@@ -106,7 +126,7 @@ __device__ inline const uint8_t* uniform(const uint8_t* p) {
 // s + 1, one stage earlier than without; a tile whose last stage has late chunks takes one line more.  Chunks of a line that are not the
 // row's are not loaded.  Measured: 255 -> 220 us, with 2880 weight rows 131 -> 112.
 template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
-__global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, int n_tiles) {
+__device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const int (&g_r0)[kSets], const int (&g_r1)[kSets]) {
   using G = Geo<R>;
   static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
   static_assert(!SPLITK || (!SWIGLU && !GROUPED), "K is split for the plain GEMM");
@@ -127,26 +147,17 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
   const int unit = (int)(bits16 & (0u - bits16));
   const bool late_at_end = SHIFT && (tail_blocks != 0 ? tail_blocks : 8) > unit;   // the last stage of K has late chunks in some row
 
-  // Lane l keeps {first m-tile, m-tiles, first row, end row} (clamped to [0, M]) of experts l, l + 64, l + 128 and l + 192;
-  // with more than 256 experts the caller's table is walked for every tile.
-  constexpr int kSets = 4;
-  int g_first[kSets], g_nt[kSets], g_r0[kSets], g_r1[kSets];
+  // Beside its experts' rows a lane keeps their {first m-tile, m-tiles}; with more than 256 experts the caller's table is walked for
+  // every tile.
+  int g_first[kSets], g_nt[kSets];
   int m_tiles = 0;
-  const bool in_registers = p.E <= 64 * kSets;
+  const bool in_registers = table_in_registers(p);
   if (!GROUPED) {
     m_tiles = (p.M + R - 1) / R;
   } else if (in_registers) {
 #pragma unroll
     for (int q = 0; q < kSets; ++q) {
-      const int e = 64 * q + lane;
-      int r0 = 0, r1 = 0;
-      if (e < p.E) {
-        r0 = p.row_offsets[e];
-        r1 = p.row_offsets[e + 1];
-        r0 = r0 < 0 ? 0 : (r0 > p.M ? p.M : r0);
-        r1 = r1 < 0 ? 0 : (r1 > p.M ? p.M : r1);
-      }
-      const int nt = r1 > r0 ? (r1 - r0 + R - 1) / R : 0;
+      const int nt = g_r1[q] > g_r0[q] ? (g_r1[q] - g_r0[q] + R - 1) / R : 0;
       int incl = nt;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
@@ -155,8 +166,6 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
       }
       g_first[q] = m_tiles + incl - nt;
       g_nt[q] = nt;
-      g_r0[q] = r0;
-      g_r1[q] = r1;
       m_tiles += __builtin_amdgcn_readlane(incl, 63);
     }
   } else {
@@ -536,16 +545,94 @@ __global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, i
 }
 
 template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
-hipError_t launch_rows(const MxArgs& p, hipStream_t s) {
+__global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, int n_tiles) {
+  int g_r0[kSets], g_r1[kSets];
+  if (GROUPED && table_in_registers(p)) load_table(p, g_r0, g_r1);
+  stream_tiles<R, SWIGLU, QUANT, GROUPED, SPLITK, SHIFT>(p, n_tiles, g_r0, g_r1);
+}
+
+// Rows per tile for the experts' table as it is, from the `rows` that the host took for the average: an expert with more rows than a
+// tile sends its weights through the load path once per tile, so where routing is uneven tall tiles take fewer rounds.  The
+// cheapest by rounds of the grid x rows that a stage loads, the same in every wave; nothing to look for (and no time spent) where no
+// expert has more than one tile.
+__device__ __forceinline__ int rows_for_table(const int (&g_r0)[kSets], const int (&g_r1)[kSets], int n_tiles, int rows) {
+  int tiles32 = 0, tiles64 = 0, tiles128 = 0, most = 0;
+#pragma unroll
+  for (int q = 0; q < kSets; ++q) {
+    const int n = g_r1[q] > g_r0[q] ? g_r1[q] - g_r0[q] : 0;
+    most = n > most ? n : most;
+    tiles32 += (n + 31) >> 5;
+    tiles64 += (n + 63) >> 6;
+    tiles128 += (n + 127) >> 7;
+  }
+  if (!__any(most > rows)) return rows;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    tiles32 += __shfl_xor(tiles32, d);
+    tiles64 += __shfl_xor(tiles64, d);
+    tiles128 += __shfl_xor(tiles128, d);
+  }
+  auto cost = [&](int tiles, int of) { return ceilf((float)tiles * (float)n_tiles / (float)gridDim.x) * (float)(of + BN); };
+  const float at64 = cost(tiles64, 64);
+  const bool tall = rows == 64 || at64 < cost(tiles32, 32);
+  const float least = tall ? at64 : cost(tiles32, 32);
+  const int taken = cost(tiles128, 128) < least ? 128 : (tall ? 64 : 32);
+  return __builtin_amdgcn_readfirstlane(taken);
+}
+
+// Expert layers on tiles of 32 or 64 rows, or (`by_table`) of more where the experts' table asks for it.  Waves that the tile
+// height has no work for end at once (a barrier waits for the others alone).  Measured, tiles by the average alone -> by the table
+// (128-row tiles with a ring per tile before that), plain, us: 128 rows of 8 experts, 28672 x 4096, all in one expert 31.8 -> 20.0 (21.0);
+// 4096 x 14336, routed by 1 / rank 61.2 -> 42.0 (49.1); 2000 rows of 128 experts, 5760 x 2880, on a quarter of them 95.9 -> 78.7 (105), in
+// one 80.2 -> 36.7 (46.4), evenly 227.3 and 227.0 (327).
+template <int R>
+constexpr bool fits_taller = Geo<R>::kThreads <= Geo<128>::kThreads && Geo<R>::kLds <= Geo<64>::kLds;
+static_assert(fits_taller<32> && fits_taller<64> && fits_taller<128>);
+template <bool SWIGLU, bool QUANT, bool SHIFT>
+__global__ __launch_bounds__(Geo<128>::kThreads) void mx_stream_by_table_kernel(MxArgs p, int n_tiles, int rows, int by_table) {
+  int g_r0[kSets], g_r1[kSets];
+  if (table_in_registers(p)) {
+    load_table(p, g_r0, g_r1);
+    if (by_table) rows = rows_for_table(g_r0, g_r1, n_tiles, rows);
+  }
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (rows == 128) {
+    stream_tiles<128, SWIGLU, QUANT, true, false, SHIFT>(p, n_tiles, g_r0, g_r1);
+  } else if (rows == 64) {
+    if (wave < Geo<64>::kThreads / 64) stream_tiles<64, SWIGLU, QUANT, true, false, SHIFT>(p, n_tiles, g_r0, g_r1);
+  } else {
+    if (wave < Geo<32>::kThreads / 64) stream_tiles<32, SWIGLU, QUANT, true, false, SHIFT>(p, n_tiles, g_r0, g_r1);
+  }
+}
+
+// workgroups for m-tiles of R rows (grouped: an upper bound of the experts' tile lists), at most one per compute unit; 0: no device
+template <bool SWIGLU, bool GROUPED, bool SPLITK>
+unsigned stream_grid(const MxArgs& p, int rows, int* n_tiles) {
   constexpr int kTileN = SWIGLU ? BN / 2 : BN;
-  const int n_tiles = (p.N + kTileN - 1) / kTileN;
+  *n_tiles = (p.N + kTileN - 1) / kTileN;
   const int cus = compute_units();
-  if (cus <= 0) return hipErrorInvalidDevice;
+  const long tiles = ((long)(p.M + rows - 1) / rows + (GROUPED ? p.E : 0)) * *n_tiles * (SPLITK ? p.slices : 1);
+  return cus <= 0 ? 0 : (unsigned)(tiles < cus ? tiles : cus);
+}
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
+hipError_t launch(const MxArgs& p, hipStream_t s) {
+  int n_tiles;
+  const unsigned grid = stream_grid<SWIGLU, GROUPED, SPLITK>(p, R, &n_tiles);
+  if (grid == 0) return hipErrorInvalidDevice;
   constexpr auto kernel = mx_stream_kernel<R, SWIGLU, QUANT, GROUPED, SPLITK, SHIFT>;
   if (hipError_t e = allow_dynamic_lds<kernel>(Geo<R>::kLds); e != hipSuccess) return e;
-  // grouped: upper bound of the experts' tile lists
-  const long tiles = ((long)(p.M + R - 1) / R + (GROUPED ? p.E : 0)) * n_tiles * (SPLITK ? p.slices : 1);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < cus ? tiles : cus)), dim3(Geo<R>::kThreads), Geo<R>::kLds, s, p, n_tiles);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Geo<R>::kThreads), Geo<R>::kLds, s, p, n_tiles);
+  return hipGetLastError();
+}
+template <bool SWIGLU, bool QUANT, bool SHIFT>
+hipError_t launch_grouped_lines(const MxArgs& p, int rows, hipStream_t s) {
+  if (rows == 128) return launch<128, SWIGLU, QUANT, true, false, SHIFT>(p, s);
+  int n_tiles;
+  const unsigned grid = stream_grid<SWIGLU, true, false>(p, rows, &n_tiles);
+  if (grid == 0) return hipErrorInvalidDevice;
+  constexpr auto kernel = mx_stream_by_table_kernel<SWIGLU, QUANT, SHIFT>;
+  if (hipError_t e = allow_dynamic_lds<kernel>(Geo<64>::kLds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Geo<128>::kThreads), Geo<64>::kLds, s, p, n_tiles, rows, p.rows_by_table);
   return hipGetLastError();
 }
 // SHIFT for experts' weights whose rows do not all start at a cache line, from HBM and over a few lines: the start of a tile costs it
@@ -563,11 +650,9 @@ bool by_lines(const MxArgs& p) {
   if (tail > unit && p.K <= 5 * BK && !p.by_lines) return false;
   return (uint64_t)p.M * row + 256 < (1ull << 32) && b_rows * row + 256 < (1ull << 32);   // room for the 128 bytes on top of an offset
 }
-template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK>
-hipError_t launch(const MxArgs& p, hipStream_t s) {
-  if constexpr (GROUPED)
-    if (by_lines<SWIGLU>(p)) return launch_rows<R, SWIGLU, QUANT, GROUPED, SPLITK, true>(p, s);
-  return launch_rows<R, SWIGLU, QUANT, GROUPED, SPLITK, false>(p, s);
+template <bool SWIGLU, bool QUANT>
+hipError_t launch_grouped(const MxArgs& p, int rows, hipStream_t s) {
+  return by_lines<SWIGLU>(p) ? launch_grouped_lines<SWIGLU, QUANT, true>(p, rows, s) : launch_grouped_lines<SWIGLU, QUANT, false>(p, rows, s);
 }
 
 // silu(gate) * up of K slices' sums P[slices][M][2N] (N gate columns, then N up columns), added up in slice order: bf16 into C, or
@@ -631,7 +716,7 @@ hipError_t launch_split(const MxArgs& p, hipStream_t s) {
   MxArgs q = p;
   q.swiglu = 0;
   q.N = p.swiglu ? 2 * p.N : p.N;
-  if (hipError_t e = launch<R, false, false, false, true>(q, s); e != hipSuccess) return e;
+  if (hipError_t e = launch<R, false, false, false, true, false>(q, s); e != hipSuccess) return e;
   if (!p.swiglu) return launch_splitk_reduce(p.P, p.C, (size_t)p.M * (size_t)p.N, p.slices, s);
   const size_t blocks = ((size_t)p.M * (p.N / 8) + 255) / 256;
   const dim3 grid((unsigned)(blocks < 4096 ? blocks : 4096));
@@ -642,14 +727,9 @@ hipError_t launch_split(const MxArgs& p, hipStream_t s) {
 template <int R>
 hipError_t launch_form(const MxArgs& p, hipStream_t s) {
   if (p.P) return launch_split<R>(p, s);
-  if (!p.row_offsets) {
-    if (p.swiglu && p.Q) return launch<R, true, true, false, false>(p, s);
-    if (p.swiglu) return launch<R, true, false, false, false>(p, s);
-    return launch<R, false, false, false, false>(p, s);
-  }
-  if (p.swiglu && p.Q) return launch<R, true, true, true, false>(p, s);
-  if (p.swiglu) return launch<R, true, false, true, false>(p, s);
-  return launch<R, false, false, true, false>(p, s);
+  if (p.swiglu && p.Q) return launch<R, true, true, false, false, false>(p, s);
+  if (p.swiglu) return launch<R, true, false, false, false, false>(p, s);
+  return launch<R, false, false, false, false, false>(p, s);
 }
 
 }  // namespace
@@ -676,7 +756,8 @@ double expected_m_tiles(int E, double rows, int R) {
 }
 }  // namespace
 
-// Shape-based dispatch; the host knows the average number of rows per expert only.  Up to 128 this kernel: it reads
+// Shape-based dispatch; the host knows the average number of rows per expert only (what it says below 128 is the least height:
+// the kernel takes taller tiles where the table is uneven, rows_for_table).  Up to 128 this kernel: it reads
 // the weights once at 4 - 5.5 TB/s (gate+up of 8 experts x 16 rows, 28672 x 4096, 92 us; 128 experts x 16 rows, 5760 x 2880, 247 us where
 // the 128-row tiles with a ring per tile took 318; 78 experts x 4 rows, 21504 x 1184, 205 against 306).  32 rows a tile up to 18 rows per
 // expert (an expert with more rows takes a second tile and its weights a second time through the load path: 36 rows on
@@ -810,6 +891,11 @@ MxStreamPlan mx_stream_plan(int M, int N, int K, bool swiglu, bool quant, int cu
 }
 
 hipError_t launch_mx_stream(const MxArgs& p, int tile_rows, hipStream_t s) {
+  if (p.row_offsets) {
+    if (p.swiglu && p.Q) return launch_grouped<true, true>(p, tile_rows, s);
+    if (p.swiglu) return launch_grouped<true, false>(p, tile_rows, s);
+    return launch_grouped<false, false>(p, tile_rows, s);
+  }
   return tile_rows == 32 ? launch_form<32>(p, s) : (tile_rows == 64 ? launch_form<64>(p, s) : launch_form<128>(p, s));
 }
 

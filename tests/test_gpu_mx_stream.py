@@ -4,7 +4,9 @@ import numpy as np
 import pytest
 import torch
 
-from avelang_amd import _lib, gemm_mxfp4_swiglu_quant_transposed_b, gemm_mxfp4_swiglu_transposed_b, quantize_mxfp4
+from avelang_amd import (_lib, gemm_mxfp4_swiglu_quant_transposed_b, gemm_mxfp4_swiglu_transposed_b,
+                         grouped_gemm_mxfp4_swiglu_quant_transposed_b, grouped_gemm_mxfp4_swiglu_transposed_b,
+                         grouped_gemm_mxfp4_transposed_b, quantize_mxfp4)
 from oracle import fp4_oracle as orc
 from tests import helpers as H
 
@@ -182,3 +184,27 @@ def test_swiglu_of_k_slices_is_cut_alike_whatever_the_result_address(gpu):
     out = torch.empty(m * n + 1, dtype=torch.bfloat16, device=gpu)[1:].view(m, n)
     gemm_mxfp4_swiglu_transposed_b(*ops, out)
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+# 260 tiles of 32 rows on 256 compute units (one round of 64-row tiles), 520 (one round of 128), few enough to stay; an average above 18 rows;
+# one expert a little taller than a tile; rows loaded by lines; more experts than a table in registers
+@pytest.mark.parametrize("rows,n,k", [([0, 128, 0, 0, 0, 0, 0, 0], 8320, 544), ([0, 0, 0, 0, 0, 128, 0, 0], 16640, 512),
+                                      ([128, 0, 0, 0, 0, 0, 0, 0], 512, 736), ([9, 47, 24, 16, 12, 8, 7, 5], 4096, 1024),
+                                      ([3, 300, 0, 1, 4, 0, 33, 11], 8320, 544), ([33] + [1] * 70, 512, 800),
+                                      ([0, 0, 130, 0, 5, 0, 0, 0], 16640, 1312), ([200] + [1] * 299, 4224, 544)])
+def test_uneven_tables_give_the_bits_of_every_tile_height(gpu, rows, n, k):
+    """The height of the tiles follows the experts' table; an output's sum does not."""
+    e, m = len(rows), sum(rows)
+    ro = torch.from_numpy(np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)).to(gpu)
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    a, b = (torch.randint(0, 256, s, dtype=torch.uint8, device=gpu, generator=g) for s in ((m, k // 2), (e, n, k // 2)))
+    a_s, b_s = (torch.randint(110, 132, s, dtype=torch.uint8, device=gpu, generator=g) for s in ((m, k // 32), (e, n, k // 32)))
+    ops = (a, a_s, b, b_s)
+    got = [(grouped_gemm_mxfp4_transposed_b(*ops, ro),), (grouped_gemm_mxfp4_swiglu_transposed_b(*ops, ro),),
+           grouped_gemm_mxfp4_swiglu_quant_transposed_b(*ops, ro)]
+    for tile_rows in (32, 64, 128):
+        want = [(_stream(gpu, ops, ro, n, tile_rows, 0, False),), (_stream(gpu, ops, ro, n // 2, tile_rows, 1, False),),
+                _stream(gpu, ops, ro, n // 2, tile_rows, 1, True)]
+        for form, (xs, ys) in enumerate(zip(got, want)):
+            for x, y in zip(xs, ys):
+                assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), (tile_rows, form)
