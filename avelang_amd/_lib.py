@@ -51,6 +51,11 @@ SIGNATURES = {
                                         ctypes.POINTER(_int), ctypes.POINTER(ctypes.c_size_t)],
     "ave_fp4_debug_gemm_mxfp4_splitk": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _int, _int, _vp],
     "ave_fp4_debug_gemm_mxfp4_stream_splitk": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _int, _int, _vp],
+    "ave_fp4_debug_gemm_mxfp4_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _vp],
+    "ave_fp4_debug_stream_plan": [_int, _int, _int, _int, _int, _int, _int, ctypes.POINTER(_int), ctypes.POINTER(_int),
+                                  ctypes.POINTER(_int), ctypes.POINTER(ctypes.c_size_t)],
+    "ave_fp4_debug_nv_plan": [_int, _int, _int, _int, _int, ctypes.POINTER(_int), ctypes.POINTER(_int), ctypes.POINTER(_int),
+                              ctypes.POINTER(_int), ctypes.POINTER(ctypes.c_size_t)],
     "ave_fp4_debug_grouped_gemm_mxfp4_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _int, _vp],
     "ave_fp4_debug_gemm_nvfp4_narrow": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, ctypes.c_size_t, _int, _int, _vp],
     "ave_fp4_gemm_mxfp4_swiglu": [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp],

@@ -806,6 +806,43 @@ int ave_fp4_debug_gemm_mxfp4_stream_splitk(const uint8_t* A, const uint8_t* A_sc
   return finish(ave::launch_mx_stream(p, tile_rows, static_cast<hipStream_t>(hip_stream)), "mxfp4 streaming kernel, split K");
 }
 
+int ave_fp4_debug_gemm_mxfp4_stream(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                    uint16_t* C, uint8_t* Q, uint8_t* Q_scale, int M, int N, int K, int swiglu, int tile_rows,
+                                    void* hip_stream) {
+  g_err[0] = 0;
+  if (int rc = check_common(A, A_scale, B, B_scale, Q ? static_cast<const void*>(Q) : C, M, N, K, 32, 16)) return rc;
+  if (M == 0 || N == 0) return 0;
+  if (tile_rows != 32 && tile_rows != 64 && tile_rows != 128) return fail_inval("tile_rows must be 32, 64 or 128, got %d.", tile_rows);
+  const ave::MxArgs p{A, A_scale, B, B_scale, Q ? nullptr : C, M, N, K, nullptr, 0, swiglu ? 1 : 0, Q, Q_scale};
+  if (!ave::mx_stream_supports(p)) return fail_inval("streaming kernel does not support M=%d N=%d K=%d.", M, N, K);
+  return finish(ave::launch_mx_stream(p, tile_rows, static_cast<hipStream_t>(hip_stream)), "mxfp4 streaming kernel");
+}
+
+int ave_fp4_debug_stream_plan(int M, int N, int K, int swiglu, int quant, int compute_units, int may_split, int* tile_rows,
+                              int* slices, int* slice_pairs, size_t* workspace_bytes) {
+  g_err[0] = 0;
+  if (compute_units <= 0 || !tile_rows || !slices || !slice_pairs || !workspace_bytes) return fail_inval("invalid argument.");
+  const ave::MxStreamPlan plan = ave::mx_stream_plan(M, N, K, swiglu != 0, quant != 0, compute_units, may_split != 0);
+  *tile_rows = plan.rows;
+  *slices = plan.slices;
+  *slice_pairs = plan.slice_pairs;
+  *workspace_bytes = plan.workspace_bytes;
+  return 0;
+}
+
+int ave_fp4_debug_nv_plan(int M, int N, int K, int compute_units, int may_split, int* kernel, int* tile_rows, int* slices,
+                          int* slice_stages, size_t* workspace_bytes) {
+  g_err[0] = 0;
+  if (compute_units <= 0 || !kernel || !tile_rows || !slices || !slice_stages || !workspace_bytes) return fail_inval("invalid argument.");
+  const ave::NvPlan plan = ave::nv_plan(M, N, K, compute_units, may_split != 0);
+  *kernel = plan.kernel;
+  *tile_rows = plan.tile_rows;
+  *slices = plan.slices;
+  *slice_stages = plan.slice_stages;
+  *workspace_bytes = plan.workspace_bytes;
+  return 0;
+}
+
 // The streaming kernel where shape-based dispatch takes it; false: somebody else's shape.
 static bool grouped_stream(ave::MxArgs& p, void* hip_stream, int* rc) {
   const int rows = ave::mx_stream_rows(p);

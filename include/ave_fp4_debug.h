@@ -40,6 +40,20 @@ int ave_fp4_debug_gemm_nvfp4_narrow(const uint8_t* A, const uint8_t* A_scale, co
 int ave_fp4_debug_gemm_mxfp4_stream_splitk(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                                            uint16_t* C, int M, int N, int K, void* workspace, size_t workspace_bytes, int tile_rows,
                                            int slice_pairs, void* hip_stream);
+/* The same kernel with K in one piece: plain, with the fused SwiGLU (swiglu != 0: B holds 2N rows) into C, or with the quantiser behind
+ * that into Q and Q_scale (C null).  K a multiple of 32 from 512 up, 16-byte aligned A and B. */
+int ave_fp4_debug_gemm_mxfp4_stream(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
+                                    uint16_t* C, uint8_t* Q, uint8_t* Q_scale, int M, int N, int K, int swiglu, int tile_rows,
+                                    void* hip_stream);
+/* Host-only diagnostics: what shape-based dispatch plans on a device with compute_units compute units, with a workspace (may_split) or
+ * without.  The MXFP4 GEMM or its fused SwiGLU forms (N outputs) on the streaming kernel: tile_rows (0: another kernel), slices
+ * of slice_pairs x 512 elements of K (1 slice: K in one piece) and the workspace bytes of their sums. */
+int ave_fp4_debug_stream_plan(int M, int N, int K, int swiglu, int quant, int compute_units, int may_split, int* tile_rows,
+                              int* slices, int* slice_pairs, size_t* workspace_bytes);
+/* The NVFP4 GEMM: kernel 0 (K below 1024, by other rules), 1 (weight-streaming), 2 (narrow tiles of tile_rows rows), 3 (256 x 256 tiles) or
+ * 4 (f16-staged tiles), slices of slice_stages x 256 elements of K and the workspace bytes of their sums. */
+int ave_fp4_debug_nv_plan(int M, int N, int K, int compute_units, int may_split, int* kernel, int* tile_rows, int* slices,
+                          int* slice_stages, size_t* workspace_bytes);
 /* Diagnostic and test hook: the grouped MXFP4 GEMM on tiles of tile_rows (32, 64 or 128) rows of A by 128 weight rows, whatever the
  * shape (K a multiple of 32 from 512 up, 16-byte aligned A and B).  swiglu: B holds 2N rows per expert; with Q and Q_scale
  * (C null) the result is quantised, rows laid out for N columns.  tile_rows with AVE_FP4_DEBUG_BY_LINES added: in the form that

@@ -208,3 +208,54 @@ def test_uneven_tables_give_the_bits_of_every_tile_height(gpu, rows, n, k):
         for form, (xs, ys) in enumerate(zip(got, want)):
             for x, y in zip(xs, ys):
                 assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), (tile_rows, form)
+
+
+# one tile and many, ragged rows and columns; two stages, an odd number of them and K % 512 of 1, 7, 8, 9 and 15 blocks
+@pytest.mark.parametrize("m,n,k", [(1, 32, 512), (33, 96, 544), (64, 160, 736), (65, 32, 768), (127, 224, 800), (128, 64, 992), (129, 352, 1248),
+                                   (200, 64, 2880), (300, 8224, 512)])
+@pytest.mark.parametrize("tile_rows", [32, 64, 128])
+def test_stream_one_matrix_with_k_in_one_piece(gpu, m, n, k, tile_rows):
+    """The forms that shape-based dispatch takes without slices: plain, SwiGLU, SwiGLU + quantiser."""
+    a, a_s = H.mx_operand(m, k, seed=m + k)
+    b, b_s = H.mx_operand(2 * n, k, seed=n + k, std=0.05)
+    ops = [H.to_dev(t, gpu) for t in (a, a_s, b, b_s)]
+
+    def run(cols, swiglu, quant):
+        c = torch.full((m, cols), float("nan"), dtype=torch.bfloat16, device=gpu)
+        q = torch.full((m, cols // 2), 0xEE, dtype=torch.uint8, device=gpu)
+        qs = torch.full((m, cols // 32), 0xEE, dtype=torch.uint8, device=gpu)
+        _lib.check(_lib.load().ave_fp4_debug_gemm_mxfp4_stream(
+            *(t.data_ptr() for t in ops), None if quant else c.data_ptr(), q.data_ptr() if quant else None,
+            qs.data_ptr() if quant else None, m, cols, k, swiglu, tile_rows, torch.cuda.current_stream(gpu).cuda_stream))
+        torch.cuda.synchronize(gpu)
+        return (q, qs) if quant else c
+
+    H.assert_mx_close(H.bits(run(2 * n, 0, False)), a, a_s, b, b_s)
+    H.assert_mx_close(H.bits(run(2 * n - 3, 0, False)), a, a_s, b[:-3], b_s[:-3])
+    fused = run(n, 1, False)
+    ok, rep = orc.check_swiglu_bf16(H.bits(fused), a, a_s, b, b_s)
+    assert ok, rep
+    want_q, want_s = quantize_mxfp4(fused)
+    q, qs = run(n, 1, True)
+    assert torch.equal(q, want_q) and torch.equal(qs, want_s)
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 256, 3776), (65, 512, 4096), (130, 256, 7200), (48, 512, 7168)])
+def test_swiglu_forms_whose_k_is_cut(gpu, m, n, k):
+    """Shapes that are planned in slices (asserted, for a device of 256 compute units): both fused forms against the oracle."""
+    lib = _lib.load()
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("planned for 256 compute units")
+    with torch.cuda.device(gpu):
+        split = [lib.ave_fp4_gemm_mxfp4_swiglu_workspace_bytes(m, n, k, quant) for quant in (0, 1)]
+    for bytes_ in split:
+        assert bytes_ > 0 and bytes_ % (m * 2 * n * 4) == 0 and bytes_ // (m * 2 * n * 4) > 1
+    a, a_s = H.mx_operand(m, k, seed=m)
+    b, b_s = H.mx_operand(2 * n, k, seed=n, std=0.05)
+    ops = [H.to_dev(t, gpu) for t in (a, a_s, b, b_s)]
+    c = gemm_mxfp4_swiglu_transposed_b(*ops)
+    ok, rep = orc.check_swiglu_bf16(H.bits(c), a, a_s, b, b_s)
+    assert ok, rep
+    q, qs = gemm_mxfp4_swiglu_quant_transposed_b(*ops)
+    want_q, want_s = quantize_mxfp4(c)
+    assert np.mean(q.cpu().numpy() != want_q.cpu().numpy()) < 1e-3 and np.mean(qs.cpu().numpy() != want_s.cpu().numpy()) < 1e-3

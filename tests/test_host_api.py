@@ -363,6 +363,85 @@ def test_split_planner_arithmetic():
     assert lib.ave_fp4_debug_split_plan(128, 128, 1024, 0, None, None, None, None) == -1
 
 
+def _stream_plan(m, n, k, swiglu, quant, may_split, cus=256):
+    rows, slices, per, ws = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    assert _lib.load().ave_fp4_debug_stream_plan(m, n, k, swiglu, quant, cus, may_split, ctypes.byref(rows), ctypes.byref(slices),
+                                                 ctypes.byref(per), ctypes.byref(ws)) == 0
+    return rows.value, slices.value, per.value, ws.value
+
+
+def _nv_plan(m, n, k, may_split, cus=256):
+    kernel, rows, slices, per, ws = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    assert _lib.load().ave_fp4_debug_nv_plan(m, n, k, cus, may_split, ctypes.byref(kernel), ctypes.byref(rows), ctypes.byref(slices),
+                                             ctypes.byref(per), ctypes.byref(ws)) == 0
+    return kernel.value, rows.value, slices.value, per.value, ws.value
+
+
+def test_streaming_plans_are_what_the_kernel_can_run():
+    """Every plan over a grid of shapes and devices: slices that all hold work and fit the compute units, a workspace of their sums."""
+    whole = cut = 0
+    for cus in (256, 64):
+        for m in (1, 16, 32, 33, 64, 65, 100, 128, 200, 513, 2048, 2049):
+            for n in (64, 512, 1792, 4096, 9216, 28672):
+                for k in (256, 512, 544, 2880, 4096, 7200, 13824, 16096):
+                    for swiglu, quant in ((0, 0), (1, 0), (1, 1)):
+                        shape = (m, n, k, swiglu, quant, cus)
+                        free, ws = _stream_plan(m, n, k, swiglu, quant, 0, cus), _stream_plan(m, n, k, swiglu, quant, 1, cus)
+                        assert free[1:] == (1, 0, 0), shape
+                        rows, slices, per, need = ws
+                        assert rows in (0, 32, 64, 128) and (rows or slices == 1), shape
+                        if rows == 0 and free[0] == 0:
+                            continue
+                        assert 512 <= k and m <= 2048 and (swiglu or m > 32), shape
+                        weight_rows, pairs = n * (2 if swiglu else 1), k // 512
+                        if slices > 1:
+                            cut += 1
+                            assert slices == -(-pairs // per) and (slices - 1) * per < pairs, shape
+                            assert slices * -(-m // rows) * -(-weight_rows // 128) <= cus, shape
+                            assert need == slices * m * weight_rows * 4, shape
+                        else:
+                            whole += 1
+                            assert (per, need) == (0, 0), shape
+                    if m <= 32 or m > 64:   # the fused forms cut K alike: quantising the one's result is the other
+                        assert _stream_plan(m, n, k, 1, 0, 1, cus)[1:] == _stream_plan(m, n, k, 1, 1, 1, cus)[1:], (m, n, k)
+    assert whole > 100 and cut > 100
+    # where the lines lie: slices for few weight rows, whole K for a K that costs the narrow-tile kernel a tail, the rings up to 32 rows
+    assert _stream_plan(128, 1792, 16096, 0, 0, 1)[1] > 1 and _stream_plan(62, 1792, 16096, 0, 0, 1)[1] > 1
+    assert _stream_plan(128, 9216, 8832, 0, 0, 1) == (64, 1, 0, 0) and _stream_plan(200, 128, 2880, 1, 1, 1) == (64, 1, 0, 0)
+    assert _stream_plan(64, 4096, 8192, 0, 0, 1)[0] == 0 and _stream_plan(32, 1792, 16096, 0, 0, 1)[0] == 0
+    assert _stream_plan(8192, 14336, 4096, 0, 0, 1)[0] == 0
+    assert _lib.load().ave_fp4_debug_stream_plan(64, 64, 512, 0, 0, 0, 0, None, None, None, None) == -1
+
+
+def test_nvfp4_plans_are_what_the_kernels_can_run():
+    seen = set()
+    for cus in (256, 64):
+        for m in (1, 16, 33, 64, 65, 128, 300, 1024, 4096):
+            for n in (64, 1000, 4096, 28672):
+                for k in (16, 256, 320, 512, 1024, 1040, 4096, 4176, 4992, 14336):
+                    for may_split in (0, 1):
+                        shape = (m, n, k, cus, may_split)
+                        kernel, rows, slices, per, need = _nv_plan(m, n, k, may_split, cus)
+                        seen.add((kernel, rows, slices > 1))
+                        if k < 256 or (k < 1024 and k % 256):
+                            assert kernel == 0, shape
+                        assert (kernel == 2) == (rows in (64, 128)) and (kernel != 1 or m <= 64), shape
+                        assert (kernel != 3 or k % 256 == 0) and (kernel != 4 or k % 64 == 0), shape
+                        if slices > 1:
+                            assert may_split and kernel in (2, 3), shape
+                            assert slices == -(-(k // 256) // per) and (slices - 1) * per < k // 256, shape
+                            assert slices * -(-m // rows) * -(-n // (128 if kernel == 2 else 256)) <= cus, shape
+                            assert need == slices * m * n * 4, shape
+                        else:
+                            assert (slices, per, need) == (1, 0, 0), shape
+    assert {kernel for kernel, _, _ in seen} >= {0, 1, 2, 3} and {(2, 64, True), (2, 128, True), (2, 64, False), (2, 128, False)} <= seen
+    # where the lines lie: rings, narrow tiles of either height, whole tiles; slices over a long K
+    assert [_nv_plan(*s, 0)[:2] for s in ((16, 28672, 4096), (64, 28672, 4096), (128, 28672, 4096), (1024, 4096, 4096))] == [
+        (1, 0), (2, 64), (2, 128), (2, 128)]
+    assert _nv_plan(4096, 4096, 14336, 1)[0] == 3 and _nv_plan(128, 4096, 14336, 1)[2] > 1 and _nv_plan(64, 5120, 13824, 1)[2] > 1
+    assert _lib.load().ave_fp4_debug_nv_plan(64, 64, 512, 0, 0, None, None, None, None, None) == -1
+
+
 def test_split_plans_beyond_the_allocation_free_scratch_are_replanned_under_it():
     """On 256 compute units some planned splits want more than the 32 MiB of partial sums that the allocation-free
     entry point holds (a few hundred rows against a K of 30000 and more).  Planned under that cap, every such shape
