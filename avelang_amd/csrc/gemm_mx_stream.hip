@@ -817,8 +817,9 @@ bool mx_swiglu_quant_in_two(int M, int N, int K, int cus) {
 //  * here: 3.3 + the larger of 0.42 - 0.5 a stage and the memory time, slices' sums 3.5 for the second launch and 7 TB/s there and back;
 //  * memory time: the weights at 7 TB/s and what is read again from L2 at 16 TB/s; a third more where rows do not start at whole
 //    128-byte lines.
-// Measured, before -> after: 128 x 1792 x 16096 52 -> 16 us, 128 x 9216 x 8832 26.8 -> 20.7, 62 x 1792 x 16096 18.5 -> 13.0,
-// 128 x 4096 x 14336 17.8 -> 15.8.
+// Measured on weights from HBM, before -> after: with a workspace 128 x 1792 x 16096 81 -> 21 us, 62 x 1792 x 16096 21.4 -> 17.1; K whole
+// 128 x 9216 x 8832 40.9 -> 31.5, without a workspace 128 x 4096 x 14336 44.7 -> 36.5 and 100 x 5120 x 13824 43.6 -> 35.0 (with one both
+// keep the narrow-tile kernel's slices, 19.3 and 19.8).
 MxStreamPlan mx_stream_plan(int M, int N, int K, bool swiglu, bool quant, int cus, bool may_split) {
   MxStreamPlan plan;
   if (cus <= 0) cus = 256;

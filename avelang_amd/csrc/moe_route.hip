@@ -1,7 +1,8 @@
 // The two steps in front of the grouped (MoE) GEMM, on the device so that the whole expert layer can
 // be recorded into one HIP graph:
 //
-//   route_top2_kernel   router logits [T, E] -> for every token its two highest-scoring experts, the
+//   route_choose_kernel, route_place_kernel
+//                       router logits [T, E] -> for every token its two highest-scoring experts, the
 //                       2T routed rows sorted by expert (stable: by token, then by rank) as a list of
 //                       token indices, the E+1 row offsets the grouped GEMM reads, and the softmax
 //                       probability of every routed row;

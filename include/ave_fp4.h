@@ -66,8 +66,8 @@ enum ave_fp4_variant {
                           per device, the weight tensors of its latest MXFP4 GEMMs: weights found among the most
                           recent ones that add up to 192 MB at most are taken to be in the 256 MB last-level cache
                           (one GEMM replayed on the same operands) and run as AVE_FP4_TILE, all others as this form */
-  AVE_FP4_SHORT = 7    /* MXFP4 plain GEMM only: 32x32 blocks of C, one wave each up to K = 512 and four waves that share K up
-                          to 2048, operands straight into registers; for small calls */
+  AVE_FP4_SHORT = 7    /* MXFP4 plain GEMM only: 32x32 blocks of C, four waves each that share K (up to 2048), operands straight
+                          into registers; for small calls */
 };
 
 /*
@@ -133,8 +133,9 @@ int ave_fp4_gemm_mxfp4_planned(const uint8_t* A, const uint8_t* A_scale, const u
  * MXFP4 gate+up GEMM with the SwiGLU activation fused into the epilogue:
  *   C[m, n] = silu(g) * u,  g = sum_k A[m,k] B[n,k],  u = sum_k A[m,k] B[N+n,k],  silu(x) = x / (1 + exp(-x)),
  * evaluated in fp32 on the fp32 accumulators, then rounded to bf16.  B [2N, K/2] and B_scale
- * [2N, K/32] hold the N gate rows followed by the N up rows; C is [M, N].  M <= 64 with N % 8 == 0
- * and K a multiple of 32 from 512 up runs on the weight-streaming kernel (AVE_FP4_DECODE); larger M with K % 512 == 0 and
+ * [2N, K/32] hold the N gate rows followed by the N up rows; C is [M, N].  M <= 32 with N % 8 == 0
+ * and K a multiple of 32 from 512 up runs on the weight-streaming kernel (AVE_FP4_DECODE); up to 64 rows on that or, where a model
+ * of their times says so, on 32- to 128-row tiles by 128 weight rows; larger M with K % 512 == 0 and
  * 16-byte-aligned scale tensors -- or any K that is a multiple of 32 from 512 up with 16-byte aligned A and B --
  * on the LDS-staged kernel (AVE_FP4_TILE: a tile is 256 rows by 128 outputs,
  * its gate and up values meet in LDS as fp32); any other shape on the shape-agnostic kernel (AVE_FP4_GENERIC).  Extends gemm_pipeline_transposed_b
@@ -219,8 +220,8 @@ int ave_fp4_grouped_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, cons
  * layer in one launch: rows row_offsets[e] .. row_offsets[e+1]-1 of A use expert e's weights B[e], which hold the N
  * gate rows followed by the N up rows (B [E, 2N, K/2], B_scale [E, 2N, K/32]); C is [total_M, N] bf16, or
  * Q [total_M, N/2] + Q_scale [total_M, N/32] with N % 32 == 0.  Every expert's rows equal what
- * ave_fp4_gemm_mxfp4_swiglu (ave_fp4_gemm_mxfp4_swiglu_quant) gives for that expert alone, bit for bit on the
- * same kernel.  K % 512 == 0 with 16-byte-aligned scale tensors, or another multiple of 32 from 512 up with
+ * ave_fp4_gemm_mxfp4_swiglu (ave_fp4_gemm_mxfp4_swiglu_quant) gives for that expert alone, bit for bit where that call adds up K
+ * in the same order: not where it cuts K into slices (its _ws form), nor up to 64 rows where it runs on the weight-streaming kernel.  K % 512 == 0 with 16-byte-aligned scale tensors, or another multiple of 32 from 512 up with
  * 16-byte-aligned A and B, takes the LDS-staged kernel; other K the shape-agnostic one (the _quant form then returns
  * AVE_FP4_EINVAL).  No counterpart in the reference.
  */
