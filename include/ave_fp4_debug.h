@@ -22,6 +22,10 @@ extern "C" {
  * 1: 256 x 128, 2: 128 x 128), and the workspace bytes (slices * M * N * 4, or 0). */
 int ave_fp4_debug_split_plan(int M, int N, int K, int compute_units, int* slices, int* slice_pairs, int* narrow_tiles,
                              size_t* workspace_bytes);
+/* The same plan when the partial sums may take at most max_workspace_bytes: the best split that fits, or none.  This is
+ * what ave_fp4_gemm_mxfp4_noalloc runs with max_workspace_bytes = AVE_FP4_NOALLOC_SCRATCH_BYTES. */
+int ave_fp4_debug_split_plan_capped(int M, int N, int K, int compute_units, size_t max_workspace_bytes, int* slices,
+                                    int* slice_pairs, int* narrow_tiles, size_t* workspace_bytes);
 /* Diagnostic and test hook: split K into slices of slice_pairs x 512 elements whatever the shape (K % 512 == 0,
  * 16-byte aligned scale tensors), on 256 x 256 tiles (narrow_tiles = 0) or on the 256 x 128 (1) or 128 x 128 (2)
  * tiles of AVE_FP4_NARROW; the workspace must hold ceil(K / 512 / slice_pairs) * M * N * 4 bytes. */
@@ -62,10 +66,6 @@ int ave_fp4_debug_nv_plan(int M, int N, int K, int compute_units, int may_split,
 int ave_fp4_debug_grouped_gemm_mxfp4_stream(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                                             const int32_t* row_offsets, uint16_t* C, uint8_t* Q, uint8_t* Q_scale, int total_M,
                                             int E, int N, int K, int swiglu, int tile_rows, void* hip_stream);
-/* The same plan when the partial sums may take at most max_workspace_bytes: the best split that fits, or none.  This is
- * what ave_fp4_gemm_mxfp4_noalloc runs with max_workspace_bytes = AVE_FP4_NOALLOC_SCRATCH_BYTES. */
-int ave_fp4_debug_split_plan_capped(int M, int N, int K, int compute_units, size_t max_workspace_bytes, int* slices,
-                                    int* slice_pairs, int* narrow_tiles, size_t* workspace_bytes);
 
 /*
  * Diagnostic, host only (no GPU needed): the output tile (tm, tn) that workgroup `pid` of the
