@@ -43,14 +43,23 @@ struct Geo {
   static constexpr int kALoads = HALF ? 4 : 8;              // 1 KB pieces of A per issuing wave and stage
   static constexpr int kDataLoads = kALoads + 4;
 };
-// a pair of stages: 256 A rows x 16 B, then B rows x 16 B in a 4 KB area of which the first 2 KB (128 rows) are
+// Scale rows.  Full form, a pair of stages: 256 A rows x 16 B, then B rows x 16 B in a 4 KB area of which the first 2 KB (128 rows) are
 // read; the second 2 KB receive what issuing waves 2 and 3 load (repeats of row 127), so that all four issuing
-// waves run the same two scale loads
+// waves run the same two scale loads.
+// HALF: chunks of 64 bytes a row, which are four pairs of stages: 128 A rows, then 128 B rows, in two buffers of 16 KB.  A load
+// instruction then touches 16 lines where 16-byte pieces touch 64 -- those were half of all lines that this form requested, and the
+// load path is what bounds it wherever the weights do not come from HBM alone (600 x 4096 x 14336: 34.3 us, without any scale loads
+// 26.7).  Four lanes fetch a row; a loading wave brings 16 of its 64 rows (A: waves 0 and 1, B: 2 and 3) with every pair of stages,
+// a whole chunk ahead.  Slot j of row r holds piece j ^ (r >> 2 & 3), so that the reads of 16 rows hit 16 different bank groups.
+// Measured, 16-byte pieces -> chunks, us: 600 x 4096 x 14336 34.3 -> 28.1, 1024 x 4096 x 14336 41.5 -> 33.3, 272 x 7680 x 10240 26.6 -> 22.2;
+// weights from HBM in one round (128 x 28672 x 4096) 18.4 -> 16.9.
 constexpr int kScalePair = 8192;
+constexpr int kScaleChunk = 16384;
 template <bool HALF>
-constexpr int kLds = Geo<HALF>::kScaleBase + 2 * kScalePair;   // 147456 / 163840
+constexpr int kLds = Geo<HALF>::kScaleBase + 2 * (HALF ? kScaleChunk : kScalePair);   // 163840 / 163840
 static_assert(kLds<false> <= 160 * 1024 && kLds<true> <= 160 * 1024, "LDS of one compute unit");
-constexpr int kScaleLoads = 2;   // loads of an issuing wave for one pair of scale rows
+template <bool HALF>
+constexpr int kScaleLoads = HALF ? 1 : 2;   // loads of an issuing wave that go out with a pair of stages
 
 // The loads of one issuing wave for one stage: eight 1 KB pieces of A to LDS addresses mda + 1024 i and four of B
 // to mdb + 1024 i, as one asm statement that the waves outside the issuing group (waves 0-3: 0, waves 4-7: 1) jump over.
@@ -211,7 +220,24 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     ga += kRowBytes;
     gb += kRowBytes;
   };
+  // HALF: 16 rows of a chunk; pieces behind the row's last whole pair are that pair's again (nobody reads them)
+  const int last_piece = p.K / (2 * BK) - 1;
+  auto issue_scale_part = [&](int chunk, int part) {
+    if (w < 4) return;
+    const int row = 16 * part + (lane >> 2);
+    int piece = k_pair0 + 4 * chunk + ((lane & 3) ^ ((lane >> 4) & 3));
+    piece = piece < last_piece ? piece : last_piece;
+    int am = m_begin + wi * 64 + row;
+    am = am < m_end ? am : m_end - 1;
+    const int r = wi < 2 ? am : b_image_row((wi & 1) * 64 + row);
+    dma16(wi < 2 ? p.As : p.Bs, (unsigned)r * row_scales + (unsigned)piece * 16,
+          lds_base + kScaleBase + (unsigned)((chunk & 1) * kScaleChunk + wi * 4096 + part * 1024));
+  };
   auto issue_scale_pair = [&](int pair) {
+    if constexpr (HALF) {   // (the fourth part of chunk 0 goes out with pair 0)
+      issue_scale_part((pair + 3) >> 2, (pair + 3) & 3);
+      return;
+    }
     dma16_scale_rows(w >> 2, issuers, lds_base + kScaleBase + (pair & 1) * kScalePair + (unsigned)wi * 1024, gas, gbs, as_off,
                      bs_off);
     gas += 16;
@@ -225,8 +251,13 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   const int b_row = wn * 64 + pi_row(rho);    // + 32 nj
   const unsigned a_frag = a_row * kRowBytes + (((4 * h) ^ ((a_row >> 1) & 7)) * 16);
   const unsigned b_frag = kOffB + b_row * kRowBytes + (((4 * h) ^ ((b_row >> 1) & 7)) * 16);
-  const unsigned a_sc = lds_base + kScaleBase + a_row * 16;             // + mi * 512
-  const unsigned b_sc = lds_base + kScaleBase + NM * 16 + b_row * 16;   // + nj * 512
+  // a fragment row's scales of pair 0, + mi (nj) * 32 rows
+  constexpr int kScaleRow = HALF ? 64 : 16;
+  const unsigned a_sc = lds_base + kScaleBase + a_row * kScaleRow + (HALF ? ((a_row >> 2) & 3) * 16 : 0);
+  const unsigned b_sc = lds_base + kScaleBase + (HALF ? kScaleChunk / 2 : NM * 16) + b_row * kScaleRow + (HALF ? ((b_row >> 2) & 3) * 16 : 0);
+  auto scale_at = [&](unsigned first, int pair) {
+    return HALF ? (first ^ (unsigned)((pair & 3) * 16)) + (unsigned)((pair >> 2) & 1) * kScaleChunk : first + (unsigned)(pair & 1) * kScalePair;
+  };
 
   v16f acc[2][2];
   v4i af0[2], bf0[2], af1[2], bf1[2];
@@ -237,8 +268,8 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   _Pragma("unroll") for (int i = 0; i < 2; ++i) dst_a[i] = lds_read16((sb) + (a_frag ^ ((KJ) * 16)) + i * 4096); \
   _Pragma("unroll") for (int i = 0; i < 2; ++i) dst_b[i] = lds_read16((sb) + (b_frag ^ ((KJ) * 16)) + i * 4096);
 #define AVE_READ_SCALE_PAIR(pair)                                                                              \
-  _Pragma("unroll") for (int i = 0; i < 2; ++i) as_pair[i] = lds_read16(a_sc + ((pair) & 1) * kScalePair + i * 512); \
-  _Pragma("unroll") for (int i = 0; i < 2; ++i) bs_pair[i] = lds_read16(b_sc + ((pair) & 1) * kScalePair + i * 512);
+  _Pragma("unroll") for (int i = 0; i < 2; ++i) as_pair[i] = lds_read16(scale_at(a_sc, pair) + i * 32 * kScaleRow); \
+  _Pragma("unroll") for (int i = 0; i < 2; ++i) bs_pair[i] = lds_read16(scale_at(b_sc, pair) + i * 32 * kScaleRow);
   // stage parity P of the pair, lane half h -> dword 2P + h of the row's 16 bytes
 #define AVE_PICK_SCALES(P)                                                                                   \
   _Pragma("unroll") for (int i = 0; i < 2; ++i) as_cur[i] = h ? as_pair[i][2 * (P) + 1] : as_pair[i][2 * (P)]; \
@@ -249,10 +280,15 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   // on the number of loads still outstanding: those issued after D(s+1), which are D(s+2) .. D(s+R-1) with the one
   // pair of scale rows that precedes an even stage among them -- fewer at the end of K.
   constexpr int kScaleIssueParity = kRing & 1;   // a stage of this parity issues a pair of scale rows with its data
-  constexpr int kWaitEven = (kRing - 2) * kDataLoads + kScaleLoads;
-  constexpr int kWaitOdd = (kRing - 2) * kDataLoads + (kRing == 4 ? kScaleLoads : 0);
+  constexpr int kWaitEven = (kRing - 2) * kDataLoads + kScaleLoads<HALF>;
+  constexpr int kWaitOdd = (kRing - 2) * kDataLoads + (kRing == 4 ? kScaleLoads<HALF> : 0);
   constexpr int kWaitTailOdd = kDataLoads;       // in front of the last two stages: D(stages-1) alone
   constexpr bool kTailIssues = kRing == 3;       // four stages from the end, stage s + R still exists for R = 3 only
+  if constexpr (HALF) {
+    issue_scale_part(0, 0);
+    issue_scale_part(0, 1);
+    issue_scale_part(0, 2);
+  }
   issue_scale_pair(0);
   issue_data(stage_buffer(0));
   issue_data(stage_buffer(1));
@@ -262,7 +298,7 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     if (kRing == 4) issue_data(stage_buffer(3));
   }
   // stage 0 has landed when only the loads issued behind it are outstanding
-  if (stages > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 1) * kDataLoads + kScaleLoads) : "memory");
+  if (stages > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 1) * kDataLoads + kScaleLoads<HALF>) : "memory");
   else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDataLoads) : "memory");
   __syncthreads();
   const bool loader = w >= 4 && upper_idle;
