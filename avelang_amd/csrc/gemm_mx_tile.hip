@@ -120,7 +120,7 @@ __device__ inline void mma_quarter(v16f (&acc)[4][2], const v4i (&bf)[4], const 
 // HBM -- a model's layers, each with weights of its own, as opposed to one GEMM replayed on operands that stay in the
 // last-level cache.  Same bits; 5 % faster on weights from HBM, 1.6 % slower on cache-resident ones (measured on
 // 8192 x 14336 x 4096), so the host chooses (launch_mx_tile).
-// CH = 4 (ungrouped pair-scale forms without touches, K % 2048 == 0; 0: 16-byte pieces per pair of stages): the scale
+// CH = 4 (ungrouped pair-scale forms without touches; 0: 16-byte pieces per pair of stages): the scale
 // rows are fetched 64 bytes at a time -- four pairs of stages -- instead of 16.  A row's scales are K / 32 bytes, 128
 // for K = 4096: with 16-byte pieces every pair of stages touches a cache line per row (512 lines for 8 KB), which costs
 // the load path as much as a tenth of the stage data does; four lanes per row touch each line twice per 4096 elements
@@ -129,14 +129,16 @@ __device__ inline void mma_quarter(v16f (&acc)[4][2], const v4i (&bf)[4], const 
 // 160 KB (so not for the forms that keep the experts' table or the touches' sink there): chunk c + 1 is requested
 // behind the barrier of the second-to-last stage of chunk c, when every wave has taken chunk c's last pair into
 // registers, and is read a stage later -- the lead the stage data has.  16-byte slot j of a row holds its piece
-// j ^ ((row >> 2) & 3) (on the source side), so that the 16 rows of a ds_read_b128 fall into 16 bank groups.
+// j ^ ((row >> 2) & 3) (on the source side), so that the 16 rows of a ds_read_b128 fall into 16 bank groups.  A last chunk of one to
+// three pairs (K no multiple of 2048) repeats the row's last piece: 272 x 20480 x 7680 54.7 -> 53.1 us, gate+up of 400 rows, 27648 x 5120,
+// 43.9 -> 43.1 against 16-byte pieces.
 template <bool SC16, bool SWIGLU = false, bool QUANT = false, bool SPLITK = false, bool TAIL = false, bool GROUPED = false,
           bool BLOCKED = false, bool TOUCH = false, int CH = 0>
 __global__ __launch_bounds__(kWaves * 64) void mx_tile_kernel(MxArgs p, int m_tiles, int n_tiles) {
   constexpr bool SC64 = CH != 0;   // chunked scale rows
   static_assert(CH == 0 || CH == 4, "scale rows per pair of stages, or in chunks of four pairs");
   static_assert(CH != 4 || (!GROUPED && !TOUCH), "four-pair chunks leave no LDS for the experts' table and the touches' sink");
-  static_assert(!SC64 || (SC16 && !SPLITK && !TAIL && !BLOCKED), "chunked scale rows: pair-scale forms on whole chunks");
+  static_assert(!SC64 || (SC16 && !SPLITK && !TAIL && !BLOCKED), "chunked scale rows: pair-scale forms");
   static_assert(!TOUCH || (SC16 && !SPLITK && !TAIL && !GROUPED && !BLOCKED), "touches: the grouped forms, and the ungrouped ones on whole pairs of stages");
   constexpr bool kTouches = GROUPED || TOUCH;
   static_assert(!BLOCKED || (SC16 && !SWIGLU && !SPLITK && !TAIL && !GROUPED), "blocked scales: the plain GEMM on whole pairs of stages");
@@ -367,8 +369,10 @@ __global__ __launch_bounds__(kWaves * 64) void mx_tile_kernel(MxArgs p, int m_ti
       const unsigned enable = (pair & 3) == 0 ? 1u : 0u;
       // (the row offsets are worked out at every call: a branch around them that the compiler can see makes it spill
       // 170 registers in the main loop)
-      const int wi = w & 3;
-      const int piece = (lane & 3) ^ ((lane >> 4) & 3);
+      // Behind the last whole chunk, where K is no multiple of 2048, a row's last piece stands in for those that it does not have.
+      const int wi = w & 3, left = p.K / (2 * BK) - 1 - pair;
+      int piece = (lane & 3) ^ ((lane >> 4) & 3);
+      piece = piece < left ? piece : left;
       unsigned ao[4], bo[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1145,12 +1149,12 @@ hipError_t launch_pair_form(const MxArgs& p, unsigned grid, hipStream_t s, int m
 // ... picked by what the launch needs: the grouped forms and the forms with touches keep the experts' table and the
 // touches' sink in LDS and fetch their scale rows per pair of stages (chunks of two pairs in the place of the two pair
 // buffers measured no faster there: 970-976 against 971-973 us on the 8-expert benchmark); the others take chunks of four
-// pairs when K is a multiple of 2048
+// pairs, the last one what is left
 template <bool SWIGLU, bool QUANT>
 hipError_t launch_pairs(const MxArgs& p, unsigned grid, hipStream_t s, int m_tiles, int n_tiles, bool touch) {
   if (p.row_offsets) return launch_pair_form<SWIGLU, QUANT, true, false, 0>(p, grid, s, m_tiles, n_tiles);
   if (touch) return launch_pair_form<SWIGLU, QUANT, false, true, 0>(p, grid, s, m_tiles, n_tiles);
-  if (p.K % (8 * BK) == 0 && !AVE_NO_SC64) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
+  if (!AVE_NO_SC64) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
   return launch_pair_form<SWIGLU, QUANT, false, false, 0>(p, grid, s, m_tiles, n_tiles);
 }
 }  // namespace
@@ -1177,7 +1181,11 @@ hipError_t launch_mx_tile(const MxArgs& p, hipStream_t s) {
   const int cus = persistent_workgroups();
   if (cus <= 0) return hipErrorInvalidDevice;
   const unsigned grid = (unsigned)(total < cus ? total : cus);
-  const bool touch = p.touch && !p.row_offsets && total > cus;   // more than one round of tiles: there is a next round to touch for
+  // Touches where there is a next round to touch for and its panels have a whole group of 32 m-tiles to share the work and the lines.
+  // With fewer rows the form without them, which has room for the 64-byte scale chunks, is the faster one, also with weights from
+  // HBM (with touches -> without, us): gate+up with SwiGLU and quantiser, 28672 x 4096, 1024 rows 70.7 -> 66.0, 2048 133.7 -> 127.9,
+  // 4096 235.8 -> 227.9, 6000 350 -> 340, but 8192 452.6 -> 470.5; plain 6000 x 4096 x 14336 176.5 -> 171.5, 8192 x 14336 x 4096 234.0 -> 249.6.
+  const bool touch = p.touch && !p.row_offsets && total > cus && m_tiles >= kXcds * kGroupM;
   if (p.swiglu) {
     if (tail_form(p)) {
       if (p.Q) return launch_form<true, true, true, true>(p, grid, kLdsBytes16, s, m_tiles, n_tiles);

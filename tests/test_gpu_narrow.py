@@ -49,6 +49,20 @@ def test_narrow_random_scales_every_kblock(gpu):
     H.assert_mx_close(c, a, a_s, b, b_s)
 
 
+@pytest.mark.parametrize("m,n,k", [(100, 300, 2048), (128, 128, 2560), (127, 264, 3584), (1, 136, 4096), (200, 1000, 6656), (65, 8, 8192)])
+def test_narrow_128_row_tiles_scale_chunks(gpu, m, n, k):
+    """128-row tiles fetch scale rows in chunks of four pairs of stages: one to four chunks, the last of one, three and four
+    pairs; scale bytes differ in every block, the 256 x 256 kernel gives the same bits."""
+    rng = np.random.default_rng(k)
+    a, a_s = H.mx_operand(m, k, seed=6)
+    b, b_s = H.mx_operand(n, k, seed=7, std=0.02)
+    a_s = (a_s.astype(np.int32) + rng.integers(-3, 4, size=a_s.shape)).clip(1, 254).astype(np.uint8)
+    b_s = (b_s.astype(np.int32) + rng.integers(-3, 4, size=b_s.shape)).clip(1, 254).astype(np.uint8)
+    c = H.run_mx(gpu, a, a_s, b, b_s, variant=NARROW)
+    H.assert_mx_close(c, a, a_s, b, b_s)
+    assert np.array_equal(c, H.run_mx(gpu, a, a_s, b, b_s, variant=TILE))
+
+
 def test_dispatch_takes_the_narrow_kernel_for_a_few_hundred_rows(gpu):
     """65..256 rows against many weight rows go to the narrow kernel by themselves: same bits as forcing it."""
     m, n, k = 128, 2048, 1024

@@ -111,6 +111,18 @@ def test_mx_tile_64_byte_scale_chunks_give_the_same_bits(gpu, m, n, k):
         H.assert_mx_close(c, a, a_s, b, b_s)
 
 
+@pytest.mark.parametrize("m,n,k", [(8192, 2304, 1536), (8200, 2304, 2560), (8192, 2304, 3584), (8192, 2304, 4608)])
+def test_mx_tile_scale_chunks_with_a_short_last_chunk(gpu, m, n, k):
+    """K of whole pairs of stages that is no multiple of 2048: a last chunk of three, one, three and one pairs, over the
+    persistent walk, against the form with touches (16-byte pieces): same bits, with scale bytes that differ in every block."""
+    rng = np.random.default_rng(k)
+    a, a_s = H.mx_operand(m, k, seed=52)
+    b, b_s = H.mx_operand(n, k, seed=53, std=0.02)
+    a_s = (a_s.astype(np.int32) + rng.integers(-3, 4, size=a_s.shape)).clip(1, 254).astype(np.uint8)
+    b_s = (b_s.astype(np.int32) + rng.integers(-3, 4, size=b_s.shape)).clip(1, 254).astype(np.uint8)
+    assert np.array_equal(H.run_mx(gpu, a, a_s, b, b_s, variant=TILE), H.run_mx(gpu, a, a_s, b, b_s, variant=6))
+
+
 def test_grouped_tile_persistent_with_empty_and_ragged_experts(gpu):
     """336 tile slots for 256 compute units: the tile loop skips the slots behind an expert's last tile and
     an expert without rows; every expert's rows equal the plain GEMM on that expert bit for bit."""
