@@ -13,8 +13,8 @@
 // barrier per stage: behind the barrier of stage j, which says that stage j has landed and stage j - 1 is consumed, stage j + ring - 1
 // is requested into the buffer of stage j - 1.  One workgroup per compute unit walks the tiles pid, pid + gridDim.x, ...
 //
-// Layout, swizzle, K order inside a stage and the epilogues are those of gemm_mx_narrow.hip; the scale rows of a pair of stages
-// (16 bytes) travel with its first stage into slots of their own.  K tail: stages = ceil(K / 256); in the last one 16-byte chunks behind
+// Layout, swizzle, K order inside a stage and the epilogues are those of gemm_mx_narrow.hip; the scale rows of one or two
+// pairs of stages (16 bytes each) travel with their first stage into slots of their own.  K tail: stages = ceil(K / 256); in the last one 16-byte chunks behind
 // the row's end repeat its last chunk, the 16 scale bytes are the row's last 16 (the row may be the tensor's last), and the
 // multiplying waves find them there and zero what is not in the row.
 #include <cmath>
@@ -31,7 +31,7 @@ constexpr int BN = 128, BK = 256;
 constexpr int kRowBytes = BK / 2;   // 128
 constexpr int kLoadWaves = 4;
 
-template <int R>   // rows of A per tile
+template <int R, bool CHUNKS>   // rows of A per tile; scale rows in chunks of two pairs of stages where LDS has room for them
 struct Geo {
   static constexpr int kWM = R == 128 ? 2 : 1;               // multiplying waves along M, R / kWM rows each
   static constexpr int kMI = R / 32 / kWM;                   // 32-row blocks of such a wave
@@ -40,17 +40,30 @@ struct Geo {
   static constexpr int kOffB = R * kRowBytes;
   static constexpr int kStage = kOffB + BN * kRowBytes;      // 20480 / 24576 / 32768
   static constexpr int kRing = R == 32 ? 7 : (R == 64 ? 6 : 4);
-  static constexpr int kScaleRows = R + BN;                  // of a pair of stages: A's, then B's, 16 bytes each
-  static constexpr int kSlot = kScaleRows * 16;              // 2560 / 3072 / 4096
-  // Pairs that stages j .. j + kRing - 1 touch at most (tiles of three stages: pairs of two and of one in turn).
-  static constexpr int kSlots = R == 128 ? 3 : 5;
+  // A chunk's 32 bytes of a row mostly lie in
+  // one line, so a load asks for half as many lines as with 16-byte pieces, which were a third of all that the kernel asked for.
+  // Slot j of row r holds piece j ^ (r >> 3 & 1): the rows of a read then fall into different banks.  For experts' weights from HBM
+  // (launch_grouped).  Measured, whole expert layers on weights from
+  // HBM, pairs -> chunks, us: 300 rows of 8 experts, 4096 / 14336, 187.0 -> 177.4; 64 rows 151.1 -> 148.2; 1000 rows of 128 experts,
+  // 2880 / 2880, 359.6 -> 351.4; 16 rows of 64, 7168 / 2048, 127.5 -> 126.7.  No gain on weights in
+  // the last-level cache (2000 rows of 16 experts, 2048 / 1024, 57.3 and 57.3).
+  static constexpr int kPairs = R == 64 || !CHUNKS ? 1 : 2;
+  static constexpr int kScaleRows = R + BN;                  // of a chunk: A's, then B's
+  static constexpr int kScaleRow = 16 * kPairs;
+  static constexpr int kSlot = kScaleRows * kScaleRow;       // chunks: 5120 / 3072 / 8192
+  // Chunks that stages j .. j + kRing - 1 touch at most, a work item having two stages or more: between a chunk's request and
+  // that of the one kSlots in front of it lie kSlots - 1 whole chunks, kRing - 1 stages or more (five stages: chunks of
+  // four and of one in turn; pairs, three stages: of two and of one).
+  static constexpr int kSlots = R == 128 ? 3 : (kPairs == 1 ? 5 : 4);
   static constexpr int kScaleBase = kRing * kStage;
-  static constexpr int kLds = kScaleBase + kSlots * kSlot;   // 156160 / 162816 / 143360
+  static constexpr int kLds = kScaleBase + kSlots * kSlot;   // chunks: 163840 / 162816 / 155648
   static constexpr int kALoads = R / 32;                     // 1 KB pieces (8 rows) of A per loading wave and stage
-  static constexpr int kData = kALoads + 4;                  // loads of a loading wave for a stage; one more with a pair's scales
-  static constexpr int kScaleLanes = kScaleRows / kLoadWaves;   // 40 / 48 / 64
+  static constexpr int kData = kALoads + 4;                  // loads of a loading wave for a stage; kPairs more with a chunk's scales
+  static constexpr int kWaveRows = kScaleRows / kLoadWaves;  // 40 / 48 / 64 scale rows of a loading wave
+  static constexpr int kLoadRows = 64 / kPairs;              // ... of which a load brings this many at most
 };
-static_assert(Geo<32>::kLds <= 160 * 1024 && Geo<64>::kLds <= 160 * 1024 && Geo<128>::kLds <= 160 * 1024, "LDS of one compute unit");
+static_assert(Geo<32, true>::kLds <= 160 * 1024 && Geo<64, true>::kLds <= 160 * 1024 && Geo<128, true>::kLds <= 160 * 1024, "LDS of one compute unit");
+static_assert(Geo<32, false>::kLds <= 160 * 1024 && Geo<64, false>::kLds <= 160 * 1024 && Geo<128, false>::kLds <= 160 * 1024, "LDS of one compute unit");
 
 __device__ inline int lds_read1(unsigned addr) {
   return *reinterpret_cast<const __attribute__((address_space(3))) unsigned char*>((uintptr_t)addr);
@@ -125,9 +138,9 @@ __device__ inline bool table_in_registers(const MxArgs& p) { return p.E <= 64 * 
 // otherwise (a "late" chunk), in either case in the slot that it has without SHIFT, so that reads stay free of bank conflicts.  Stage s waits for line
 // s + 1, one stage earlier than without; a tile whose last stage has late chunks takes one line more.  Chunks of a line that are not the
 // row's are not loaded.  Measured: 255 -> 220 us, with 2880 weight rows 131 -> 112.
-template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT, bool CHUNKS>
 __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const int (&g_r0)[kSets], const int (&g_r1)[kSets]) {
-  using G = Geo<R>;
+  using G = Geo<R, CHUNKS>;
   static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
   static_assert(!SPLITK || (!SWIGLU && !GROUPED), "K is split for the plain GEMM");
   static_assert(!SHIFT || GROUPED, "by lines: the experts' weights only");
@@ -231,7 +244,9 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     unsigned a_off[G::kALoads], b_off[4];
     int a_chunk[G::kALoads], b_chunk[4];
     unsigned a_late = 0, b_late = 0;   // SHIFT: bit i: this lane's chunk of load i is a late one
-    const uint8_t *ga = nullptr, *gb = nullptr, *gs = nullptr;
+    const uint8_t *ga = nullptr, *gb = nullptr, *gs[G::kPairs] = {};
+    const int s_piece = lane % G::kPairs;   // (of its slot; its piece of the row: s_from)
+    int s_from = 0;
     int s = 0, s_end = 0;      // stage (SHIFT: line) of the tile that goes out next, and the one behind its last
     unsigned to = lds_base, slot_to = lds_base + G::kScaleBase;
     unsigned with_scales = 0;  // bit i: the stage issued i stages ago brought a pair of scale rows
@@ -270,11 +285,17 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
         // (SHIFT: a late chunk is that of the stage before; the offsets are from one stage in front of line s)
         ga = p.A + (size_t)s * kRowBytes - (SHIFT ? kRowBytes : 0);
         gb = p.B + expert_rows * row_bytes + (size_t)s * kRowBytes - (SHIFT ? kRowBytes : 0);
-        const int sr = wi * G::kScaleLanes + (lane < G::kScaleLanes ? lane : 0);
-        int am = m_begin + sr;
-        am = am < m_end ? am : m_end - 1;
-        gs = sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
-        gs += (size_t)(s >> 1) * 16;
+#pragma unroll
+        for (int l = 0; l < G::kPairs; ++l) {
+          const int in_wave = l * G::kLoadRows + lane / G::kPairs;
+          const int sr = wi * G::kWaveRows + (in_wave < G::kWaveRows ? in_wave : 0);
+          int am = m_begin + sr;
+          am = am < m_end ? am : m_end - 1;
+          gs[l] = sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
+        }
+        // (kLoadRows is 0 or 32 mod 64 and kWaveRows a multiple of 8: the same piece in both loads)
+        if (G::kPairs == 1) gs[0] += (size_t)(s >> 1) * 16;
+        if (G::kPairs == 2) s_from = s_piece ^ ((wi * G::kWaveRows + lane / G::kPairs) >> 3 & 1);
       }
       if (!SHIFT && tail_blocks != 0 && s == stages - 1) {   // chunks behind the row's end: its last chunk again
 #pragma unroll
@@ -284,11 +305,20 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
         for (int i = 0; i < 4; ++i)
           if (b_chunk[i] >= tail_blocks) b_off[i] -= (unsigned)(b_chunk[i] - (tail_blocks - 1)) * 16;
       }
-      const bool scales = (s & 1) == 0 && (!SHIFT || s < s_last);
+      const bool scales = (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) && (!SHIFT || s < s_last);
       if (scales) {
-        if (pair_tail != 0 && s + 2 >= stages) gs -= 16 - pair_tail;   // (K >= 512: there are 16 bytes in front of the row's end)
-        load_scale_rows<G::kScaleLanes>(gs, __builtin_amdgcn_readfirstlane(slot_to) + (unsigned)wi * (G::kScaleLanes * 16));
-        gs += 16;
+        const unsigned first = __builtin_amdgcn_readfirstlane(slot_to) + (unsigned)wi * (G::kWaveRows * G::kScaleRow);
+        if constexpr (G::kPairs == 1) {
+          if (pair_tail != 0 && s + 2 >= stages) gs[0] -= 16 - pair_tail;   // (K >= 512: there are 16 bytes in front of the row's end)
+          load_scale_rows<G::kWaveRows>(gs[0], first);
+          gs[0] += 16;
+        } else {
+          // the last pair's piece, and those behind it, are the row's last 16 bytes
+          unsigned at = (unsigned)((s >> 1) + s_from) * 16;
+          at = at < row_scales - 16 ? at : row_scales - 16;
+          load_scale_rows<64>(gs[0] + at, first);
+          load_scale_rows<2 * (G::kWaveRows - G::kLoadRows)>(gs[1] + at, first + 1024);
+        }
         slot_to = slot_to + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot_to + G::kSlot;
       }
       with_scales = (with_scales << 1) | (scales ? 1u : 0u);
@@ -318,14 +348,14 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     for (int i = 0; i < G::kRing - 1 && more; ++i) more = issue();
     for (int j = 0; j < issued; ++j) {
       // Stage j (SHIFT: line j + 1) has landed when only the loads of the stages behind it are outstanding: `ahead` of them, each kData
-      // loads and one more for those that brought scale rows (fewer than there are is safe, and waits a little longer).
+      // loads and kPairs more for those that brought scale rows (fewer than there are is safe, and waits a little longer).
       constexpr int kAhead = G::kRing - 2 - (SHIFT ? 1 : 0);   // (while there is more to issue)
       const int ahead = __builtin_amdgcn_readfirstlane(issued - 1 - (SHIFT ? 1 : 0) - j);
       if (ahead >= kAhead) {
         const int c = __popc(__builtin_amdgcn_readfirstlane((int)(with_scales & ((1u << kAhead) - 1))));
-        if (c >= 3) wait_vm<kAhead * G::kData + 3>();
-        else if (c == 2) wait_vm<kAhead * G::kData + 2>();
-        else if (!SHIFT || c == 1) wait_vm<kAhead * G::kData + 1>();   // (not SHIFT: every two stages in a row hold the first stage of a pair)
+        if (c >= 3) wait_vm<kAhead * G::kData + 3 * G::kPairs>();
+        else if (c == 2) wait_vm<kAhead * G::kData + 2 * G::kPairs>();
+        else if ((G::kPairs == 1 && !SHIFT) || c == 1) wait_vm<kAhead * G::kData + G::kPairs>();   // (pairs, not SHIFT: every two stages in a row hold the first stage of a pair)
         else wait_vm<kAhead * G::kData>();
       } else if (ahead == 4) {
         wait_vm<4 * G::kData>();
@@ -352,7 +382,9 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
   const int b_row = wn * 64 + pi_row(rho);    // + 32 nj
   const unsigned a_frag = (unsigned)(a_row * kRowBytes + (((4 * h) ^ ((a_row >> 1) & 7)) * 16));
   const unsigned b_frag = (unsigned)(G::kOffB + b_row * kRowBytes + (((4 * h) ^ ((b_row >> 1) & 7)) * 16));
-  const unsigned a_sc = (unsigned)a_row * 16, b_sc = (unsigned)(R + b_row) * 16;   // in a slot, + 512 per 32 rows
+  // a row's piece 0 in a slot, + kScaleRow * 32 per 32 rows; piece 1 at the address with bit 4 the other way
+  const unsigned a_sc = (unsigned)(a_row * G::kScaleRow + (G::kPairs == 2 ? (a_row >> 3 & 1) * 16 : 0));
+  const unsigned b_sc = (unsigned)((R + b_row) * G::kScaleRow + (G::kPairs == 2 ? (b_row >> 3 & 1) * 16 : 0));
   unsigned sb = lds_base, slot = lds_base + G::kLds - G::kSlot;
   auto next_buffer = [&]() { sb = sb + G::kStage == lds_base + G::kScaleBase ? lds_base : sb + G::kStage; };
   while (next_tile()) {
@@ -382,11 +414,14 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
       for (int j = 0; j < MI; ++j) acc[i][j] = v16f{};
     int as_cur[MI], bs_cur[2];
     // the dword of a row's 16 scale bytes for stage parity P and this lane's half: 2 P + h
+    int s = s_first;
+    auto piece = [&]() { return G::kPairs == 2 ? (unsigned)((s - s_first) & 2) * 8 : 0u; };   // stage s: 0 or 16
     auto read_scales = [&](int P) {
+      const unsigned at = slot + (unsigned)(2 * P + h) * 4, as = a_sc ^ piece(), bs = b_sc ^ piece();
 #pragma unroll
-      for (int i = 0; i < MI; ++i) as_cur[i] = lds_read4(slot + a_sc + i * 512 + (unsigned)(2 * P + h) * 4);
+      for (int i = 0; i < MI; ++i) as_cur[i] = lds_read4(at + as + i * (32 * G::kScaleRow));
 #pragma unroll
-      for (int i = 0; i < 2; ++i) bs_cur[i] = lds_read4(slot + b_sc + i * 512 + (unsigned)(2 * P + h) * 4);
+      for (int i = 0; i < 2; ++i) bs_cur[i] = lds_read4(at + bs + i * (32 * G::kScaleRow));
     };
     v4i af[4][MI], bf[4][2];   // the fragments of a whole stage: all requested before the first is waited for
     auto read_frags = [&]() {
@@ -401,8 +436,9 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     };
     // stages of whole pairs end here
     const int whole = pair_tail == 0 || s_last < stages ? s_last : (stages - 1) & ~1;
-    auto next_slot = [&]() { slot = slot + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot + G::kSlot; };
-    int s = s_first;
+    auto next_slot = [&]() {   // a stage that starts a chunk
+      if (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) slot = slot + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot + G::kSlot;
+    };
     auto behind_the_last_stage = [&]() {
       if (late_at_end) {
         __syncthreads();
@@ -412,7 +448,7 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     if (G::kWM > 1 && m_begin + m_wave >= m_end) {   // no rows for this wave: the barriers and the positions, nothing else
       for (; s < s_last; ++s) {
         __syncthreads();
-        if ((s & 1) == 0) next_slot();
+        next_slot();
         next_buffer();
       }
       behind_the_last_stage();
@@ -420,7 +456,7 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     }
     for (; s < whole; ++s) {
       __syncthreads();   // the stage has landed
-      if ((s & 1) == 0) next_slot();
+      next_slot();
       read_scales(s & 1);
       read_frags();
 #pragma unroll
@@ -446,25 +482,25 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     // A block that is not there is zeros under the scale 2^0.
     for (; s < s_last; ++s) {
       __syncthreads();
-      if ((s & 1) == 0) next_slot();
+      next_slot();
       const int blocks = s == stages - 1 && tail_blocks != 0 ? tail_blocks : 8;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int block = p.tail_four_apart ? 4 * h + j : 2 * j + h;
         const bool have = block < blocks;
-        const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (have ? block : 0));
+        const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (have ? block : 0)), as = a_sc ^ piece(), bs = b_sc ^ piece();
         const v4i none = {0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
           const v4i f = lds_read16(sb + late(a_late[i], block) + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
-          const int sc = lds_read1(at + a_sc + i * 512);
+          const int sc = lds_read1(at + as + i * (32 * G::kScaleRow));
           af[j][i] = have ? f : none;
           as_cur[i] = have ? sc : 0x7f;
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const v4i f = lds_read16(sb + late(b_late[i], block) + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
-          const int sc = lds_read1(at + b_sc + i * 512);
+          const int sc = lds_read1(at + bs + i * (32 * G::kScaleRow));
           bf[j][i] = have ? f : none;
           bs_cur[i] = have ? sc : 0x7f;
         }
@@ -544,11 +580,11 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
   }
 }
 
-template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
-__global__ __launch_bounds__(Geo<R>::kThreads) void mx_stream_kernel(MxArgs p, int n_tiles) {
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT, bool CHUNKS>
+__global__ __launch_bounds__((Geo<R, CHUNKS>::kThreads)) void mx_stream_kernel(MxArgs p, int n_tiles) {
   int g_r0[kSets], g_r1[kSets];
   if (GROUPED && table_in_registers(p)) load_table(p, g_r0, g_r1);
-  stream_tiles<R, SWIGLU, QUANT, GROUPED, SPLITK, SHIFT>(p, n_tiles, g_r0, g_r1);
+  stream_tiles<R, SWIGLU, QUANT, GROUPED, SPLITK, SHIFT, CHUNKS>(p, n_tiles, g_r0, g_r1);
 }
 
 // Rows per tile for the experts' table as it is, from the `rows` that the host took for the average: an expert with more rows than a
@@ -585,11 +621,13 @@ __device__ __forceinline__ int rows_for_table(const int (&g_r0)[kSets], const in
 // (128-row tiles with a ring per tile before that), plain, us: 128 rows of 8 experts, 28672 x 4096, all in one expert 31.8 -> 20.0 (21.0);
 // 4096 x 14336, routed by 1 / rank 61.2 -> 42.0 (49.1); 2000 rows of 128 experts, 5760 x 2880, on a quarter of them 95.9 -> 78.7 (105), in
 // one 80.2 -> 36.7 (46.4), evenly 227.3 and 227.0 (327).
+template <bool CHUNKS>
+constexpr int kTallestLds = CHUNKS ? Geo<32, true>::kLds : Geo<64, false>::kLds;
 template <int R>
-constexpr bool fits_taller = Geo<R>::kThreads <= Geo<128>::kThreads && Geo<R>::kLds <= Geo<64>::kLds;
+constexpr bool fits_taller = Geo<R, true>::kThreads <= Geo<128, true>::kThreads && Geo<R, true>::kLds <= kTallestLds<true> && Geo<R, false>::kLds <= kTallestLds<false>;
 static_assert(fits_taller<32> && fits_taller<64> && fits_taller<128>);
-template <bool SWIGLU, bool QUANT, bool SHIFT>
-__global__ __launch_bounds__(Geo<128>::kThreads) void mx_stream_by_table_kernel(MxArgs p, int n_tiles, int rows, int by_table) {
+template <bool SWIGLU, bool QUANT, bool SHIFT, bool CHUNKS>
+__global__ __launch_bounds__((Geo<128, true>::kThreads)) void mx_stream_by_table_kernel(MxArgs p, int n_tiles, int rows, int by_table) {
   int g_r0[kSets], g_r1[kSets];
   if (table_in_registers(p)) {
     load_table(p, g_r0, g_r1);
@@ -597,11 +635,11 @@ __global__ __launch_bounds__(Geo<128>::kThreads) void mx_stream_by_table_kernel(
   }
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   if (rows == 128) {
-    stream_tiles<128, SWIGLU, QUANT, true, false, SHIFT>(p, n_tiles, g_r0, g_r1);
+    stream_tiles<128, SWIGLU, QUANT, true, false, SHIFT, CHUNKS>(p, n_tiles, g_r0, g_r1);
   } else if (rows == 64) {
-    if (wave < Geo<64>::kThreads / 64) stream_tiles<64, SWIGLU, QUANT, true, false, SHIFT>(p, n_tiles, g_r0, g_r1);
+    if (wave < Geo<64, true>::kThreads / 64) stream_tiles<64, SWIGLU, QUANT, true, false, SHIFT, CHUNKS>(p, n_tiles, g_r0, g_r1);
   } else {
-    if (wave < Geo<32>::kThreads / 64) stream_tiles<32, SWIGLU, QUANT, true, false, SHIFT>(p, n_tiles, g_r0, g_r1);
+    if (wave < Geo<32, true>::kThreads / 64) stream_tiles<32, SWIGLU, QUANT, true, false, SHIFT, CHUNKS>(p, n_tiles, g_r0, g_r1);
   }
 }
 
@@ -614,25 +652,26 @@ unsigned stream_grid(const MxArgs& p, int rows, int* n_tiles) {
   const long tiles = ((long)(p.M + rows - 1) / rows + (GROUPED ? p.E : 0)) * *n_tiles * (SPLITK ? p.slices : 1);
   return cus <= 0 ? 0 : (unsigned)(tiles < cus ? tiles : cus);
 }
-template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT>
+template <int R, bool SWIGLU, bool QUANT, bool GROUPED, bool SPLITK, bool SHIFT, bool CHUNKS>
 hipError_t launch(const MxArgs& p, hipStream_t s) {
   int n_tiles;
   const unsigned grid = stream_grid<SWIGLU, GROUPED, SPLITK>(p, R, &n_tiles);
   if (grid == 0) return hipErrorInvalidDevice;
-  constexpr auto kernel = mx_stream_kernel<R, SWIGLU, QUANT, GROUPED, SPLITK, SHIFT>;
-  if (hipError_t e = allow_dynamic_lds<kernel>(Geo<R>::kLds); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Geo<R>::kThreads), Geo<R>::kLds, s, p, n_tiles);
+  constexpr auto kernel = mx_stream_kernel<R, SWIGLU, QUANT, GROUPED, SPLITK, SHIFT, CHUNKS>;
+  using G = Geo<R, CHUNKS>;
+  if (hipError_t e = allow_dynamic_lds<kernel>(G::kLds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(G::kThreads), G::kLds, s, p, n_tiles);
   return hipGetLastError();
 }
-template <bool SWIGLU, bool QUANT, bool SHIFT>
+template <bool SWIGLU, bool QUANT, bool SHIFT, bool CHUNKS>
 hipError_t launch_grouped_lines(const MxArgs& p, int rows, hipStream_t s) {
-  if (rows == 128) return launch<128, SWIGLU, QUANT, true, false, SHIFT>(p, s);
+  if (rows == 128) return launch<128, SWIGLU, QUANT, true, false, SHIFT, CHUNKS>(p, s);
   int n_tiles;
   const unsigned grid = stream_grid<SWIGLU, true, false>(p, rows, &n_tiles);
   if (grid == 0) return hipErrorInvalidDevice;
-  constexpr auto kernel = mx_stream_by_table_kernel<SWIGLU, QUANT, SHIFT>;
-  if (hipError_t e = allow_dynamic_lds<kernel>(Geo<64>::kLds); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(Geo<128>::kThreads), Geo<64>::kLds, s, p, n_tiles, rows, p.rows_by_table);
+  constexpr auto kernel = mx_stream_by_table_kernel<SWIGLU, QUANT, SHIFT, CHUNKS>;
+  if (hipError_t e = allow_dynamic_lds<kernel>(kTallestLds<CHUNKS>); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3((Geo<128, true>::kThreads)), kTallestLds<CHUNKS>, s, p, n_tiles, rows, p.rows_by_table);
   return hipGetLastError();
 }
 // SHIFT for experts' weights whose rows do not all start at a cache line, from HBM and over a few lines: the start of a tile costs it
@@ -652,7 +691,10 @@ bool by_lines(const MxArgs& p) {
 }
 template <bool SWIGLU, bool QUANT>
 hipError_t launch_grouped(const MxArgs& p, int rows, hipStream_t s) {
-  return by_lines<SWIGLU>(p) ? launch_grouped_lines<SWIGLU, QUANT, true>(p, rows, s) : launch_grouped_lines<SWIGLU, QUANT, false>(p, rows, s);
+  if (by_lines<SWIGLU>(p)) return launch_grouped_lines<SWIGLU, QUANT, true, true>(p, rows, s);
+  // chunks of scale rows from the weights' size on where they come from HBM (Geo): both sides measured there
+  const bool from_hbm = (uint64_t)p.E * p.N * (SWIGLU ? 2 : 1) * (uint64_t)(p.K / 2) >= (64u << 20) || p.by_lines;
+  return from_hbm ? launch_grouped_lines<SWIGLU, QUANT, false, true>(p, rows, s) : launch_grouped_lines<SWIGLU, QUANT, false, false>(p, rows, s);
 }
 
 // silu(gate) * up of K slices' sums P[slices][M][2N] (N gate columns, then N up columns), added up in slice order: bf16 into C, or
@@ -716,7 +758,7 @@ hipError_t launch_split(const MxArgs& p, hipStream_t s) {
   MxArgs q = p;
   q.swiglu = 0;
   q.N = p.swiglu ? 2 * p.N : p.N;
-  if (hipError_t e = launch<R, false, false, false, true, false>(q, s); e != hipSuccess) return e;
+  if (hipError_t e = launch<R, false, false, false, true, false, false>(q, s); e != hipSuccess) return e;
   if (!p.swiglu) return launch_splitk_reduce(p.P, p.C, (size_t)p.M * (size_t)p.N, p.slices, s);
   const size_t blocks = ((size_t)p.M * (p.N / 8) + 255) / 256;
   const dim3 grid((unsigned)(blocks < 4096 ? blocks : 4096));
@@ -727,9 +769,9 @@ hipError_t launch_split(const MxArgs& p, hipStream_t s) {
 template <int R>
 hipError_t launch_form(const MxArgs& p, hipStream_t s) {
   if (p.P) return launch_split<R>(p, s);
-  if (p.swiglu && p.Q) return launch<R, true, true, false, false, false>(p, s);
-  if (p.swiglu) return launch<R, true, false, false, false, false>(p, s);
-  return launch<R, false, false, false, false, false>(p, s);
+  if (p.swiglu && p.Q) return launch<R, true, true, false, false, false, false>(p, s);
+  if (p.swiglu) return launch<R, true, false, false, false, false, false>(p, s);
+  return launch<R, false, false, false, false, false, false>(p, s);
 }
 
 }  // namespace

@@ -11,6 +11,7 @@ from oracle import fp4_oracle as orc
 from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
+NARROW = 4
 
 
 def _stream(gpu, ops, ro, n, tile_rows, swiglu, quant):
@@ -49,6 +50,50 @@ def test_stream_matches_oracle_and_its_own_fused_forms(gpu, rows, n, k, tile_row
             assert ok, (x, rep)
     want_q, want_s = quantize_mxfp4(fused)
     assert torch.equal(q, want_q) and torch.equal(qs, want_s)
+
+
+# chunks of two pairs of scale rows: items of two, three, five, six and nine stages, several to a workgroup, so that short chunks (one
+# stage, two stages) follow each other in the slots; scale bytes differ in every block, so a piece of another pair or row shows
+@pytest.mark.parametrize("k", [512, 672, 1056, 1536, 2144])
+@pytest.mark.parametrize("tile_rows", [32, 64, 128])
+def test_stream_scale_chunks_over_several_tiles(gpu, k, tile_rows):
+    e, n = 90, 384   # three n-tiles: 270 and more tiles on 256 compute units
+    rows = [1 + 7 * x % 40 for x in range(e)]
+    m = sum(rows)
+    ro = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    rng = np.random.default_rng(k)
+    a, a_s = H.mx_operand(m, k, seed=k)
+    b, b_s = H.mx_operand(e * n, k, seed=k + 1, std=0.05)
+    a_s = (a_s.astype(np.int32) + rng.integers(-3, 4, size=a_s.shape)).clip(1, 254).astype(np.uint8)
+    b_s = (b_s.astype(np.int32) + rng.integers(-3, 4, size=b_s.shape)).clip(1, 254).astype(np.uint8)
+    b, b_s = b.reshape(e, n, k // 2), b_s.reshape(e, n, k // 32)
+    ops = [H.to_dev(t, gpu) for t in (a, a_s, b, b_s)]
+    dro = torch.from_numpy(ro).to(gpu)
+    c = H.bits(_stream(gpu, ops, dro, n, tile_rows | 0x1000, 0, False))   # (the form for weights from HBM)
+    assert np.array_equal(c, H.bits(_stream(gpu, ops, dro, n, tile_rows, 0, False)))
+    for x in (0, 38, e - 1):
+        r0, r1 = int(ro[x]), int(ro[x + 1])
+        H.assert_mx_close(c[r0:r1], a[r0:r1], a_s[r0:r1], b[x], b_s[x])
+    for x in range(0, e, 7):   # the narrow-tile kernel adds up in this order
+        r0, r1 = int(ro[x]), int(ro[x + 1])
+        assert np.array_equal(c[r0:r1], H.run_mx(gpu, a[r0:r1], a_s[r0:r1], b[x], b_s[x], variant=NARROW)), x
+
+
+# weights just beyond 64 MB on K of two stages and a tail: chunks without the form by lines; and just below
+@pytest.mark.parametrize("k,n", [(672, 2240), (672, 2216), (992, 1504)])
+@pytest.mark.parametrize("tile_rows", [32, 64, 128])
+def test_stream_scale_chunks_by_the_weights_size(gpu, k, n, tile_rows):
+    e = 90
+    ro = np.arange(e + 1, dtype=np.int32) * 3
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(k + n)
+    a, b = (torch.randint(0, 256, (*s, k // 2), generator=gen, device=gpu, dtype=torch.uint8) for s in ((3 * e,), (e, n)))
+    a_s, b_s = (torch.randint(118, 130, (*s, k // 32), generator=gen, device=gpu, dtype=torch.uint8) for s in ((3 * e,), (e, n)))
+    c = H.bits(_stream(gpu, [a, a_s, b, b_s], torch.from_numpy(ro).to(gpu), n, tile_rows, 0, False))
+    for x in range(0, e, 8):
+        r = slice(3 * x, 3 * x + 3)
+        want = H.run_mx(gpu, *(t.cpu().numpy() for t in (a[r], a_s[r], b[x], b_s[x])), variant=NARROW)
+        assert np.array_equal(c[r], want), x
 
 
 # every offset of a row from its line (K / 32 mod 8), last stages that end in front of, at and behind a line's end, two to nine stages
