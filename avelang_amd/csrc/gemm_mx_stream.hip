@@ -44,7 +44,7 @@ struct Geo {
   // one line, so a load asks for half as many lines as with 16-byte pieces, which were a third of all that the kernel asked for.
   // Slot j of row r holds piece j ^ (r >> 3 & 1): the rows of a read then fall into different banks.  For experts' weights from HBM
   // (launch_grouped).  Measured, whole expert layers on weights from
-  // HBM, pairs -> chunks, us: 300 rows of 8 experts, 4096 / 14336, 187.0 -> 177.4; 64 rows 151.1 -> 148.2; 1000 rows of 128 experts,
+  // HBM, pairs -> chunks, us: 300 rows of 8 experts, 4096 / 14336, 187.0 -> 177.4; 64 rows 150.6 -> 148.2 - 150.4; 1000 rows of 128 experts,
   // 2880 / 2880, 359.6 -> 351.4; 16 rows of 64, 7168 / 2048, 127.5 -> 126.7.  No gain on weights in
   // the last-level cache (2000 rows of 16 experts, 2048 / 1024, 57.3 and 57.3).
   static constexpr int kPairs = R == 64 || !CHUNKS ? 1 : 2;
