@@ -244,12 +244,12 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     unsigned a_off[G::kALoads], b_off[4];
     int a_chunk[G::kALoads], b_chunk[4];
     unsigned a_late = 0, b_late = 0;   // SHIFT: bit i: this lane's chunk of load i is a late one
-    const uint8_t *ga = nullptr, *gb = nullptr, *gs[G::kPairs] = {};
-    const int s_piece = lane % G::kPairs;   // (of its slot; its piece of the row: s_from)
-    int s_from = 0;
+    const uint8_t *ga = nullptr, *gb = nullptr, *gs = nullptr;
+    [[maybe_unused]] const uint8_t* gs_up = nullptr;   // chunks: rows 32 .. of the wave's, and the piece of a row that this lane fetches
+    [[maybe_unused]] int s_from = 0;
     int s = 0, s_end = 0;      // stage (SHIFT: line) of the tile that goes out next, and the one behind its last
     unsigned to = lds_base, slot_to = lds_base + G::kScaleBase;
-    unsigned with_scales = 0;  // bit i: the stage issued i stages ago brought a pair of scale rows
+    unsigned with_scales = 0;  // bit i: the stage issued i stages ago brought scale rows
     int issued = 0;
     auto issue = [&]() {       // false: nothing left
       if (s == s_end) {
@@ -285,17 +285,24 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
         // (SHIFT: a late chunk is that of the stage before; the offsets are from one stage in front of line s)
         ga = p.A + (size_t)s * kRowBytes - (SHIFT ? kRowBytes : 0);
         gb = p.B + expert_rows * row_bytes + (size_t)s * kRowBytes - (SHIFT ? kRowBytes : 0);
-#pragma unroll
-        for (int l = 0; l < G::kPairs; ++l) {
-          const int in_wave = l * G::kLoadRows + lane / G::kPairs;
-          const int sr = wi * G::kWaveRows + (in_wave < G::kWaveRows ? in_wave : 0);
+        if constexpr (G::kPairs == 1) {
+          const int sr = wi * G::kWaveRows + (lane < G::kWaveRows ? lane : 0);
           int am = m_begin + sr;
           am = am < m_end ? am : m_end - 1;
-          gs[l] = sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
+          gs = sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
+          gs += (size_t)(s >> 1) * 16;
+        } else {
+          auto scale_row = [&](int in_wave) {
+            const int sr = wi * G::kWaveRows + (in_wave < G::kWaveRows ? in_wave : 0);
+            int am = m_begin + sr;
+            am = am < m_end ? am : m_end - 1;
+            return sr < R ? p.As + (size_t)am * row_scales : p.Bs + (expert_rows + (unsigned)b_image_row(sr - R)) * row_scales;
+          };
+          gs = scale_row(lane >> 1);
+          gs_up = scale_row(G::kLoadRows + (lane >> 1));
+          // (kLoadRows is 32 and kWaveRows a multiple of 8: the same piece in both loads)
+          s_from = (lane & 1) ^ ((wi * G::kWaveRows + (lane >> 1)) >> 3 & 1);
         }
-        // (kLoadRows is 0 or 32 mod 64 and kWaveRows a multiple of 8: the same piece in both loads)
-        if (G::kPairs == 1) gs[0] += (size_t)(s >> 1) * 16;
-        if (G::kPairs == 2) s_from = s_piece ^ ((wi * G::kWaveRows + lane / G::kPairs) >> 3 & 1);
       }
       if (!SHIFT && tail_blocks != 0 && s == stages - 1) {   // chunks behind the row's end: its last chunk again
 #pragma unroll
@@ -307,17 +314,17 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
       }
       const bool scales = (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) && (!SHIFT || s < s_last);
       if (scales) {
-        const unsigned first = __builtin_amdgcn_readfirstlane(slot_to) + (unsigned)wi * (G::kWaveRows * G::kScaleRow);
         if constexpr (G::kPairs == 1) {
-          if (pair_tail != 0 && s + 2 >= stages) gs[0] -= 16 - pair_tail;   // (K >= 512: there are 16 bytes in front of the row's end)
-          load_scale_rows<G::kWaveRows>(gs[0], first);
-          gs[0] += 16;
+          if (pair_tail != 0 && s + 2 >= stages) gs -= 16 - pair_tail;   // (K >= 512: there are 16 bytes in front of the row's end)
+          load_scale_rows<G::kWaveRows>(gs, __builtin_amdgcn_readfirstlane(slot_to) + (unsigned)wi * (G::kWaveRows * 16));
+          gs += 16;
         } else {
+          const unsigned first = __builtin_amdgcn_readfirstlane(slot_to) + (unsigned)wi * (G::kWaveRows * 32);
           // the last pair's piece, and those behind it, are the row's last 16 bytes
           unsigned at = (unsigned)((s >> 1) + s_from) * 16;
           at = at < row_scales - 16 ? at : row_scales - 16;
-          load_scale_rows<64>(gs[0] + at, first);
-          load_scale_rows<2 * (G::kWaveRows - G::kLoadRows)>(gs[1] + at, first + 1024);
+          load_scale_rows<64>(gs + at, first);
+          load_scale_rows<2 * (G::kWaveRows - G::kLoadRows)>(gs_up + at, first + 1024);
         }
         slot_to = slot_to + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot_to + G::kSlot;
       }
@@ -413,15 +420,23 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
 #pragma unroll
       for (int j = 0; j < MI; ++j) acc[i][j] = v16f{};
     int as_cur[MI], bs_cur[2];
-    // the dword of a row's 16 scale bytes for stage parity P and this lane's half: 2 P + h
-    int s = s_first;
-    auto piece = [&]() { return G::kPairs == 2 ? (unsigned)((s - s_first) & 2) * 8 : 0u; };   // stage s: 0 or 16
-    auto read_scales = [&](int P) {
-      const unsigned at = slot + (unsigned)(2 * P + h) * 4, as = a_sc ^ piece(), bs = b_sc ^ piece();
+    // The dword of a row's 16 scale bytes for stage parity P and this lane's half: 2 P + h; chunks: of the piece `piece` bytes into the
+    // slot.  (What differs between pairs and chunks is spelled out where it stands, with nothing of the chunks left in the pair forms:
+    // one expression for both made the compiler order the pair forms' address arithmetic differently, 1 - 4 % slower on 64- and
+    // 128-row tiles: gate+up with quantiser 70 x 2560 x 1792 7.72 -> 7.98 us, plain 100 x 4096 x 2048 7.97 -> 8.15.)
+    auto read_scales = [&](int P, [[maybe_unused]] unsigned piece) {
+      if constexpr (G::kPairs == 1) {
 #pragma unroll
-      for (int i = 0; i < MI; ++i) as_cur[i] = lds_read4(at + as + i * (32 * G::kScaleRow));
+        for (int i = 0; i < MI; ++i) as_cur[i] = lds_read4(slot + a_sc + i * 512 + (unsigned)(2 * P + h) * 4);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) bs_cur[i] = lds_read4(at + bs + i * (32 * G::kScaleRow));
+        for (int i = 0; i < 2; ++i) bs_cur[i] = lds_read4(slot + b_sc + i * 512 + (unsigned)(2 * P + h) * 4);
+      } else {
+        const unsigned at = slot + (unsigned)(2 * P + h) * 4, as = a_sc ^ piece, bs = b_sc ^ piece;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) as_cur[i] = lds_read4(at + as + i * 1024);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) bs_cur[i] = lds_read4(at + bs + i * 1024);
+      }
     };
     v4i af[4][MI], bf[4][2];   // the fragments of a whole stage: all requested before the first is waited for
     auto read_frags = [&]() {
@@ -436,9 +451,8 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     };
     // stages of whole pairs end here
     const int whole = pair_tail == 0 || s_last < stages ? s_last : (stages - 1) & ~1;
-    auto next_slot = [&]() {   // a stage that starts a chunk
-      if (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) slot = slot + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot + G::kSlot;
-    };
+    auto next_slot = [&]() { slot = slot + G::kSlot == lds_base + G::kLds ? lds_base + G::kScaleBase : slot + G::kSlot; };
+    int s = s_first;
     auto behind_the_last_stage = [&]() {
       if (late_at_end) {
         __syncthreads();
@@ -448,7 +462,7 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     if (G::kWM > 1 && m_begin + m_wave >= m_end) {   // no rows for this wave: the barriers and the positions, nothing else
       for (; s < s_last; ++s) {
         __syncthreads();
-        next_slot();
+        if (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) next_slot();
         next_buffer();
       }
       behind_the_last_stage();
@@ -456,8 +470,8 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     }
     for (; s < whole; ++s) {
       __syncthreads();   // the stage has landed
-      next_slot();
-      read_scales(s & 1);
+      if (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) next_slot();
+      read_scales(s & 1, G::kPairs == 1 ? 0u : (unsigned)((s - s_first) & 2) * 8);
       read_frags();
 #pragma unroll
       for (int nj = 0; nj < 2; ++nj)
@@ -482,25 +496,25 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
     // A block that is not there is zeros under the scale 2^0.
     for (; s < s_last; ++s) {
       __syncthreads();
-      next_slot();
+      if (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) next_slot();
       const int blocks = s == stages - 1 && tail_blocks != 0 ? tail_blocks : 8;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int block = p.tail_four_apart ? 4 * h + j : 2 * j + h;
         const bool have = block < blocks;
-        const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (have ? block : 0)), as = a_sc ^ piece(), bs = b_sc ^ piece();
+        const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (have ? block : 0));
         const v4i none = {0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
           const v4i f = lds_read16(sb + late(a_late[i], block) + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
-          const int sc = lds_read1(at + as + i * (32 * G::kScaleRow));
+          const int sc = lds_read1(at + (G::kPairs == 1 ? a_sc : a_sc ^ ((unsigned)((s - s_first) & 2) * 8)) + i * (32 * G::kScaleRow));
           af[j][i] = have ? f : none;
           as_cur[i] = have ? sc : 0x7f;
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const v4i f = lds_read16(sb + late(b_late[i], block) + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
-          const int sc = lds_read1(at + bs + i * (32 * G::kScaleRow));
+          const int sc = lds_read1(at + (G::kPairs == 1 ? b_sc : b_sc ^ ((unsigned)((s - s_first) & 2) * 8)) + i * (32 * G::kScaleRow));
           bf[j][i] = have ? f : none;
           bs_cur[i] = have ? sc : 0x7f;
         }
