@@ -862,10 +862,12 @@ int ave_fp4_debug_grouped_gemm_mxfp4_stream(const uint8_t* A, const uint8_t* A_s
   if (total_M == 0 || N == 0) return 0;
   if (!row_offsets) return fail_inval("null row_offsets pointer.");
   const bool by_lines = (tile_rows & AVE_FP4_DEBUG_BY_LINES) != 0;
-  tile_rows &= ~AVE_FP4_DEBUG_BY_LINES;
+  const int scale_chunks = (tile_rows & AVE_FP4_DEBUG_SCALE_CHUNKS) ? 1 : ((tile_rows & AVE_FP4_DEBUG_SCALE_PAIRS) ? -1 : 0);
+  tile_rows &= ~(AVE_FP4_DEBUG_BY_LINES | AVE_FP4_DEBUG_SCALE_CHUNKS | AVE_FP4_DEBUG_SCALE_PAIRS);
   if (tile_rows != 32 && tile_rows != 64 && tile_rows != 128) return fail_inval("tile_rows must be 32, 64 or 128, got %d.", tile_rows);
   ave::MxArgs p{A, A_scale, B, B_scale, Q ? nullptr : C, total_M, N, K, row_offsets, E, swiglu ? 1 : 0, Q, Q_scale};
   p.by_lines = by_lines ? 1 : 0;
+  p.scale_chunks = scale_chunks;
   if (!ave::mx_stream_supports(p)) return fail_inval("streaming kernel does not support total_M=%d N=%d K=%d.", total_M, N, K);
   return finish(ave::launch_mx_stream(p, tile_rows, static_cast<hipStream_t>(hip_stream)), "grouped mxfp4 streaming kernel");
 }

@@ -43,10 +43,8 @@ struct Geo {
   // A chunk's 32 bytes of a row mostly lie in
   // one line, so a load asks for half as many lines as with 16-byte pieces, which were a third of all that the kernel asked for.
   // Slot j of row r holds piece j ^ (r >> 3 & 1): the rows of a read then fall into different banks.  For experts' weights from HBM
-  // (launch_grouped).  Measured, whole expert layers on weights from
-  // HBM, pairs -> chunks, us: 300 rows of 8 experts, 4096 / 14336, 187.0 -> 177.4; 64 rows 150.6 -> 148.2 - 150.4; 1000 rows of 128 experts,
-  // 2880 / 2880, 359.6 -> 351.4; 16 rows of 64, 7168 / 2048, 127.5 -> 126.7.  No gain on weights in
-  // the last-level cache (2000 rows of 16 experts, 2048 / 1024, 57.3 and 57.3).
+  // (scale_chunks, with the figures).  Whole expert layers, pairs -> chunks, us: 300 rows of 8 experts, 4096 / 14336, 187.0 -> 177.4; 1000
+  // rows of 128 experts, 2880 / 2880, 359.6 -> 351.4; level at 64 rows of 8 experts.
   static constexpr int kPairs = R == 64 || !CHUNKS ? 1 : 2;
   static constexpr int kScaleRows = R + BN;                  // of a chunk: A's, then B's
   static constexpr int kScaleRow = 16 * kPairs;
@@ -703,12 +701,32 @@ bool by_lines(const MxArgs& p) {
   if (tail > unit && p.K <= 5 * BK && !p.by_lines) return false;
   return (uint64_t)p.M * row + 256 < (1ull << 32) && b_rows * row + 256 < (1ull << 32);   // room for the 128 bytes on top of an offset
 }
+// Scale rows in chunks of two pairs of stages: for experts' weights of 64 MB and more, which in a model of many layers come from HBM,
+// over so many stages that the lines saved outweigh the second load of a chunk (rows of one to three chunks have none to save).
+// Pairs -> chunks, 70 - 300 MB of weights, 4096 (K = 2880: 2880) weight rows, 4 / 14 (32-row tiles) and 50 / 100 rows (128-row tiles) of each
+// expert, time by chunks over time by pairs:
+//  * rows that start at a line, weights from HBM: K = 768 - 1536 0.99 - 1.01 (1280 beyond 256 MB 0.98 - 1.00), 1792 and 2048 0.97 - 1.00,
+//    2816 0.96 - 1.00, 4096 0.94 - 1.00, 14336 0.89 - 0.97;
+//  * the same weights still in the last-level cache (below 256 MB; a layer replayed alone): K = 768 - 1536 1.01 - 1.05, 2048 0.96 - 1.03,
+//    4096 0.98 - 1.05, 7168 0.93 - 1.00 -- the price of the rule up to K = 4096;
+//  * by lines, from HBM: 32-row tiles K = 1056 1.00 - 1.02, 1312 1.00 - 1.01, 1568 0.99 - 1.00, 2880 0.97 - 0.99; 128-row tiles K = 1056 - 1312
+//    1.00 - 1.06, 1696 1.01 - 1.03, 2080 0.98 - 1.03, 2880 0.98 - 1.01, 4256 0.97 - 0.99.
+template <bool SWIGLU>
+bool scale_chunks(const MxArgs& p, int rows, bool lines) {
+  if (p.scale_chunks != 0) return p.scale_chunks > 0;
+  if (p.by_lines) return true;
+  const uint64_t bytes = (uint64_t)p.E * p.N * (SWIGLU ? 2 : 1) * (uint64_t)(p.K / 2);
+  if (bytes < (64u << 20)) return false;
+  if (lines) return p.K > (rows == 128 ? 8 * BK : 6 * BK);
+  return p.K > (bytes > (256u << 20) ? 4 * BK : 6 * BK);
+}
 template <bool SWIGLU, bool QUANT>
 hipError_t launch_grouped(const MxArgs& p, int rows, hipStream_t s) {
-  if (by_lines<SWIGLU>(p)) return launch_grouped_lines<SWIGLU, QUANT, true, true>(p, rows, s);
-  // chunks of scale rows from the weights' size on where they come from HBM (Geo): both sides measured there
-  const bool from_hbm = (uint64_t)p.E * p.N * (SWIGLU ? 2 : 1) * (uint64_t)(p.K / 2) >= (64u << 20) || p.by_lines;
-  return from_hbm ? launch_grouped_lines<SWIGLU, QUANT, false, true>(p, rows, s) : launch_grouped_lines<SWIGLU, QUANT, false, false>(p, rows, s);
+  const bool lines = by_lines<SWIGLU>(p), chunks = scale_chunks<SWIGLU>(p, rows, lines);
+  if (lines && chunks) return launch_grouped_lines<SWIGLU, QUANT, true, true>(p, rows, s);
+  if (lines) return launch_grouped_lines<SWIGLU, QUANT, true, false>(p, rows, s);
+  if (chunks) return launch_grouped_lines<SWIGLU, QUANT, false, true>(p, rows, s);
+  return launch_grouped_lines<SWIGLU, QUANT, false, false>(p, rows, s);
 }
 
 // silu(gate) * up of K slices' sums P[slices][M][2N] (N gate columns, then N up columns), added up in slice order: bf16 into C, or

@@ -29,11 +29,13 @@ struct MxArgs {
                                //   expected to come from HBM rather than from the last-level cache)
   int tail_four_apart = 0;     // grouped streaming kernel: order of addition behind the last whole 512 elements of K, as in the
                                //   256 x 256 kernel (1) or as in the narrow-tile kernel (0)
-  int by_lines = 0;            // grouped streaming kernel: 1 = by cache lines of the rows whatever the sizes (as far as offsets have room)
+  int by_lines = 0;            // grouped streaming kernel: 1 = by cache lines of the rows whatever the sizes (as far as offsets have room),
+                               //   and scale rows in chunks
   int rows_by_table = 0;       // grouped streaming kernel: 1 = taller tiles than asked for where the experts' table is uneven
   int blocked_scales = 0;      // 1: As and Bs are in the 128 x 4 blocked layout (plain GEMM, K % 512 == 0): padded to
                                //   128 rows and 4 columns, 512-byte tiles in row-major tile order, scale (r, c) of a
                                //   tile at byte (r % 32) * 16 + (r / 32) * 4 + c
+  int scale_chunks = 0;        // grouped streaming kernel: scale rows in chunks (1) or by pairs of stages (-1) whatever the sizes
 };
 
 __host__ __device__ inline int q_row_cols(const MxArgs& p) { return p.q_n > 0 ? p.q_n : p.N; }

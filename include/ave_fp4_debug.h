@@ -61,8 +61,12 @@ int ave_fp4_debug_nv_plan(int M, int N, int K, int compute_units, int may_split,
 /* Diagnostic and test hook: the grouped MXFP4 GEMM on tiles of tile_rows (32, 64 or 128) rows of A by 128 weight rows, whatever the
  * shape (K a multiple of 32 from 512 up, 16-byte aligned A and B).  swiglu: B holds 2N rows per expert; with Q and Q_scale
  * (C null) the result is quantised, rows laid out for N columns.  tile_rows with AVE_FP4_DEBUG_BY_LINES added: in the form that
- * loads the rows by whole cache lines, where not all of them start at one (the same bits). */
+ * loads the rows by whole cache lines, where not all of them start at one, and the scale rows in chunks of 32 bytes (32- and 128-row
+ * tiles); with AVE_FP4_DEBUG_SCALE_CHUNKS or AVE_FP4_DEBUG_SCALE_PAIRS added: the scale rows in such chunks, or 16 bytes at a time.  The
+ * same bits in every form. */
 #define AVE_FP4_DEBUG_BY_LINES 0x1000
+#define AVE_FP4_DEBUG_SCALE_CHUNKS 0x2000
+#define AVE_FP4_DEBUG_SCALE_PAIRS 0x4000
 int ave_fp4_debug_grouped_gemm_mxfp4_stream(const uint8_t* A, const uint8_t* A_scale, const uint8_t* B, const uint8_t* B_scale,
                                             const int32_t* row_offsets, uint16_t* C, uint8_t* Q, uint8_t* Q_scale, int total_M,
                                             int E, int N, int K, int swiglu, int tile_rows, void* hip_stream);

@@ -12,6 +12,7 @@ from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
 NARROW = 4
+BY_LINES, CHUNKS, PAIRS = 0x1000, 0x2000, 0x4000   # include/ave_fp4_debug.h
 
 
 def _stream(gpu, ops, ro, n, tile_rows, swiglu, quant):
@@ -79,7 +80,7 @@ def test_stream_scale_chunks_over_several_tiles(gpu, k, tile_rows):
         assert np.array_equal(c[r0:r1], H.run_mx(gpu, a[r0:r1], a_s[r0:r1], b[x], b_s[x], variant=NARROW)), x
 
 
-# weights just beyond 64 MB on K of two stages and a tail: chunks without the form by lines; and just below
+# chunks without the form by lines on K of two stages and a tail, around 64 MB of weights
 @pytest.mark.parametrize("k,n", [(672, 2240), (672, 2216), (992, 1504)])
 @pytest.mark.parametrize("tile_rows", [32, 64, 128])
 def test_stream_scale_chunks_by_the_weights_size(gpu, k, n, tile_rows):
@@ -89,11 +90,47 @@ def test_stream_scale_chunks_by_the_weights_size(gpu, k, n, tile_rows):
     gen.manual_seed(k + n)
     a, b = (torch.randint(0, 256, (*s, k // 2), generator=gen, device=gpu, dtype=torch.uint8) for s in ((3 * e,), (e, n)))
     a_s, b_s = (torch.randint(118, 130, (*s, k // 32), generator=gen, device=gpu, dtype=torch.uint8) for s in ((3 * e,), (e, n)))
-    c = H.bits(_stream(gpu, [a, a_s, b, b_s], torch.from_numpy(ro).to(gpu), n, tile_rows, 0, False))
+    c = H.bits(_stream(gpu, [a, a_s, b, b_s], torch.from_numpy(ro).to(gpu), n, tile_rows | CHUNKS, 0, False))
     for x in range(0, e, 8):
         r = slice(3 * x, 3 * x + 3)
         want = H.run_mx(gpu, *(t.cpu().numpy() for t in (a[r], a_s[r], b[x], b_s[x])), variant=NARROW)
         assert np.array_equal(c[r], want), x
+
+
+# two (one chunk), five (chunks of four and one in turn, the tightest use of the slots, with and without a tail), eight and nine stages;
+# 270 tiles and more
+@pytest.mark.parametrize("k", [512, 1120, 1280, 2048, 2304])
+@pytest.mark.parametrize("tile_rows", [32, 128])
+def test_stream_scale_chunks_and_pairs_give_the_same_bits_in_every_form(gpu, k, tile_rows):
+    e, n = 90, 192
+    ro = torch.arange(e + 1, dtype=torch.int32, device=gpu) * 5
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(k)
+    a, b = (torch.randint(0, 256, (*s, k // 2), generator=gen, device=gpu, dtype=torch.uint8) for s in ((5 * e,), (e, 2 * n)))
+    a_s, b_s = (torch.randint(118, 130, (*s, k // 32), generator=gen, device=gpu, dtype=torch.uint8) for s in ((5 * e,), (e, 2 * n)))
+    for cols, swiglu, quant in ((2 * n, 0, False), (n, 1, False), (n, 1, True)):
+        want = _stream(gpu, (a, a_s, b, b_s), ro, cols, tile_rows | PAIRS, swiglu, quant)
+        for flags in (CHUNKS, BY_LINES, BY_LINES | PAIRS):   # (by lines: where rows do not all start at one)
+            got = _stream(gpu, (a, a_s, b, b_s), ro, cols, tile_rows | flags, swiglu, quant)
+            for x, y in zip(want, got) if quant else ((want, got),):
+                assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), flags
+
+
+# weights of 64 MB and more on both sides of the rule: rows at lines K = 1536 | 1792, by lines K = 1056 | 1568 (32 rows a tile), 2080 (128)
+@pytest.mark.parametrize("k,n", [(1536, 4400), (1792, 3776), (1056, 6368), (1568, 4288), (2080, 3232)])
+@pytest.mark.parametrize("tile_rows", [32, 128])
+def test_stream_scale_rows_by_rule(gpu, k, n, tile_rows):
+    e = 20
+    ro = torch.arange(e + 1, dtype=torch.int32, device=gpu) * 3
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(k)
+    a, b = (torch.randint(0, 256, (*s, k // 2), generator=gen, device=gpu, dtype=torch.uint8) for s in ((3 * e,), (e, n)))
+    a_s, b_s = (torch.randint(118, 130, (*s, k // 32), generator=gen, device=gpu, dtype=torch.uint8) for s in ((3 * e,), (e, n)))
+    assert b.numel() >= 64 << 20
+    got = [_stream(gpu, (a, a_s, b, b_s), ro, n, tile_rows | flags, 0, False).view(torch.int16) for flags in (0, CHUNKS, PAIRS)]
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    want = H.run_mx(gpu, *(t.cpu().numpy() for t in (a[-3:], a_s[-3:], b[-1], b_s[-1])), variant=NARROW)
+    assert np.array_equal(H.bits(got[0][-3:].view(torch.bfloat16)), want)
 
 
 # every offset of a row from its line (K / 32 mod 8), last stages that end in front of, at and behind a line's end, two to nine stages
