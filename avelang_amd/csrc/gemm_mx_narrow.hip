@@ -11,7 +11,8 @@
 // Everything else follows gemm_mx_tile.hip: global -> LDS with global_load_lds_dwordx4 issued by waves 0-3,
 // source-side XOR swizzle, scales as 16-byte rows per pair of stages, eight waves (two per SIMD), here of
 // 64 (m) x 64 (n) each = 2 x 2 accumulator blocks of v_mfma_scale_f32_32x32x64_f8f6f4, the barrier of a stage in
-// front of its last K quarter.  K % 512 == 0, 16-byte aligned scale tensors.
+// front of its last K quarter.  16-byte aligned scale tensors; K of any multiple of 32 from 512 up (slices of K: of whole 512s).  In
+// tiles without upper rows (HALF, and the last ones of a matrix) waves 4-7 load; long K on 128-row tiles: scale rows in 64-byte chunks.
 //
 // SWIGLU: B holds the N gate rows followed by the N up rows and a tile is 256 rows of C by 64 outputs.  The 64
 // B-image rows of wave (wm, wn) are the gate rows (first 32) and the up rows (last 32) of outputs 32 wn .. 32 wn + 31,
@@ -43,23 +44,22 @@ struct Geo {
   static constexpr int kALoads = HALF ? 4 : 8;              // 1 KB pieces of A per issuing wave and stage
   static constexpr int kDataLoads = kALoads + 4;
 };
-// Scale rows.  Full form, a pair of stages: 256 A rows x 16 B, then B rows x 16 B in a 4 KB area of which the first 2 KB (128 rows) are
+// Scale rows.  By pairs of stages: 256 A rows x 16 B, then B rows x 16 B in a 4 KB area of which the first 2 KB (128 rows) are
 // read; the second 2 KB receive what issuing waves 2 and 3 load (repeats of row 127), so that all four issuing
 // waves run the same two scale loads.
-// HALF: chunks of 64 bytes a row, which are four pairs of stages: 128 A rows, then 128 B rows, in two buffers of 16 KB.  A load
-// instruction then touches 16 lines where 16-byte pieces touch 64 -- those were half of all lines that this form requested, and the
-// load path is what bounds it wherever the weights do not come from HBM alone (600 x 4096 x 14336: 34.3 us, without any scale loads
-// 26.7).  Four lanes fetch a row; a loading wave brings 16 of its 64 rows (A: waves 0 and 1, B: 2 and 3) with every pair of stages,
-// a whole chunk ahead.  Slot j of row r holds piece j ^ (r >> 2 & 3), so that the reads of 16 rows hit 16 different bank groups.
-// Measured, 16-byte pieces -> chunks, us: 600 x 4096 x 14336 34.3 -> 28.1, 1024 x 4096 x 14336 41.5 -> 33.3, 272 x 7680 x 10240 26.6 -> 22.2;
-// weights from HBM in one round (128 x 28672 x 4096) 18.4 -> 16.9.
+// CHUNKS (128-row tiles): 64 bytes a row, which are four pairs of stages: 128 A rows, then 128 B rows, in two buffers of 16 KB.  A load
+// instruction then touches 16 lines where 16-byte pieces touch 64 -- those are half as many as the data lines, and the
+// load path is what bounds this form wherever the weights do not come from HBM alone (600 x 4096 x 14336: 34.3 us, without any scale
+// loads 26.7).  Four lanes fetch a row; a loading wave brings 16 of its 64 rows (A: waves 0 and 1, B: 2 and 3) with every pair of stages:
+// three parts of a chunk with the pairs in front of it, the fourth with the chunk's first pair.  Slot j of row r holds piece
+// j ^ (r >> 2 & 3), so that the reads of 16 rows hit 16 different bank groups.  Where they pay: scale_chunks.
 constexpr int kScalePair = 8192;
 constexpr int kScaleChunk = 16384;
-template <bool HALF>
-constexpr int kLds = Geo<HALF>::kScaleBase + 2 * (HALF ? kScaleChunk : kScalePair);   // 163840 / 163840
-static_assert(kLds<false> <= 160 * 1024 && kLds<true> <= 160 * 1024, "LDS of one compute unit");
-template <bool HALF>
-constexpr int kScaleLoads = HALF ? 1 : 2;   // loads of an issuing wave that go out with a pair of stages
+template <bool HALF, bool CHUNKS>
+constexpr int kLds = Geo<HALF>::kScaleBase + 2 * (CHUNKS ? kScaleChunk : kScalePair);   // full 163840, HALF 147456, chunks 163840
+static_assert(kLds<false, false> <= 160 * 1024 && kLds<true, false> <= 160 * 1024 && kLds<true, true> <= 160 * 1024, "LDS of one compute unit");
+template <bool CHUNKS>
+constexpr int kScaleLoads = CHUNKS ? 1 : 2;   // loads of an issuing wave that go out with a pair of stages
 
 // The loads of one issuing wave for one stage: eight 1 KB pieces of A to LDS addresses mda + 1024 i and four of B
 // to mdb + 1024 i, as one asm statement that the waves outside the issuing group (waves 0-3: 0, waves 4-7: 1) jump over.
@@ -130,13 +130,14 @@ __device__ inline void mma_quarter(v16f (&acc)[2][2], const v4i (&bf)[2], const 
   }                                                           \
   __builtin_amdgcn_sched_barrier(0);
 
-template <bool SWIGLU, bool QUANT = false, bool SPLITK = false, bool HALF = false>
+template <bool SWIGLU, bool QUANT = false, bool SPLITK = false, bool HALF = false, bool CHUNKS = false>
 __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, int n_tiles) {
   using G = Geo<HALF>;
   constexpr int kRowsTile = G::kRows, kOffB = G::kOffB, kStage = G::kStage, kRing = G::kRing, kScaleBase = G::kScaleBase;
   constexpr int kDataLoads = G::kDataLoads;
   static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
   static_assert(!SPLITK || !SWIGLU, "K is split for the plain GEMM");
+  static_assert(HALF || !CHUNKS, "the full form's ring leaves no LDS for chunks");
   constexpr int kTileN = SWIGLU ? NN / 2 : NN;   // output columns per tile
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x;
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     ga += kRowBytes;
     gb += kRowBytes;
   };
-  // HALF: 16 rows of a chunk; pieces behind the row's last whole pair are that pair's again (nobody reads them)
+  // chunks: 16 rows of one; pieces behind the row's last whole pair are that pair's again (nobody reads them)
   const int last_piece = p.K / (2 * BK) - 1;
   auto issue_scale_part = [&](int chunk, int part) {
     if (w < 4) return;
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
           lds_base + kScaleBase + (unsigned)((chunk & 1) * kScaleChunk + wi * 4096 + part * 1024));
   };
   auto issue_scale_pair = [&](int pair) {
-    if constexpr (HALF) {   // (the fourth part of chunk 0 goes out with pair 0)
+    if constexpr (CHUNKS) {   // (the fourth part of chunk 0 goes out with pair 0)
       issue_scale_part((pair + 3) >> 2, (pair + 3) & 3);
       return;
     }
@@ -252,11 +253,11 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   const unsigned a_frag = a_row * kRowBytes + (((4 * h) ^ ((a_row >> 1) & 7)) * 16);
   const unsigned b_frag = kOffB + b_row * kRowBytes + (((4 * h) ^ ((b_row >> 1) & 7)) * 16);
   // a fragment row's scales of pair 0, + mi (nj) * 32 rows
-  constexpr int kScaleRow = HALF ? 64 : 16;
-  const unsigned a_sc = lds_base + kScaleBase + a_row * kScaleRow + (HALF ? ((a_row >> 2) & 3) * 16 : 0);
-  const unsigned b_sc = lds_base + kScaleBase + (HALF ? kScaleChunk / 2 : NM * 16) + b_row * kScaleRow + (HALF ? ((b_row >> 2) & 3) * 16 : 0);
+  constexpr int kScaleRow = CHUNKS ? 64 : 16;
+  const unsigned a_sc = lds_base + kScaleBase + a_row * kScaleRow + (CHUNKS ? ((a_row >> 2) & 3) * 16 : 0);
+  const unsigned b_sc = lds_base + kScaleBase + (CHUNKS ? kScaleChunk / 2 : NM * 16) + b_row * kScaleRow + (CHUNKS ? ((b_row >> 2) & 3) * 16 : 0);
   auto scale_at = [&](unsigned first, int pair) {
-    return HALF ? (first ^ (unsigned)((pair & 3) * 16)) + (unsigned)((pair >> 2) & 1) * kScaleChunk : first + (unsigned)(pair & 1) * kScalePair;
+    return CHUNKS ? (first ^ (unsigned)((pair & 3) * 16)) + (unsigned)((pair >> 2) & 1) * kScaleChunk : first + (unsigned)(pair & 1) * kScalePair;
   };
 
   v16f acc[2][2];
@@ -280,11 +281,11 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
   // on the number of loads still outstanding: those issued after D(s+1), which are D(s+2) .. D(s+R-1) with the one
   // pair of scale rows that precedes an even stage among them -- fewer at the end of K.
   constexpr int kScaleIssueParity = kRing & 1;   // a stage of this parity issues a pair of scale rows with its data
-  constexpr int kWaitEven = (kRing - 2) * kDataLoads + kScaleLoads<HALF>;
-  constexpr int kWaitOdd = (kRing - 2) * kDataLoads + (kRing == 4 ? kScaleLoads<HALF> : 0);
+  constexpr int kWaitEven = (kRing - 2) * kDataLoads + kScaleLoads<CHUNKS>;
+  constexpr int kWaitOdd = (kRing - 2) * kDataLoads + (kRing == 4 ? kScaleLoads<CHUNKS> : 0);
   constexpr int kWaitTailOdd = kDataLoads;       // in front of the last two stages: D(stages-1) alone
   constexpr bool kTailIssues = kRing == 3;       // four stages from the end, stage s + R still exists for R = 3 only
-  if constexpr (HALF) {
+  if constexpr (CHUNKS) {
     issue_scale_part(0, 0);
     issue_scale_part(0, 1);
     issue_scale_part(0, 2);
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(512) void mx_narrow_kernel(MxArgs p, int m_tiles, i
     if (kRing == 4) issue_data(stage_buffer(3));
   }
   // stage 0 has landed when only the loads issued behind it are outstanding
-  if (stages > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 1) * kDataLoads + kScaleLoads<HALF>) : "memory");
+  if (stages > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 1) * kDataLoads + kScaleLoads<CHUNKS>) : "memory");
   else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDataLoads) : "memory");
   __syncthreads();
   const bool loader = w >= 4 && upper_idle;
@@ -553,20 +554,33 @@ bool mx_narrow_preferred(const MxArgs& p) {
 }
 
 namespace {
-template <bool SWIGLU, bool QUANT, bool HALF>
+template <bool SWIGLU, bool QUANT, bool HALF, bool CHUNKS>
 hipError_t launch_narrow(const MxArgs& p, hipStream_t s, int n_tiles) {
+  constexpr auto kernel = mx_narrow_kernel<SWIGLU, QUANT, false, HALF, CHUNKS>;
   const int m_tiles = (p.M + Geo<HALF>::kRows - 1) / Geo<HALF>::kRows;
-  if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<SWIGLU, QUANT, false, HALF>>(kLds<HALF>); e != hipSuccess) return e;
-  hipLaunchKernelGGL((mx_narrow_kernel<SWIGLU, QUANT, false, HALF>), dim3((unsigned)((long)m_tiles * n_tiles)), dim3(512), kLds<HALF>, s, p,
-                     m_tiles, n_tiles);
+  if (hipError_t e = allow_dynamic_lds<kernel>(kLds<HALF, CHUNKS>); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((long)m_tiles * n_tiles)), dim3(512), (kLds<HALF, CHUNKS>), s, p, m_tiles, n_tiles);
   return hipGetLastError();
 }
-template <bool HALF>
+template <bool HALF, bool CHUNKS>
 hipError_t launch_narrow_form(const MxArgs& p, hipStream_t s, int n_tiles) {
-  if (p.swiglu && p.Q) return launch_narrow<true, true, HALF>(p, s, n_tiles);
-  if (p.swiglu) return launch_narrow<true, false, HALF>(p, s, n_tiles);
-  return launch_narrow<false, false, HALF>(p, s, n_tiles);
+  if (p.swiglu && p.Q) return launch_narrow<true, true, HALF, CHUNKS>(p, s, n_tiles);
+  if (p.swiglu) return launch_narrow<true, false, HALF, CHUNKS>(p, s, n_tiles);
+  return launch_narrow<false, false, HALF, CHUNKS>(p, s, n_tiles);
 }
+// 128-row tiles: scale rows in chunks from K = 3072 up, from 5120 where one row of tiles takes more than three quarters of the compute units.  The
+// four parts of the first chunk that go out in front of the first stage cost 0.25 - 0.4 us, which a short K does not earn back.  Time by
+// chunks over time by pairs, weights from HBM | replayed from the last-level cache:
+//  * up to 192 tiles a row (70 - 600 rows): K = 512 1.05 - 1.11 | 1.05 - 1.10, 1024 1.04 - 1.06 | 1.04 - 1.06, 2048 0.97 - 1.04 | 1.02 - 1.06, 2560 0.95 -
+//    1.02 | 1.01 - 1.05, 2816 0.98 - 1.03 | 1.03 - 1.07, 3072 0.93 - 1.00 | 0.98 - 1.07, 4096 0.89 - 0.98 | 0.91 - 1.02, 8192 0.85 - 0.95 | 0.87 -
+//    1.04, 14336 0.85 - 0.90 | 0.79 - 0.91;
+//  * 216 to 256 tiles in one row, on eight cards: K = 3072 0.97 - 1.07 | 1.00 - 1.20, 4096 0.95 - 1.07 (on average 1.01) | 0.96 - 1.18, 5120
+//    0.93 - 1.03 | 0.96 - 1.31, 6144 0.92 - 1.01 | 0.95 - 1.28, 8192 0.93 - 1.05 | 0.94 - 1.25, 14336 0.88 - 0.96 | 0.94 - 1.11: a full chip's
+//    weights of 60 MB and more, replayed alone, come from the cache more slowly in chunks on some cards; why was not found (turning the
+//    order of the parts from tile to tile changes nothing).
+// us, pairs -> chunks: 600 x 4096 x 14336 34.3 -> 28.1, 1024 x 4096 x 14336 41.5 -> 33.3, 272 x 7680 x 10240 26.6 -> 22.2; 100 x 4096 x 512, which
+// is by pairs, 4.56 -> 4.88.  Slices of K are in chunks whatever their length (one to ten pairs: 0.89 - 1.07 | 0.92 - 1.07, on average 0.96 | 0.99).
+bool scale_chunks(const MxArgs& p, int n_tiles, int cus) { return p.K >= (4L * n_tiles > 3L * cus ? 20 : 12) * BK; }
 }  // namespace
 
 // 128-row tiles (waves 0-3 multiply, waves 4-7 load, a ring of four stages) where no tile would have upper rows
@@ -577,22 +591,23 @@ hipError_t launch_mx_narrow(const MxArgs& p, hipStream_t s) {
   const int n_tiles = (p.N + tile_n - 1) / tile_n;
   // 128-row tiles also for more rows while they do not outnumber the compute units: twice the workgroups
   const int cus = compute_units();
-  if (p.M <= 128 || (cus > 0 && (long)((p.M + 127) / 128) * n_tiles <= cus)) return launch_narrow_form<true>(p, s, n_tiles);
-  return launch_narrow_form<false>(p, s, n_tiles);
+  if (p.M <= 128 || (cus > 0 && (long)((p.M + 127) / 128) * n_tiles <= cus))
+    return scale_chunks(p, n_tiles, cus) ? launch_narrow_form<true, true>(p, s, n_tiles) : launch_narrow_form<true, false>(p, s, n_tiles);
+  return launch_narrow_form<false, false>(p, s, n_tiles);
 }
 
 hipError_t launch_mx_narrow_splitk(const MxArgs& p, hipStream_t s) {
   const int n_tiles = (p.N + NN - 1) / NN;
   if (p.M <= 128 || p.half_rows) {
     const int m_tiles = (p.M + 127) / 128;
-    if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<false, false, true, true>>(kLds<true>); e != hipSuccess) return e;
-    hipLaunchKernelGGL((mx_narrow_kernel<false, false, true, true>), dim3((unsigned)(m_tiles * n_tiles * p.slices)),
-                       dim3(512), kLds<true>, s, p, m_tiles, n_tiles);
+    constexpr auto kernel = mx_narrow_kernel<false, false, true, true, true>;
+    if (hipError_t e = allow_dynamic_lds<kernel>(kLds<true, true>); e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(m_tiles * n_tiles * p.slices)), dim3(512), (kLds<true, true>), s, p, m_tiles, n_tiles);
   } else {
     const int m_tiles = (p.M + NM - 1) / NM;
-    if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<false, false, true>>(kLds<false>); e != hipSuccess) return e;
+    if (hipError_t e = allow_dynamic_lds<mx_narrow_kernel<false, false, true>>(kLds<false, false>); e != hipSuccess) return e;
     hipLaunchKernelGGL((mx_narrow_kernel<false, false, true>), dim3((unsigned)(m_tiles * n_tiles * p.slices)), dim3(512),
-                       kLds<false>, s, p, m_tiles, n_tiles);
+                       (kLds<false, false>), s, p, m_tiles, n_tiles);
   }
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   return launch_splitk_reduce(p.P, p.C, (size_t)p.M * (size_t)p.N, p.slices, s);

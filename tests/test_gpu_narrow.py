@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from avelang_amd import _lib, gemm_mxfp4_transposed_b
+from avelang_amd import _lib, gemm_mxfp4_swiglu_transposed_b, gemm_mxfp4_transposed_b
 from oracle import fp4_oracle as orc
 from tests import helpers as H
 
@@ -49,10 +49,11 @@ def test_narrow_random_scales_every_kblock(gpu):
     H.assert_mx_close(c, a, a_s, b, b_s)
 
 
-@pytest.mark.parametrize("m,n,k", [(100, 300, 2048), (128, 128, 2560), (127, 264, 3584), (1, 136, 4096), (200, 1000, 6656), (65, 8, 8192)])
+@pytest.mark.parametrize("m,n,k", [(100, 300, 2048), (128, 128, 2560), (127, 264, 3584), (1, 136, 4096), (200, 1000, 6656), (65, 8, 8192),
+                                   (127, 264, 3072)])
 def test_narrow_128_row_tiles_scale_chunks(gpu, m, n, k):
-    """128-row tiles fetch scale rows in chunks of four pairs of stages: one to four chunks, the last of one, three and four
-    pairs; scale bytes differ in every block, the 256 x 256 kernel gives the same bits."""
+    """128-row tiles fetch scale rows in chunks of four pairs of stages from six pairs (K = 3072) up: two to four chunks, the
+    last of one to four pairs; below, by pairs.  Scale bytes differ in every block, the 256 x 256 kernel gives the same bits."""
     rng = np.random.default_rng(k)
     a, a_s = H.mx_operand(m, k, seed=6)
     b, b_s = H.mx_operand(n, k, seed=7, std=0.02)
@@ -61,6 +62,20 @@ def test_narrow_128_row_tiles_scale_chunks(gpu, m, n, k):
     c = H.run_mx(gpu, a, a_s, b, b_s, variant=NARROW)
     H.assert_mx_close(c, a, a_s, b, b_s)
     assert np.array_equal(c, H.run_mx(gpu, a, a_s, b, b_s, variant=TILE))
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 136, 3040), (100, 264, 3072), (129, 72, 3104), (65, 200, 4576), (100, 13360, 4608), (100, 13360, 5120)])
+def test_narrow_128_row_tiles_with_a_k_tail_and_fused_forms(gpu, m, n, k):
+    """By pairs (3040, and 4608 on 209 tiles) and in chunks with and without a K tail, plain and with the fused SwiGLU; scale bytes
+    differ in every block."""
+    rng = np.random.default_rng(k)
+    a, a_s = H.mx_operand(m, k, seed=8)
+    b, b_s = H.mx_operand(2 * n, k, seed=9, std=0.05)
+    a_s, b_s = ((s.astype(np.int32) + rng.integers(-3, 4, size=s.shape)).clip(1, 254).astype(np.uint8) for s in (a_s, b_s))
+    H.assert_mx_close(H.run_mx(gpu, a, a_s, b, b_s, variant=NARROW), a, a_s, b, b_s)
+    fused = gemm_mxfp4_swiglu_transposed_b(*(H.to_dev(t, gpu) for t in (a, a_s, b, b_s)), variant=NARROW)
+    ok, rep = orc.check_swiglu_bf16(H.bits(fused), a, a_s, b, b_s)
+    assert ok, rep
 
 
 def test_dispatch_takes_the_narrow_kernel_for_a_few_hundred_rows(gpu):
