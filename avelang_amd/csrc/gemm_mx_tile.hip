@@ -40,10 +40,6 @@
 #include "tile_common.hpp"
 #include "tile_map.hpp"
 
-#ifndef AVE_NO_SC64
-#define AVE_NO_SC64 0   // 1: build without the 64-byte scale chunk forms (A/B measurements)
-#endif
-
 namespace ave {
 namespace {
 
@@ -129,15 +125,16 @@ __device__ inline void mma_quarter(v16f (&acc)[4][2], const v4i (&bf)[4], const 
 // 160 KB (so not for the forms that keep the experts' table or the touches' sink there): chunk c + 1 is requested
 // behind the barrier of the second-to-last stage of chunk c, when every wave has taken chunk c's last pair into
 // registers, and is read a stage later -- the lead the stage data has.  16-byte slot j of a row holds its piece
-// j ^ ((row >> 2) & 3) (on the source side), so that the 16 rows of a ds_read_b128 fall into 16 bank groups.  A last chunk of one to
-// three pairs (K no multiple of 2048) repeats the row's last piece: 272 x 20480 x 7680 54.7 -> 53.1 us, gate+up of 400 rows, 27648 x 5120,
-// 43.9 -> 43.1 against 16-byte pieces.
+// j ^ ((row >> 2) & 3) (on the source side), so that the 16 rows of a ds_read_b128 fall into 16 bank groups.  PART: K is no
+// multiple of 2048, and the last chunk, of one to three pairs, repeats the row's last piece (a form of its own,
+// because the clamp in the main loop cost whole chunks 0.5 - 1.4 %: 8192 x 14336 x 4096 241.2 -> 242.4 us, 1500 x 12288 x 4096 54.2 -> 54.9).
 template <bool SC16, bool SWIGLU = false, bool QUANT = false, bool SPLITK = false, bool TAIL = false, bool GROUPED = false,
-          bool BLOCKED = false, bool TOUCH = false, int CH = 0>
+          bool BLOCKED = false, bool TOUCH = false, int CH = 0, bool PART = false>
 __global__ __launch_bounds__(kWaves * 64) void mx_tile_kernel(MxArgs p, int m_tiles, int n_tiles) {
   constexpr bool SC64 = CH != 0;   // chunked scale rows
   static_assert(CH == 0 || CH == 4, "scale rows per pair of stages, or in chunks of four pairs");
   static_assert(CH != 4 || (!GROUPED && !TOUCH), "four-pair chunks leave no LDS for the experts' table and the touches' sink");
+  static_assert(SC64 || !PART, "a part of a chunk");
   static_assert(!SC64 || (SC16 && !SPLITK && !TAIL && !BLOCKED), "chunked scale rows: pair-scale forms");
   static_assert(!TOUCH || (SC16 && !SPLITK && !TAIL && !GROUPED && !BLOCKED), "touches: the grouped forms, and the ungrouped ones on whole pairs of stages");
   constexpr bool kTouches = GROUPED || TOUCH;
@@ -369,10 +366,12 @@ __global__ __launch_bounds__(kWaves * 64) void mx_tile_kernel(MxArgs p, int m_ti
       const unsigned enable = (pair & 3) == 0 ? 1u : 0u;
       // (the row offsets are worked out at every call: a branch around them that the compiler can see makes it spill
       // 170 registers in the main loop)
-      // Behind the last whole chunk, where K is no multiple of 2048, a row's last piece stands in for those that it does not have.
-      const int wi = w & 3, left = p.K / (2 * BK) - 1 - pair;
+      const int wi = w & 3;
       int piece = (lane & 3) ^ ((lane >> 4) & 3);
-      piece = piece < left ? piece : left;
+      if constexpr (PART) {   // behind the last whole chunk a row's last piece stands in for those that it does not have
+        const int left = p.K / (2 * BK) - 1 - pair;
+        piece = piece < left ? piece : left;
+      }
       unsigned ao[4], bo[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1138,24 +1137,24 @@ bool mx_tile_blocked_supports(const MxArgs& p) {
 namespace {
 // one pair-scale form on whole pairs of stages: SWIGLU / QUANT epilogue, grouped or not, with or without touches, scale
 // rows in chunks of CH pairs (0: per pair)
-template <bool SWIGLU, bool QUANT, bool GROUPED, bool TOUCH, int CH>
+template <bool SWIGLU, bool QUANT, bool GROUPED, bool TOUCH, int CH, bool PART = false>
 hipError_t launch_pair_form(const MxArgs& p, unsigned grid, hipStream_t s, int m_tiles, int n_tiles) {
   constexpr int lds_bytes = CH == 4 ? kLdsBytes64 : kLdsBytes16;
-  if (hipError_t e = allow_dynamic_lds<mx_tile_kernel<true, SWIGLU, QUANT, false, false, GROUPED, false, TOUCH, CH>>(lds_bytes); e != hipSuccess) return e;
-  hipLaunchKernelGGL((mx_tile_kernel<true, SWIGLU, QUANT, false, false, GROUPED, false, TOUCH, CH>), dim3(grid), dim3(kWaves * 64), lds_bytes, s,
-                     p, m_tiles, n_tiles);
+  constexpr auto kernel = mx_tile_kernel<true, SWIGLU, QUANT, false, false, GROUPED, false, TOUCH, CH, PART>;
+  if (hipError_t e = allow_dynamic_lds<kernel>(lds_bytes); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kWaves * 64), lds_bytes, s, p, m_tiles, n_tiles);
   return hipGetLastError();
 }
 // ... picked by what the launch needs: the grouped forms and the forms with touches keep the experts' table and the
 // touches' sink in LDS and fetch their scale rows per pair of stages (chunks of two pairs in the place of the two pair
 // buffers measured no faster there: 970-976 against 971-973 us on the 8-expert benchmark); the others take chunks of four
-// pairs, the last one what is left
+// pairs, the last one what is left (272 x 20480 x 7680 54.7 -> 53.1 us, gate+up of 400 rows, 27648 x 5120, 43.9 -> 43.1)
 template <bool SWIGLU, bool QUANT>
 hipError_t launch_pairs(const MxArgs& p, unsigned grid, hipStream_t s, int m_tiles, int n_tiles, bool touch) {
   if (p.row_offsets) return launch_pair_form<SWIGLU, QUANT, true, false, 0>(p, grid, s, m_tiles, n_tiles);
   if (touch) return launch_pair_form<SWIGLU, QUANT, false, true, 0>(p, grid, s, m_tiles, n_tiles);
-  if (!AVE_NO_SC64) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
-  return launch_pair_form<SWIGLU, QUANT, false, false, 0>(p, grid, s, m_tiles, n_tiles);
+  if (p.K % (8 * BK) == 0) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
+  return launch_pair_form<SWIGLU, QUANT, false, false, 4, true>(p, grid, s, m_tiles, n_tiles);
 }
 }  // namespace
 
