@@ -126,7 +126,7 @@ __device__ inline void mma_quarter(v16f (&acc)[4][2], const v4i (&bf)[4], const 
 // behind the barrier of the second-to-last stage of chunk c, when every wave has taken chunk c's last pair into
 // registers, and is read a stage later -- the lead the stage data has.  16-byte slot j of a row holds its piece
 // j ^ ((row >> 2) & 3) (on the source side), so that the 16 rows of a ds_read_b128 fall into 16 bank groups.  PART: K is no
-// multiple of 2048, and the last chunk, of one to three pairs, repeats the row's last piece (a form of its own,
+// multiple of 2048, and the last chunk, of one to three pairs, repeats the row's last piece (launch_pairs: from which K; a form of its own,
 // because the clamp in the main loop cost whole chunks 0.5 - 1.4 %: 8192 x 14336 x 4096 241.2 -> 242.4 us, 1500 x 12288 x 4096 54.2 -> 54.9).
 template <bool SC16, bool SWIGLU = false, bool QUANT = false, bool SPLITK = false, bool TAIL = false, bool GROUPED = false,
           bool BLOCKED = false, bool TOUCH = false, int CH = 0, bool PART = false>
@@ -1148,13 +1148,18 @@ hipError_t launch_pair_form(const MxArgs& p, unsigned grid, hipStream_t s, int m
 // ... picked by what the launch needs: the grouped forms and the forms with touches keep the experts' table and the
 // touches' sink in LDS and fetch their scale rows per pair of stages (chunks of two pairs in the place of the two pair
 // buffers measured no faster there: 970-976 against 971-973 us on the 8-expert benchmark); the others take chunks of four
-// pairs, the last one what is left (272 x 20480 x 7680 54.7 -> 53.1 us, gate+up of 400 rows, 27648 x 5120, 43.9 -> 43.1)
+// pairs for whole chunks and from K = 3584 up, where the last chunk is what is left: with fewer stages the loads of a part of a chunk that
+// is not there, and eight of them in front of the first stage where pairs have two, cost more than the lines saved.  Time by chunks over
+// time by pairs, K no multiple of 2048, 1024 - 8192 rows, plain and SwiGLU, weights from HBM | from the last-level cache: K = 512 1.01 - 1.03 |
+// 1.00 - 1.04, 1024 1.00 - 1.02 | 1.01 - 1.03, 1536 0.98 - 1.02 | 0.97 - 1.03, 2560 0.99 - 1.02 | 0.96 - 1.04, 3072 0.99 - 1.01 | 0.97 - 1.02, 3584
+// 0.98 - 1.00 | 0.99 - 1.03, 4608 0.97 - 1.00 | 0.99 - 1.03, 7680 0.92 - 0.99 | 0.99 - 1.01, 13824 0.89 - 1.00 | 0.99 - 1.01.
 template <bool SWIGLU, bool QUANT>
 hipError_t launch_pairs(const MxArgs& p, unsigned grid, hipStream_t s, int m_tiles, int n_tiles, bool touch) {
   if (p.row_offsets) return launch_pair_form<SWIGLU, QUANT, true, false, 0>(p, grid, s, m_tiles, n_tiles);
   if (touch) return launch_pair_form<SWIGLU, QUANT, false, true, 0>(p, grid, s, m_tiles, n_tiles);
   if (p.K % (8 * BK) == 0) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
-  return launch_pair_form<SWIGLU, QUANT, false, false, 4, true>(p, grid, s, m_tiles, n_tiles);
+  if (p.K >= 14 * BK) return launch_pair_form<SWIGLU, QUANT, false, false, 4, true>(p, grid, s, m_tiles, n_tiles);
+  return launch_pair_form<SWIGLU, QUANT, false, false, 0>(p, grid, s, m_tiles, n_tiles);
 }
 }  // namespace
 

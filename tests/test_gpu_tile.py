@@ -111,10 +111,12 @@ def test_mx_tile_64_byte_scale_chunks_give_the_same_bits(gpu, m, n, k):
         H.assert_mx_close(c, a, a_s, b, b_s)
 
 
-@pytest.mark.parametrize("m,n,k", [(8192, 2304, 1536), (8200, 2304, 2560), (8192, 2304, 3584), (8192, 2304, 4608)])
+@pytest.mark.parametrize("m,n,k", [(8192, 2304, 1536), (8200, 2304, 2560), (8192, 2304, 3584), (8192, 2304, 4608),
+                                   (8192, 2304, 5120)])
 def test_mx_tile_scale_chunks_with_a_short_last_chunk(gpu, m, n, k):
-    """K of whole pairs of stages that is no multiple of 2048: a last chunk of three, one, three and one pairs, over the
-    persistent walk, against the form with touches (16-byte pieces): same bits, with scale bytes that differ in every block."""
+    """K of whole pairs of stages that is no multiple of 2048, over the persistent walk, against the form with touches (16-byte
+    pieces): a last chunk of three, one and two pairs from K = 3584 up, 16-byte pieces below: same bits, with scale bytes that
+    differ in every block."""
     rng = np.random.default_rng(k)
     a, a_s = H.mx_operand(m, k, seed=52)
     b, b_s = H.mx_operand(n, k, seed=53, std=0.02)
