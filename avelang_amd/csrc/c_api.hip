@@ -128,6 +128,16 @@ int ave_fp4_debug_tiles_per_workgroup(int n_tiles, int compute_units, int t_max,
   return ave::tiles_per_workgroup(n_tiles, compute_units, t_max, step);
 }
 
+int ave_fp4_debug_tile_form(int M, int N, int K, int swiglu, int compute_units, int touch, int* touches, int* chunks) {
+  g_err[0] = 0;
+  if (M <= 0 || N <= 0 || K <= 0 || compute_units <= 0 || touch < 0 || touch > 2 || !touches || !chunks)
+    return fail_inval("tile form of M=%d N=%d K=%d on %d compute units, touch %d.", M, N, K, compute_units, touch);
+  const ave::MxTileForm form = ave::mx_tile_form(M, N, K, swiglu != 0, touch, compute_units);
+  *touches = form.touch ? 1 : 0;
+  *chunks = form.chunks ? 1 : 0;
+  return 0;
+}
+
 int ave_fp4_debug_weights_from_hbm(const void* B, size_t bytes) { return weights_likely_from_hbm(B, bytes) ? 1 : 0; }
 
 int ave_fp4_debug_map_tile(int pid, int m_tiles, int n_tiles, int* tm, int* tn) {
@@ -276,7 +286,7 @@ int ave_fp4_gemm_mxfp4_ex(const uint8_t* A, const uint8_t* A_scale, const uint8_
     case AVE_FP4_TILE:
     case AVE_FP4_TILE_STREAMED:
       if (!ave::mx_tile_supports(p)) return fail_inval("tile kernel does not support M=%d N=%d K=%d.", M, N, K);
-      p.touch = variant == AVE_FP4_TILE_STREAMED ? 1 : 0;
+      p.touch = variant == AVE_FP4_TILE_STREAMED ? 2 : 0;
       return finish(ave::launch_mx_tile(p, s), "mxfp4 tile kernel");
     case AVE_FP4_DECODE:
       if (!ave::mx_decode_supports(p)) return fail_inval("decode kernel does not support M=%d N=%d K=%d.", M, N, K);
@@ -613,7 +623,7 @@ int ave_fp4_gemm_mxfp4_swiglu_ex(const uint8_t* A, const uint8_t* A_scale, const
       return finish(ave::launch_mx_generic(p, s), "mxfp4 swiglu generic kernel");
     case AVE_FP4_TILE:
     case AVE_FP4_TILE_STREAMED:
-      p.touch = variant == AVE_FP4_TILE_STREAMED ? 1 : 0;
+      p.touch = variant == AVE_FP4_TILE_STREAMED ? 2 : 0;
       if (!ave::mx_tile_supports(p))
         return fail_inval("swiglu tile kernel does not support M=%d N=%d K=%d (K a multiple of 32 from 512 up; K %% 512 == 0 wants 16-byte aligned scales).", M, N, K);
       return finish(ave::launch_mx_tile(p, s), "mxfp4 swiglu tile kernel");

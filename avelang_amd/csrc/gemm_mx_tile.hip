@@ -115,7 +115,7 @@ __device__ inline void mma_quarter(v16f (&acc)[4][2], const v4i (&bf)[4], const 
 // TOUCH (ungrouped pair-scale forms, plain or with the fused epilogues): the look-ahead touches of the grouped form for a plain GEMM whose weights come from
 // HBM -- a model's layers, each with weights of its own, as opposed to one GEMM replayed on operands that stay in the
 // last-level cache.  Same bits; 5 % faster on weights from HBM, 1.6 % slower on cache-resident ones (measured on
-// 8192 x 14336 x 4096), so the host chooses (launch_mx_tile).
+// 8192 x 14336 x 4096), so the host chooses (mx_tile_form).
 // CH = 4 (ungrouped pair-scale forms without touches; 0: 16-byte pieces per pair of stages): the scale
 // rows are fetched 64 bytes at a time -- four pairs of stages -- instead of 16.  A row's scales are K / 32 bytes, 128
 // for K = 4096: with 16-byte pieces every pair of stages touches a cache line per row (512 lines for 8 KB), which costs
@@ -126,7 +126,7 @@ __device__ inline void mma_quarter(v16f (&acc)[4][2], const v4i (&bf)[4], const 
 // behind the barrier of the second-to-last stage of chunk c, when every wave has taken chunk c's last pair into
 // registers, and is read a stage later -- the lead the stage data has.  16-byte slot j of a row holds its piece
 // j ^ ((row >> 2) & 3) (on the source side), so that the 16 rows of a ds_read_b128 fall into 16 bank groups.  PART: K is no
-// multiple of 2048, and the last chunk, of one to three pairs, repeats the row's last piece (launch_pairs: from which K; a form of its own,
+// multiple of 2048, and the last chunk, of one to three pairs, repeats the row's last piece (mx_tile_form: from which K; a form of its own,
 // because the clamp in the main loop cost whole chunks 0.5 - 1.4 %: 8192 x 14336 x 4096 241.2 -> 242.4 us, 1500 x 12288 x 4096 54.2 -> 54.9).
 template <bool SC16, bool SWIGLU = false, bool QUANT = false, bool SPLITK = false, bool TAIL = false, bool GROUPED = false,
           bool BLOCKED = false, bool TOUCH = false, int CH = 0, bool PART = false>
@@ -1147,21 +1147,38 @@ hipError_t launch_pair_form(const MxArgs& p, unsigned grid, hipStream_t s, int m
 }
 // ... picked by what the launch needs: the grouped forms and the forms with touches keep the experts' table and the
 // touches' sink in LDS and fetch their scale rows per pair of stages (chunks of two pairs in the place of the two pair
-// buffers measured no faster there: 970-976 against 971-973 us on the 8-expert benchmark); the others take chunks of four
-// pairs for whole chunks and from K = 3584 up, where the last chunk is what is left: with fewer stages the loads of a part of a chunk that
-// is not there, and eight of them in front of the first stage where pairs have two, cost more than the lines saved.  Time by chunks over
-// time by pairs, K no multiple of 2048, 1024 - 8192 rows, plain and SwiGLU, weights from HBM | from the last-level cache: K = 512 1.01 - 1.03 |
-// 1.00 - 1.04, 1024 1.00 - 1.02 | 1.01 - 1.03, 1536 0.98 - 1.02 | 0.97 - 1.03, 2560 0.99 - 1.02 | 0.96 - 1.04, 3072 0.99 - 1.01 | 0.97 - 1.02, 3584
-// 0.98 - 1.00 | 0.99 - 1.03, 4608 0.97 - 1.00 | 0.99 - 1.03, 7680 0.92 - 0.99 | 0.99 - 1.01, 13824 0.89 - 1.00 | 0.99 - 1.01.
+// buffers measured no faster there: 970-976 against 971-973 us on the 8-expert benchmark)
 template <bool SWIGLU, bool QUANT>
-hipError_t launch_pairs(const MxArgs& p, unsigned grid, hipStream_t s, int m_tiles, int n_tiles, bool touch) {
+hipError_t launch_pairs(const MxArgs& p, unsigned grid, hipStream_t s, int m_tiles, int n_tiles, int cus) {
   if (p.row_offsets) return launch_pair_form<SWIGLU, QUANT, true, false, 0>(p, grid, s, m_tiles, n_tiles);
-  if (touch) return launch_pair_form<SWIGLU, QUANT, false, true, 0>(p, grid, s, m_tiles, n_tiles);
+  const MxTileForm form = mx_tile_form(p.M, p.N, p.K, SWIGLU, p.touch, cus);
+  if (form.touch) return launch_pair_form<SWIGLU, QUANT, false, true, 0>(p, grid, s, m_tiles, n_tiles);
+  if (!form.chunks) return launch_pair_form<SWIGLU, QUANT, false, false, 0>(p, grid, s, m_tiles, n_tiles);
   if (p.K % (8 * BK) == 0) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
-  if (p.K >= 14 * BK) return launch_pair_form<SWIGLU, QUANT, false, false, 4, true>(p, grid, s, m_tiles, n_tiles);
-  return launch_pair_form<SWIGLU, QUANT, false, false, 0>(p, grid, s, m_tiles, n_tiles);
+  return launch_pair_form<SWIGLU, QUANT, false, false, 4, true>(p, grid, s, m_tiles, n_tiles);
 }
 }  // namespace
+
+// Touches (touch: 0 none, 1 for weights that are expected from HBM, 2 whatever their origin and the rows): K of whole pairs of stages and a
+// next round to touch for.  They go out for whole groups of 32 rows of tiles, which share the work and the lines, and their sink leaves no
+// LDS for chunks; so with fewer rows the form would touch nothing and lose the chunks, and 1 is taken from 32 rows of tiles up.
+// Weights from HBM, us, that form -> the chunks: gate+up with SwiGLU and quantiser, 28672 x 4096, 1024 rows 70.7 -> 66.0, 2048 133.7 -> 127.9, 4096
+// 235.8 -> 227.9, 6000 350 -> 340, but 8192 452.6 -> 470.5; plain 6000 x 4096 x 14336 176.5 -> 171.5, 8192 x 14336 x 4096 234.0 -> 249.6.
+//
+// Without touches, scale rows in chunks of four pairs of stages for whole chunks, and from K = 3584 up where the last chunk is what is left:
+// with fewer stages the loads of a part of a chunk that is not there, and eight of them in front of the first stage where pairs have two,
+// cost more than the lines saved.  Time by chunks over time by pairs, K no multiple of 2048, 1024 - 8192 rows, plain and SwiGLU, weights
+// from HBM | from the last-level cache: K = 512 1.01 - 1.04 | 1.00 - 1.04, 1024 1.00 - 1.02 | 1.01 - 1.03, 1536 0.98 - 1.02 | 0.96 - 1.03, 2560 0.99 -
+// 1.02 | 0.96 - 1.04, 3072 0.99 - 1.01 | 0.97 - 1.02, 3584 0.98 - 1.00 | 0.97 - 1.03, 4608 0.97 - 1.00 | 0.99 - 1.03, 7680 0.92 - 0.99 | 0.99 -
+// 1.01, 13824 0.89 - 1.00 | 0.99 - 1.01.
+MxTileForm mx_tile_form(int M, int N, int K, bool swiglu, int touch, int cus) {
+  MxTileForm form;
+  if (K % (2 * BK) != 0) return form;
+  const long m_tiles = ((long)M + BM - 1) / BM, n_tiles = swiglu ? ((long)N + BN / 2 - 1) / (BN / 2) : ((long)N + BN - 1) / BN;
+  form.touch = touch != 0 && m_tiles * n_tiles > cus && (touch == 2 || m_tiles >= kXcds * kGroupM);
+  form.chunks = !form.touch && (K % (8 * BK) == 0 || K >= 14 * BK);
+  return form;
+}
 
 hipError_t launch_mx_tile(const MxArgs& p, hipStream_t s) {
   if (p.blocked_scales) {
@@ -1185,21 +1202,16 @@ hipError_t launch_mx_tile(const MxArgs& p, hipStream_t s) {
   const int cus = persistent_workgroups();
   if (cus <= 0) return hipErrorInvalidDevice;
   const unsigned grid = (unsigned)(total < cus ? total : cus);
-  // Touches where there is a next round to touch for and its panels have a whole group of 32 m-tiles to share the work and the lines.
-  // With fewer rows the form without them, which has room for the 64-byte scale chunks, is the faster one, also with weights from
-  // HBM (with touches -> without, us): gate+up with SwiGLU and quantiser, 28672 x 4096, 1024 rows 70.7 -> 66.0, 2048 133.7 -> 127.9,
-  // 4096 235.8 -> 227.9, 6000 350 -> 340, but 8192 452.6 -> 470.5; plain 6000 x 4096 x 14336 176.5 -> 171.5, 8192 x 14336 x 4096 234.0 -> 249.6.
-  const bool touch = p.touch && !p.row_offsets && total > cus && m_tiles >= kXcds * kGroupM;
   if (p.swiglu) {
     if (tail_form(p)) {
       if (p.Q) return launch_form<true, true, true, true>(p, grid, kLdsBytes16, s, m_tiles, n_tiles);
       return launch_form<true, true, false, true>(p, grid, kLdsBytes16, s, m_tiles, n_tiles);
     }
-    if (p.Q) return launch_pairs<true, true>(p, grid, s, m_tiles, n_tiles, touch);
-    return launch_pairs<true, false>(p, grid, s, m_tiles, n_tiles, touch);
+    if (p.Q) return launch_pairs<true, true>(p, grid, s, m_tiles, n_tiles, cus);
+    return launch_pairs<true, false>(p, grid, s, m_tiles, n_tiles, cus);
   }
   if (tail_form(p)) return launch_form<true, false, false, true>(p, grid, kLdsBytes16, s, m_tiles, n_tiles);
-  return launch_pairs<false, false>(p, grid, s, m_tiles, n_tiles, touch);
+  return launch_pairs<false, false>(p, grid, s, m_tiles, n_tiles, cus);
 }
 
 }  // namespace ave

@@ -25,8 +25,8 @@ struct MxArgs {
   int slices = 1;              //   K slices of slice_pairs x 512 elements each (the last one what is left)
   int slice_pairs = 0;
   int half_rows = 0;           //   narrow-tile kernel only: 1 = the slices run on its 128-row tiles
-  int touch = 0;               // 256 x 256 kernel, plain GEMM: 1 = look-ahead touches of the next round's panels (weights
-                               //   expected to come from HBM rather than from the last-level cache)
+  int touch = 0;               // 256 x 256 kernel, ungrouped: look-ahead touches of the next round's panels, 1 = weights expected to come from
+                               //   HBM rather than from the last-level cache, 2 = asked for (mx_tile_form)
   int tail_four_apart = 0;     // grouped streaming kernel: order of addition behind the last whole 512 elements of K, as in the
                                //   256 x 256 kernel (1) or as in the narrow-tile kernel (0)
   int by_lines = 0;            // grouped streaming kernel: 1 = by cache lines of the rows whatever the sizes (as far as offsets have room),
@@ -52,6 +52,14 @@ struct SplitPlan {
 SplitPlan mx_tile_split_plan(int M, int N, int K, size_t max_workspace_bytes = ~(size_t)0);
 SplitPlan mx_tile_split_plan_for(int M, int N, int K, int compute_units,
                                  size_t max_workspace_bytes = ~(size_t)0);   // host arithmetic only
+
+// How launch_mx_tile runs an ungrouped GEMM or fused SwiGLU (N outputs) on aligned scale tensors: with look-ahead touches, with scale
+// rows in chunks of four pairs of stages, or neither.  touch as in MxArgs.
+struct MxTileForm {
+  bool touch = false;
+  bool chunks = false;
+};
+MxTileForm mx_tile_form(int M, int N, int K, bool swiglu, int touch, int compute_units);   // host arithmetic only
 
 // The streaming kernel for the ungrouped MXFP4 GEMM and its fused SwiGLU forms (gemm_mx_stream.hip): rows per tile, 0 where
 // another kernel is the faster one; K in slices of slice_pairs x 512 elements (a K tail with the last one) whose sums take

@@ -61,11 +61,14 @@ enum ave_fp4_variant {
                           which come from HBM (a model's layers, each with weights of its own) are in the last-level
                           cache when their stage loads ask for them; takes effect with K % 512 == 0, 16-byte aligned
                           scale tensors and more 256 x 256 tiles than compute units, and is AVE_FP4_TILE otherwise.
+                          Requests go out for whole groups of 32 rows of tiles (8192 rows of A); with fewer the form runs
+                          and requests nothing.
                           Same bits as AVE_FP4_TILE; on 8192 x 14336 x 4096 7 % faster on weights from HBM, 1 %
                           slower on cache-resident ones.  Also for the fused SwiGLU forms.  Shape-based dispatch keeps,
                           per device, the weight tensors of its latest MXFP4 GEMMs: weights found among the most
                           recent ones that add up to 192 MB at most are taken to be in the 256 MB last-level cache
-                          (one GEMM replayed on the same operands) and run as AVE_FP4_TILE, all others as this form */
+                          (one GEMM replayed on the same operands) and run as AVE_FP4_TILE, all others from 32 rows of tiles
+                          up as this form */
   AVE_FP4_SHORT = 7    /* MXFP4 plain GEMM only: 32x32 blocks of C, four waves each that share K (up to 2048), operands straight
                           into registers; for small calls */
 };

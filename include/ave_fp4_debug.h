@@ -139,9 +139,16 @@ int ave_fp4_debug_stream_read_write(const void* src, size_t bytes, void* dst, si
 int ave_fp4_debug_tiles_per_workgroup(int n_tiles, int compute_units, int t_max, int step);
 
 /*
+ * Diagnostic, host only: the form in which the 256 x 256 kernel runs the MXFP4 GEMM, or its fused SwiGLU forms (N outputs), on 16-byte
+ * aligned scale tensors and compute_units compute units: with look-ahead touches (touches = 1), with scale rows in 64-byte chunks (chunks = 1)
+ * or with neither.  touch: 0 for AVE_FP4_TILE, 1 for shape-based dispatch of weights expected from HBM, 2 for AVE_FP4_TILE_STREAMED.
+ */
+int ave_fp4_debug_tile_form(int M, int N, int K, int swiglu, int compute_units, int touch, int* touches, int* chunks);
+
+/*
  * Diagnostic, host only: the hint that shape-based dispatch of the MXFP4 GEMMs takes before it launches the 256 x 256
- * kernel -- 1 when a weight tensor at address B of `bytes` bytes is expected to come from HBM (the kernel then runs
- * with look-ahead touches, AVE_FP4_TILE_STREAMED), 0 when it is expected in the last-level cache.  The call RECORDS B
+ * kernel -- 1 when a weight tensor at address B of `bytes` bytes is expected to come from HBM (from 32 rows of tiles up the kernel
+ * then runs with look-ahead touches, ave_fp4_debug_tile_form), 0 when it is expected in the last-level cache.  The call RECORDS B
  * as the device's most recent weight tensor, exactly as a GEMM call does: the library keeps the last eight per device,
  * most recent first, and takes a tensor to be resident when it is found among the most recent ones whose sizes add up
  * to 192 MB at most.  Nothing is launched and B is not dereferenced.

@@ -560,6 +560,27 @@ def test_weights_from_hbm_hint_models_the_last_level_cache():
     assert [(hint(big1, 150 * mb), hint(big2, 150 * mb)) for _ in range(3)] == [(1, 1)] * 3
 
 
+def test_form_of_the_wide_tile_kernel():
+    """AVE_FP4_TILE_STREAMED (2) takes the form with look-ahead touches wherever there is a next round of tiles, shape-based dispatch
+    on weights from HBM (1) from 32 rows of tiles up; scale rows in chunks only without touches, for whole chunks of K and from 3584 up."""
+    lib = _lib.load()
+
+    def form(m, n, k, swiglu, touch, cus=256):
+        touches, chunks = ctypes.c_int(-1), ctypes.c_int(-1)
+        assert lib.ave_fp4_debug_tile_form(m, n, k, swiglu, cus, touch, ctypes.byref(touches), ctypes.byref(chunks)) == 0
+        return touches.value, chunks.value
+
+    assert form(4100, 4300, 512, 0, 2) == (1, 0) and form(4100, 4300, 512, 0, 1) == (0, 0)      # 17 rows of tiles
+    assert form(4100, 4300, 2048, 0, 2) == (1, 0) and form(4100, 4300, 2048, 0, 1) == (0, 1)
+    assert form(7936, 14336, 4096, 0, 1) == (0, 1) and form(7937, 14336, 4096, 0, 1) == (1, 0)  # 31 | 32
+    assert form(8192, 1024, 4096, 1, 1) == (0, 1) and form(8192, 1025, 4096, 1, 1) == (1, 0)    # 256 tiles of 128 outputs | more
+    assert form(8192, 2048, 4096, 0, 2) == (0, 1) and form(8192, 2049, 4096, 0, 2) == (1, 0)
+    assert form(8192, 2304, 768, 0, 2) == (0, 0)                                                # no whole pairs of stages
+    for k, chunks in ((512, 0), (1536, 0), (2048, 1), (2560, 0), (3072, 0), (3584, 1), (4096, 1), (4608, 1)):
+        assert form(8192, 14336, k, 0, 0) == (0, chunks), k
+    assert lib.ave_fp4_debug_tile_form(8192, 14336, 4096, 0, 256, 3, None, None) == -1
+
+
 def test_tiles_per_workgroup_of_the_weight_streaming_kernels():
     """One round of workgroups while ceil(tiles / CUs) fits the most tiles a workgroup takes; beyond that balanced
     rounds instead of a full round and a nearly empty one.  Every choice covers all tiles."""
