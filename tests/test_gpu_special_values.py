@@ -15,7 +15,8 @@ GENERIC, TILE, DECODE, NARROW, TILE_STREAMED = 1, 2, 3, 4, 6
                                            (300, 260, 2048, TILE),            # scale rows in 64-byte chunks
                                            (300, 260, 768, TILE),             # scales per stage
                                            (100, 300, 1024, NARROW), (200, 130, 1056, NARROW),
-                                           (2100, 9000, 512, TILE_STREAMED)])  # more tiles than compute units: touches
+                                           (2100, 9000, 512, TILE_STREAMED),  # more tiles than compute units: the form with touches
+                                           (8200, 2100, 512, TILE_STREAMED)])  # ... and a whole group of 32 rows of tiles: they go out
 def test_mxfp4_nan_scale_bytes(gpu, m, n, k, variant):
     a, a_s = H.mx_operand(m, k, seed=1)
     b, b_s = H.mx_operand(n, k, seed=2, std=0.05)

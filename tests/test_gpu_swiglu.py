@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from avelang_amd import (gemm_mxfp4_swiglu_quant_transposed_b, gemm_mxfp4_swiglu_transposed_b,
+from avelang_amd import (_lib, gemm_mxfp4_swiglu_quant_transposed_b, gemm_mxfp4_swiglu_transposed_b,
                          gemm_mxfp4_transposed_b, grouped_gemm_mxfp4_swiglu_quant_transposed_b,
                          grouped_gemm_mxfp4_swiglu_transposed_b, quantize_mxfp4)
 from oracle import fp4_oracle as orc
@@ -58,9 +58,8 @@ def test_swiglu_tile_kernel(gpu, m, n, k):
 
 
 def test_swiglu_tile_kernel_with_look_ahead_touches_gives_the_same_bits(gpu):
-    """More tiles than compute units: the form that touches the next round's weight panels (TILE_STREAMED, what dispatch
-    takes for weights it has not just seen) against the form without, for the fused SwiGLU and for SwiGLU + quantiser
-    (two calls in a row on the same weights run first the one form, then the other)."""
+    """More tiles than compute units, 17 rows of them: the form with touches (TILE_STREAMED; none go out below 32 rows) against the
+    form without for the fused SwiGLU; SwiGLU + quantiser, which dispatch runs without touches here, against the two calls."""
     m, n, k = 4100, 2100, 512
     a, a_s, b, b_s = _operands(m, n, k, seed=77)
     want = _run(gpu, a, a_s, b, b_s, TILE)
@@ -75,6 +74,30 @@ def test_swiglu_tile_kernel_with_look_ahead_touches_gives_the_same_bits(gpu):
     want_q, want_s = quantize_mxfp4(gemm_mxfp4_swiglu_transposed_b(*ops, variant=TILE))
     for q, sc in ((q1, s1), (q2, s2)):
         assert torch.equal(q, want_q) and torch.equal(sc, want_s)
+
+
+@pytest.mark.parametrize("k", [512, 2048, 4608])
+def test_swiglu_tile_kernel_with_touches_of_whole_groups_gives_the_same_bits(gpu, k):
+    """33 rows of tiles, 297 tiles: the touches go out (at a tile's start, and eight stages before its end), for the fused SwiGLU and,
+    through dispatch on weights it has not seen, for SwiGLU + quantiser; the same call again runs the form without."""
+    m, n = 8200, 1120
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(k)
+    a, b = (torch.randint(0, 256, (r, k // 2), generator=gen, device=gpu, dtype=torch.uint8) for r in (m, 2 * n))
+    a_s, b_s = (torch.randint(110, 122, (r, k // 32), generator=gen, device=gpu, dtype=torch.uint8) for r in (m, 2 * n))
+    want = gemm_mxfp4_swiglu_transposed_b(a, a_s, b, b_s, variant=TILE)
+    assert torch.equal(gemm_mxfp4_swiglu_transposed_b(a, a_s, b, b_s, variant=6).view(torch.int16), want.view(torch.int16))
+    last = slice(m - 20, m)
+    ok, rep = orc.check_swiglu_bf16(H.bits(want[last]), *(t.cpu().numpy() for t in (a[last], a_s[last], b, b_s)))
+    assert ok, rep
+    want_q, want_s = quantize_mxfp4(want)
+    lib = _lib.load()
+    with torch.cuda.device(gpu):
+        for other in range(1, 9):   # eight other weight tensors: the next call's are not among the latest
+            lib.ave_fp4_debug_weights_from_hbm(other << 12, 192 << 20)
+    for _ in range(2):
+        q, q_s = gemm_mxfp4_swiglu_quant_transposed_b(a, a_s, b, b_s)
+        assert torch.equal(q, want_q) and torch.equal(q_s, want_s)
 
 
 @pytest.mark.parametrize("m,n,k", [(300, 264, 2048), (4100, 2112, 2048), (130, 1000, 4096)])

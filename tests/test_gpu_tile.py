@@ -75,9 +75,9 @@ def test_mx_tile_more_tiles_than_compute_units(gpu, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(8192, 2400, 512), (8200, 2100, 1024), (4100, 4300, 512), (300, 300, 512), (8192, 2304, 768)])
 def test_mx_tile_with_look_ahead_touches_gives_the_same_bits(gpu, m, n, k):
     """The form for weights that come from HBM (TILE_STREAMED: touches of the next round's panels; whole groups of 32
-    m-tiles, a ragged group, a single round, a K it does not apply to) against the form without: same bits.  Shape-based
-    dispatch takes one or the other by whether the weights are those of the previous call, so two calls in a row on
-    the same operands run both."""
+    m-tiles, a ragged group, fewer than a group, a single round, a K it does not apply to) against the form without: same
+    bits.  From 32 m-tiles up shape-based dispatch takes one or the other by whether the weights are those of the previous
+    call, so two calls in a row on the same operands run both."""
     TILE_STREAMED = 6
     a, a_s = H.mx_operand(m, k, seed=40)
     b, b_s = H.mx_operand(n, k, seed=41, std=0.02)
@@ -96,7 +96,7 @@ def test_mx_tile_with_look_ahead_touches_gives_the_same_bits(gpu, m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [(300, 520, 2048), (4100, 4300, 2048), (257, 130, 4096), (1000, 777, 6144), (8192, 2100, 4096), (65, 3000, 8192)])
 def test_mx_tile_64_byte_scale_chunks_give_the_same_bits(gpu, m, n, k):
-    """K % 2048 == 0 without touches: the scale rows are fetched 64 bytes at a time into one chunk buffer (one, two, three
+    """K % 2048 == 0 in the form without touches: the scale rows are fetched 64 bytes at a time into one chunk buffer (one, two, three
     and four chunks; one tile per workgroup and the persistent walk; ragged last tiles).  The form with touches keeps
     the 16-byte pieces per pair of stages: same MFMAs on the same scale bytes, so the same bits.  Scale bytes differ in
     every block of every row, so a piece taken from the wrong row, chunk or slot changes the result."""
