@@ -141,7 +141,7 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
   using G = Geo<R, CHUNKS>;
   static_assert(SWIGLU || !QUANT, "the fused quantiser follows the fused SwiGLU");
   static_assert(!SPLITK || (!SWIGLU && !GROUPED), "K is split for the plain GEMM");
-  static_assert(!SHIFT || GROUPED, "by lines: the experts' weights only");
+  static_assert((!SHIFT && !CHUNKS) || GROUPED, "by lines, scale rows in chunks: the experts' weights only");
   constexpr int kTileN = SWIGLU ? BN / 2 : BN;   // output columns per tile
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x;
@@ -496,30 +496,73 @@ __device__ __forceinline__ void stream_tiles(const MxArgs& p, int n_tiles, const
       __syncthreads();
       if (G::kPairs == 1 ? (s & 1) == 0 : ((s - s_first) & 3) == 0) next_slot();
       const int blocks = s == stages - 1 && tail_blocks != 0 ? tail_blocks : 8;
+      if constexpr (GROUPED) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int block = p.tail_four_apart ? 4 * h + j : 2 * j + h;
-        const bool have = block < blocks;
-        const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (have ? block : 0));
-        const v4i none = {0, 0, 0, 0};
+        for (int j = 0; j < 4; ++j) {
+          const int block = p.tail_four_apart ? 4 * h + j : 2 * j + h;
+          const bool have = block < blocks;
+          const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (have ? block : 0));
+          const v4i none = {0, 0, 0, 0};
 #pragma unroll
-        for (int i = 0; i < MI; ++i) {
-          const v4i f = lds_read16(sb + late(a_late[i], block) + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
-          const int sc = lds_read1(at + (G::kPairs == 1 ? a_sc : a_sc ^ ((unsigned)((s - s_first) & 2) * 8)) + i * (32 * G::kScaleRow));
-          af[j][i] = have ? f : none;
-          as_cur[i] = have ? sc : 0x7f;
+          for (int i = 0; i < MI; ++i) {
+            const v4i f = lds_read16(sb + late(a_late[i], block) + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
+            const int sc = lds_read1(at + (G::kPairs == 1 ? a_sc : a_sc ^ ((unsigned)((s - s_first) & 2) * 8)) + i * (32 * G::kScaleRow));
+            af[j][i] = have ? f : none;
+            as_cur[i] = have ? sc : 0x7f;
+          }
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const v4i f = lds_read16(sb + late(b_late[i], block) + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
+            const int sc = lds_read1(at + (G::kPairs == 1 ? b_sc : b_sc ^ ((unsigned)((s - s_first) & 2) * 8)) + i * (32 * G::kScaleRow));
+            bf[j][i] = have ? f : none;
+            bs_cur[i] = have ? sc : 0x7f;
+          }
+#pragma unroll
+          for (int nj = 0; nj < 2; ++nj)
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<0, 0>(bf[j][nj], af[j][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
         }
+      } else {
+        // One matrix: all of the stage's fragments and scales are requested before the first is waited for, as in the stages above.
+        // Left to the compiler, the plain form's 64-row tiles and all 128-row tiles waited for them one by one: 250 x 1280 x 1376 8.07 ->
+        // 7.45 us, 220 x 1536 x 4480 13.7 -> 13.1, 100 x 2048 x 2944 10.8 -> 10.1.  (Grouped, this order was 4 % slower in places, 5 %
+        // faster in others.)
+        int as_tail[4][MI], bs_tail[4][2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const v4i f = lds_read16(sb + late(b_late[i], block) + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
-          const int sc = lds_read1(at + (G::kPairs == 1 ? b_sc : b_sc ^ ((unsigned)((s - s_first) & 2) * 8)) + i * (32 * G::kScaleRow));
-          bf[j][i] = have ? f : none;
-          bs_cur[i] = have ? sc : 0x7f;
+        for (int j = 0; j < 4; ++j) {
+          const int block = p.tail_four_apart ? 4 * h + j : 2 * j + h;
+          const unsigned at = slot + (unsigned)(16 - pair_tail + 8 * (s & 1) + (block < blocks ? block : 0));
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            af[j][i] = lds_read16(sb + (unsigned)((a_row + 32 * i) * kRowBytes + ((block ^ ((a_row >> 1) & 7)) * 16)));
+            as_tail[j][i] = lds_read1(at + a_sc + i * 512);
+          }
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            bf[j][i] = lds_read16(sb + (unsigned)(G::kOffB + (b_row + 32 * i) * kRowBytes + ((block ^ ((b_row >> 1) & 7)) * 16)));
+            bs_tail[j][i] = lds_read1(at + b_sc + i * 512);
+          }
         }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int nj = 0; nj < 2; ++nj)
+        for (int j = 0; j < 4; ++j) {
+          const bool have = (p.tail_four_apart ? 4 * h + j : 2 * j + h) < blocks;
+          const v4i none = {0, 0, 0, 0};
 #pragma unroll
-          for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<0, 0>(bf[j][nj], af[j][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
+          for (int i = 0; i < MI; ++i) {
+            af[j][i] = have ? af[j][i] : none;
+            as_cur[i] = have ? as_tail[j][i] : 0x7f;
+          }
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            bf[j][i] = have ? bf[j][i] : none;
+            bs_cur[i] = have ? bs_tail[j][i] : 0x7f;
+          }
+#pragma unroll
+          for (int nj = 0; nj < 2; ++nj)
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) acc[nj][mi] = mfma32<0, 0>(bf[j][nj], af[j][mi], acc[nj][mi], bs_cur[nj], as_cur[mi]);
+        }
       }
       next_buffer();
     }
@@ -711,6 +754,8 @@ bool by_lines(const MxArgs& p) {
 //    4096 0.98 - 1.05, 7168 0.93 - 1.00 -- the price of the rule up to K = 4096;
 //  * by lines, from HBM: 32-row tiles K = 1056 1.00 - 1.02, 1312 1.00 - 1.01, 1568 0.99 - 1.00, 2880 0.97 - 0.99; 128-row tiles K = 1056 - 1312
 //    1.00 - 1.06, 1696 1.01 - 1.03, 2080 0.98 - 1.03, 2880 0.98 - 1.01, 4256 0.97 - 0.99.
+// Tables of random routing, 20 - 170 rows on average: 0.92 - 1.00 (one in 64 of those calls 1.03); the same few rows behind a whole tile in every
+// expert, which routing does not give, up to 1.2 (51 x 137 rows, 6656 x 6144).
 template <bool SWIGLU>
 bool scale_chunks(const MxArgs& p, int rows, bool lines) {
   if (p.scale_chunks != 0) return p.scale_chunks > 0;
