@@ -568,19 +568,22 @@ hipError_t launch_narrow_form(const MxArgs& p, hipStream_t s, int n_tiles) {
   if (p.swiglu) return launch_narrow<true, false, HALF, CHUNKS>(p, s, n_tiles);
   return launch_narrow<false, false, HALF, CHUNKS>(p, s, n_tiles);
 }
-// 128-row tiles: scale rows in chunks from K = 3072 up, from 5120 where one row of tiles takes more than three quarters of the compute units.  The
-// four parts of the first chunk that go out in front of the first stage cost 0.25 - 0.4 us, which a short K does not earn back.  Time by
-// chunks over time by pairs, weights from HBM | replayed from the last-level cache:
-//  * up to 192 tiles a row (70 - 600 rows): K = 512 1.05 - 1.11 | 1.05 - 1.10, 1024 1.04 - 1.06 | 1.04 - 1.06, 2048 0.97 - 1.04 | 1.02 - 1.06, 2560 0.95 -
-//    1.02 | 1.01 - 1.05, 2816 0.98 - 1.03 | 1.03 - 1.07, 3072 0.93 - 1.00 | 0.98 - 1.07, 4096 0.89 - 0.98 | 0.91 - 1.02, 8192 0.85 - 0.95 | 0.87 -
-//    1.04, 14336 0.85 - 0.90 | 0.79 - 0.91;
+// 128-row tiles: scale rows in chunks from K = 3072 up, and for 2560 (no tail) on 24 tiles and more; from 5120 where one row of tiles takes
+// more than three quarters of the compute units.  The four parts of the first chunk that go out in front of the first stage cost 0.25 -
+// 0.4 us, which a short K does not earn back.  Time by chunks over time by pairs, weights from HBM | replayed from the last-level cache:
+//  * up to 192 tiles a row (70 - 600 rows): K = 512 1.05 - 1.13 | 1.05 - 1.10, 1024 1.03 - 1.07 | 1.03 - 1.06, 2048 0.97 - 1.05 | 1.01 - 1.06, 2560
+//    0.95 - 1.00 from 24 tiles up, 0.98 - 1.02 below | 1.01 - 1.05, 2816 0.98 - 1.03 | 1.02 - 1.07, 3072 0.92 - 1.00 | 0.98 - 1.07, 4096 0.89 - 0.98 |
+//    0.91 - 1.04, 8192 0.85 - 0.95 | 0.87 - 1.04, 14336 0.83 - 0.90 | 0.79 - 1.02;
 //  * 216 to 256 tiles in one row, on eight cards: K = 3072 0.97 - 1.07 | 1.00 - 1.20, 4096 0.95 - 1.07 (on average 1.01) | 0.96 - 1.18, 5120
 //    0.93 - 1.03 | 0.96 - 1.31, 6144 0.92 - 1.01 | 0.95 - 1.28, 8192 0.93 - 1.05 | 0.94 - 1.25, 14336 0.88 - 0.96 | 0.94 - 1.11: a full chip's
 //    weights of 60 MB and more, replayed alone, come from the cache more slowly in chunks on some cards; why was not found (turning the
 //    order of the parts from tile to tile changes nothing).
 // us, pairs -> chunks: 600 x 4096 x 14336 34.3 -> 28.1, 1024 x 4096 x 14336 41.5 -> 33.3, 272 x 7680 x 10240 26.6 -> 22.2; 100 x 4096 x 512, which
 // is by pairs, 4.56 -> 4.88.  Slices of K are in chunks whatever their length (one to ten pairs: 0.89 - 1.07 | 0.92 - 1.07, on average 0.96 | 0.99).
-bool scale_chunks(const MxArgs& p, int n_tiles, int cus) { return p.K >= (4L * n_tiles > 3L * cus ? 20 : 12) * BK; }
+bool scale_chunks(const MxArgs& p, int n_tiles, int cus) {
+  if (4L * n_tiles > 3L * cus) return p.K >= 20 * BK;
+  return p.K >= 12 * BK || (p.K == 10 * BK && (long)((p.M + 127) / 128) * n_tiles >= 24);
+}
 }  // namespace
 
 // 128-row tiles (waves 0-3 multiply, waves 4-7 load, a ring of four stages) where no tile would have upper rows

@@ -50,10 +50,10 @@ def test_narrow_random_scales_every_kblock(gpu):
 
 
 @pytest.mark.parametrize("m,n,k", [(100, 300, 2048), (128, 128, 2560), (127, 264, 3584), (1, 136, 4096), (200, 1000, 6656), (65, 8, 8192),
-                                   (127, 264, 3072)])
+                                   (127, 264, 3072), (130, 1600, 2560)])
 def test_narrow_128_row_tiles_scale_chunks(gpu, m, n, k):
-    """128-row tiles fetch scale rows in chunks of four pairs of stages from six pairs (K = 3072) up: two to four chunks, the
-    last of one to four pairs; below, by pairs.  Scale bytes differ in every block, the 256 x 256 kernel gives the same bits."""
+    """128-row tiles fetch scale rows in chunks of four pairs of stages from six pairs (K = 3072) up, and for
+    five on 24 tiles and more: two to four chunks, the last of one to four pairs; below, by pairs.  Scale bytes differ in every block, the 256 x 256 kernel gives the same bits."""
     rng = np.random.default_rng(k)
     a, a_s = H.mx_operand(m, k, seed=6)
     b, b_s = H.mx_operand(n, k, seed=7, std=0.02)
