@@ -127,7 +127,7 @@ __device__ inline void mma_quarter(v16f (&acc)[4][2], const v4i (&bf)[4], const 
 // registers, and is read a stage later -- the lead the stage data has.  16-byte slot j of a row holds its piece
 // j ^ ((row >> 2) & 3) (on the source side), so that the 16 rows of a ds_read_b128 fall into 16 bank groups.  PART: K is no
 // multiple of 2048, and the last chunk, of one to three pairs, repeats the row's last piece (mx_tile_form: from which K; a form of its own,
-// because the clamp in the main loop cost whole chunks 0.5 - 1.4 %: 8192 x 14336 x 4096 241.2 -> 242.4 us, 1500 x 12288 x 4096 54.2 -> 54.9).
+// because the clamp in the main loop costs whole chunks 0.5 - 1.4 %: 8192 x 14336 x 4096 241.2 -> 242.4 us, 1500 x 12288 x 4096 54.2 -> 54.9).
 template <bool SC16, bool SWIGLU = false, bool QUANT = false, bool SPLITK = false, bool TAIL = false, bool GROUPED = false,
           bool BLOCKED = false, bool TOUCH = false, int CH = 0, bool PART = false>
 __global__ __launch_bounds__(kWaves * 64) void mx_tile_kernel(MxArgs p, int m_tiles, int n_tiles) {
@@ -1147,14 +1147,17 @@ hipError_t launch_pair_form(const MxArgs& p, unsigned grid, hipStream_t s, int m
 }
 // ... picked by what the launch needs: the grouped forms and the forms with touches keep the experts' table and the
 // touches' sink in LDS and fetch their scale rows per pair of stages (chunks of two pairs in the place of the two pair
-// buffers measured no faster there: 970-976 against 971-973 us on the 8-expert benchmark)
+// buffers measured no faster there: 970-976 against 971-973 us on the 8-expert benchmark).
+// Whole chunks with the quantiser run the PART form below K = 8192 all the same: its main loop is the slower one by 0.5 %, its tile ends
+// the faster, as the two are compiled (PART over whole, weights from HBM | from the cache, 700 - 6000 rows: K = 2048 0.97 - 0.99 | 0.99 - 1.00,
+// 4096 0.98 - 1.00 | 1.00, 6144 0.98 - 1.00 | 1.00, 8192 0.99 - 1.01 | 1.00 - 1.01).
 template <bool SWIGLU, bool QUANT>
 hipError_t launch_pairs(const MxArgs& p, unsigned grid, hipStream_t s, int m_tiles, int n_tiles, int cus) {
   if (p.row_offsets) return launch_pair_form<SWIGLU, QUANT, true, false, 0>(p, grid, s, m_tiles, n_tiles);
   const MxTileForm form = mx_tile_form(p.M, p.N, p.K, SWIGLU, p.touch, cus);
   if (form.touch) return launch_pair_form<SWIGLU, QUANT, false, true, 0>(p, grid, s, m_tiles, n_tiles);
   if (!form.chunks) return launch_pair_form<SWIGLU, QUANT, false, false, 0>(p, grid, s, m_tiles, n_tiles);
-  if (p.K % (8 * BK) == 0) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
+  if (p.K % (8 * BK) == 0 && !(QUANT && p.K < 32 * BK)) return launch_pair_form<SWIGLU, QUANT, false, false, 4>(p, grid, s, m_tiles, n_tiles);
   return launch_pair_form<SWIGLU, QUANT, false, false, 4, true>(p, grid, s, m_tiles, n_tiles);
 }
 }  // namespace

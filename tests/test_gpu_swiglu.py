@@ -76,10 +76,11 @@ def test_swiglu_tile_kernel_with_look_ahead_touches_gives_the_same_bits(gpu):
         assert torch.equal(q, want_q) and torch.equal(sc, want_s)
 
 
-@pytest.mark.parametrize("k", [512, 2048, 4608])
+@pytest.mark.parametrize("k", [512, 2048, 4608, 8192])
 def test_swiglu_tile_kernel_with_touches_of_whole_groups_gives_the_same_bits(gpu, k):
     """33 rows of tiles, 297 tiles: the touches go out (at a tile's start, and eight stages before its end), for the fused SwiGLU and,
-    through dispatch on weights it has not seen, for SwiGLU + quantiser; the same call again runs the form without."""
+    through dispatch on weights it has not seen, for SwiGLU + quantiser; the same call again runs the form without (scale rows by
+    pairs, and in whole and short chunks)."""
     m, n = 8200, 1120
     gen = torch.Generator(device=gpu)
     gen.manual_seed(k)
