@@ -1058,7 +1058,10 @@ SplitPlan mx_tile_split_plan_for(int M, int N, int K, int cus, size_t max_worksp
   const long narrow_tiles = (long)((M + BM - 1) / BM) * ((N + 127) / 128);   // 256 x 128 tiles
   const long half_tiles = (long)((M + 127) / 128) * ((N + 127) / 128);       // 128 x 128 tiles
   // per stage: 1.65 on 256 x 256 tiles, 0.85 on 256 x 128 tiles (three stage buffers), 0.72 on 128 x 128 tiles
-  // (four, and waves of their own for the loads); the unsplit call takes the best tiling that fits the compute units
+  // (four, and waves of their own for the loads); the unsplit call takes the best tiling that fits the compute units.
+  // (0.72 is from before those tiles fetched long scale rows in chunks: 300 - 600 rows x 4096 x 8192 - 14336 take 0.58 - 0.62 from HBM
+  // now, 0.37 - 0.43 from the cache.  Not refitted, so K may be cut where one launch is as fast; mx_stream_plan has the same tiles at
+  // 0.47 or the memory time, whichever is longer.)
   const double unsplit = (half_tiles <= cus ? 0.72 : (narrow_tiles <= cus ? 0.85 : 1.65)) * 2 * pairs + 5.0;
   double best = unsplit * 0.85;   // a split must save 15 %
   // the slices run on 256 x 256 tiles, or on the 256 x 128 or 128 x 128 tiles of the narrow-tile kernel
